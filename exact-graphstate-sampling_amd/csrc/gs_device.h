@@ -16,10 +16,18 @@ constexpr int kBigStepLog2 = 30;        // one-slot steps of at least 2^30 coset
 constexpr int kDefaultGridLog2OneBig = 14;  // width 34: 1.231 -> 1.196 s per sample; width 30 prefers 2^12
 constexpr int kDefaultTTGridLog2 = 14;  // gather sweeps of the two-table engine (latency-bound gathers: the
                                          // width-31 IBM sample 0.276 s at 2^9 blocks, 0.121 s at 2^14)
-constexpr int kFenceBlocks = 64;    // sweeps of at most this many blocks reduce in their last block
+constexpr int kFenceBlocks = 64;    // launches of at most this many blocks reduce in each string's last block
+// Several strings per launch (one arena each): as many as fit in kSlotBytes of device memory, at most one chunk of
+// strings, and only arenas of which at least kMinSlots fit.  A sweep of a few thousand cosets takes about 9 us whether
+// it runs one string or 32, so a plan far below the chip's size is bound by its launches.  Per string, one at a time
+// against together (complex64): 64 strings of the n = 24 plan 108 -> 2.2 us, 32 of the n = 40 one (width 14) 274 ->
+// 12 us, 32 at width 20 600 -> 81 us, 32 at width 24 1210 -> 733 us (833 with 1 GiB), 8 at width 25 2120 -> 1840 us; at
+// width 26 (512 MB arenas) one string fills the chip and 7 together gain nothing (4.26 ms either way).
+constexpr size_t kSlotBytes = size_t(1) << 32;
+constexpr int kMinSlots = 8;
 constexpr int kPartStride = 8;      // doubles per block partial (write norms + fused next-step norms)
 constexpr size_t kPartDoubles = size_t(kPartStride) << kMaxGridLog2;
-constexpr int kCounters = 1;
+constexpr int kCounters = 64;      // one per string of a launch
 
 // Canonical routing of the 2 * ntq terms of a step onto the outputs tau (after the host relabels the offsets):
 //   kRoute1     m = 1: every term feeds tau 0
@@ -127,6 +135,11 @@ struct Ctl {
     int pad;
 };
 
+// Whether a sweep's blocks reduce their own partials (one block per string, or few blocks in all): see sweep_epilogue.
+__device__ __host__ __forceinline__ bool reduces_in_kernel(unsigned blocks, unsigned strings) {
+    return blocks == 1 || blocks * strings <= unsigned(kFenceBlocks);
+}
+
 // Modes of the chain (how norms become a branch and bookkeeping).
 enum ChainMode { kChain = 0, kChain1 = 1, kRun = 2 };
 
@@ -156,6 +169,10 @@ struct Epi {
     unsigned pend_nblk;
     int pend_nq, pend_k, pend_role, pend_next, pend_sweep;
     int quiet;                 // 1: leave the per-string outputs (bits, cond, out) to another block
+    // Launches of several strings (gridDim.y > 1): string y of the launch has its own arena (slot_entries apart), block
+    // partials (slot_part doubles apart), chain state, counter and per-string buffers.
+    uint64_t slot_entries;
+    uint32_t slot_part;
 };
 
 }  // namespace gs

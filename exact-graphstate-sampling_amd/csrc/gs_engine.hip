@@ -72,13 +72,20 @@ __device__ float2 to_storage<float2>(double2 v) { return make_float2(float(v.x),
 template <>
 __device__ double2 to_storage<double2>(double2 v) { return v; }
 
+// Start of a chain, one block per string of the launch.
 template <class S>
-__global__ void init_kernel(S* mem, Ctl* ctl) {
-    mem[0] = to_storage<S>(make_double2(1.0, 0.0));
+__global__ void init_kernel(S* mem, Ctl* ctl, uint64_t slot_entries) {
+    mem[blockIdx.x * slot_entries] = to_storage<S>(make_double2(1.0, 0.0));
     Ctl c{};
     c.prev = 1;
     c.nstored = 1;
-    *ctl = c;
+    ctl[blockIdx.x] = c;
+}
+
+// Arena entry 0 of every string of the launch (its amplitude after the last step), 16 bytes per string.
+template <class S>
+__global__ void amp_kernel(const S* mem, uint64_t slot_entries, unsigned char* amp) {
+    *reinterpret_cast<S*>(amp + size_t(blockIdx.x) * 16) = mem[blockIdx.x * slot_entries];
 }
 
 __global__ void init_ctl_kernel(Ctl* ctl, double prev, double logscale) {
@@ -290,6 +297,12 @@ struct gs_engine {
         int fgrid = 1;
     };
     std::vector<Launch> launch;
+    // several strings per launch: `strings` of them, each with an arena of its own in `slots` (see ensure_slots)
+    int strings = 1;                // strings of the launches being enqueued (1: the engine's own arena)
+    void* slots = nullptr;          // [nslots] arenas, then the block partials
+    double* slot_part[2] = {nullptr, nullptr};
+    int nslots = 0;
+    bool own_buffers = true;        // false: buffers of the scratch array (gs_prob_noalloc), which allocates nothing
     double* part = nullptr;         // per-block partials of the running sweep (part_buf[0])
     double* part_buf[2] = {nullptr, nullptr};   // alternate between sweeps: one may hold partials still unreduced
     int cur_part = 0;               // the buffer the next sweep writes
@@ -360,6 +373,43 @@ int ns_of(const gs_engine* e) { return e->plan.ns; }
 // Partial sums per block of each sweep kind (Gram 4, direct 2, write 2, write + Gram 6, write + direct 4).
 int partials_of(int sweep) { return sweep == kGram ? 4 : sweep == kWriteGram ? 6 : sweep == kWriteDirect ? 4 : 2; }
 
+// Arena of the launches being enqueued, and the distance of their strings' arenas and partials.
+void* arena_of(const gs_engine* e) { return e->strings > 1 ? e->slots : e->arena; }
+uint64_t slot_entries(const gs_engine* e) { return uint64_t(1) << e->plan.R; }
+// Doubles of one string's block partials: a sweep has at most one block per 2^8 arena entries.
+uint32_t slot_part_doubles(const gs_engine* e) {
+    return uint32_t(kPartStride) << std::min(kMaxGridLog2, std::max(0, e->plan.R - 8));
+}
+
+// Make room for up to `want` strings per launch; returns how many the engine can run at once (1: one by one, also when
+// the memory is not there).  Runs of diagonal steps keep pattern sums for one string only, so plans with such runs
+// (2^20 cosets and more) run one string at a time, as do engines whose sweeps are timed one by one.
+int ensure_slots(gs_engine* e, int64_t want) {
+    if (want < 2 || !e->own_buffers || e->profile || !e->hrun.empty()) return 1;
+    const size_t arena = slot_entries(e) * e->esz;
+    const size_t part = size_t(slot_part_doubles(e)) * sizeof(double);
+    const size_t each = arena + 2 * part;
+    const int most = int(std::min<size_t>(gs_engine::kChunk, kSlotBytes / each));
+    if (most < kMinSlots) return 1;
+    int n = 2;
+    while (n < want && n < most) n = std::min(2 * n, most);
+    if (n > e->nslots) {
+        if (hipStreamSynchronize(e->stream) != hipSuccess) return 1;
+        (void)hipFree(e->slots);
+        e->slots = nullptr;
+        e->nslots = 0;
+        if (hipMalloc(&e->slots, each * size_t(n)) != hipSuccess) {
+            (void)hipGetLastError();
+            e->slots = nullptr;
+            return 1;
+        }
+        e->nslots = n;
+        e->slot_part[0] = reinterpret_cast<double*>(static_cast<unsigned char*>(e->slots) + arena * size_t(n));
+        e->slot_part[1] = e->slot_part[0] + size_t(slot_part_doubles(e)) * size_t(n);
+    }
+    return int(std::min<int64_t>(n, want));
+}
+
 // Reduce the partials the last sweep left (one-block kernel) before a launch that does not reduce them itself.
 int flush_pending(gs_engine* e) {
     if (!e->pend_nblk) return 0;
@@ -370,7 +420,7 @@ int flush_pending(gs_engine* e) {
     int sw = e->pend_sweep;
     e->pend_nblk = 0;
     void* rargs[] = {&cpart, &nblk, &ctl, &ep, &sw};
-    HIP_TRY(hipLaunchKernel(reduce_kernel_ptr(sw), dim3(1), dim3(kThreads), rargs, 0, e->stream));
+    HIP_TRY(hipLaunchKernel(reduce_kernel_ptr(sw), dim3(1, e->strings), dim3(kThreads), rargs, 0, e->stream));
     return 0;
 }
 
@@ -382,7 +432,7 @@ int launch_sweep(gs_engine* e, int k, int sweep, const Epi& epi) {
     const bool fused = sweep == kWriteGram || sweep == kWriteDirect;
     const KStep* sp = (fused ? e->dfused : e->dplain) + k;
     const int grid = fused ? L.fgrid : L.grid;
-    void* mem = e->arena;
+    void* mem = arena_of(e);
     Epi ep = epi;
     const KStep& hs = (fused ? e->hfused : e->hplain)[size_t(k)];
     const int live_r = hs.nk + (hs.ntq == 4 ? 2 : hs.ntq == 2 ? 1 : 0);
@@ -398,11 +448,11 @@ int launch_sweep(gs_engine* e, int k, int sweep, const Epi& epi) {
         ep.pend_next = e->pend_epi.next;
         ep.pend_sweep = e->pend_sweep;
         e->cur_ctl ^= 1;
-        e->ctl = e->ctl_base + e->cur_ctl;
+        e->ctl = e->ctl_base + e->cur_ctl * gs_engine::kChunk;
         ep.ctl_out = e->ctl;
         e->pend_nblk = 0;
     }
-    double* part = e->part_buf[e->cur_part];
+    double* part = (e->strings > 1 ? e->slot_part : e->part_buf)[e->cur_part];
     void* args[] = {&sp, &mem, &part, &ctl, &ep};
     hipEvent_t a = nullptr, b = nullptr;
     if (e->profile) {
@@ -410,14 +460,14 @@ int launch_sweep(gs_engine* e, int k, int sweep, const Epi& epi) {
         HIP_TRY(hipEventCreate(&b));
         HIP_TRY(hipEventRecord(a, e->stream));
     }
-    HIP_TRY(hipLaunchKernel(fn, dim3(grid), dim3(kThreads), args, 0, e->stream));
+    HIP_TRY(hipLaunchKernel(fn, dim3(grid, e->strings), dim3(kThreads), args, 0, e->stream));
     if (e->profile) {                   // the sweep kernel alone (the reduce kernel, if any, is not timed here)
         HIP_TRY(hipEventRecord(b, e->stream));
         e->pev.push_back(a);
         e->pev.push_back(b);
         e->pev_tag.push_back(k * 8 + sweep);
     }
-    if (grid > kFenceBlocks) {          // the blocks only stored their partials: the next sweep reduces them
+    if (!reduces_in_kernel(unsigned(grid), unsigned(e->strings))) {   // the blocks only stored their partials
         e->pend_part = part;
         e->pend_nblk = unsigned(grid);
         e->pend_sweep = sweep;
@@ -449,10 +499,10 @@ int launch_small(gs_engine* e, void* fn, Epi epi, int k) {
     Ctl* ctl = e->ctl;
     if (k >= 0) {
         void* args[] = {&ctl, &epi, &k};
-        HIP_TRY(hipLaunchKernel(fn, dim3(1), dim3(1), args, 0, e->stream));
+        HIP_TRY(hipLaunchKernel(fn, dim3(1, e->strings), dim3(1), args, 0, e->stream));
     } else {
         void* args[] = {&ctl, &epi};
-        HIP_TRY(hipLaunchKernel(fn, dim3(1), dim3(1), args, 0, e->stream));
+        HIP_TRY(hipLaunchKernel(fn, dim3(1, e->strings), dim3(1), args, 0, e->stream));
     }
     return 0;
 }
@@ -460,11 +510,11 @@ int launch_small(gs_engine* e, void* fn, Epi epi, int k) {
 int launch_init(gs_engine* e) {
     Ctl* ctl = e->ctl;
     if (e->storage == GS_C64) {
-        float2* mem = static_cast<float2*>(e->arena);
-        hipLaunchKernelGGL(init_kernel<float2>, dim3(1), dim3(1), 0, e->stream, mem, ctl);
+        float2* mem = static_cast<float2*>(arena_of(e));
+        hipLaunchKernelGGL(init_kernel<float2>, dim3(e->strings), dim3(1), 0, e->stream, mem, ctl, slot_entries(e));
     } else {
-        double2* mem = static_cast<double2*>(e->arena);
-        hipLaunchKernelGGL(init_kernel<double2>, dim3(1), dim3(1), 0, e->stream, mem, ctl);
+        double2* mem = static_cast<double2*>(arena_of(e));
+        hipLaunchKernelGGL(init_kernel<double2>, dim3(e->strings), dim3(1), 0, e->stream, mem, ctl, slot_entries(e));
     }
     HIP_TRY(hipGetLastError());
     return 0;
@@ -558,8 +608,9 @@ int norm_for(const gs_engine* e, int mode, int k, int forced_bit, bool forced_st
     return kGram;
 }
 
-// Enqueue steps k0..k1-1 of one string.  forced_h: host copy of the string's forced bits (nullptr when every step is
-// sampled); device pointers address this string's slot.  Per step: [norm sweep, when the previous write could not
+// Enqueue steps k0..k1-1 of e->strings strings (one unless the caller set it).  forced_h: host copy of the first
+// string's forced bits (nullptr when every step is sampled; the others have the same '?' steps); device pointers
+// address the first string's slot, the others follow.  Per step: [norm sweep, when the previous write could not
 // fold it in] -> write sweep, whose last block does the bookkeeping and decides the next step.
 int enqueue_run(gs_engine* e, int mode, int k0, int k1, const int8_t* forced_h, const int8_t* forced_d, const double* U_d,
                 int8_t* bits_d, double* cond_d, double* out_d) {
@@ -574,6 +625,8 @@ int enqueue_run(gs_engine* e, int mode, int k0, int k1, const int8_t* forced_h, 
     base.out = out_d;
     base.counter = e->counter;
     base.plain = e->dplain;
+    base.slot_entries = slot_entries(e);
+    base.slot_part = slot_part_doubles(e);
     if (k0 == k1) return launch_small(e, publish_kernel_ptr(), base, -1);
     const bool fstr = forced_h != nullptr && mode == kChain;
     auto fb = [&](int k) { return forced_h ? int(forced_h[k]) : -1; };
@@ -593,13 +646,13 @@ int enqueue_run(gs_engine* e, int mode, int k0, int k1, const int8_t* forced_h, 
         if (ke - k >= 2) {
             if (int rc = flush_pending(e)) return rc;
             const KStep* sp = e->dplain;
-            void* mem = e->arena;
+            void* mem = arena_of(e);
             Ctl* ctl = e->ctl;
             Epi ep = base;
             int a = k, b = ke, d = decided ? 1 : 0;
             void* args[] = {&sp, &mem, &ctl, &ep, &a, &b, &d};
-            HIP_TRY(hipLaunchKernel(small_run_kernel_ptr(e->storage), dim3(1), dim3(small_run_threads()), args, 0,
-                                    e->stream));
+            HIP_TRY(hipLaunchKernel(small_run_kernel_ptr(e->storage), dim3(1, e->strings), dim3(small_run_threads()),
+                                    args, 0, e->stream));
             decided = false;
             k = ke - 1;
             continue;
@@ -1270,6 +1323,7 @@ void free_engine(gs_engine* e) {
     (void)hipFree(e->dfused);
     (void)hipFree(e->dlogical);
     (void)hipFree(e->part_buf[0]);
+    (void)hipFree(e->slots);
     (void)hipFree(e->counter);
     (void)hipFree(e->ctl_base);
     (void)hipFree(e->d_forced);
@@ -1328,10 +1382,43 @@ std::complex<double> read_amp(const gs_engine* e, int slot) {
     return {v[0], v[1]};
 }
 
-// Copy arena entry 0 into the string's amplitude slot (ordered on the stream).
+// Copy arena entry 0 of the strings in flight into their amplitude slots (ordered on the stream).
 int enqueue_amp(gs_engine* e, int slot) {
-    HIP_TRY(hipMemcpyAsync(e->d_amp + size_t(slot) * 16, e->arena, e->esz, hipMemcpyDeviceToDevice, e->stream));
+    unsigned char* out = e->d_amp + size_t(slot) * 16;
+    if (e->storage == GS_C64)
+        hipLaunchKernelGGL(amp_kernel<float2>, dim3(e->strings), dim3(1), 0, e->stream,
+                           static_cast<const float2*>(arena_of(e)), slot_entries(e), out);
+    else
+        hipLaunchKernelGGL(amp_kernel<double2>, dim3(e->strings), dim3(1), 0, e->stream,
+                           static_cast<const double2*>(arena_of(e)), slot_entries(e), out);
+    HIP_TRY(hipGetLastError());
     return 0;
+}
+
+// Enqueue the chains of a chunk of cnt strings (slots 0 .. cnt-1 of the per-string buffers) from the start, several per
+// launch where the engine has room.  In the hybrid modes the strings of a launch have the same '?' steps, since those
+// decide which sweeps a step needs.
+int enqueue_strings(gs_engine* e, int mode, int cnt, bool forced, bool amp) {
+    const int ns = ns_of(e);
+    const int most = ensure_slots(e, cnt);
+    auto alike = [&](int a, int b) {
+        for (int k = 0; k < ns; k++)
+            if ((e->h_forced[size_t(a) * ns + k] < 0) != (e->h_forced[size_t(b) * ns + k] < 0)) return false;
+        return true;
+    };
+    int rc = 0;
+    for (int i = 0; i < cnt && !rc; i += e->strings) {
+        e->strings = 1;
+        while (e->strings < most && i + e->strings < cnt && (mode != kRun || alike(i, i + e->strings))) e->strings++;
+        if ((rc = launch_init(e))) break;
+        const size_t at = size_t(i) * ns;
+        if ((rc = enqueue_run(e, mode, 0, ns, forced ? e->h_forced + at : nullptr, forced ? e->d_forced + at : nullptr,
+                              e->d_U + at, e->d_bits + at, e->d_cond + at, e->d_out + size_t(i) * 4)))
+            break;
+        if (amp) rc = enqueue_amp(e, i);
+    }
+    e->strings = 1;
+    return rc;
 }
 
 int check_bits(const int8_t* b, int64_t n, bool allow_q) {
@@ -1352,14 +1439,7 @@ int run_forced(gs_engine* e, int mode, const int8_t* bits, int64_t nstr, double*
         memcpy(e->h_forced, bits + s0 * ns, size_t(cnt) * ns);
         HIP_TRY(hipMemcpyAsync(e->d_forced, e->h_forced, size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
         if (int rc = begin_timing(e)) return rc;
-        for (int i = 0; i < cnt; i++) {
-            if (int rc = launch_init(e)) return rc;
-            if (int rc = enqueue_run(e, mode, 0, ns, e->h_forced + size_t(i) * ns, e->d_forced + size_t(i) * ns, e->d_U,
-                                     e->d_bits + size_t(i) * ns, e->d_cond + size_t(i) * ns, e->d_out + size_t(i) * 4))
-                return rc;
-            if (amp)
-                if (int rc = enqueue_amp(e, i)) return rc;
-        }
+        if (int rc = enqueue_strings(e, mode, cnt, true, amp != nullptr)) return rc;
         if (int rc = end_timing(e)) return rc;
         HIP_TRY(hipMemcpyAsync(e->h_out, e->d_out, size_t(cnt) * 4 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
         if (cond)
@@ -1454,7 +1534,7 @@ int gs_engine_create(const gs_plan* plan, int storage, int device, gs_engine** o
               dev_alloc((void**)&e->dlogical, sizeof(KStep) * nsz) &&
               dev_alloc((void**)&e->part_buf[0], 2 * sizeof(double) * kPartDoubles) &&
               dev_alloc((void**)&e->counter, sizeof(unsigned) * kCounters) &&
-              dev_alloc((void**)&e->ctl_base, 2 * sizeof(Ctl)) && dev_alloc((void**)&e->d_forced, C * nsz) &&
+              dev_alloc((void**)&e->ctl_base, 2 * C * sizeof(Ctl)) && dev_alloc((void**)&e->d_forced, C * nsz) &&
               dev_alloc((void**)&e->d_U, sizeof(double) * C * nsz) && dev_alloc((void**)&e->d_bits, C * nsz) &&
               dev_alloc((void**)&e->d_cond, sizeof(double) * C * nsz) &&
               dev_alloc((void**)&e->d_out, sizeof(double) * C * 4) && dev_alloc((void**)&e->d_amp, 16 * C) &&
@@ -1513,12 +1593,7 @@ int gs_sample(gs_engine* eng, uint64_t seed, int64_t first, int64_t count, int s
         }
         HIP_TRY(hipMemcpyAsync(e->d_U, e->h_U, sizeof(double) * size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
         if (int rc = begin_timing(e)) return rc;
-        for (int i = 0; i < cnt; i++) {
-            if (int rc = launch_init(e)) return rc;
-            if (int rc = enqueue_run(e, kChain, 0, ns, nullptr, nullptr, e->d_U + size_t(i) * ns,
-                                     e->d_bits + size_t(i) * ns, e->d_cond + size_t(i) * ns, e->d_out + size_t(i) * 4))
-                return rc;
-        }
+        if (int rc = enqueue_strings(e, kChain, cnt, false, false)) return rc;
         if (int rc = end_timing(e)) return rc;
         HIP_TRY(hipMemcpyAsync(e->h_bits, e->d_bits, size_t(cnt) * ns, hipMemcpyDeviceToHost, e->stream));
         HIP_TRY(hipMemcpyAsync(e->h_out, e->d_out, size_t(cnt) * 4 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
@@ -1550,13 +1625,7 @@ int gs_hybrid(gs_engine* eng, const int8_t* bits, int64_t nstr, uint64_t seed, i
         HIP_TRY(hipMemcpyAsync(e->d_forced, e->h_forced, size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
         HIP_TRY(hipMemcpyAsync(e->d_U, e->h_U, sizeof(double) * size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
         if (int rc = begin_timing(e)) return rc;
-        for (int i = 0; i < cnt; i++) {
-            if (int rc = launch_init(e)) return rc;
-            if (int rc = enqueue_run(e, kRun, 0, ns, e->h_forced + size_t(i) * ns, e->d_forced + size_t(i) * ns,
-                                     e->d_U + size_t(i) * ns, e->d_bits + size_t(i) * ns, e->d_cond + size_t(i) * ns,
-                                     e->d_out + size_t(i) * 4))
-                return rc;
-        }
+        if (int rc = enqueue_strings(e, kRun, cnt, true, false)) return rc;
         if (int rc = end_timing(e)) return rc;
         HIP_TRY(hipMemcpyAsync(e->h_bits, e->d_bits, size_t(cnt) * ns, hipMemcpyDeviceToHost, e->stream));
         HIP_TRY(hipMemcpyAsync(e->h_cond, e->d_cond, size_t(cnt) * ns * sizeof(double), hipMemcpyDeviceToHost, e->stream));
@@ -2040,6 +2109,7 @@ extern "C" int gs_prob_noalloc(const gs_plan* plan, int storage, int device, con
     if (device < 0 || device >= ndev || device >= kMaxScratchDevices) return fail(16, "device index out of range");
     HIP_TRY(hipSetDevice(device));
     gs_engine e;                                       // host-side plan of the launches; no device memory of its own
+    e.own_buffers = false;
     e.run_max = 0;                                     // no runs of diagonal steps (their pattern sums need 32 MB)
     e.plan = plan->p;
     e.storage = storage;

@@ -431,6 +431,19 @@ __device__ void decide(Ctl& c, const Epi& e, int k, int norm, const double* red)
     c.w[3] = m1.y * sc;
 }
 
+// The per-string buffers of the epilogue's arguments for this block's string (blockIdx.y).
+__device__ __forceinline__ Epi slot_epi(const Epi& e) {
+    Epi s = e;
+    const size_t y = blockIdx.y, at = y * size_t(e.ns);
+    if (s.forced) s.forced += at;
+    s.U += at;
+    s.bits += at;
+    s.cond += at;
+    s.out += 4 * y;
+    s.counter += y;
+    return s;
+}
+
 // Block-wide sum of v[NQ] over the NT threads in a fixed order (a butterfly inside each 64-lane wave, then the wave
 // sums in wave order by one thread: two barriers instead of a log2(NT)-level tree); the result is in sh[0][*].
 template <int NQ, int NT = kThreads>
@@ -495,10 +508,10 @@ __device__ __forceinline__ void reduce_partials(double (&sh)[kThreads / 64][NQ],
     block_tree_sum<NQ>(sh, r, t);
 }
 
-// End of a sweep block: the block's sums go to its partial slot.  Grids of at most kFenceBlocks blocks finish in
-// the kernel: the last block to arrive (agent-scope counter) reduces and runs the chain.  Larger grids end here and
-// sweep_reduce_kernel follows on the stream: an agent-scope release per block writes back the XCD's L2 each time
-// (tens of ns per block), which a launch boundary does once.
+// End of a sweep block: the block's sums go to its partial slot.  Launches of at most kFenceBlocks blocks finish in
+// the kernel: the last block of a string to arrive (agent-scope counter) reduces and runs the chain; a string's only
+// block does so at once.  Larger launches end here and sweep_reduce_kernel follows on the stream: an agent-scope
+// release per block writes back the XCD's L2 each time (tens of ns per block), which a launch boundary does once.
 template <int NQ>
 __device__ void sweep_epilogue(double (&acc)[NQ], double* part, Ctl* ctl, const Epi& e, int sweep) {
     // block sum (wave butterfly, then the 4 waves in order)
@@ -509,27 +522,37 @@ __device__ void sweep_epilogue(double (&acc)[NQ], double* part, Ctl* ctl, const 
     __shared__ int s_last;
     const int t = threadIdx.x;
     const unsigned nblk = gridDim.x;
-    const bool inkernel = nblk <= unsigned(kFenceBlocks);
+    const bool inkernel = reduces_in_kernel(nblk, gridDim.y);
     if ((t & 63) == 0)
 #pragma unroll
         for (int q = 0; q < NQ; q++) sh[t >> 6][q] = acc[q];
     __syncthreads();
     if (t == 0) {
         double* mine = part + size_t(blockIdx.x) * kPartStride;
+        double red[NQ];
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
             double v = sh[0][q];
 #pragma unroll
             for (int w = 1; w < kThreads / 64; w++) v += sh[w][q];
-            if (inkernel) __hip_atomic_store(mine + q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            else mine[q] = v;
+            red[q] = v;
         }
-        if (inkernel) {
-            const unsigned done = __hip_atomic_fetch_add(e.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        if (nblk == 1) {
+            chain_step<NQ>(red, ctl, slot_epi(e), sweep);
+        } else {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+                if (inkernel) __hip_atomic_store(mine + q, red[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else mine[q] = red[q];
+            }
+        }
+        if (inkernel && nblk > 1) {
+            const unsigned done = __hip_atomic_fetch_add(e.counter + blockIdx.y, 1u, __ATOMIC_ACQ_REL,
+                                                         __HIP_MEMORY_SCOPE_AGENT);
             s_last = done == nblk - 1;
         }
     }
-    if (!inkernel) return;
+    if (!inkernel || nblk == 1) return;
     __syncthreads();
     if (!s_last) return;
     __atomic_thread_fence(__ATOMIC_ACQUIRE);
@@ -538,14 +561,17 @@ __device__ void sweep_epilogue(double (&acc)[NQ], double* part, Ctl* ctl, const 
     double red[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; q++) red[q] = sh[0][q];
-    chain_step<NQ>(red, ctl, e, sweep);
-    __hip_atomic_store(e.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    chain_step<NQ>(red, ctl, slot_epi(e), sweep);
+    __hip_atomic_store(e.counter + blockIdx.y, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Reduction and chain logic of a sweep of nblk > kFenceBlocks blocks (one block, launched after the sweep).
+// Reduction and chain logic of a sweep whose blocks left their partials (one block per string, launched after the
+// sweep).
 template <int NQ>
 __global__ __launch_bounds__(kThreads) void sweep_reduce_kernel(const double* __restrict__ part, unsigned nblk,
                                                                 Ctl* __restrict__ ctl, Epi e, int sweep) {
+    ctl += blockIdx.y;
+    part += size_t(blockIdx.y) * e.slot_part;
     if (ctl->dead) return;
     __shared__ double sh[kThreads / 64][NQ];
     const int t = threadIdx.x;
@@ -554,7 +580,7 @@ __global__ __launch_bounds__(kThreads) void sweep_reduce_kernel(const double* __
     double red[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; q++) red[q] = sh[0][q];
-    chain_step<NQ>(red, ctl, e, sweep);
+    chain_step<NQ>(red, ctl, slot_epi(e), sweep);
 }
 
 // The chain step of block partials a previous sweep left unreduced, run at the start of the next sweep by every block
@@ -564,14 +590,14 @@ template <int NQ>
 __device__ void pending_reduce_step(Ctl& cl, const Ctl* ctl, const Epi& epi, Ctl* shc) {
     __shared__ double sh[kThreads / 64][NQ];
     const int t = threadIdx.x;
-    reduce_partials<NQ>(sh, epi.pend_part, epi.pend_nblk, t, false);
+    reduce_partials<NQ>(sh, epi.pend_part + size_t(blockIdx.y) * epi.slot_part, epi.pend_nblk, t, false);
     if (t == 0) {
         Ctl c = *ctl;
         if (!c.dead) {
             double red[NQ];
 #pragma unroll
             for (int q = 0; q < NQ; q++) red[q] = sh[0][q];
-            Epi ep = epi;
+            Epi ep = slot_epi(epi);
             ep.k = epi.pend_k;
             ep.role = epi.pend_role;
             ep.next = epi.pend_next;
@@ -579,7 +605,7 @@ __device__ void pending_reduce_step(Ctl& cl, const Ctl* ctl, const Epi& epi, Ctl
             chain_step<NQ>(red, &c, ep, epi.pend_sweep);
         }
         *shc = c;
-        if (blockIdx.x == 0) *epi.ctl_out = c;
+        if (blockIdx.x == 0) epi.ctl_out[blockIdx.y] = c;
     }
     __syncthreads();
     cl = *shc;
@@ -611,6 +637,9 @@ __global__ __launch_bounds__(kThreads) void sweep_kernel(const KStep* __restrict
     const KStep& s = *sp;
     const int nk = s.nk;
     const int tid = threadIdx.x;
+    mem += uint64_t(blockIdx.y) * epi.slot_entries;   // this block's string
+    part += size_t(blockIdx.y) * epi.slot_part;
+    ctl += blockIdx.y;
     constexpr int lt = LV + 8;                     // log2 cosets per tile
 
     // parity bits of a coordinate: bit 0 output sign, bit 1 next-step slot index, bit 2 next-step sign, bit 3 the
@@ -714,7 +743,7 @@ __global__ __launch_bounds__(kThreads) void sweep_kernel(const KStep* __restrict
     Ctl* cur = ctl;
     Ctl cl;
     if (epi.pend_nblk) {
-        cur = epi.ctl_out;
+        cur = epi.ctl_out + blockIdx.y;
         if (active) {
             load_tile(a_tb ^ a_it, e);
             first_loaded = true;
@@ -864,11 +893,11 @@ __global__ __launch_bounds__(kThreads) void sweep_kernel(const KStep* __restrict
 // single-thread chain kernels
 
 __global__ void decide_kernel(Ctl* ctl, Epi e, int k) {
-    Ctl& c = *ctl;
-    if (!c.dead) decide(c, e, k, -1, nullptr);
+    Ctl& c = ctl[blockIdx.y];
+    if (!c.dead) decide(c, slot_epi(e), k, -1, nullptr);
 }
 
-__global__ void publish_kernel(Ctl* ctl, Epi e) { publish(*ctl, e); }
+__global__ void publish_kernel(Ctl* ctl, Epi e) { publish(ctl[blockIdx.y], slot_epi(e)); }
 
 // ---------------------------------------------------------------------------------------------------------------
 // A run of small steps in one block.  The head and tail of a plan are steps of a few thousand cosets, where a sweep
@@ -981,8 +1010,11 @@ __device__ __forceinline__ void small_pass_any(const KStep& s, S* mem, int sweep
 // run steps need none, growth steps use the stored norm, forced chain strings use direct norms, sampled steps Gram.
 template <class S>
 __global__ __launch_bounds__(kSmallThreads) void small_run_kernel(const KStep* __restrict__ steps, S* __restrict__ mem,
-                                                                  Ctl* __restrict__ ctl, Epi e, int k0, int k1,
+                                                                  Ctl* __restrict__ ctl, Epi epi, int k0, int k1,
                                                                   int decided0) {
+    const Epi e = slot_epi(epi);
+    mem += uint64_t(blockIdx.y) * epi.slot_entries;
+    ctl += blockIdx.y;
     __shared__ double sh[kSmallThreads / 64][4];
     __shared__ int s_dead;
     __shared__ Ctl c;               // the chain state, in LDS while the run lasts
