@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "../../include/gsamp_amd.h"
+#include "gs_gf2.h"
 #include "gs_plan.h"
 
 namespace {
@@ -40,6 +41,7 @@ constexpr int kWaves = 4;            // waves per block, each on its own part of
 constexpr int kRChunks = 64;         // chunks of the first reduction stage per lane group
 constexpr int kBThreads = kLanes * kWaves;
 constexpr int64_t kMinItems = 1024;  // work items (blocks) a step launch should have before tiles get coarser
+constexpr int kMaxSums = 8;          // per-lane sums of one item: the norms of one or two steps, or their G_k(x)
 
 struct BStep {
     uint64_t cols[40];
@@ -48,6 +50,7 @@ struct BStep {
     double mre[2][2], mim[2][2];
     int nk, ntq, m;
     int tau0[4], tau1[4], par[4];
+    uint32_t t0m, t1m, parm;     // tau0, tau1, par as bit masks over the offsets
 };
 
 struct BItem {
@@ -60,10 +63,29 @@ struct BItem {
     int pad;
 };
 
+// Two consecutive steps as one sweep (see make_pair).  L1, the live table between them, splits into W, the span of
+// step k+1's slot offsets (relative to its first) and step k's g, and a complement C inside the span of step k's
+// columns.  A super-coset a + W (a in C) is closed under both steps: its NI step-k cosets i (at a ^ D[i]) give the
+// elements (i, t) at a ^ D[i] ^ t g, which are all the slots of its NU step-(k+1) cosets, so a lane takes it from step
+// k's inputs to step k+1's outputs without the table between them ever being stored.
+struct BPair {
+    uint64_t cols[40];   // columns of the super-coset coordinates
+    uint64_t D[4];
+    uint64_t lab[4];     // D[i], or D[i] ^ g where it is labelled output 1: the base address of step k's coset
+    uint64_t g, d1, d2;  // step k's g; step k+1's second and third offsets relative to the first
+    uint64_t o0;         // step k+1's first offset
+    uint8_t pn[40];      // per coordinate: bit 0 step k's sign, bit 1 step k+1's sign, bits 2-3 step k+1's slot index
+    uint8_t pd[4], pg;   // the same of D[i] (bit 4: the output index it is labelled with) and of g
+    uint8_t pc;          // the same of step k+1's first offset
+    int nk;              // super-coset coordinates
+    int ni, mo, deg;     // step-k cosets, outputs of step k, 1 when g is among the slot offsets of step k+1 (NU = 1)
+};
+
 struct BInst {           // device view of one instance
     void* mem;           // [2^R][B] forward arena
     void* lam;           // [2^R][B] adjoint arena (gradient mode)
     const BStep* steps;  // [ns]
+    const BPair* pairs;  // [ns]: the sweep of steps k and k+1, where one is taken
     const int8_t* bitsT; // [ns][B] forced bits, step-major
     double* prev;        // [B]
     int* dead;           // [B]
@@ -71,8 +93,8 @@ struct BInst {           // device view of one instance
     double* logp;        // [B]
     double* amp;         // [B][2]
     double* grad;        // [B][ns][2][2]: G_k(x) re, im (gradient mode)
-    double* part;        // [groups][max items per group][64][4]
-    double* cpart;       // [groups][kRChunks][64][4]: chunk sums of the item partials
+    double* part;        // [groups][items of the step per group][nq][64]: the items' nq sums
+    double* cpart;       // [groups][kRChunks][nq][64]: chunk sums of the item partials
     int B, ns, pad0, pad1;
 };
 
@@ -192,17 +214,19 @@ struct Walk {
 // per-(instance, lane group) reduction runs in batch_reduce_kernel after the step, at a launch boundary).
 template <int NQ>
 __device__ void lane_store(const BInst& I, const BItem& it, int wave, int lane, const double (&v)[NQ]) {
-    __shared__ double sh[kWaves][kLanes][NQ];
+    __shared__ double sh[kWaves][NQ][kLanes];
 #pragma unroll
-    for (int q = 0; q < NQ; q++) sh[wave][lane][q] = v[q];
+    for (int q = 0; q < NQ; q++) sh[wave][q][lane] = v[q];
     __syncthreads();
-    if (wave != 0) return;
-    double* part = I.part + ((size_t(it.group) * size_t(it.count) + size_t(it.index)) * kLanes + lane) * 4;
+    double* part = I.part + (size_t(it.group) * size_t(it.count) + size_t(it.index)) * (NQ * kLanes);
 #pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        double t = sh[0][lane][q];
-        for (int w = 1; w < kWaves; w++) t += sh[w][lane][q];
-        part[q] = t;
+    for (int q0 = 0; q0 < NQ; q0 += kWaves) {            // wave w adds up sums w, w + 4, ...
+        const int q = q0 + wave;
+        if (q >= NQ) break;
+        double t = sh[0][q][lane];
+#pragma unroll
+        for (int w = 1; w < kWaves; w++) t += sh[w][q][lane];
+        part[q * kLanes + lane] = t;
     }
 }
 
@@ -424,65 +448,470 @@ __global__ __launch_bounds__(kBThreads) void batch_back_kernel(const BInst* __re
     lane_store<4>(I, it, wave, lane, val);
 }
 
-// After step k, in two fixed-order stages: batch_chunk_kernel sums the items' partials (cnt[inst] items per lane
-// group) in kRChunks chunks of consecutive items, one block of kWaves waves per (lane group, chunk) -- wave w takes
-// items w, w + kWaves, ... of the chunk -- and batch_reduce_kernel sums the chunks per (instance, lane), then runs
-// chain1 bookkeeping (mode 0: cond, prev, dead; gsamp2.cpp:67) or stores the gradient entry G_k (mode 1).
+// ---- two steps per sweep (BPair)
+//
+// A single step's sweep is bound by HBM: it reads and writes one table (n = 70 band 26, 64 lanes, 2^22 cosets: 4.3 GB
+// in 0.85 ms, 5.0 TB/s) and its FP64 work takes a quarter of that time.  Two steps in one sweep move the same bytes
+// once instead of twice.  Everything that depends on the super-coset alone (addresses, signs, slot indices) is
+// wave-uniform and kept in scalar registers; a lane holds the NI * NQ inputs of its string.  The table between the
+// steps is rounded to the storage type in registers, so the results are the single steps' bit for bit up to the order
+// of the FP64 sums over the cosets.
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    return (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(v >> 32)))) << 32) |
+           uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
+}
+__device__ __forceinline__ double2 flip_if(double2 a, uint32_t s) {          // (-1)^s a
+    const int m = int(s << 31);
+    return make_double2(__hiloint2double(__double2hiint(a.x) ^ m, __double2loint(a.x)),
+                        __hiloint2double(__double2hiint(a.y) ^ m, __double2loint(a.y)));
+}
+__device__ __forceinline__ void route_one(double2 (&A)[2][2], double2 w, uint32_t t0, uint32_t t1, uint32_t neg) {
+    const double2 ws = flip_if(w, neg);
+    if (t0) A[1][0] = cadd(A[1][0], w); else A[0][0] = cadd(A[0][0], w);     // uniform branches
+    if (t1) A[1][1] = cadd(A[1][1], ws); else A[0][1] = cadd(A[0][1], ws);
+}
+
+// Super-cosets a wave gathers at once: about 8 loads in flight per lane for 8-byte entries, 4 for 16-byte ones.
+template <class S>
+constexpr int pair_lu(int loads) {
+    const int most = sizeof(S) == 8 ? 8 : 4;
+    return loads * 4 <= most ? 2 : loads * 2 <= most ? 1 : 0;
+}
+
+// The super-cosets of one wave (as Walk, with uniform state): U at a time, Gray-ordered groups.
+template <int LU>
+struct PairWalk {
+    static constexpr int U = 1 << LU;
+    const uint64_t* cols;                     // in LDS
+    const int* pn;
+    uint64_t cstart, base, ubase[U];
+    uint32_t p, up[U];
+    int lsub, lu;
+    bool on;
+    __device__ __forceinline__ uint64_t col(int j) const { return uniform64(cols[j]); }
+    __device__ __forceinline__ uint32_t nib(int j) const { return uint32_t(__builtin_amdgcn_readfirstlane(pn[j])); }
+    __device__ PairWalk(const BItem& it, const BPair& P, uint64_t* scols, int* spn, int wave) : cols(scols), pn(spn) {
+        for (int j = threadIdx.x; j < P.nk; j += blockDim.x) {
+            scols[j] = P.cols[j];
+            spn[j] = P.pn[j];
+        }
+        __syncthreads();
+        const int lw = it.lg >= 2 ? 2 : it.lg;
+        on = wave < (1 << lw);
+        lsub = it.lg - lw;
+        cstart = it.c0 | (uint64_t(wave) << lsub);
+        base = 0;
+        p = 0;
+        for (int j = lsub; j < P.nk; j++)
+            if ((cstart >> j) & 1) {
+                base ^= col(j);
+                p ^= nib(j);
+            }
+        lu = lsub < LU ? lsub : LU;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            ubase[u] = 0;
+            up[u] = 0;
+#pragma unroll
+            for (int j = 0; j < LU; j++)
+                if (j < lu && ((u >> j) & 1)) {
+                    ubase[u] ^= col(j);
+                    up[u] ^= nib(j);
+                }
+        }
+    }
+    __device__ uint64_t groups() const { return on ? uint64_t(1) << (lsub - lu) : 0; }
+    __device__ bool valid(int u) const { return u < (1 << lu); }
+    __device__ int own(int u) const { return u & ((1 << lu) - 1); }
+    __device__ void next(uint64_t t) {
+        const int j = lu + __builtin_ctzll(t);
+        base ^= col(j);
+        p ^= nib(j);
+    }
+    __device__ uint64_t index(uint64_t t, int u) const { return cstart | ((t ^ (t >> 1)) << lu) | uint64_t(u); }
+};
+
+// Uniform per-launch constants of a pair.
+struct PairRegs {
+    uint64_t lab[4], off[4], g, d1, d2, o0, g1;
+    uint32_t pd[4], pg, pc, t0m, t1m, parm, u0m, u1m, uparm;
+    int m1;
+    __device__ PairRegs(const BPair& P, const BStep& s0, const BStep& s1) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            lab[i] = P.lab[i];
+            off[i] = s0.off[i];
+            pd[i] = P.pd[i];
+        }
+        g = P.g; d1 = P.d1; d2 = P.d2; o0 = P.o0; pg = P.pg; pc = P.pc;
+        g1 = s1.g;
+        m1 = s1.m;
+        t0m = s0.t0m; t1m = s0.t1m; parm = s0.parm;
+        u0m = s1.t0m; u1m = s1.t1m; uparm = s1.parm;
+    }
+    // slot of step k+1 at element (i, t) of the super-coset with parities pa, and its coset's sign
+    __device__ uint32_t slot(uint32_t pa, int i, int t) const { return ((pa ^ pd[i] ^ (t ? pg : 0) ^ pc) >> 2) & 3; }
+    __device__ uint32_t sign(uint32_t pa, int c) const { return ((pa ^ (c ? pg : 0) ^ pc) >> 1) & 1; }
+    // output 0 of step-(k+1) coset c of the super-coset at a
+    __device__ uint64_t out(uint64_t a, uint32_t pa, int c) const {
+        const uint32_t j = slot(pa, 0, c);
+        return a ^ (c ? g : 0) ^ o0 ^ ((j & 1) ? d1 : 0) ^ ((j & 2) ? d2 : 0);
+    }
+};
+
+// Slot sums of step-k coset i: A[t][x], t the element label (output index t ^ label bit).
+template <class S, int NQ>
+__device__ __forceinline__ void pair_route0(const PairRegs& r, const S (&v)[NQ], uint32_t pa, int i,
+                                            double2 (&A)[2][2]) {
+    A[0][0] = A[0][1] = A[1][0] = A[1][1] = make_double2(-0.0, -0.0);
+    const uint32_t pc = (pa ^ r.pd[i]) & 1, sw = (r.pd[i] >> 4) & 1;
+#pragma unroll
+    for (int q = 0; q < NQ; q++)
+        route_one(A, Sto<S>::wide(v[q]), ((r.t0m >> q) & 1) ^ sw, ((r.t1m >> q) & 1) ^ sw, pc ^ ((r.parm >> q) & 1));
+}
+
+// Slot sums of step-(k+1) coset c from the elements e[i][t] (already rounded to the storage type).
+template <int NI, int MO, bool DEG>
+__device__ __forceinline__ void pair_route1(const PairRegs& r, const double2 (&e)[NI][MO], uint32_t pa, int c,
+                                            double2 (&A)[2][2]) {
+    A[0][0] = A[0][1] = A[1][0] = A[1][1] = make_double2(-0.0, -0.0);
+    const uint32_t sg = r.sign(pa, c);
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int t = 0; t < MO; t++) {
+            if (!DEG && t != c) continue;
+            const uint32_t j = r.slot(pa, i, t);
+            route_one(A, e[i][t], (r.u0m >> j) & 1, (r.u1m >> j) & 1, sg ^ ((r.uparm >> j) & 1));
+        }
+}
+
+template <class S, int NQ, int NI, int MO, bool DEG>
+__global__ __launch_bounds__(kBThreads) void pair_step_kernel(const BInst* __restrict__ insts,
+                                                              const BItem* __restrict__ items, BLaunch L) {
+    constexpr int NU = DEG ? 1 : MO, LU = pair_lu<S>(NI * NQ), U = 1 << LU;
+    const BItem it = items[blockIdx.x];
+    const BInst& I = insts[it.inst];
+    const int k = L.k;
+    const BStep& s0 = I.steps[k];
+    const BStep& s1 = I.steps[k + 1];
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int B = I.B;
+    const int b = it.group * kLanes + lane;
+    const int b0 = I.bitsT[size_t(k) * B + b], b1 = I.bitsT[size_t(k + 1) * B + b];
+    const double2 w0 = make_double2(s0.mre[b0][0], s0.mim[b0][0]), w1 = make_double2(s0.mre[b0][1], s0.mim[b0][1]);
+    const double2 x0 = make_double2(s1.mre[b1][0], s1.mim[b1][0]), x1 = make_double2(s1.mre[b1][1], s1.mim[b1][1]);
+    S* __restrict__ mem = static_cast<S*>(I.mem);
+    S* __restrict__ cp = L.copy ? static_cast<S*>(L.copy[it.inst]) : nullptr;
+    const PairRegs r(I.pairs[k], s0, s1);
+    __shared__ uint64_t scols[40];
+    __shared__ int spn[40];
+    PairWalk<LU> wk(it, I.pairs[k], scols, spn, wave);
+    const uint64_t ng = wk.groups();
+    double nb[2] = {0, 0};
+    for (uint64_t t = 0; t < ng; t++) {
+        if (t) wk.next(t);
+        S v[U][NI][NQ];
+        // every load first and unconditionally (see batch_step_kernel): super-cosets u >= 2^lu of a short range repeat
+        // the ones before them and are discarded
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+#pragma unroll
+                for (int q = 0; q < NQ; q++)
+                    v[u][i][q] = Sto<S>::ld(mem + (wk.base ^ wk.ubase[u] ^ r.lab[i] ^ r.off[q]) * B + b);
+        if (cp)
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int i = 0; i < NI; i++)
+#pragma unroll
+                    for (int q = 0; q < NQ; q++)
+                        if (wk.valid(u)) Sto<S>::st(cp + ((wk.index(t, u) * NI + i) * NQ + q) * B + b, v[u][i][q]);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t pa = wk.p ^ wk.up[u];
+            const uint64_t a = wk.base ^ wk.ubase[u];
+            const bool mine = wk.valid(u);
+            double2 e[NI][MO];
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                double2 A[2][2];
+                pair_route0<S, NQ>(r, v[u][i], pa, i, A);
+#pragma unroll
+                for (int m = 0; m < MO; m++) {
+                    const double2 o = cfma(w0, A[m][0], cmul(w1, A[m][1]));
+                    if (mine) nb[0] += norm2(o);
+                    e[i][m] = Sto<S>::wide(Sto<S>::narrow(o));
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < NU; c++) {
+                double2 A[2][2];
+                pair_route1<NI, MO, DEG>(r, e, pa, c, A);
+                const double2 f0 = cfma(x0, A[0][0], cmul(x1, A[0][1]));
+                const double2 f1 = cfma(x0, A[1][0], cmul(x1, A[1][1]));
+                if (!mine) continue;
+                const uint64_t at = r.out(a, pa, c);
+                Sto<S>::st(mem + at * B + b, Sto<S>::narrow(f0));
+                nb[1] += norm2(f0);
+                if (r.m1 == 2) {
+                    Sto<S>::st(mem + (at ^ r.g1) * B + b, Sto<S>::narrow(f1));
+                    nb[1] += norm2(f1);
+                }
+            }
+        }
+    }
+    if (!L.bookkeeping) return;
+    lane_store<2>(I, it, wave, lane, nb);
+}
+
+// Put a compact copy of a pair's input table back into the forward arena.
+template <class S, int NQ, int NI, int MO, bool DEG>
+__global__ __launch_bounds__(kBThreads) void pair_restore_kernel(const BInst* __restrict__ insts,
+                                                                 const BItem* __restrict__ items, BLaunch L) {
+    constexpr int LU = pair_lu<S>(NI * NQ), U = 1 << LU;
+    const BItem it = items[blockIdx.x];
+    const BInst& I = insts[it.inst];
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int B = I.B;
+    const int b = it.group * kLanes + lane;
+    S* __restrict__ mem = static_cast<S*>(I.mem);
+    const S* __restrict__ cp = static_cast<const S*>(L.copy[it.inst]);
+    if (!cp) return;
+    const PairRegs r(I.pairs[L.k], I.steps[L.k], I.steps[L.k + 1]);
+    __shared__ uint64_t scols[40];
+    __shared__ int spn[40];
+    PairWalk<LU> wk(it, I.pairs[L.k], scols, spn, wave);
+    const uint64_t ng = wk.groups();
+    for (uint64_t t = 0; t < ng; t++) {
+        if (t) wk.next(t);
+        S v[U][NI][NQ];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+#pragma unroll
+                for (int q = 0; q < NQ; q++)
+                    v[u][i][q] = Sto<S>::ld(cp + ((wk.index(t, wk.own(u)) * NI + i) * NQ + q) * B + b);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+#pragma unroll
+                for (int q = 0; q < NQ; q++)
+                    Sto<S>::st(mem + (wk.base ^ wk.ubase[u] ^ r.lab[i] ^ r.off[q]) * B + b, v[u][i][q]);
+    }
+}
+
+// Backward through both steps: the copy of step k's input gives the table between them again (in registers), lambda
+// goes from step k+1's outputs to step k's inputs, and both gradients are summed.
+template <class S, int NQ, int NI, int MO, bool DEG>
+__global__ __launch_bounds__(kBThreads) void pair_back_kernel(const BInst* __restrict__ insts,
+                                                              const BItem* __restrict__ items, BLaunch L) {
+    constexpr int NU = DEG ? 1 : MO, LU = pair_lu<S>(NI * NQ + 2 * NU), U = 1 << LU;
+    const BItem it = items[blockIdx.x];
+    const BInst& I = insts[it.inst];
+    const int k = L.k;
+    const BStep& s0 = I.steps[k];
+    const BStep& s1 = I.steps[k + 1];
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int B = I.B;
+    const int b = it.group * kLanes + lane;
+    const int b0 = I.bitsT[size_t(k) * B + b], b1 = I.bitsT[size_t(k + 1) * B + b];
+    const double2 w0 = make_double2(s0.mre[b0][0], s0.mim[b0][0]), w1 = make_double2(s0.mre[b0][1], s0.mim[b0][1]);
+    const double2 x0 = make_double2(s1.mre[b1][0], s1.mim[b1][0]), x1 = make_double2(s1.mre[b1][1], s1.mim[b1][1]);
+    S* __restrict__ lam = static_cast<S*>(I.lam);
+    const S* __restrict__ cp = static_cast<const S*>(L.copy[it.inst]);
+    const PairRegs r(I.pairs[k], s0, s1);
+    const uint64_t gq = r.m1 == 2 ? r.g1 : 0;
+    __shared__ uint64_t scols[40];
+    __shared__ int spn[40];
+    PairWalk<LU> wk(it, I.pairs[k], scols, spn, wave);
+    const uint64_t ng = wk.groups();
+    double2 ga[2] = {make_double2(0, 0), make_double2(0, 0)}, gb[2] = {ga[0], ga[0]};   // G_k(x), G_{k+1}(x)
+    for (uint64_t t = 0; t < ng; t++) {
+        if (t) wk.next(t);
+        S v[U][NI][NQ], l2[U][NU][2];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+#pragma unroll
+                for (int q = 0; q < NQ; q++)
+                    v[u][i][q] = Sto<S>::ld(cp + ((wk.index(t, wk.own(u)) * NI + i) * NQ + q) * B + b);
+#pragma unroll
+            for (int c = 0; c < NU; c++) {
+                const uint64_t at = r.out(wk.base ^ wk.ubase[u], wk.p ^ wk.up[u], c);
+                l2[u][c][0] = Sto<S>::ld(lam + at * B + b);
+                l2[u][c][1] = Sto<S>::ld(lam + (at ^ gq) * B + b);     // a one-output step reads its output twice
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t pa = wk.p ^ wk.up[u];
+            const uint64_t a = wk.base ^ wk.ubase[u];
+            double2 e[NI][MO], l1[NI][MO];
+            double2 ha[2] = {ga[0], ga[1]}, hb[2] = {gb[0], gb[1]};
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                double2 A[2][2];
+                pair_route0<S, NQ>(r, v[u][i], pa, i, A);
+#pragma unroll
+                for (int m = 0; m < MO; m++)
+                    e[i][m] = Sto<S>::wide(Sto<S>::narrow(cfma(w0, A[m][0], cmul(w1, A[m][1]))));
+            }
+#pragma unroll
+            for (int c = 0; c < NU; c++) {
+                double2 A[2][2];
+                pair_route1<NI, MO, DEG>(r, e, pa, c, A);
+                const double2 m0 = Sto<S>::wide(l2[u][c][0]);
+                const double2 m1 = r.m1 == 2 ? Sto<S>::wide(l2[u][c][1]) : make_double2(0, 0);
+#pragma unroll
+                for (int x = 0; x < 2; x++) {
+                    hb[x] = cfma(m0, A[0][x], hb[x]);
+                    if (r.m1 == 2) hb[x] = cfma(m1, A[1][x], hb[x]);
+                }
+                const double2 y0 = cmul(x1, m0), y1 = cmul(x1, m1);
+                const uint32_t sg = r.sign(pa, c);
+#pragma unroll
+                for (int i = 0; i < NI; i++)
+#pragma unroll
+                    for (int m = 0; m < MO; m++) {
+                        if (!DEG && m != c) continue;
+                        const uint32_t j = r.slot(pa, i, m);
+                        const double2 lt = ((r.u0m >> j) & 1) ? m1 : m0;
+                        const double2 y = ((r.u1m >> j) & 1) ? y1 : y0;
+                        l1[i][m] = Sto<S>::wide(Sto<S>::narrow(cfma(x0, lt, flip_if(y, sg ^ ((r.uparm >> j) & 1)))));
+                    }
+            }
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                double2 A[2][2];
+                pair_route0<S, NQ>(r, v[u][i], pa, i, A);
+#pragma unroll
+                for (int x = 0; x < 2; x++)
+#pragma unroll
+                    for (int m = 0; m < MO; m++) ha[x] = cfma(l1[i][m], A[m][x], ha[x]);
+            }
+            if (!wk.valid(u)) continue;             // gradient terms and stores of the wave's own super-cosets only
+#pragma unroll
+            for (int x = 0; x < 2; x++) {
+                ga[x] = ha[x];
+                gb[x] = hb[x];
+            }
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const uint32_t pc = (pa ^ r.pd[i]) & 1, sw = (r.pd[i] >> 4) & 1;
+#pragma unroll
+                for (int q = 0; q < NQ; q++) {
+                    const uint32_t t0 = ((r.t0m >> q) & 1) ^ sw, t1 = ((r.t1m >> q) & 1) ^ sw;
+                    const double2 m0 = MO == 2 && t0 ? l1[i][MO - 1] : l1[i][0];
+                    const double2 m1 = MO == 2 && t1 ? l1[i][MO - 1] : l1[i][0];
+                    const double2 out = cfma(w0, m0, flip_if(cmul(w1, m1), pc ^ ((r.parm >> q) & 1)));
+                    Sto<S>::st(lam + (a ^ r.lab[i] ^ r.off[q]) * B + b, Sto<S>::narrow(out));
+                }
+            }
+        }
+    }
+    const double val[8] = {ga[0].x, ga[0].y, ga[1].x, ga[1].y, gb[0].x, gb[0].y, gb[1].x, gb[1].y};
+    lane_store<8>(I, it, wave, lane, val);
+}
+
+// After a sweep of STEPS steps from step k, batch_reduce_kernel sums the items' partials (cnt[inst] items per lane
+// group) per (instance, lane) in a fixed order over kRWaves waves and runs chain1 bookkeeping (GRAD false: cond, prev,
+// dead; gsamp2.cpp:67) or stores the gradient entries G_k.  Above kDirectItems items batch_chunk_kernel first sums
+// kRChunks chunks of consecutive items over many blocks, and the reduction takes the chunks.  One stage for few items:
+// the second launch costs 4 us and the 64 chunk sums of a lane were a serial chain of 12-16 us.
+constexpr int kRWaves = 8;
+constexpr int kDirectItems = 256;
 __host__ __device__ inline int chunk_items(int count) { return (count + kRChunks - 1) / kRChunks; }
 
+template <int NQ>
 __global__ __launch_bounds__(kBThreads) void batch_chunk_kernel(const BInst* __restrict__ insts,
-                                                               const int* __restrict__ cnt, int mode) {
+                                                               const int* __restrict__ cnt) {
     const int inst = blockIdx.y, group = blockIdx.x / kRChunks, chunk = blockIdx.x % kRChunks;
     const int lane = threadIdx.x & (kLanes - 1), wave = threadIdx.x / kLanes;
     const BInst& I = insts[inst];
     const int count = cnt[inst];
-    if (count == 0 || group >= I.B / kLanes) return;
+    if (count <= kDirectItems || group >= I.B / kLanes) return;
     const int per = chunk_items(count);
     const int i0 = chunk * per, i1 = min(count, i0 + per);
     if (i0 >= i1) return;
-    const int nq = mode == 0 ? 1 : 4;
-    const double* gp = I.part + size_t(group) * size_t(count) * kLanes * 4;
-    double tot[4] = {0, 0, 0, 0};
+    const double* gp = I.part + size_t(group) * size_t(count) * (NQ * kLanes);
+    double tot[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) tot[q] = 0;
     for (int i = i0 + wave; i < i1; i += kWaves)
-        for (int q = 0; q < nq; q++) tot[q] += gp[(size_t(i) * kLanes + lane) * 4 + q];
-    __shared__ double sh[kWaves][kLanes][4];
-    for (int q = 0; q < 4; q++) sh[wave][lane][q] = tot[q];
+#pragma unroll
+        for (int q = 0; q < NQ; q++) tot[q] += gp[(size_t(i) * NQ + q) * kLanes + lane];
+    __shared__ double sh[kWaves][NQ][kLanes];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) sh[wave][q][lane] = tot[q];
     __syncthreads();
     if (wave != 0) return;
-    double* out = I.cpart + ((size_t(group) * kRChunks + chunk) * kLanes + lane) * 4;
-    for (int q = 0; q < nq; q++) {
-        double t = sh[0][lane][q];
-        for (int w = 1; w < kWaves; w++) t += sh[w][lane][q];
-        out[q] = t;
+    double* out = I.cpart + (size_t(group) * kRChunks + chunk) * (NQ * kLanes);
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        double t = sh[0][q][lane];
+        for (int w = 1; w < kWaves; w++) t += sh[w][q][lane];
+        out[q * kLanes + lane] = t;
     }
 }
 
-__global__ __launch_bounds__(kLanes) void batch_reduce_kernel(const BInst* __restrict__ insts,
-                                                              const int* __restrict__ cnt, int k, int mode) {
-    const int inst = blockIdx.y, group = blockIdx.x, lane = threadIdx.x;
+template <int STEPS, bool GRAD>
+__global__ __launch_bounds__(kLanes * kRWaves) void batch_reduce_kernel(const BInst* __restrict__ insts,
+                                                                        const int* __restrict__ cnt, int k) {
+    constexpr int NQ = STEPS * (GRAD ? 4 : 1);
+    const int inst = blockIdx.y, group = blockIdx.x;
+    const int lane = threadIdx.x & (kLanes - 1), wave = threadIdx.x / kLanes;
     const BInst& I = insts[inst];
     const int count = cnt[inst];
     if (count == 0 || group >= I.B / kLanes) return;
-    const int b = group * kLanes + lane;
-    const int nq = mode == 0 ? 1 : 4;
-    double tot[4] = {0, 0, 0, 0};
-    const int nchunks = (count + chunk_items(count) - 1) / chunk_items(count);
-    const double* gp = I.cpart + size_t(group) * kRChunks * kLanes * 4;
-    for (int c = 0; c < nchunks; c++)
-        for (int q = 0; q < nq; q++) tot[q] += gp[(size_t(c) * kLanes + lane) * 4 + q];
-    const int ns = I.ns;
-    if (mode == 1) {
-        double* G = I.grad + (size_t(b) * ns + k) * 4;
-        for (int q = 0; q < 4; q++) G[q] = tot[q];
-        return;
+    const bool direct = count <= kDirectItems;
+    const int n = direct ? count : (count + chunk_items(count) - 1) / chunk_items(count);
+    const double* gp = direct ? I.part + size_t(group) * size_t(count) * (NQ * kLanes)
+                              : I.cpart + size_t(group) * kRChunks * (NQ * kLanes);
+    double tot[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) tot[q] = 0;
+    for (int c = wave; c < n; c += kRWaves)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) tot[q] += gp[(size_t(c) * NQ + q) * kLanes + lane];
+    __shared__ double sh[kRWaves][NQ][kLanes];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) sh[wave][q][lane] = tot[q];
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        tot[q] = sh[0][q][lane];
+#pragma unroll
+        for (int w = 1; w < kRWaves; w++) tot[q] += sh[w][q][lane];
     }
-    if (!I.dead[b]) {
-        I.cond[size_t(b) * ns + k] = tot[0] / (2 * I.prev[b]);
-        I.prev[b] = tot[0];
-        if (tot[0] <= 0) {
-            for (int q = k; q < ns; q++) I.cond[size_t(b) * ns + q] = 0;
-            I.dead[b] = 1;
+    const int b = group * kLanes + lane, ns = I.ns;
+    if constexpr (GRAD) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) I.grad[(size_t(b) * ns + k) * 4 + q] = tot[q];
+    } else {
+        double prev = I.prev[b];
+        bool dead = I.dead[b] != 0;
+#pragma unroll
+        for (int j = 0; j < STEPS; j++) {
+            if (dead) break;
+            I.cond[size_t(b) * ns + k + j] = tot[j] / (2 * prev);
+            prev = tot[j];
+            if (prev <= 0) {
+                for (int q = k + j; q < ns; q++) I.cond[size_t(b) * ns + q] = 0;
+                I.dead[b] = 1;
+                dead = true;
+            }
         }
+        I.prev[b] = prev;
     }
 }
 
@@ -549,12 +978,17 @@ struct gs_batch {
     std::vector<void*> allocs;
     int maxns = 0;
     // per step: work items (device) and their count; tuning: log2 cosets per item per step
-    std::vector<BItem*> ditems;
+    std::vector<BItem*> ditems;           // in item_mem
+    void* item_mem = nullptr;
     std::vector<int> nitems;
+    std::vector<char> chunked;            // per step: some lane group has more than kDirectItems items
     std::vector<std::vector<int>> lg;     // [inst][step]
     int lg_default = 8;                   // smallest tile (sizes the partial buffers); steps start at 2^9
     std::vector<int> nq;                  // per step: most slots per coset among the instances (kernel variant)
     std::vector<int> nq_exact;            // per step: 1 if every instance at the step has nq slots per coset
+    std::vector<std::vector<BPair>> hpairs;   // [inst][step]: steps k and k+1 as one sweep (ni 0: not possible)
+    std::vector<char> unit;               // per step: steps of the sweep that starts there (1, 2; 0: inside a pair)
+    bool pairs_on = true;
     int* dcnt = nullptr;                  // device [maxns][ninst]: items per lane group of instance i at step k
     int maxgroups = 1;
     int lu = 2;                           // log2 cosets a lane gathers at once
@@ -589,42 +1023,189 @@ T* dalloc(gs_batch* b, size_t n) {
     return static_cast<T*>(p);
 }
 
+// Steps k and k+1 of a plan as one sweep (see BPair); false when a super-coset cannot be closed or would write a slot
+// that another super-coset still reads.
+bool make_pair(const gs::StepInfo& s0, const gs::StepInfo& s1, BPair& p) {
+    using gs::GfBasis;
+    using gs::parity;
+    memset(&p, 0, sizeof p);
+    GfBasis live;                                     // L1: the columns of step k (its output 0), then g
+    for (uint64_t c : s0.cols)
+        if (!live.add(c)) return false;
+    if (s0.m == 2 && !live.add(s0.g)) return false;
+    const int lg1 = s1.ntq == 4 ? 2 : s1.ntq == 2 ? 1 : 0;
+    uint64_t d[4] = {0, 0, 0, 0};
+    for (int j = 1; j < s1.ntq; j++) d[j] = s1.off[j] ^ s1.off[0];
+    if (s1.ntq == 4 && (d[3] != (d[1] ^ d[2]))) return false;
+    GfBasis next;                                     // the same space as step k+1 reads it: its columns, then d1, d2
+    for (uint64_t c : s1.cols)
+        if (!live.has(c) || !next.add(c)) return false;
+    for (int j = 1; j <= lg1; j++)
+        if (!live.has(d[j]) || !next.add(d[j])) return false;
+    if (next.n != live.n || !live.has(s1.off[0])) return false;
+    // parities of an address of L1: bit 0 step k's sign, bit 1 step k+1's, bits 2-3 its slot, bit 4 step k's output
+    auto nib = [&](uint64_t x) {
+        uint64_t c0 = 0, c1 = 0;
+        (void)live.solve(x, c0);
+        (void)next.solve(x, c1);
+        const uint64_t m0 = (uint64_t(1) << s0.nk) - 1, m1 = (uint64_t(1) << s1.nk) - 1;
+        return uint8_t(parity(c0 & m0 & s0.rhoc) | (parity(c1 & m1 & s1.rhoc) << 1) | (int((c1 >> s1.nk) & 3) << 2) |
+                       (int((c0 >> s0.nk) & 1) << 4));
+    };
+    GfBasis slots;
+    for (int j = 1; j <= lg1; j++) (void)slots.add(d[j]);
+    p.deg = s0.m == 2 && slots.has(s0.g);
+    p.mo = s0.m;
+    p.ni = p.deg ? s1.ntq / 2 : s1.ntq;
+    if (p.deg) p.D[1] = p.ni == 2 ? (d[1] != s0.g ? d[1] : d[2]) : 0;
+    else
+        for (int i = 1; i < p.ni; i++) p.D[i] = d[i];
+    GfBasis W;
+    if (s0.m == 2) (void)W.add(s0.g);
+    for (int i = 1; i < p.ni; i++) (void)W.add(p.D[i]);
+    GfBasis C;
+    for (uint64_t c : s0.cols)
+        if (W.add(c)) {
+            (void)C.add(c);
+            p.cols[p.nk] = c;
+            p.pn[p.nk++] = nib(c);
+        }
+    if (W.n != live.n) return false;
+    p.g = s0.g;
+    p.d1 = d[1];
+    p.d2 = lg1 == 2 ? d[2] : 0;
+    p.o0 = s1.off[0];
+    p.pg = s0.m == 2 ? nib(s0.g) : 0;
+    p.pc = nib(s1.off[0]);
+    for (int i = 0; i < p.ni; i++) {
+        p.pd[i] = nib(p.D[i]);
+        p.lab[i] = p.D[i] ^ ((p.pd[i] & 16) ? s0.g : 0);
+    }
+    // slots read and written relative to the super-coset's base: no two super-cosets may meet on a written slot
+    std::vector<uint64_t> rd, wr;
+    for (int i = 0; i < p.ni; i++)
+        for (int q = 0; q < s0.ntq; q++) rd.push_back(p.lab[i] ^ s0.off[q]);
+    for (int c = 0; c < (p.deg ? 1 : p.mo); c++)
+        for (int j = 0; j < s1.ntq; j++) {
+            const uint64_t at = (c ? s0.g : 0) ^ s1.off[0] ^ d[j];
+            wr.push_back(at);
+            if (s1.m == 2) wr.push_back(at ^ s1.g);
+        }
+    auto clash = [&](const std::vector<uint64_t>& x, const std::vector<uint64_t>& y) {
+        for (uint64_t u : x)
+            for (uint64_t v : y)
+                if (u != v && C.has(u ^ v)) return true;
+        return false;
+    };
+    return !clash(wr, rd) && !clash(wr, wr) && !clash(rd, rd);
+}
+
+// Which sweeps the step sequence takes: single steps, or two at once where every instance that is still running has
+// the same kind of pair.  A pair saves the write and the read of the table between its steps (and a launch), so the
+// pairs are the disjoint ones that save the most.
+void choose_units(gs_batch* bt) {
+    const int ns = bt->maxns;
+    bt->unit.assign(size_t(ns), 1);
+    if (!bt->pairs_on) return;
+    constexpr double kLaunch = 40e6;                      // bytes moved in the time a launch and its reduction take
+    std::vector<double> gain(size_t(ns), -1.0), best(size_t(ns) + 2, 0.0);
+    for (int k = 0; k + 1 < ns; k++) {
+        double g = kLaunch;
+        const BPair* first = nullptr;
+        int ntq = 0;
+        bool ok = true;
+        for (size_t i = 0; i < bt->plans.size() && ok; i++) {
+            const gs::Plan& P = bt->plans[i];
+            if (k >= P.ns) continue;
+            const BPair& p = bt->hpairs[i][size_t(k)];
+            if (k + 1 >= P.ns || !p.ni) {
+                ok = false;
+            } else if (!first) {
+                first = &p;
+                ntq = P.steps[size_t(k)].ntq;
+            } else {
+                ok = p.ni == first->ni && p.mo == first->mo && p.deg == first->deg && P.steps[size_t(k)].ntq == ntq;
+            }
+            g += 2.0 * double(bt->B[i]) * double(bt->esz) * double(uint64_t(p.mo) << P.steps[size_t(k)].nk);
+        }
+        if (ok && first) gain[size_t(k)] = g;
+    }
+    for (int k = ns - 1; k >= 0; k--)
+        best[size_t(k)] = std::max(best[size_t(k) + 1], gain[size_t(k)] + best[size_t(k) + 2]);
+    for (int k = 0; k < ns; k++)
+        if (gain[size_t(k)] > 0 && gain[size_t(k)] + best[size_t(k) + 2] > best[size_t(k) + 1]) {
+            bt->unit[size_t(k)] = 2;
+            bt->unit[size_t(k) + 1] = 0;
+            k++;
+        }
+}
+
+// Cosets (or super-cosets of a pair) of instance i's sweep at step k, log2, and log2 of the step-k cosets in each.
+void sweep_size(const gs_batch* bt, size_t i, int k, int& nk, int& inner) {
+    nk = bt->plans[i].steps[size_t(k)].nk;
+    inner = 0;
+    if (bt->unit[size_t(k)] != 2) return;
+    const BPair& p = bt->hpairs[i][size_t(k)];
+    inner = p.ni == 4 ? 2 : p.ni == 2 ? 1 : 0;
+    nk = p.nk;
+}
+
+// log2 (super-)cosets per work item.  Tiles set per step index (by hand or by the autotuner, often on a larger batch)
+// are made finer, down to 2^kFinestTile cosets, while the launch has fewer than kMinItems items: one item per block,
+// and a launch of a few dozen blocks leaves the chip idle while each wave walks a long range (five width-11 plans of
+// 128 lanes: 40 blocks of 2^8 cosets took 30 us a step).  A pair's backward sums take twice the room per item, so its
+// tiles start one step coarser.
+constexpr int kFinestTile = 4;
+int item_lg(const gs_batch* bt, size_t i, int k, int shrink, bool& finer) {
+    int nk, inner;
+    sweep_size(bt, i, k, nk, inner);
+    const int floor = std::min(nk, std::max(0, kFinestTile - inner));
+    int lg = bt->lg[i][size_t(k)];
+    if (bt->unit[size_t(k)] == 2) lg = std::max(lg, bt->lg_default + 1);
+    lg = std::min(nk, std::max(lg - inner - shrink, floor));
+    finer = finer || lg > floor;
+    return lg;
+}
+
 int build_items(gs_batch* bt) {
-    for (auto* p : bt->ditems) (void)hipFree(p);
+    (void)hipFree(bt->item_mem);
+    bt->item_mem = nullptr;
+    std::vector<BItem> all;                               // the lists of every step, in one allocation
+    std::vector<size_t> at(size_t(bt->maxns), 0);
     const size_t ni = bt->plans.size();
     std::vector<int> cnt(size_t(bt->maxns) * ni, 0);
     bt->maxgroups = 1;
     for (size_t i = 0; i < ni; i++) bt->maxgroups = std::max(bt->maxgroups, bt->B[i] / kLanes);
     bt->ditems.assign(size_t(bt->maxns), nullptr);
     bt->nitems.assign(size_t(bt->maxns), 0);
+    bt->chunked.assign(size_t(bt->maxns), 0);
     bt->nq.assign(size_t(bt->maxns), 1);
     bt->nq_exact.assign(size_t(bt->maxns), 0);
+    choose_units(bt);
     for (int k = 0; k < bt->maxns; k++) {
-        // Tiles set per step index (by hand or by the autotuner, often on a larger batch) are made finer for this
-        // step, down to 2^lg_default cosets, while the step has fewer than kMinItems items: one item per block, and
-        // a launch of a few hundred blocks leaves most of the chip idle while each wave walks a long coset range.
+        if (!bt->unit[size_t(k)]) continue;
         int shrink = 0;
         for (;; shrink++) {
             int64_t tot = 0;
             bool finer = false;
-            for (size_t i = 0; i < bt->plans.size(); i++) {
-                const gs::Plan& P = bt->plans[i];
-                if (k >= P.ns) continue;
-                const int nk = P.steps[size_t(k)].nk;
-                const int lg = std::min(nk, std::max(bt->lg[i][size_t(k)] - shrink, std::min(nk, bt->lg_default)));
-                tot += int64_t(bt->B[i] / kLanes) << (nk - lg);
-                finer = finer || lg > std::min(nk, bt->lg_default);
+            for (size_t i = 0; i < ni; i++) {
+                if (k >= bt->plans[i].ns) continue;
+                int nk, inner;
+                sweep_size(bt, i, k, nk, inner);
+                tot += int64_t(bt->B[i] / kLanes) << (nk - item_lg(bt, i, k, shrink, finer));
             }
             if (tot >= kMinItems || !finer) break;
         }
         std::vector<BItem> items;
-        for (size_t i = 0; i < bt->plans.size(); i++) {
-            const gs::Plan& P = bt->plans[i];
-            if (k >= P.ns) continue;
-            const int nk = P.steps[size_t(k)].nk;
-            const int lg = std::min(nk, std::max(bt->lg[i][size_t(k)] - shrink, std::min(nk, bt->lg_default)));
+        for (size_t i = 0; i < ni; i++) {
+            if (k >= bt->plans[i].ns) continue;
+            int nk, inner;
+            bool finer = false;
+            sweep_size(bt, i, k, nk, inner);
+            const int lg = item_lg(bt, i, k, shrink, finer);
             const int count = 1 << (nk - lg);
             cnt[size_t(k) * ni + i] = count;
+            if (count > kDirectItems) bt->chunked[size_t(k)] = 1;
             const int ng = bt->B[i] / kLanes;
             for (int o = 0; o < ng * count; o++) {
                 // group-major (every coset range of lane group 0, then group 1, ...) or, with xcd_items == 2,
@@ -658,13 +1239,16 @@ int build_items(gs_batch* bt) {
             if (k < bt->plans[i].ns && bt->plans[i].steps[size_t(k)].ntq != nqk) exact = 0;
         bt->nq_exact[size_t(k)] = exact;
         bt->nitems[size_t(k)] = int(items.size());
-        void* d = nullptr;
-        if (hipMalloc(&d, std::max<size_t>(items.size() * sizeof(BItem), 16)) != hipSuccess)
-            return bfail(11, "work-item allocation failed");
-        if (hipMemcpy(d, items.data(), items.size() * sizeof(BItem), hipMemcpyHostToDevice) != hipSuccess)
-            return bfail(17, "work-item upload failed");
-        bt->ditems[size_t(k)] = static_cast<BItem*>(d);
+        at[size_t(k)] = all.size();
+        all.insert(all.end(), items.begin(), items.end());
     }
+    if (hipMalloc(&bt->item_mem, std::max<size_t>(all.size() * sizeof(BItem), 16)) != hipSuccess) {
+        bt->item_mem = nullptr;
+        return bfail(11, "work-item allocation failed");
+    }
+    if (hipMemcpy(bt->item_mem, all.data(), all.size() * sizeof(BItem), hipMemcpyHostToDevice) != hipSuccess)
+        return bfail(17, "work-item upload failed");
+    for (int k = 0; k < bt->maxns; k++) bt->ditems[size_t(k)] = static_cast<BItem*>(bt->item_mem) + at[size_t(k)];
     if (!bt->dcnt && hipMalloc(&bt->dcnt, std::max<size_t>(cnt.size() * sizeof(int), 16)) != hipSuccess) {
         bt->dcnt = nullptr;
         return bfail(11, "count table allocation failed");
@@ -674,15 +1258,15 @@ int build_items(gs_batch* bt) {
     return 0;
 }
 
-// Largest number of items any (instance, group) may have in a step at the smallest tile gs_batch_set_tile accepts
-// (2^lg_default cosets): sizes the partial buffers.
-int max_items(const gs_batch* bt, size_t i) {
-    int m = 1;
-    for (int k = 0; k < bt->plans[i].ns; k++) {
-        const int nk = bt->plans[i].steps[size_t(k)].nk;
-        m = std::max(m, 1 << (nk - std::min(nk, bt->lg_default)));
-    }
-    return m;
+// Doubles of one lane group's partials of instance i: four sums per lane of every item of a step at the smallest tile
+// gs_batch_set_tile accepts (2^lg_default cosets; a pair's eight at twice that tile), and the items of a launch that
+// was made finer (fewer than 2 kMinItems over all groups).
+size_t part_doubles(const gs_batch* bt, size_t i) {
+    size_t m = 1;
+    for (const gs::StepInfo& s : bt->plans[i].steps)
+        m = std::max(m, size_t(1) << (s.nk - std::min(s.nk, bt->lg_default)));
+    const size_t fine = 2 * size_t(kMinItems) * kLanes / size_t(bt->B[i]);
+    return kLanes * std::max(4 * m, size_t(kMaxSums) * std::max<size_t>(fine, 1));
 }
 
 // Instantiation of kernel K<S, NQ, LU, EX> for NQ in {1, 2, 4}, LU in 0..3, EX (every instance has NQ slots at the
@@ -700,6 +1284,21 @@ int max_items(const gs_batch* bt, size_t i) {
         return nullptr;                                                                                            \
     }()
 
+// Instantiation of pair kernel K<S, NQ, NI, MO, DEG> for the step's slots and the kind of pair.
+#define GS_PV(K, S, nq, ni, mo, deg)                                                                               \
+    case (nq) * 32 + (ni) * 4 + (mo) * 2 + (deg) - 2: return reinterpret_cast<const void*>(&K<S, nq, ni, mo, deg>);
+#define GS_PVN(K, S, nq)                                                                                           \
+    GS_PV(K, S, nq, 1, 1, 0) GS_PV(K, S, nq, 1, 2, 0) GS_PV(K, S, nq, 1, 2, 1)                                      \
+    GS_PV(K, S, nq, 2, 1, 0) GS_PV(K, S, nq, 2, 2, 0) GS_PV(K, S, nq, 2, 2, 1)                                      \
+    GS_PV(K, S, nq, 4, 1, 0) GS_PV(K, S, nq, 4, 2, 0)
+#define GS_PAIR_VARIANT(K, S, nq, p)                                                                               \
+    [&]() -> const void* {                                                                                         \
+        switch ((nq) * 32 + (p).ni * 4 + (p).mo * 2 + (p).deg - 2) {                                                \
+            GS_PVN(K, S, 1) GS_PVN(K, S, 2) GS_PVN(K, S, 4)                                                        \
+        }                                                                                                          \
+        return nullptr;                                                                                            \
+    }()
+
 enum BKernel { kBStep, kBRestore, kBBack };
 
 template <class S>
@@ -708,7 +1307,14 @@ int launch_batch(gs_batch* bt, BKernel kind, int k, BLaunch L) {
     if (n == 0) return 0;
     const int nq = bt->nq[size_t(k)], lu = bt->lu;
     const bool ex = bt->nq_exact[size_t(k)] != 0;
-    const void* fn = kind == kBStep ? GS_BATCH_VARIANT(batch_step_kernel, S, nq, lu, ex)
+    const BPair* pair = nullptr;
+    if (bt->unit[size_t(k)] == 2)
+        for (size_t i = 0; i < bt->plans.size() && !pair; i++)
+            if (k < bt->plans[i].ns) pair = &bt->hpairs[i][size_t(k)];
+    const void* fn = pair ? (kind == kBStep ? GS_PAIR_VARIANT(pair_step_kernel, S, nq, *pair)
+                             : kind == kBRestore ? GS_PAIR_VARIANT(pair_restore_kernel, S, nq, *pair)
+                                                 : GS_PAIR_VARIANT(pair_back_kernel, S, nq, *pair))
+                   : kind == kBStep ? GS_BATCH_VARIANT(batch_step_kernel, S, nq, lu, ex)
                    : kind == kBRestore ? GS_BATCH_VARIANT(batch_restore_kernel, S, nq, lu, ex)
                                        : GS_BATCH_VARIANT(batch_back_kernel, S, nq, lu, ex);
     if (!fn) return bfail(16, "no kernel variant");
@@ -719,20 +1325,29 @@ int launch_batch(gs_batch* bt, BKernel kind, int k, BLaunch L) {
                                                                                       : bfail(17, "step launch failed");
 }
 
-// Per-(instance, lane) reduction of step k's item partials: mode 0 chain bookkeeping, mode 1 gradient entry.
-int launch_reduce(gs_batch* bt, int k, int mode) {
-    if (bt->nitems[size_t(k)] == 0) return 0;
-    hipLaunchKernelGGL(batch_chunk_kernel, dim3(bt->maxgroups * kRChunks, int(bt->plans.size())), dim3(kBThreads), 0,
-                       bt->stream, bt->dinst, bt->dcnt + size_t(k) * bt->plans.size(), mode);
-    hipLaunchKernelGGL(batch_reduce_kernel, dim3(bt->maxgroups, int(bt->plans.size())), dim3(kLanes), 0, bt->stream,
-                       bt->dinst, bt->dcnt + size_t(k) * bt->plans.size(), k, mode);
+// Per-(instance, lane) reduction of the item partials of the sweep at step k: chain bookkeeping or gradient entries.
+template <int STEPS, bool GRAD>
+int launch_reduce_t(gs_batch* bt, int k) {
+    const int* cnt = bt->dcnt + size_t(k) * bt->plans.size();
+    const int ninst = int(bt->plans.size());
+    if (bt->chunked[size_t(k)])
+        hipLaunchKernelGGL((batch_chunk_kernel<STEPS * (GRAD ? 4 : 1)>), dim3(bt->maxgroups * kRChunks, ninst),
+                           dim3(kBThreads), 0, bt->stream, bt->dinst, cnt);
+    hipLaunchKernelGGL((batch_reduce_kernel<STEPS, GRAD>), dim3(bt->maxgroups, ninst), dim3(kLanes * kRWaves), 0,
+                       bt->stream, bt->dinst, cnt, k);
     return hipGetLastError() == hipSuccess ? 0 : bfail(17, "reduce launch failed");
+}
+
+int launch_reduce(gs_batch* bt, int k, bool grad) {
+    if (bt->nitems[size_t(k)] == 0) return 0;
+    if (bt->unit[size_t(k)] == 2) return grad ? launch_reduce_t<2, true>(bt, k) : launch_reduce_t<2, false>(bt, k);
+    return grad ? launch_reduce_t<1, true>(bt, k) : launch_reduce_t<1, false>(bt, k);
 }
 
 template <class S>
 int launch_step(gs_batch* bt, int k, int bookkeeping, void* const* copy) {
     if (int rc = launch_batch<S>(bt, kBStep, k, BLaunch{k, bookkeeping, copy})) return rc;
-    return bookkeeping ? launch_reduce(bt, k, 0) : 0;
+    return bookkeeping ? launch_reduce(bt, k, false) : 0;
 }
 
 template <class S>
@@ -740,6 +1355,7 @@ int enqueue_t(gs_batch* bt, bool record_steps) {
     const int ninst = int(bt->plans.size());
     hipLaunchKernelGGL(batch_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
     for (int k = 0; k < bt->maxns; k++) {
+        if (!bt->unit[size_t(k)]) continue;               // the second step of a pair
         if (int rc = launch_step<S>(bt, k, 1, nullptr)) return rc;
         if (record_steps && bt->nitems[size_t(k)] && hipEventRecord(bt->step_ev[size_t(k)], bt->stream) != hipSuccess)
             return bfail(17, "event record failed");
@@ -803,6 +1419,15 @@ void free_grad(gs_batch* bt) {
     bt->seg = 0;
 }
 
+// First step of segment s's sweeps: its sweeps are those that start in steps s seg .. (s + 1) seg - 1, so a pair that
+// straddles the boundary belongs to the earlier segment (the pairs, and with them the order of every sum, do not
+// depend on seg).
+int seg_first(const gs_batch* bt, int seg, int s) {
+    int k = std::min(s * seg, bt->maxns);
+    while (k < bt->maxns && !bt->unit[size_t(k)]) k++;
+    return k;
+}
+
 // Allocate the adjoint arenas and the copies for segments of `seg` steps.
 int alloc_grad(gs_batch* bt, int seg) {
     free_grad(bt);
@@ -826,8 +1451,8 @@ int alloc_grad(gs_batch* bt, int seg) {
     bt->stack.assign(size_t(seg), std::vector<void*>(ni, nullptr));
     for (int sgi = 0; sgi < nseg; sgi++)
         for (size_t i = 0; i < ni; i++) {
-            const int k = sgi * seg;
-            if (k >= bt->plans[i].ns) continue;
+            const int k = seg_first(bt, seg, sgi);
+            if (k >= bt->plans[i].ns || k >= (sgi + 1) * seg) continue;
             if (!(bt->ckpt[size_t(sgi)][i] = galloc(copy_entries(bt, i, k) * bt->esz))) return bfail(11, "checkpoint allocation failed");
         }
     for (int j = 0; j < seg; j++)
@@ -835,7 +1460,7 @@ int alloc_grad(gs_batch* bt, int seg) {
             size_t mx = 0;
             for (int sgi = 0; sgi < nseg; sgi++) {
                 const int k = sgi * seg + j;
-                if (k < bt->plans[i].ns) mx = std::max(mx, copy_entries(bt, i, k));
+                if (k < bt->plans[i].ns && bt->unit[size_t(k)]) mx = std::max(mx, copy_entries(bt, i, k));
             }
             if (mx && !(bt->stack[size_t(j)][i] = galloc(mx * bt->esz))) return bfail(11, "segment stack allocation failed");
         }
@@ -850,12 +1475,15 @@ size_t grad_bytes(const gs_batch* bt, int seg) {
     size_t tot = 0;
     const int nseg = (bt->maxns + seg - 1) / seg;
     for (size_t i = 0; i < bt->plans.size(); i++) {
-        for (int sgi = 0; sgi < nseg; sgi++)
-            if (sgi * seg < bt->plans[i].ns) tot += copy_entries(bt, i, sgi * seg);
+        for (int sgi = 0; sgi < nseg; sgi++) {
+            const int k = seg_first(bt, seg, sgi);
+            if (k < bt->plans[i].ns && k < (sgi + 1) * seg) tot += copy_entries(bt, i, k);
+        }
         for (int j = 0; j < seg; j++) {
             size_t mx = 0;
             for (int sgi = 0; sgi < nseg; sgi++)
-                if (sgi * seg + j < bt->plans[i].ns) mx = std::max(mx, copy_entries(bt, i, sgi * seg + j));
+                if (sgi * seg + j < bt->plans[i].ns && bt->unit[size_t(sgi * seg + j)])
+                    mx = std::max(mx, copy_entries(bt, i, sgi * seg + j));
             tot += mx;
         }
     }
@@ -908,7 +1536,8 @@ int grad_t(gs_batch* bt) {
     for (int k = 0; k < ns; k++)
         for (int i = 0; i < ninst; i++)
             host[size_t(k) * ninst + i] = k / seg == last ? bt->stack[size_t(k - last * seg)][size_t(i)]
-                                        : (k % seg == 0 ? bt->ckpt[size_t(k / seg)][size_t(i)] : nullptr);
+                                        : (k == seg_first(bt, seg, k / seg) ? bt->ckpt[size_t(k / seg)][size_t(i)]
+                                                                            : nullptr);
     for (int j = 0; j < seg; j++)
         for (int i = 0; i < ninst; i++) host[size_t(ns + j) * ninst + i] = bt->stack[size_t(j)][size_t(i)];
     for (int s = 0; s < nseg; s++)
@@ -920,20 +1549,24 @@ int grad_t(gs_batch* bt) {
     (void)hipEventRecord(e0, bt->stream);
     hipLaunchKernelGGL(batch_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
     for (int k = 0; k < ns; k++)
-        if (int rc = launch_step<S>(bt, k, 1, fwd_ptr(k))) return rc;
+        if (bt->unit[size_t(k)])
+            if (int rc = launch_step<S>(bt, k, 1, fwd_ptr(k))) return rc;
     hipLaunchKernelGGL(batch_finish_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
     (void)hipEventRecord(em, bt->stream);
     hipLaunchKernelGGL(batch_lambda_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
     for (int s = last; s >= 0; s--) {
         const int k0 = s * seg, k1 = std::min(ns, k0 + seg);
-        if (s != last) {                                    // recompute the segment from its checkpoint
-            if (int rc = launch_batch<S>(bt, kBRestore, k0, BLaunch{k0, 0, ck_ptr(s)})) return rc;
-            for (int k = k0; k < k1; k++)
-                if (int rc = launch_step<S>(bt, k, 0, rec_ptr(k - k0))) return rc;
+        const int kf = seg_first(bt, seg, s);
+        if (s != last && kf < k1) {                         // recompute the segment from its checkpoint
+            if (int rc = launch_batch<S>(bt, kBRestore, kf, BLaunch{kf, 0, ck_ptr(s)})) return rc;
+            for (int k = kf; k < k1; k++)
+                if (bt->unit[size_t(k)])
+                    if (int rc = launch_step<S>(bt, k, 0, rec_ptr(k - k0))) return rc;
         }
-        for (int k = k1 - 1; k >= k0; k--) {
+        for (int k = k1 - 1; k >= kf; k--) {
+            if (!bt->unit[size_t(k)]) continue;
             if (int rc = launch_batch<S>(bt, kBBack, k, BLaunch{k, 0, rec_ptr(k - k0)})) return rc;
-            if (int rc = launch_reduce(bt, k, 1)) return rc;
+            if (int rc = launch_reduce(bt, k, true)) return rc;
         }
     }
     (void)hipEventRecord(e1, bt->stream);
@@ -966,7 +1599,7 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
     bt->lu = storage == GS_C64 ? 2 : 1;
     auto bail = [&](int rc) {
         for (void* p : bt->allocs) (void)hipFree(p);
-        for (auto* p : bt->ditems) (void)hipFree(p);
+        (void)hipFree(bt->item_mem);
         delete bt;
         return rc;
     };
@@ -1004,6 +1637,9 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
                 s.tau0[j] = si.tau0[j];
                 s.tau1[j] = si.tau1[j];
                 s.par[j] = si.par[j];
+                s.t0m |= uint32_t(si.tau0[j] & 1) << j;
+                s.t1m |= uint32_t(si.tau1[j] & 1) << j;
+                s.parm |= uint32_t(si.par[j] & 1) << j;
             }
             s.g = si.g;
             s.rhoc = si.rhoc;
@@ -1016,21 +1652,41 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
             s.ntq = si.ntq;
             s.m = si.m;
         }
-        BStep* ds = dalloc<BStep>(bt, hs.size());
-        if (!ds || hipMemcpy(ds, hs.data(), hs.size() * sizeof(BStep), hipMemcpyHostToDevice) != hipSuccess)
+        std::vector<BPair> hp(size_t(P.ns));
+        for (int k = 0; k < P.ns; k++)
+            if (k + 1 >= P.ns || !make_pair(P.steps[size_t(k)], P.steps[size_t(k) + 1], hp[size_t(k)])) hp[size_t(k)].ni = 0;
+        // the instance's small buffers in one allocation: descriptors first, uploaded in one copy
+        size_t used = 0;
+        auto take = [&](size_t bytes) {
+            const size_t at = used;
+            used += (bytes + 255) & ~size_t(255);
+            return at;
+        };
+        const size_t o_steps = take(hs.size() * sizeof(BStep)), o_pairs = take(hp.size() * sizeof(BPair)), head = used;
+        const size_t o_bits = take(size_t(P.ns) * B), o_prev = take(sizeof(double) * B), o_dead = take(sizeof(int) * B),
+                     o_cond = take(sizeof(double) * size_t(B) * P.ns), o_logp = take(sizeof(double) * B),
+                     o_amp = take(sizeof(double) * 2 * B),
+                     o_cpart = take(sizeof(double) * size_t(B / kLanes) * kRChunks * kLanes * kMaxSums),
+                     o_part = take(sizeof(double) * size_t(B / kLanes) * part_doubles(bt, size_t(i)));
+        char* mem = dalloc<char>(bt, used);
+        if (!mem) return bail(bfail(11, "batch buffer allocation failed"));
+        std::vector<char> up(head);
+        if (!hs.empty()) memcpy(up.data() + o_steps, hs.data(), hs.size() * sizeof(BStep));
+        if (!hp.empty()) memcpy(up.data() + o_pairs, hp.data(), hp.size() * sizeof(BPair));
+        if (head && hipMemcpy(mem, up.data(), head, hipMemcpyHostToDevice) != hipSuccess)
             return bail(bfail(17, "plan upload failed"));
-        bt->hsteps.push_back(hs);
-        I.steps = ds;
-        I.bitsT = dalloc<int8_t>(bt, size_t(P.ns) * B);
-        I.prev = dalloc<double>(bt, size_t(B));
-        I.dead = dalloc<int>(bt, size_t(B));
-        I.cond = dalloc<double>(bt, size_t(B) * P.ns);
-        I.logp = dalloc<double>(bt, size_t(B));
-        I.amp = dalloc<double>(bt, size_t(B) * 2);
-        I.part = dalloc<double>(bt, size_t(B / kLanes) * size_t(max_items(bt, size_t(i))) * kLanes * 4);
-        I.cpart = dalloc<double>(bt, size_t(B / kLanes) * kRChunks * kLanes * 4);
-        if (!I.bitsT || !I.prev || !I.dead || !I.cond || !I.logp || !I.amp || !I.part || !I.cpart)
-            return bail(bfail(11, "batch buffer allocation failed"));
+        bt->hsteps.push_back(std::move(hs));
+        bt->hpairs.push_back(std::move(hp));
+        I.steps = reinterpret_cast<BStep*>(mem + o_steps);
+        I.pairs = reinterpret_cast<BPair*>(mem + o_pairs);
+        I.bitsT = reinterpret_cast<int8_t*>(mem + o_bits);
+        I.prev = reinterpret_cast<double*>(mem + o_prev);
+        I.dead = reinterpret_cast<int*>(mem + o_dead);
+        I.cond = reinterpret_cast<double*>(mem + o_cond);
+        I.logp = reinterpret_cast<double*>(mem + o_logp);
+        I.amp = reinterpret_cast<double*>(mem + o_amp);
+        I.cpart = reinterpret_cast<double*>(mem + o_cpart);
+        I.part = reinterpret_cast<double*>(mem + o_part);
         bt->hinst.push_back(I);
     }
     bt->dinst = dalloc<BInst>(bt, bt->hinst.size());
@@ -1051,7 +1707,7 @@ void gs_batch_destroy(gs_batch* bt) {
     drop_graph(bt);
     free_grad(bt);
     for (void* p : bt->allocs) (void)hipFree(p);
-    for (auto* p : bt->ditems) (void)hipFree(p);
+    (void)hipFree(bt->item_mem);
     (void)hipFree(bt->dcnt);
     for (auto& ev : bt->step_ev) (void)hipEventDestroy(ev);
     (void)hipEventDestroy(bt->ev0);
@@ -1095,6 +1751,19 @@ int gs_batch_set_unroll(gs_batch* bt, int lu) {
     if (!bt || lu < 0 || lu > 3) return bfail(16, "unroll must be 0..3");
     bt->lu = lu;
     drop_graph(bt);
+    return 0;
+}
+
+// Two consecutive steps per sweep where the plans allow it (on, default) or one (off); the results differ at most by
+// the order of FP64 sums.  A gradient's copies are laid out anew by its next call.
+int gs_batch_set_pairs(gs_batch* bt, int on) {
+    if (!bt) return bfail(16, "null batch");
+    bt->pairs_on = on != 0;
+    drop_graph(bt);
+    (void)hipSetDevice(bt->device);
+    (void)hipStreamSynchronize(bt->stream);
+    free_grad(bt);
+    bt->items_dirty = true;
     return 0;
 }
 
@@ -1152,6 +1821,7 @@ int gs_batch_score(gs_batch* bt, const int8_t* const* bits, double* const* log2p
             float t = 0;
             if (bt->nitems[size_t(k)] && hipEventElapsedTime(&t, bt->ev0, bt->step_ev[size_t(k)]) == hipSuccess)
                 bt->step_ms[size_t(k)] = t;
+            else if (k > 0 && !bt->unit[size_t(k)]) bt->step_ms[size_t(k)] = bt->step_ms[size_t(k) - 1];   // pair
         }
     for (size_t i = 0; i < bt->plans.size(); i++) {
         const BInst& I = bt->hinst[i];

@@ -22,7 +22,7 @@ ABI_SYMBOLS = ("gs_plan_load", "gs_plan_parse", "gs_plan_info", "gs_plan_destroy
                "gs_engine_destroy", "gs_prob", "gs_chain", "gs_sample", "gs_hybrid", "gs_prefix", "gs_resume",
                "gs_last_device_ms", "gs_last_error", "gs_profile_enable", "gs_profile_read",
                "gs_step_geometry", "gs_step_columns", "gs_set_fusion", "gs_set_fused4", "gs_set_grid_log2", "gs_set_grid_log2_one_slot", "gs_set_small_steps", "gs_set_walk", "gs_set_xcd_blocks", "gs_set_plain_pairs", "gs_set_fused_run", "gs_set_diag_runs", "gs_step_run", "gs_set_fold_reduce", "gs_race_check", "gs_copy_probe", "gs_batch_create", "gs_batch_destroy", "gs_batch_score",
-               "gs_batch_use_graph", "gs_batch_set_tile", "gs_batch_set_unroll", "gs_batch_set_xcd_items", "gs_batch_last_ms", "gs_batch_last_error",
+               "gs_batch_use_graph", "gs_batch_set_tile", "gs_batch_set_unroll", "gs_batch_set_xcd_items", "gs_batch_set_pairs", "gs_batch_last_ms", "gs_batch_last_error",
                "gs_batch_set_matrices", "gs_batch_grad", "gs_batch_grad_ms", "gs_tt_plan_load", "gs_tt_plan_info",
                "gs_tt_plan_destroy", "gs_tt_engine_create", "gs_tt_engine_destroy", "gs_tt_prob", "gs_tt_chain",
                "gs_tt_sample", "gs_tt_hybrid", "gs_tt_prefix", "gs_tt_resume", "gs_tt_dp", "gs_tt_last_error", "gs_tt_set_grid_log2",
@@ -98,6 +98,7 @@ def library():
         "gs_batch_set_tile": (I, [P, I, I, I]),
         "gs_batch_set_xcd_items": (I, [P, I]),
         "gs_batch_set_unroll": (I, [P, I]),
+        "gs_batch_set_pairs": (I, [P, I]),
         "gs_tt_plan_load": (I, [ctypes.c_char_p, I, pp]),
         "gs_tt_plan_info": (I, [P, ip, ip, ip]),
         "gs_tt_set_grid_log2": (I, [P, I]),
@@ -466,6 +467,10 @@ class BatchEngine:
     def set_unroll(self, lu):
         """log2 cosets each lane gathers at once (0..3)."""
         self._check(library().gs_batch_set_unroll(self._h, int(lu)))
+
+    def set_pairs(self, on):
+        """Two consecutive steps per sweep where the plans allow it (True, default) or one."""
+        self._check(library().gs_batch_set_pairs(self._h, 1 if on else 0))
 
     def score(self, bits, want_cond=True, want_amp=True):
         """bits: list (per plan) of int8 [lanes_i, ns_i].  Returns lists of log2p [lanes_i], cond [lanes_i, ns_i],
