@@ -75,6 +75,19 @@ struct KStep {
     int sgg, sgk;          // kWriteGram1: next step's sign parity of g, and its constant (pmask[2]: per coordinate)
 };
 
+// Runs of small steps (gs_small.hip): one block of kSmallThreads per string, the slots a run touches in LDS.
+constexpr int kSmallThreads = 512;
+constexpr int kSmallMaxNk = 12;     // cosets of a step, log2
+constexpr int kSmallSteps = 64;     // steps of a run
+struct SStep {
+    uint32_t cols[kSmallMaxNk];     // LDS index of each coset coordinate's column (0 beyond nk), as the plain descriptor's
+    uint32_t off[4], g;             // of the coset offsets (beyond ntq: the first again) and of g
+    uint32_t rho;                   // sign mask over the coordinates
+    uint32_t route;                 // a bit per offset: output of its x = 0 term | of its x = 1 term << 4 | its par << 8
+    int nk, ntq, m, growth, pad;
+    double mre[2][2], mim[2][2];
+};
+
 // One step of the two-table (gather-form) engine as its kernels see it: output cp of the new table gathers the inputs
 // u = pdep(cp, pivmask) ^ kspan[t] of the old one (c = u & lowmask, x = the bit r of u).  pdep is linear in cp:
 // output coordinate j goes to the physical bit dep[j].

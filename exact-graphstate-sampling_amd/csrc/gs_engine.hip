@@ -25,6 +25,7 @@
 
 #include "../../include/gsamp_amd.h"
 #include "gs_device.h"
+#include "gs_gf2.h"
 #include "gs_plan.h"
 
 namespace gs {
@@ -35,7 +36,7 @@ void* decide_kernel_ptr();
 void* publish_kernel_ptr();
 void* reduce_kernel_ptr(int sweep);
 void* small_run_kernel_ptr(int storage);
-int small_run_threads();
+size_t small_run_lds(size_t tab_bytes);
 void* reduce1_kernel_ptr();
 void* run_hist_kernel_ptr(int storage);
 void* run_apply_kernel_ptr(int storage);
@@ -340,7 +341,12 @@ struct gs_engine {
     int grid_cap = kDefaultGridLog2;  // log2 of the most blocks a sweep launches
     int grid_cap1 = kDefaultGridLog2One;  // ... a plain sweep of a one-slot step
     int grid_cap1_big = kDefaultGridLog2OneBig;  // ... of a one-slot step with at least 2^kBigStepLog2 cosets
-    int small_nk = 10;              // runs of steps with nk <= small_nk go to one single-block launch (-1: never)
+    // runs of small steps (gs_small.hip): descriptors, the run each step belongs to (-1: none), log2 slots of each run
+    int small_nk = 10;              // steps with at most 2^small_nk cosets (-1: no runs)
+    std::vector<SStep> hsmall;
+    std::vector<int> small_at, small_dim;
+    SStep* dsmall = nullptr;
+    bool fresh = false;             // the next launch starts the strings' chains
     int walk = 0;                   // tile order: 0 forward, 1 reverse on odd steps, 2 reverse on every step
     int fused_run = -1;             // log2 run of the fused layout (-1: the storage's default)
     int xcd_blocks = 1;             // XCD-contiguous block coordinates in every sweep
@@ -424,7 +430,10 @@ int flush_pending(gs_engine* e) {
     return 0;
 }
 
+int launch_init(gs_engine* e);
+
 int launch_sweep(gs_engine* e, int k, int sweep, const Epi& epi) {
+    if (int rc = launch_init(e)) return rc;
     const auto& L = e->launch[size_t(k)];
     void* fn = sweep == kGram ? L.gram : sweep == kDirect ? L.direct : sweep == kWrite ? L.write
              : sweep == kWriteGram ? L.wgram : L.wdirect;
@@ -494,7 +503,9 @@ int collect_profile(gs_engine* e) {
     return 0;
 }
 
-int launch_small(gs_engine* e, void* fn, Epi epi, int k) {
+// A kernel of one thread per string: the decision of step k, or the string's outputs (k = -1).
+int launch_single(gs_engine* e, void* fn, Epi epi, int k) {
+    if (int rc = launch_init(e)) return rc;
     if (int rc = flush_pending(e)) return rc;
     Ctl* ctl = e->ctl;
     if (k >= 0) {
@@ -507,7 +518,16 @@ int launch_small(gs_engine* e, void* fn, Epi epi, int k) {
     return 0;
 }
 
+// The strings' chains start with the next launch: a run of small steps starts them itself, anything else is preceded
+// by a launch that does.
+int start_chain(gs_engine* e) {
+    e->fresh = true;
+    return 0;
+}
+
 int launch_init(gs_engine* e) {
+    if (!e->fresh) return 0;
+    e->fresh = false;
     Ctl* ctl = e->ctl;
     if (e->storage == GS_C64) {
         float2* mem = static_cast<float2*>(arena_of(e));
@@ -530,6 +550,7 @@ int run_from(const gs_engine* e, int k, int k1) {
 // A run of diagonal steps: pattern sums (one pass), their reduction, the run's decisions and bookkeeping (one block),
 // the product pass; its stored norm goes to the chain state.
 int launch_run(gs_engine* e, int ri, const Epi& base, bool gram) {
+    if (int rc = launch_init(e)) return rc;
     if (int rc = flush_pending(e)) return rc;
     const RStep& rs = e->hrun[size_t(ri)];
     const RStep* rp = e->drun + ri;
@@ -588,7 +609,7 @@ int launch_run(gs_engine* e, int ri, const Epi& base, bool gram) {
             return 0;
         }))
         return rc;
-    if (nblk > unsigned(kFenceBlocks)) {
+    if (!reduces_in_kernel(nblk, 1)) {
         const double* cpart = part;
         int sw = kWrite;
         void* rargs[] = {&cpart, &nblk, &ctl, &ea, &sw};
@@ -627,13 +648,13 @@ int enqueue_run(gs_engine* e, int mode, int k0, int k1, const int8_t* forced_h, 
     base.plain = e->dplain;
     base.slot_entries = slot_entries(e);
     base.slot_part = slot_part_doubles(e);
-    if (k0 == k1) return launch_small(e, publish_kernel_ptr(), base, -1);
+    if (k0 == k1) return launch_single(e, publish_kernel_ptr(), base, -1);
     const bool fstr = forced_h != nullptr && mode == kChain;
     auto fb = [&](int k) { return forced_h ? int(forced_h[k]) : -1; };
     bool decided = false;
     for (int k = k0; k < k1; k++) {
         int ke = k;                                       // a run of two or more small steps: one launch
-        while (e->small_nk >= 0 && ke < k1 && e->hplain[size_t(ke)].nk <= e->small_nk) ke++;
+        while (ke < k1 && e->small_at[size_t(ke)] >= 0 && e->small_at[size_t(ke)] == e->small_at[size_t(k)]) ke++;
         if (const int ri = run_from(e, k, k1); ri >= 0) {   // a run of diagonal steps decides its own steps
             const RStep& rs = e->hrun[size_t(ri)];
             const int kn = rs.k0 + rs.j;            // a paired run's product pass can also decide the next step
@@ -645,14 +666,17 @@ int enqueue_run(gs_engine* e, int mode, int k0, int k1, const int8_t* forced_h, 
         }
         if (ke - k >= 2) {
             if (int rc = flush_pending(e)) return rc;
+            const SStep* ss = e->dsmall;
             const KStep* sp = e->dplain;
             void* mem = arena_of(e);
             Ctl* ctl = e->ctl;
             Epi ep = base;
-            int a = k, b = ke, d = decided ? 1 : 0;
-            void* args[] = {&sp, &mem, &ctl, &ep, &a, &b, &d};
-            HIP_TRY(hipLaunchKernel(small_run_kernel_ptr(e->storage), dim3(1, e->strings), dim3(small_run_threads()),
-                                    args, 0, e->stream));
+            int a = k, b = ke, d = decided ? 1 : 0, start = e->fresh ? 1 : 0;
+            int tab = int(std::max<size_t>(16, e->esz << e->small_dim[size_t(e->small_at[size_t(k)])]));
+            void* args[] = {&ss, &sp, &mem, &ctl, &ep, &a, &b, &d, &start, &tab};
+            HIP_TRY(hipLaunchKernel(small_run_kernel_ptr(e->storage), dim3(1, e->strings), dim3(kSmallThreads), args,
+                                    small_run_lds(size_t(tab)), e->stream));
+            e->fresh = false;
             decided = false;
             k = ke - 1;
             continue;
@@ -665,7 +689,7 @@ int enqueue_run(gs_engine* e, int mode, int k0, int k1, const int8_t* forced_h, 
                 ep.role = kRoleNorm;
                 if (int rc = launch_sweep(e, k, nm, ep)) return rc;
             } else {
-                if (int rc = launch_small(e, decide_kernel_ptr(), base, k)) return rc;
+                if (int rc = launch_single(e, decide_kernel_ptr(), base, k)) return rc;
             }
         }
         Epi ep = base;
@@ -1194,6 +1218,90 @@ void build_runs(gs_engine* e) {
     }
 }
 
+// Runs of small steps: consecutive steps of at most 2^small_nk cosets (2^kSmallMaxNk at most) whose slots together span
+// a subspace that fits the LDS.  A slot's index is its bits at the pivots of the subspace's reduced basis (pivots the
+// lowest set bits, so the unit bits of the arena stay the low bits of the index).
+void build_small(gs_engine* e) {
+    const Plan& P = e->plan;
+    e->hsmall.assign(size_t(std::max(P.ns, 1)), SStep{});
+    e->small_at.assign(size_t(std::max(P.ns, 1)), -1);
+    e->small_dim.clear();
+    const size_t room = size_t(64) << 10;                 // bytes of table
+    const int lim = std::min(e->small_nk, kSmallMaxNk);
+    auto slots_of = [](const KStep& s) {
+        std::vector<uint64_t> v(s.cols, s.cols + s.nk);
+        v.insert(v.end(), s.off, s.off + s.ntq);
+        if (s.m == 2) v.push_back(s.g);
+        return v;
+    };
+    for (int k = 0; k < P.ns;) {
+        if (e->hplain[size_t(k)].nk > lim) {
+            k++;
+            continue;
+        }
+        GfBasis span;
+        int end = k;
+        while (end < P.ns && e->hplain[size_t(end)].nk <= lim && end - k < kSmallSteps) {
+            GfBasis next = span;
+            for (uint64_t v : slots_of(e->hplain[size_t(end)])) (void)next.add(v);
+            if ((e->esz << next.n) > room) break;
+            span = next;
+            end++;
+        }
+        if (end == k) {                                   // a single step that does not fit
+            k++;
+            continue;
+        }
+        // fully reduced basis with the lowest set bits as pivots
+        std::vector<uint64_t> rows;
+        for (int b = 0; b < 64; b++)
+            if (span.row[b]) rows.push_back(span.row[b]);
+        std::vector<int> piv;
+        for (size_t r = 0; r < rows.size();) {
+            int low = 64;
+            size_t at = r;
+            for (size_t i = r; i < rows.size(); i++)
+                if (__builtin_ctzll(rows[i]) < low) {
+                    low = __builtin_ctzll(rows[i]);
+                    at = i;
+                }
+            std::swap(rows[r], rows[at]);
+            for (size_t i = 0; i < rows.size(); i++)
+                if (i != r && ((rows[i] >> low) & 1)) rows[i] ^= rows[r];
+            piv.push_back(low);
+            r++;
+        }
+        auto index_of = [&](uint64_t x) {
+            uint32_t i = 0;
+            for (size_t r = 0; r < piv.size(); r++) i |= uint32_t((x >> piv[r]) & 1) << r;
+            return i;
+        };
+        for (int q = k; q < end; q++) {
+            const KStep& s = e->hplain[size_t(q)];
+            SStep& d = e->hsmall[size_t(q)];
+            for (int j = 0; j < s.nk; j++) d.cols[j] = index_of(s.cols[j]);
+            for (int j = 0; j < 4; j++) d.off[j] = index_of(s.off[j < s.ntq ? j : 0]);
+            d.g = s.m == 2 ? index_of(s.g) : 0;
+            d.rho = uint32_t(s.pmask[0]);
+            d.nk = s.nk;
+            d.ntq = s.ntq;
+            d.m = s.m;
+            d.growth = s.growth;
+            for (int j = 0; j < s.ntq; j++) {             // the canonical routes (see Route)
+                const int t0 = s.route == kRouteMixA || s.route == kRouteMixB ? j & 1 : 0;
+                const int t1 = s.route == kRoute1 ? 0 : s.route == kRouteSplit ? 1 : s.route == kRouteMixA ? 1 - (j & 1)
+                                                                                                        : (j & 1);
+                d.route |= uint32_t(t0) << j | uint32_t(t1) << (4 + j) | ((s.parmask >> j) & 1) << (8 + j);
+            }
+            memcpy(d.mre, s.mre, sizeof d.mre);
+            memcpy(d.mim, s.mim, sizeof d.mim);
+            e->small_at[size_t(q)] = int(e->small_dim.size());
+        }
+        e->small_dim.push_back(span.n);
+        k = end;
+    }
+}
+
 int build_steps(gs_engine* e) {
     const Plan& P = e->plan;
     e->hplain.assign(size_t(P.ns), KStep{});
@@ -1283,6 +1391,7 @@ int build_steps(gs_engine* e) {
         e->fusable[size_t(k)] = 1;
     }
     build_runs(e);
+    build_small(e);
     return 0;
 }
 
@@ -1293,6 +1402,7 @@ int upload_descriptors(gs_engine* e, bool logical) {
     if (ns) {
         HIP_TRY(hipMemcpy(e->dplain, e->hplain.data(), sizeof(KStep) * ns, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(e->dfused, e->hfused.data(), sizeof(KStep) * ns, hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(e->dsmall, e->hsmall.data(), sizeof(SStep) * ns, hipMemcpyHostToDevice));
         if (logical) HIP_TRY(hipMemcpy(e->dlogical, e->hlogical.data(), sizeof(KStep) * ns, hipMemcpyHostToDevice));
     }
     if (e->hrun.empty()) return 0;
@@ -1322,6 +1432,7 @@ void free_engine(gs_engine* e) {
     (void)hipFree(e->dplain);
     (void)hipFree(e->dfused);
     (void)hipFree(e->dlogical);
+    (void)hipFree(e->dsmall);
     (void)hipFree(e->part_buf[0]);
     (void)hipFree(e->slots);
     (void)hipFree(e->counter);
@@ -1410,7 +1521,7 @@ int enqueue_strings(gs_engine* e, int mode, int cnt, bool forced, bool amp) {
     for (int i = 0; i < cnt && !rc; i += e->strings) {
         e->strings = 1;
         while (e->strings < most && i + e->strings < cnt && (mode != kRun || alike(i, i + e->strings))) e->strings++;
-        if ((rc = launch_init(e))) break;
+        if ((rc = start_chain(e))) break;
         const size_t at = size_t(i) * ns;
         if ((rc = enqueue_run(e, mode, 0, ns, forced ? e->h_forced + at : nullptr, forced ? e->d_forced + at : nullptr,
                               e->d_U + at, e->d_bits + at, e->d_cond + at, e->d_out + size_t(i) * 4)))
@@ -1532,6 +1643,7 @@ int gs_engine_create(const gs_plan* plan, int storage, int device, gs_engine** o
     const size_t nsz = size_t(std::max(ns, 1));
     bool ok = dev_alloc((void**)&e->dplain, sizeof(KStep) * nsz) && dev_alloc((void**)&e->dfused, sizeof(KStep) * nsz) &&
               dev_alloc((void**)&e->dlogical, sizeof(KStep) * nsz) &&
+              dev_alloc((void**)&e->dsmall, sizeof(SStep) * nsz) &&
               dev_alloc((void**)&e->part_buf[0], 2 * sizeof(double) * kPartDoubles) &&
               dev_alloc((void**)&e->counter, sizeof(unsigned) * kCounters) &&
               dev_alloc((void**)&e->ctl_base, 2 * C * sizeof(Ctl)) && dev_alloc((void**)&e->d_forced, C * nsz) &&
@@ -1659,7 +1771,7 @@ int gs_prefix(gs_engine* eng, const int8_t* bits, int K, double* table_reim, int
     for (int k = K; k < ns; k++) e->h_forced[k] = 0;
     HIP_TRY(hipMemcpyAsync(e->d_forced, e->h_forced, size_t(ns), hipMemcpyHostToDevice, e->stream));
     if (int rc = begin_timing(e)) return rc;
-    if (int rc = launch_init(e)) return rc;
+    if (int rc = start_chain(e)) return rc;
     if (int rc = enqueue_run(e, kRun, 0, K, e->h_forced, e->d_forced, e->d_U, e->d_bits, e->d_cond, e->d_out)) return rc;
     if (int rc = end_timing(e)) return rc;
     void* doffs = nullptr;
@@ -1784,6 +1896,7 @@ int gs_resume(gs_engine* eng, const int8_t* bits, int K, int nslices, const doub
             rc = fail(17, "resume upload failed");
             break;
         }
+        e->fresh = false;
         hipLaunchKernelGGL(init_ctl_kernel, dim3(1), dim3(1), 0, e->stream, e->ctl, norm, L);
         if ((rc = begin_timing(e))) break;
         if ((rc = enqueue_run(e, kRun, K, ns, e->h_forced, e->d_forced, e->d_U, e->d_bits, e->d_cond, e->d_out))) break;
@@ -1954,12 +2067,16 @@ int gs_set_walk(gs_engine* eng, int mode) {
     return upload_descriptors(eng, false);
 }
 
-// Steps with at most 2^nk cosets run, in runs of two or more, in one single-block launch (nk -1: never; default 10).
+// Steps with at most 2^nk cosets run, in runs of two or more, in one single-block launch (nk -1: never; default 10; runs
+// are cut where their slots would not fit the LDS, and steps beyond 2^12 cosets always take sweeps).
 int gs_set_small_steps(gs_engine* eng, int nk) {
     if (!eng) return fail(16, "null engine");
     if (nk < -1 || nk > 20) return fail(16, "small-step limit must be -1..20");
+    HIP_TRY(hipSetDevice(eng->device));
+    HIP_TRY(hipStreamSynchronize(eng->stream));
     eng->small_nk = nk;
-    return 0;
+    build_small(eng);
+    return upload_descriptors(eng, false);
 }
 
 // Runs of at most max_steps consecutive diagonal steps (2..8; 0 or 1: off; default 8) of at least 2^min_nk cosets
@@ -2148,6 +2265,8 @@ extern "C" int gs_prob_noalloc(const gs_plan* plan, int storage, int device, con
     e.d_cond = reinterpret_cast<double*>(base + o_cond);
     e.dplain = reinterpret_cast<KStep*>(base + o_plain);
     e.dfused = reinterpret_cast<KStep*>(base + o_fused);
+    static_assert(sizeof(SStep) <= sizeof(double) * gs_engine::kChunk, "the uniforms' buffer holds a descriptor per step");
+    e.dsmall = reinterpret_cast<SStep*>(base + o_U);       // forced strings draw no uniforms
     e.arena = base + o_arena;
     // host staging in ordinary (pageable) memory; the null stream; no timing events
     std::vector<int8_t> h_forced(C * nsz);
@@ -2160,6 +2279,7 @@ extern "C" int gs_prob_noalloc(const gs_plan* plan, int storage, int device, con
     if (ns > 0) {
         HIP_TRY(hipMemcpy(e.dplain, e.hplain.data(), sizeof(KStep) * size_t(ns), hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(e.dfused, e.hfused.data(), sizeof(KStep) * size_t(ns), hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(e.dsmall, e.hsmall.data(), sizeof(SStep) * size_t(ns), hipMemcpyHostToDevice));
     }
     // the sweeps' block counter must start at 0 (a kernel fill, not a memset node: callers may capture this)
     hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(64), 0, e.stream, e.counter, kCounters);

@@ -1,0 +1,10 @@
+// The sweep kernels of a complex128 arena.
+#include "gs_sweep.h"
+
+namespace gs {
+
+void* sweep_kernel_c128(int lr, int vg, int ntq, int route, int sweep, int route2) {
+    return sweep_for<double2>(lr, vg, ntq, route, sweep, route2);
+}
+
+}  // namespace gs
