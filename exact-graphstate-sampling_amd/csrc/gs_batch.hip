@@ -31,10 +31,18 @@
 #include <vector>
 
 #include "../../include/gsamp_amd.h"
-#include "gs_gf2.h"
+#include "gs_pair.h"
 #include "gs_plan.h"
 
 namespace {
+
+using gs::flip_if;
+using gs::make_pair;
+using gs::pair_route0;
+using gs::pair_route1;
+using gs::PairDesc;
+using gs::PairRegs;
+using gs::PairSteps;
 
 constexpr int kLanes = 64;           // strings per wave (one lane group)
 constexpr int kWaves = 4;            // waves per block, each on its own part of the coset range
@@ -63,29 +71,11 @@ struct BItem {
     int pad;
 };
 
-// Two consecutive steps as one sweep (see make_pair).  L1, the live table between them, splits into W, the span of
-// step k+1's slot offsets (relative to its first) and step k's g, and a complement C inside the span of step k's
-// columns.  A super-coset a + W (a in C) is closed under both steps: its NI step-k cosets i (at a ^ D[i]) give the
-// elements (i, t) at a ^ D[i] ^ t g, which are all the slots of its NU step-(k+1) cosets, so a lane takes it from step
-// k's inputs to step k+1's outputs without the table between them ever being stored.
-struct BPair {
-    uint64_t cols[40];   // columns of the super-coset coordinates
-    uint64_t D[4];
-    uint64_t lab[4];     // D[i], or D[i] ^ g where it is labelled output 1: the base address of step k's coset
-    uint64_t g, d1, d2;  // step k's g; step k+1's second and third offsets relative to the first
-    uint64_t o0;         // step k+1's first offset
-    uint8_t pn[40];      // per coordinate: bit 0 step k's sign, bit 1 step k+1's sign, bits 2-3 step k+1's slot index
-    uint8_t pd[4], pg;   // the same of D[i] (bit 4: the output index it is labelled with) and of g
-    uint8_t pc;          // the same of step k+1's first offset
-    int nk;              // super-coset coordinates
-    int ni, mo, deg;     // step-k cosets, outputs of step k, 1 when g is among the slot offsets of step k+1 (NU = 1)
-};
-
 struct BInst {           // device view of one instance
     void* mem;           // [2^R][B] forward arena
     void* lam;           // [2^R][B] adjoint arena (gradient mode)
     const BStep* steps;  // [ns]
-    const BPair* pairs;  // [ns]: the sweep of steps k and k+1, where one is taken
+    const PairDesc* pairs;  // [ns]: the sweep of steps k and k+1, where one is taken
     const int8_t* bitsT; // [ns][B] forced bits, step-major
     double* prev;        // [B]
     int* dead;           // [B]
@@ -448,7 +438,7 @@ __global__ __launch_bounds__(kBThreads) void batch_back_kernel(const BInst* __re
     lane_store<4>(I, it, wave, lane, val);
 }
 
-// ---- two steps per sweep (BPair)
+// ---- two steps per sweep (PairDesc)
 //
 // A single step's sweep is bound by HBM: it reads and writes one table (n = 70 band 26, 64 lanes, 2^22 cosets: 4.3 GB
 // in 0.85 ms, 5.0 TB/s) and its FP64 work takes a quarter of that time.  Two steps in one sweep move the same bytes
@@ -460,17 +450,6 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
     return (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(v >> 32)))) << 32) |
            uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
 }
-__device__ __forceinline__ double2 flip_if(double2 a, uint32_t s) {          // (-1)^s a
-    const int m = int(s << 31);
-    return make_double2(__hiloint2double(__double2hiint(a.x) ^ m, __double2loint(a.x)),
-                        __hiloint2double(__double2hiint(a.y) ^ m, __double2loint(a.y)));
-}
-__device__ __forceinline__ void route_one(double2 (&A)[2][2], double2 w, uint32_t t0, uint32_t t1, uint32_t neg) {
-    const double2 ws = flip_if(w, neg);
-    if (t0) A[1][0] = cadd(A[1][0], w); else A[0][0] = cadd(A[0][0], w);     // uniform branches
-    if (t1) A[1][1] = cadd(A[1][1], ws); else A[0][1] = cadd(A[0][1], ws);
-}
-
 // Super-cosets a wave gathers at once: about 8 loads in flight per lane for 8-byte entries, 4 for 16-byte ones.
 template <class S>
 constexpr int pair_lu(int loads) {
@@ -490,7 +469,7 @@ struct PairWalk {
     bool on;
     __device__ __forceinline__ uint64_t col(int j) const { return uniform64(cols[j]); }
     __device__ __forceinline__ uint32_t nib(int j) const { return uint32_t(__builtin_amdgcn_readfirstlane(pn[j])); }
-    __device__ PairWalk(const BItem& it, const BPair& P, uint64_t* scols, int* spn, int wave) : cols(scols), pn(spn) {
+    __device__ PairWalk(const BItem& it, const PairDesc& P, uint64_t* scols, int* spn, int wave) : cols(scols), pn(spn) {
         for (int j = threadIdx.x; j < P.nk; j += blockDim.x) {
             scols[j] = P.cols[j];
             spn[j] = P.pn[j];
@@ -531,59 +510,8 @@ struct PairWalk {
     __device__ uint64_t index(uint64_t t, int u) const { return cstart | ((t ^ (t >> 1)) << lu) | uint64_t(u); }
 };
 
-// Uniform per-launch constants of a pair.
-struct PairRegs {
-    uint64_t lab[4], off[4], g, d1, d2, o0, g1;
-    uint32_t pd[4], pg, pc, t0m, t1m, parm, u0m, u1m, uparm;
-    int m1;
-    __device__ PairRegs(const BPair& P, const BStep& s0, const BStep& s1) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            lab[i] = P.lab[i];
-            off[i] = s0.off[i];
-            pd[i] = P.pd[i];
-        }
-        g = P.g; d1 = P.d1; d2 = P.d2; o0 = P.o0; pg = P.pg; pc = P.pc;
-        g1 = s1.g;
-        m1 = s1.m;
-        t0m = s0.t0m; t1m = s0.t1m; parm = s0.parm;
-        u0m = s1.t0m; u1m = s1.t1m; uparm = s1.parm;
-    }
-    // slot of step k+1 at element (i, t) of the super-coset with parities pa, and its coset's sign
-    __device__ uint32_t slot(uint32_t pa, int i, int t) const { return ((pa ^ pd[i] ^ (t ? pg : 0) ^ pc) >> 2) & 3; }
-    __device__ uint32_t sign(uint32_t pa, int c) const { return ((pa ^ (c ? pg : 0) ^ pc) >> 1) & 1; }
-    // output 0 of step-(k+1) coset c of the super-coset at a
-    __device__ uint64_t out(uint64_t a, uint32_t pa, int c) const {
-        const uint32_t j = slot(pa, 0, c);
-        return a ^ (c ? g : 0) ^ o0 ^ ((j & 1) ? d1 : 0) ^ ((j & 2) ? d2 : 0);
-    }
-};
-
-// Slot sums of step-k coset i: A[t][x], t the element label (output index t ^ label bit).
-template <class S, int NQ>
-__device__ __forceinline__ void pair_route0(const PairRegs& r, const S (&v)[NQ], uint32_t pa, int i,
-                                            double2 (&A)[2][2]) {
-    A[0][0] = A[0][1] = A[1][0] = A[1][1] = make_double2(-0.0, -0.0);
-    const uint32_t pc = (pa ^ r.pd[i]) & 1, sw = (r.pd[i] >> 4) & 1;
-#pragma unroll
-    for (int q = 0; q < NQ; q++)
-        route_one(A, Sto<S>::wide(v[q]), ((r.t0m >> q) & 1) ^ sw, ((r.t1m >> q) & 1) ^ sw, pc ^ ((r.parm >> q) & 1));
-}
-
-// Slot sums of step-(k+1) coset c from the elements e[i][t] (already rounded to the storage type).
-template <int NI, int MO, bool DEG>
-__device__ __forceinline__ void pair_route1(const PairRegs& r, const double2 (&e)[NI][MO], uint32_t pa, int c,
-                                            double2 (&A)[2][2]) {
-    A[0][0] = A[0][1] = A[1][0] = A[1][1] = make_double2(-0.0, -0.0);
-    const uint32_t sg = r.sign(pa, c);
-#pragma unroll
-    for (int i = 0; i < NI; i++)
-#pragma unroll
-        for (int t = 0; t < MO; t++) {
-            if (!DEG && t != c) continue;
-            const uint32_t j = r.slot(pa, i, t);
-            route_one(A, e[i][t], (r.u0m >> j) & 1, (r.u1m >> j) & 1, sg ^ ((r.uparm >> j) & 1));
-        }
+__device__ __forceinline__ PairSteps pair_steps(const BStep& s0, const BStep& s1) {
+    return PairSteps{s0.off, s1.g, s1.m, s0.t0m, s0.t1m, s0.parm, s1.t0m, s1.t1m, s1.parm};
 }
 
 template <class S, int NQ, int NI, int MO, bool DEG>
@@ -604,7 +532,7 @@ __global__ __launch_bounds__(kBThreads) void pair_step_kernel(const BInst* __res
     const double2 x0 = make_double2(s1.mre[b1][0], s1.mim[b1][0]), x1 = make_double2(s1.mre[b1][1], s1.mim[b1][1]);
     S* __restrict__ mem = static_cast<S*>(I.mem);
     S* __restrict__ cp = L.copy ? static_cast<S*>(L.copy[it.inst]) : nullptr;
-    const PairRegs r(I.pairs[k], s0, s1);
+    const PairRegs r(I.pairs[k], pair_steps(s0, s1));
     __shared__ uint64_t scols[40];
     __shared__ int spn[40];
     PairWalk<LU> wk(it, I.pairs[k], scols, spn, wave);
@@ -650,7 +578,7 @@ __global__ __launch_bounds__(kBThreads) void pair_step_kernel(const BInst* __res
 #pragma unroll
             for (int c = 0; c < NU; c++) {
                 double2 A[2][2];
-                pair_route1<NI, MO, DEG>(r, e, pa, c, A);
+                pair_route1<NI, MO, DEG>(r, e, pa, pa, c, A);
                 const double2 f0 = cfma(x0, A[0][0], cmul(x1, A[0][1]));
                 const double2 f1 = cfma(x0, A[1][0], cmul(x1, A[1][1]));
                 if (!mine) continue;
@@ -682,7 +610,7 @@ __global__ __launch_bounds__(kBThreads) void pair_restore_kernel(const BInst* __
     S* __restrict__ mem = static_cast<S*>(I.mem);
     const S* __restrict__ cp = static_cast<const S*>(L.copy[it.inst]);
     if (!cp) return;
-    const PairRegs r(I.pairs[L.k], I.steps[L.k], I.steps[L.k + 1]);
+    const PairRegs r(I.pairs[L.k], pair_steps(I.steps[L.k], I.steps[L.k + 1]));
     __shared__ uint64_t scols[40];
     __shared__ int spn[40];
     PairWalk<LU> wk(it, I.pairs[L.k], scols, spn, wave);
@@ -727,7 +655,7 @@ __global__ __launch_bounds__(kBThreads) void pair_back_kernel(const BInst* __res
     const double2 x0 = make_double2(s1.mre[b1][0], s1.mim[b1][0]), x1 = make_double2(s1.mre[b1][1], s1.mim[b1][1]);
     S* __restrict__ lam = static_cast<S*>(I.lam);
     const S* __restrict__ cp = static_cast<const S*>(L.copy[it.inst]);
-    const PairRegs r(I.pairs[k], s0, s1);
+    const PairRegs r(I.pairs[k], pair_steps(s0, s1));
     const uint64_t gq = r.m1 == 2 ? r.g1 : 0;
     __shared__ uint64_t scols[40];
     __shared__ int spn[40];
@@ -768,7 +696,7 @@ __global__ __launch_bounds__(kBThreads) void pair_back_kernel(const BInst* __res
 #pragma unroll
             for (int c = 0; c < NU; c++) {
                 double2 A[2][2];
-                pair_route1<NI, MO, DEG>(r, e, pa, c, A);
+                pair_route1<NI, MO, DEG>(r, e, pa, pa, c, A);
                 const double2 m0 = Sto<S>::wide(l2[u][c][0]);
                 const double2 m1 = r.m1 == 2 ? Sto<S>::wide(l2[u][c][1]) : make_double2(0, 0);
 #pragma unroll
@@ -986,7 +914,7 @@ struct gs_batch {
     int lg_default = 8;                   // smallest tile (sizes the partial buffers); steps start at 2^9
     std::vector<int> nq;                  // per step: most slots per coset among the instances (kernel variant)
     std::vector<int> nq_exact;            // per step: 1 if every instance at the step has nq slots per coset
-    std::vector<std::vector<BPair>> hpairs;   // [inst][step]: steps k and k+1 as one sweep (ni 0: not possible)
+    std::vector<std::vector<PairDesc>> hpairs;   // [inst][step]: steps k and k+1 as one sweep (ni 0: not possible)
     std::vector<char> unit;               // per step: steps of the sweep that starts there (1, 2; 0: inside a pair)
     bool pairs_on = true;
     int* dcnt = nullptr;                  // device [maxns][ninst]: items per lane group of instance i at step k
@@ -1023,83 +951,6 @@ T* dalloc(gs_batch* b, size_t n) {
     return static_cast<T*>(p);
 }
 
-// Steps k and k+1 of a plan as one sweep (see BPair); false when a super-coset cannot be closed or would write a slot
-// that another super-coset still reads.
-bool make_pair(const gs::StepInfo& s0, const gs::StepInfo& s1, BPair& p) {
-    using gs::GfBasis;
-    using gs::parity;
-    memset(&p, 0, sizeof p);
-    GfBasis live;                                     // L1: the columns of step k (its output 0), then g
-    for (uint64_t c : s0.cols)
-        if (!live.add(c)) return false;
-    if (s0.m == 2 && !live.add(s0.g)) return false;
-    const int lg1 = s1.ntq == 4 ? 2 : s1.ntq == 2 ? 1 : 0;
-    uint64_t d[4] = {0, 0, 0, 0};
-    for (int j = 1; j < s1.ntq; j++) d[j] = s1.off[j] ^ s1.off[0];
-    if (s1.ntq == 4 && (d[3] != (d[1] ^ d[2]))) return false;
-    GfBasis next;                                     // the same space as step k+1 reads it: its columns, then d1, d2
-    for (uint64_t c : s1.cols)
-        if (!live.has(c) || !next.add(c)) return false;
-    for (int j = 1; j <= lg1; j++)
-        if (!live.has(d[j]) || !next.add(d[j])) return false;
-    if (next.n != live.n || !live.has(s1.off[0])) return false;
-    // parities of an address of L1: bit 0 step k's sign, bit 1 step k+1's, bits 2-3 its slot, bit 4 step k's output
-    auto nib = [&](uint64_t x) {
-        uint64_t c0 = 0, c1 = 0;
-        (void)live.solve(x, c0);
-        (void)next.solve(x, c1);
-        const uint64_t m0 = (uint64_t(1) << s0.nk) - 1, m1 = (uint64_t(1) << s1.nk) - 1;
-        return uint8_t(parity(c0 & m0 & s0.rhoc) | (parity(c1 & m1 & s1.rhoc) << 1) | (int((c1 >> s1.nk) & 3) << 2) |
-                       (int((c0 >> s0.nk) & 1) << 4));
-    };
-    GfBasis slots;
-    for (int j = 1; j <= lg1; j++) (void)slots.add(d[j]);
-    p.deg = s0.m == 2 && slots.has(s0.g);
-    p.mo = s0.m;
-    p.ni = p.deg ? s1.ntq / 2 : s1.ntq;
-    if (p.deg) p.D[1] = p.ni == 2 ? (d[1] != s0.g ? d[1] : d[2]) : 0;
-    else
-        for (int i = 1; i < p.ni; i++) p.D[i] = d[i];
-    GfBasis W;
-    if (s0.m == 2) (void)W.add(s0.g);
-    for (int i = 1; i < p.ni; i++) (void)W.add(p.D[i]);
-    GfBasis C;
-    for (uint64_t c : s0.cols)
-        if (W.add(c)) {
-            (void)C.add(c);
-            p.cols[p.nk] = c;
-            p.pn[p.nk++] = nib(c);
-        }
-    if (W.n != live.n) return false;
-    p.g = s0.g;
-    p.d1 = d[1];
-    p.d2 = lg1 == 2 ? d[2] : 0;
-    p.o0 = s1.off[0];
-    p.pg = s0.m == 2 ? nib(s0.g) : 0;
-    p.pc = nib(s1.off[0]);
-    for (int i = 0; i < p.ni; i++) {
-        p.pd[i] = nib(p.D[i]);
-        p.lab[i] = p.D[i] ^ ((p.pd[i] & 16) ? s0.g : 0);
-    }
-    // slots read and written relative to the super-coset's base: no two super-cosets may meet on a written slot
-    std::vector<uint64_t> rd, wr;
-    for (int i = 0; i < p.ni; i++)
-        for (int q = 0; q < s0.ntq; q++) rd.push_back(p.lab[i] ^ s0.off[q]);
-    for (int c = 0; c < (p.deg ? 1 : p.mo); c++)
-        for (int j = 0; j < s1.ntq; j++) {
-            const uint64_t at = (c ? s0.g : 0) ^ s1.off[0] ^ d[j];
-            wr.push_back(at);
-            if (s1.m == 2) wr.push_back(at ^ s1.g);
-        }
-    auto clash = [&](const std::vector<uint64_t>& x, const std::vector<uint64_t>& y) {
-        for (uint64_t u : x)
-            for (uint64_t v : y)
-                if (u != v && C.has(u ^ v)) return true;
-        return false;
-    };
-    return !clash(wr, rd) && !clash(wr, wr) && !clash(rd, rd);
-}
-
 // Which sweeps the step sequence takes: single steps, or two at once where every instance that is still running has
 // the same kind of pair.  A pair saves the write and the read of the table between its steps (and a launch), so the
 // pairs are the disjoint ones that save the most.
@@ -1111,13 +962,13 @@ void choose_units(gs_batch* bt) {
     std::vector<double> gain(size_t(ns), -1.0), best(size_t(ns) + 2, 0.0);
     for (int k = 0; k + 1 < ns; k++) {
         double g = kLaunch;
-        const BPair* first = nullptr;
+        const PairDesc* first = nullptr;
         int ntq = 0;
         bool ok = true;
         for (size_t i = 0; i < bt->plans.size() && ok; i++) {
             const gs::Plan& P = bt->plans[i];
             if (k >= P.ns) continue;
-            const BPair& p = bt->hpairs[i][size_t(k)];
+            const PairDesc& p = bt->hpairs[i][size_t(k)];
             if (k + 1 >= P.ns || !p.ni) {
                 ok = false;
             } else if (!first) {
@@ -1145,7 +996,7 @@ void sweep_size(const gs_batch* bt, size_t i, int k, int& nk, int& inner) {
     nk = bt->plans[i].steps[size_t(k)].nk;
     inner = 0;
     if (bt->unit[size_t(k)] != 2) return;
-    const BPair& p = bt->hpairs[i][size_t(k)];
+    const PairDesc& p = bt->hpairs[i][size_t(k)];
     inner = p.ni == 4 ? 2 : p.ni == 2 ? 1 : 0;
     nk = p.nk;
 }
@@ -1307,7 +1158,7 @@ int launch_batch(gs_batch* bt, BKernel kind, int k, BLaunch L) {
     if (n == 0) return 0;
     const int nq = bt->nq[size_t(k)], lu = bt->lu;
     const bool ex = bt->nq_exact[size_t(k)] != 0;
-    const BPair* pair = nullptr;
+    const PairDesc* pair = nullptr;
     if (bt->unit[size_t(k)] == 2)
         for (size_t i = 0; i < bt->plans.size() && !pair; i++)
             if (k < bt->plans[i].ns) pair = &bt->hpairs[i][size_t(k)];
@@ -1652,9 +1503,9 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
             s.ntq = si.ntq;
             s.m = si.m;
         }
-        std::vector<BPair> hp(size_t(P.ns));
+        std::vector<PairDesc> hp(size_t(P.ns));
         for (int k = 0; k < P.ns; k++)
-            if (k + 1 >= P.ns || !make_pair(P.steps[size_t(k)], P.steps[size_t(k) + 1], hp[size_t(k)])) hp[size_t(k)].ni = 0;
+            if (k + 1 >= P.ns || !make_pair(P.steps[size_t(k)], P.steps[size_t(k) + 1], false, hp[size_t(k)])) hp[size_t(k)].ni = 0;
         // the instance's small buffers in one allocation: descriptors first, uploaded in one copy
         size_t used = 0;
         auto take = [&](size_t bytes) {
@@ -1662,7 +1513,7 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
             used += (bytes + 255) & ~size_t(255);
             return at;
         };
-        const size_t o_steps = take(hs.size() * sizeof(BStep)), o_pairs = take(hp.size() * sizeof(BPair)), head = used;
+        const size_t o_steps = take(hs.size() * sizeof(BStep)), o_pairs = take(hp.size() * sizeof(PairDesc)), head = used;
         const size_t o_bits = take(size_t(P.ns) * B), o_prev = take(sizeof(double) * B), o_dead = take(sizeof(int) * B),
                      o_cond = take(sizeof(double) * size_t(B) * P.ns), o_logp = take(sizeof(double) * B),
                      o_amp = take(sizeof(double) * 2 * B),
@@ -1672,13 +1523,13 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
         if (!mem) return bail(bfail(11, "batch buffer allocation failed"));
         std::vector<char> up(head);
         if (!hs.empty()) memcpy(up.data() + o_steps, hs.data(), hs.size() * sizeof(BStep));
-        if (!hp.empty()) memcpy(up.data() + o_pairs, hp.data(), hp.size() * sizeof(BPair));
+        if (!hp.empty()) memcpy(up.data() + o_pairs, hp.data(), hp.size() * sizeof(PairDesc));
         if (head && hipMemcpy(mem, up.data(), head, hipMemcpyHostToDevice) != hipSuccess)
             return bail(bfail(17, "plan upload failed"));
         bt->hsteps.push_back(std::move(hs));
         bt->hpairs.push_back(std::move(hp));
         I.steps = reinterpret_cast<BStep*>(mem + o_steps);
-        I.pairs = reinterpret_cast<BPair*>(mem + o_pairs);
+        I.pairs = reinterpret_cast<PairDesc*>(mem + o_pairs);
         I.bitsT = reinterpret_cast<int8_t*>(mem + o_bits);
         I.prev = reinterpret_cast<double*>(mem + o_prev);
         I.dead = reinterpret_cast<int*>(mem + o_dead);

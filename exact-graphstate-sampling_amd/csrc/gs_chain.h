@@ -137,6 +137,16 @@ __device__ void chain_step(const double (&red)[NQ], Ctl* ctl, const Epi& e, int 
         return;
     } else if (e.role == kRoleNorm) {
         decide(c, e, e.k, sweep, red);
+    } else if (NQ == 2 && e.role == kRolePair) {
+        finish_write(c, e, e.k, red[0], red[0]);
+        if (!c.dead) {
+            decide(c, e, e.k + 1, -1, nullptr);
+            finish_write(c, e, e.k + 1, red[1], red[1]);
+        }
+        if (!c.dead) {
+            if (e.k + 2 == e.k1) publish(c, e);
+            else if (e.next == kNextDecide) decide(c, e, e.k + 2, -1, nullptr);
+        }
     } else {
         finish_write(c, e, e.k, red[0], red[1]);
         if (!c.dead) {

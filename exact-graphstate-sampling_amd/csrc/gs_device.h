@@ -10,6 +10,10 @@ namespace gs {
 constexpr int kThreads = 256;       // threads per sweep block (4 waves of 64)
 constexpr int kMaxGridLog2 = 14;    // at most 16384 blocks per sweep; beyond that each block loops over tiles
 constexpr int kDefaultGridLog2 = 9;     // measured best for the width-30 sweeps (a few waves per SIMD suffice)
+// Chain sweeps of two steps: 2^10 blocks, 2^12 from 2^26 super-cosets on, 2^9 with 16-byte entries.  At 2^9 / 2^10 / 2^12
+// blocks a complex64 string takes 584 / 581 / 689 us at width 24 and 8.74 / 8.60 / 8.34 ms at width 29, a complex128 one
+// 89 / 97 / 97 us at width 20 and 4.13 / 4.56 / 4.42 ms at width 26.
+constexpr int kDefaultGridLog2Pair = 10, kDefaultGridLog2PairBig = 12, kBigPairLog2 = 26, kDefaultGridLog2PairWide = 9;
 constexpr int kDefaultGridLog2One = 12; // plain sweeps of one-slot steps: one load per thread and tile, so more waves
                                         // (width 34, 1-slot norm passes: 691 -> 343 ms per sample at 2^12 blocks)
 constexpr int kBigStepLog2 = 30;        // one-slot steps of at least 2^30 cosets take more blocks still:
@@ -159,7 +163,8 @@ enum ChainMode { kChain = 0, kChain1 = 1, kRun = 2 };
 // What the last block of a sweep does after the sweep (kRoleStored: record the stored table's norm only -- the
 // product pass of a run of diagonal steps, whose decisions and bookkeeping were made before it).
 // kRoleStoredGram: the same, then the next step's decision from the Gram matrix the product pass summed.
-enum EpiRole { kRoleNorm = 0, kRoleWrite = 1, kRoleStored = 2, kRoleStoredGram = 3 };
+// kRolePair: a chain-mode sweep of steps k and k+1, whose sums are the two steps' written norms.
+enum EpiRole { kRoleNorm = 0, kRoleWrite = 1, kRoleStored = 2, kRoleStoredGram = 3, kRolePair = 4 };
 // Write role: what follows step k.
 enum Next { kNextPublish = -2, kNextDecide = -1, kNextFusedGram = kGram, kNextFusedDirect = kDirect, kNextSweep = 3 };
 

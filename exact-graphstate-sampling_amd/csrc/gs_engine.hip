@@ -27,6 +27,7 @@
 #include "gs_device.h"
 #include "gs_gf2.h"
 #include "gs_plan.h"
+#include "gs_pstep.h"
 
 namespace gs {
 void* sweep_kernel_for(int storage, int lr, int vg, int ntq, int route, int sweep, int route2);
@@ -37,6 +38,7 @@ void* publish_kernel_ptr();
 void* reduce_kernel_ptr(int sweep);
 void* small_run_kernel_ptr(int storage);
 size_t small_run_lds(size_t tab_bytes);
+void* pair_sweep_kernel_ptr(int storage, int nq, int ni, int mo, int deg);
 void* reduce1_kernel_ptr();
 void* run_hist_kernel_ptr(int storage);
 void* run_apply_kernel_ptr(int storage);
@@ -339,6 +341,7 @@ struct gs_engine {
     bool allow_fusion = true;
     bool allow_fused4 = true;       // fold a four-slot next step's norms into the write (two pairing coordinates)
     int grid_cap = kDefaultGridLog2;  // log2 of the most blocks a sweep launches
+    int grid_cap2 = 0;              // ... of two steps (0: the defaults by size and storage)
     int grid_cap1 = kDefaultGridLog2One;  // ... a plain sweep of a one-slot step
     int grid_cap1_big = kDefaultGridLog2OneBig;  // ... of a one-slot step with at least 2^kBigStepLog2 cosets
     // runs of small steps (gs_small.hip): descriptors, the run each step belongs to (-1: none), log2 slots of each run
@@ -346,6 +349,11 @@ struct gs_engine {
     std::vector<SStep> hsmall;
     std::vector<int> small_at, small_dim;
     SStep* dsmall = nullptr;
+    // chain mode: steps k and k+1 as one sweep (gs_pair.hip)
+    bool allow_pairs = true;
+    std::vector<PStep> hpair;
+    std::vector<void*> pair_fn;     // the sweep of the pair that starts at a step, or nullptr
+    PStep* dpair = nullptr;
     bool fresh = false;             // the next launch starts the strings' chains
     int walk = 0;                   // tile order: 0 forward, 1 reverse on odd steps, 2 reverse on every step
     int fused_run = -1;             // log2 run of the fused layout (-1: the storage's default)
@@ -484,6 +492,28 @@ int launch_sweep(gs_engine* e, int k, int sweep, const Epi& epi) {
         e->pend_epi.pend_nblk = 0;
         e->cur_part ^= 1;
         if (e->fold_r < 0) return flush_pending(e);
+    }
+    return 0;
+}
+
+// The sweep of steps k and k+1 of a chain-mode string (both weights known, no scale).
+int launch_pair(gs_engine* e, int k, const Epi& epi) {
+    if (int rc = launch_init(e)) return rc;
+    if (int rc = flush_pending(e)) return rc;
+    const PStep* pp = e->dpair + k;
+    void* mem = arena_of(e);
+    double* part = e->strings > 1 ? e->slot_part[0] : e->part_buf[0];
+    Ctl* ctl = e->ctl;
+    Epi ep = epi;
+    const int grid = 1 << e->hpair[size_t(k)].lg_grid;
+    void* args[] = {&pp, &mem, &part, &ctl, &ep};
+    HIP_TRY(hipLaunchKernel(e->pair_fn[size_t(k)], dim3(grid, e->strings), dim3(kThreads), args, 0, e->stream));
+    if (!reduces_in_kernel(unsigned(grid), unsigned(e->strings))) {
+        const double* cpart = part;
+        unsigned nblk = unsigned(grid);
+        int sw = kWrite;
+        void* rargs[] = {&cpart, &nblk, &ctl, &ep, &sw};
+        HIP_TRY(hipLaunchKernel(reduce_kernel_ptr(sw), dim3(1, e->strings), dim3(kThreads), rargs, 0, e->stream));
     }
     return 0;
 }
@@ -695,6 +725,14 @@ int enqueue_run(gs_engine* e, int mode, int k0, int k1, const int8_t* forced_h, 
         Epi ep = base;
         ep.k = k;
         ep.role = kRoleWrite;
+        if (mode == kChain1 && e->allow_pairs && !e->profile && k + 1 < k1 && e->pair_fn[size_t(k)]) {
+            ep.role = kRolePair;
+            ep.next = k + 2 == k1 ? kNextPublish : run_from(e, k + 2, k1) >= 0 ? kNextSweep : kNextDecide;
+            if (int rc = launch_pair(e, k, ep)) return rc;
+            decided = ep.next != kNextSweep;
+            k++;
+            continue;
+        }
         int sweep = kWrite;
         if (k + 1 == k1) {
             ep.next = kNextPublish;
@@ -1302,6 +1340,68 @@ void build_small(gs_engine* e) {
     }
 }
 
+// Pairs of steps of the chain mode: steps outside the runs of small and of diagonal steps whose super-cosets give a
+// thread one aligned 16-byte run per slot and leave step k+1's slot index the same over the threads' coordinates.  Each
+// saves the write and the read of the table between its steps and a launch; the pairs are the disjoint ones that save
+// the most.
+void build_pairs(gs_engine* e) {
+    const Plan& P = e->plan;
+    const size_t ns = size_t(P.ns);
+    e->hpair.assign(std::max<size_t>(ns, 1), PStep{});
+    e->pair_fn.assign(std::max<size_t>(ns, 1), nullptr);
+    if (!e->own_buffers) return;                          // prob only
+    const int lr = e->storage == GS_C64 ? 1 : 0;
+    std::vector<char> taken(ns, 0);
+    for (size_t k = 0; k < ns; k++) taken[k] = e->small_at[k] >= 0;
+    for (const RStep& r : e->hrun)
+        for (int i = 0; i < r.j; i++) taken[size_t(r.k0 + i)] = 1;
+    std::vector<double> best(ns + 2, 0.0), gain(ns, 0.0);
+    std::vector<void*> fn(ns, nullptr);
+    for (size_t k = 0; k + 1 < ns; k++) {
+        if (taken[k] || taken[k + 1]) continue;
+        const StepInfo &s0 = P.steps[k], &s1 = P.steps[k + 1];
+        PStep& p = e->hpair[k];
+        if (!make_pair(s0, s1, true, p.d) || p.d.nk < lr + 8 || (lr && p.d.cols[0] != 1)) continue;
+        bool fits = true;
+        for (int j = 0; j < lr + 8; j++) fits = fits && !(p.d.pn[j] & 12);
+        if (!fits) continue;
+        if (lr)
+            for (int j = 1; j < p.d.nk; j++)              // the run's bit in coordinate 0 only
+                if (p.d.cols[j] & 1) {
+                    p.d.cols[j] ^= 1;
+                    p.d.pn[j] ^= p.d.pn[0];
+                }
+        for (int q = 0; q < s0.ntq; q++) {
+            p.off[q] = s0.off[q];
+            p.t0m |= uint32_t(s0.tau0[q] & 1) << q;
+            p.t1m |= uint32_t(s0.tau1[q] & 1) << q;
+            p.parm |= uint32_t(s0.par[q] & 1) << q;
+        }
+        for (int q = 0; q < s1.ntq; q++) {
+            p.u0m |= uint32_t(s1.tau0[q] & 1) << q;
+            p.u1m |= uint32_t(s1.tau1[q] & 1) << q;
+            p.uparm |= uint32_t(s1.par[q] & 1) << q;
+        }
+        p.g1 = s1.g;
+        p.m1 = s1.m;
+        p.ntq = s0.ntq;
+        p.xcd = e->xcd_blocks;
+        const int tiles = p.d.nk - lr - 8;
+        const int cap = e->grid_cap2 ? e->grid_cap2 : !lr ? kDefaultGridLog2PairWide
+                      : p.d.nk >= kBigPairLog2 ? kDefaultGridLog2PairBig : kDefaultGridLog2Pair;
+        p.lg_grid = std::min(tiles, cap);
+        p.lg_iter = tiles - p.lg_grid;
+        fn[k] = pair_sweep_kernel_ptr(e->storage, s0.ntq, p.d.ni, p.d.mo, p.d.deg);
+        if (fn[k]) gain[k] = 20e6 + 2.0 * double(e->esz) * double(uint64_t(s0.m) << s0.nk);
+    }
+    for (size_t k = ns; k-- > 0;) best[k] = std::max(best[k + 1], fn[k] ? gain[k] + best[k + 2] : 0.0);
+    for (size_t k = 0; k < ns; k++)
+        if (fn[k] && gain[k] + best[k + 2] > best[k + 1]) {
+            e->pair_fn[k] = fn[k];
+            k++;
+        }
+}
+
 int build_steps(gs_engine* e) {
     const Plan& P = e->plan;
     e->hplain.assign(size_t(P.ns), KStep{});
@@ -1392,6 +1492,7 @@ int build_steps(gs_engine* e) {
     }
     build_runs(e);
     build_small(e);
+    build_pairs(e);
     return 0;
 }
 
@@ -1402,6 +1503,7 @@ int upload_descriptors(gs_engine* e, bool logical) {
     if (ns) {
         HIP_TRY(hipMemcpy(e->dplain, e->hplain.data(), sizeof(KStep) * ns, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(e->dfused, e->hfused.data(), sizeof(KStep) * ns, hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(e->dpair, e->hpair.data(), sizeof(PStep) * ns, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(e->dsmall, e->hsmall.data(), sizeof(SStep) * ns, hipMemcpyHostToDevice));
         if (logical) HIP_TRY(hipMemcpy(e->dlogical, e->hlogical.data(), sizeof(KStep) * ns, hipMemcpyHostToDevice));
     }
@@ -1433,6 +1535,7 @@ void free_engine(gs_engine* e) {
     (void)hipFree(e->dfused);
     (void)hipFree(e->dlogical);
     (void)hipFree(e->dsmall);
+    (void)hipFree(e->dpair);
     (void)hipFree(e->part_buf[0]);
     (void)hipFree(e->slots);
     (void)hipFree(e->counter);
@@ -1643,7 +1746,7 @@ int gs_engine_create(const gs_plan* plan, int storage, int device, gs_engine** o
     const size_t nsz = size_t(std::max(ns, 1));
     bool ok = dev_alloc((void**)&e->dplain, sizeof(KStep) * nsz) && dev_alloc((void**)&e->dfused, sizeof(KStep) * nsz) &&
               dev_alloc((void**)&e->dlogical, sizeof(KStep) * nsz) &&
-              dev_alloc((void**)&e->dsmall, sizeof(SStep) * nsz) &&
+              dev_alloc((void**)&e->dsmall, sizeof(SStep) * nsz) && dev_alloc((void**)&e->dpair, sizeof(PStep) * nsz) &&
               dev_alloc((void**)&e->part_buf[0], 2 * sizeof(double) * kPartDoubles) &&
               dev_alloc((void**)&e->counter, sizeof(unsigned) * kCounters) &&
               dev_alloc((void**)&e->ctl_base, 2 * C * sizeof(Ctl)) && dev_alloc((void**)&e->d_forced, C * nsz) &&
@@ -2000,6 +2103,7 @@ static int set_grid_caps(gs_engine* eng, int lg, bool one_slot_only) {
     HIP_TRY(hipSetDevice(eng->device));
     HIP_TRY(hipStreamSynchronize(eng->stream));
     if (!one_slot_only) eng->grid_cap = lg ? lg : kDefaultGridLog2;
+    if (!one_slot_only) eng->grid_cap2 = lg;
     eng->grid_cap1 = lg ? lg : kDefaultGridLog2One;
     eng->grid_cap1_big = lg ? lg : kDefaultGridLog2OneBig;
     if (int rc = build_steps(eng)) return rc;
@@ -2076,6 +2180,7 @@ int gs_set_small_steps(gs_engine* eng, int nk) {
     HIP_TRY(hipStreamSynchronize(eng->stream));
     eng->small_nk = nk;
     build_small(eng);
+    build_pairs(eng);
     return upload_descriptors(eng, false);
 }
 
@@ -2159,6 +2264,13 @@ int gs_race_check(gs_engine* eng, int k, int layout, int64_t* counts) {
     (void)hipFree(dcnt);
     for (int i = 0; i < 4; i++) counts[i] = int64_t(h[i]);
     return rc;
+}
+
+// Chain mode: two steps per sweep where the plan allows it (default on) or one.
+int gs_set_pairs(gs_engine* eng, int on) {
+    if (!eng) return fail(16, "null engine");
+    eng->allow_pairs = on != 0;
+    return 0;
 }
 
 // Turn the folding of the next step's norms into the previous write off or on (for measurements; default on).

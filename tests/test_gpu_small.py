@@ -1,5 +1,5 @@
-"""Runs of small steps (one block per string, table in LDS) against one sweep per step: the same bits, and log2 Pr and
-conditionals to the order of their FP64 sums (at most 2^14 terms: 1e-12)."""
+"""Runs of small steps (one block per string, table in LDS) and chain-mode pairs of steps against one sweep per step: the
+same bits and amplitudes, and log2 Pr and conditionals to the order of their FP64 sums (at most 2^14 terms: 1e-12)."""
 import numpy as np
 import pytest
 
@@ -33,6 +33,7 @@ def test_small_runs_equal_single_sweeps(shape, limit, storage, tmp_path):
     K = inst.N // 2
     print(shape, limit, storage, flush=True)
     with gs.Engine(plan, storage) as e:
+        e.set_pairs(False)
         got = []
         for nk in (limit, -1):
             e.set_small_steps(nk)
@@ -48,3 +49,22 @@ def test_small_runs_equal_single_sweeps(shape, limit, storage, tmp_path):
         else:
             assert np.allclose(a, b, rtol=tol, atol=tol * 1e-3), np.max(np.abs(a - b))
 
+
+@pytest.mark.parametrize("storage", [gs.C64, gs.C128])
+@pytest.mark.parametrize("shape", [(34, 14, 3, 0), (40, 18, 3, 12), (60, 24, 4, 0), (52, 21, 8, 0)])
+@pytest.mark.parametrize("grid", [2, 0])
+def test_chain_pairs_equal_single_steps(shape, storage, grid, tmp_path):
+    inst, plan = _inst(shape, tmp_path)
+    given = np.random.default_rng(6).integers(0, 2, size=(3, inst.N)).astype(np.int8)
+    print(shape, storage, grid, flush=True)
+    with gs.Engine(plan, storage) as e:
+        e.set_grid_log2(grid)
+        two = e.chain(given)
+        one_by_one = [e.chain(g) for g in given]
+        e.set_pairs(False)
+        one = e.chain(given)
+    assert np.array_equal(two[2], one[2])                   # the tables are the same, bit for bit
+    assert np.max(np.abs(two[0] - one[0])) < 1e-11
+    assert np.allclose(two[1], one[1], rtol=1e-12, atol=0)
+    for j in range(3):
+        assert np.array_equal(two[j], np.concatenate([r[j] for r in one_by_one]))
