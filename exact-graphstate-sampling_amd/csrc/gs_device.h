@@ -18,6 +18,9 @@ constexpr int kDefaultGridLog2One = 12; // plain sweeps of one-slot steps: one l
                                         // (width 34, 1-slot norm passes: 691 -> 343 ms per sample at 2^12 blocks)
 constexpr int kBigStepLog2 = 30;        // one-slot steps of at least 2^30 cosets take more blocks still:
 constexpr int kDefaultGridLog2OneBig = 14;  // width 34: 1.231 -> 1.196 s per sample; width 30 prefers 2^12
+// The write that folds in the next step's norms holds 4-8 outputs per thread and wants fewer blocks: width 26 5.65 ms per
+// sample at 2^11 blocks, 5.72 / 5.78 / 7.30 at 2^10 / 2^12 / 2^14; width 29 18.1 ms at 2^10 - 2^12, 18.3 at 2^14.
+constexpr int kDefaultTTFoldGridLog2 = 11;
 constexpr int kDefaultTTGridLog2 = 14;  // gather sweeps of the two-table engine (latency-bound gathers: the
                                          // width-31 IBM sample 0.276 s at 2^9 blocks, 0.121 s at 2^14)
 constexpr int kFenceBlocks = 64;    // launches of at most this many blocks reduce in each string's last block
@@ -110,6 +113,20 @@ struct TStep {
     // pdelta, a tile bit, or -1 (no pairing).
     uint64_t pdelta, pD;
     int ph, ptd;
+};
+
+// The write of a two-table step that folds in the next step's norms (gather_fold_kernel).  Output-space vectors: the
+// directions dvec (low parts of the next step's kernel vectors) and the partner direction pdelta, with their images in
+// the old table's input space; the other coordinates are output bits pos[0..], 8 of the threads, then the blocks', then
+// the tiles'.
+struct TFold {
+    uint64_t dvec[2], dimg[2], pdelta, pimg;
+    uint64_t rho;              // next step's sign mask over the entries
+    uint32_t xk;               // bit e: x of the next step's input e relative to input 0
+    int ptd;                   // the partner's input t is this output's input t ^ ptd
+    int nd2, share, pure;
+    int lg_grid, lg_iter;
+    uint8_t pos[40];
 };
 
 // A run of consecutive diagonal steps: one-slot, one-output steps with slot offset 0 over the same live table.  Step i

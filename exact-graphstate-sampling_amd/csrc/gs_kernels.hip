@@ -1,5 +1,5 @@
-// The other kernels of the engines: reductions after a sweep, one-thread chain kernels, runs of diagonal steps, and the
-// gather sweeps of the two-table engine; and the table of all of them the engines launch from.
+// The other kernels of the engines: reductions after a sweep, one-thread chain kernels, runs of diagonal steps; and the
+// table of all of them the engines launch from.
 #include "gs_sweep.h"
 
 namespace gs {
@@ -289,147 +289,6 @@ __global__ __launch_bounds__(kThreads) void run_apply_kernel(const RStep* __rest
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Two-table (gather-form) steps (gsamp.cpp:21-29, :39-55; dp.cpp:44-53).  Output cp gathers its 2^nker inputs; S0 sums
-// the x = 0 terms, S1 the x = 1 terms with sign (-1)^{parity(c & rho)}; the outputs are M[b][0] S0 + M[b][1] S1.
-// Norm pass (SWEEP = kDirect): both branch norms |M[b][0] S0 + M[b][1] S1|^2 summed directly (the reference's chain).
-// Write pass (kWrite): w0 S0 + w1 S1 stored at nw[cp] (contiguous), with w from the chain's decision or, for the
-// amplitude engine, from wext[4k..4k+3] (the job's per-vertex weights).  NKS = 2^nker inputs per output.  Output
-// bits 0..7 are the thread index, then the block index, then the tile index (groups of 4 tiles per thread, see
-// below; one tile at a time when a block has fewer than 4).
-template <class S, int SWEEP, int NKS>
-__global__ __launch_bounds__(kThreads) void gather_kernel(const TStep* __restrict__ tp, const S* __restrict__ old,
-                                                          S* __restrict__ nw, double* __restrict__ part,
-                                                          Ctl* __restrict__ ctl, Epi epi,
-                                                          const double* __restrict__ wext) {
-    if (ctl->dead) return;
-    const TStep& s = *tp;
-    const int tid = threadIdx.x;
-    uint64_t a_thr = 0;
-#pragma unroll
-    for (int b = 0; b < 8; b++)
-        if (b < s.rn && ((tid >> b) & 1)) a_thr ^= s.dep[b];
-    const bool active = s.rn >= 8 || tid < (1 << s.rn);
-    uint64_t a_blk = 0;
-    for (int b = 0; b < s.lg_grid; b++)
-        if ((blockIdx.x >> b) & 1) a_blk ^= s.dep[8 + b];
-    const int jit = 8 + s.lg_grid;
-    const int niter = 1 << s.lg_iter;
-    double2 M[2][2], w0 = make_double2(0, 0), w1 = w0;
-    if constexpr (SWEEP == kDirect) {
-        const KStep& ms = epi.plain[epi.k];
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int x = 0; x < 2; x++) M[b][x] = make_double2(ms.mre[b][x], ms.mim[b][x]);
-    } else {
-        const double* w = wext ? wext + 4 * epi.k : ctl->w;
-        w0 = make_double2(w[0], w[1]);
-        w1 = make_double2(w[2], w[3]);
-    }
-    uint64_t ks[NKS];
-#pragma unroll
-    for (int t = 0; t < NKS; t++) ks[t] = s.kspan[t];
-    const uint64_t lowmask = s.lowmask, xbit = s.xbit, rho = s.rho;
-    double acc[2] = {0, 0};
-    // One output from its NKS gathered inputs (u0: its address before the kernel span): S0, S1, then the branch norms
-    // (norm pass) or the write at cp.
-    auto output = [&](const S (&v)[NKS], uint64_t u0, uint64_t cp) {
-        double2 S0 = make_double2(0, 0), S1 = S0;
-#pragma unroll
-        for (int t = 0; t < NKS; t++) {
-            const uint64_t u = u0 ^ ks[t];
-            const double2 x = Cx<S>::widen(v[t]);
-            if (u & xbit) S1 = cadd(S1, negate_if(x, __popcll(u & lowmask & rho) & 1));
-            else S0 = cadd(S0, x);
-        }
-        if constexpr (SWEEP == kDirect) {
-            add_norm(acc[0], cfma(M[0][0], S0, cmul(M[0][1], S1)));
-            add_norm(acc[1], cfma(M[1][0], S0, cmul(M[1][1], S1)));
-        } else {
-            const double2 o = cfma(w0, S0, cmul(w1, S1));
-            const S so = Cx<S>::narrow(o);
-            Run<S, 1>::store(nw, cp, {so});
-            add_norm(acc[0], o);
-            add_norm(acc[1], Cx<S>::widen(so));
-        }
-    };
-    const uint64_t ab = a_thr ^ a_blk;
-    const uint64_t cb = (uint64_t(blockIdx.x) << 8) | uint64_t(tid);
-    constexpr int U = 4;        // tiles per iteration (every gather of the U tiles in flight at once)
-    if (niter >= U) {
-        // Tiles of a group: j & 1 selects output bit jit, j >> 1 the second direction -- the partner direction
-        // pdelta when the step has one (tiles j = 2, 3 then reuse the loads of tiles 0, 1, permuted by ptd: each
-        // table entry is read once instead of twice), else output bit jit + 1.  The other tile bits (jit + 1 ..
-        // rn - 1 without h, the second direction's top bit) take a Gray walk over the groups.
-        const bool share = s.ph >= 0;
-        const int h = share ? s.ph : jit + 1;
-        const uint64_t d0 = s.dep[jit];
-        const uint64_t D = share ? s.pD : s.dep[jit + 1];
-        const uint64_t dc = share ? s.pdelta : uint64_t(1) << (jit + 1);
-        const int td = s.ptd;
-        uint64_t a_g = 0, c_g = 0;
-        for (int g = 0; g < niter / U; g++) {
-            if (g) {
-                int b = jit + 1 + __builtin_ctz(unsigned(g));
-                if (b >= h) b++;
-                a_g ^= s.dep[b];
-                c_g ^= uint64_t(1) << b;
-            }
-            if (!active) continue;
-            S v[U][NKS];
-            if (share) {
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const uint64_t u0 = ab ^ a_g ^ (j ? d0 : 0);
-#pragma unroll
-                    for (int t = 0; t < NKS; t++) v[j][t] = old[(u0 ^ ks[t]) & lowmask];
-#pragma unroll
-                    for (int t = 0; t < NKS; t++) {           // v[j][t ^ td] by selects (no indexed registers)
-                        S x = v[j][0];
-#pragma unroll
-                        for (int q = 1; q < NKS; q++)
-                            if ((t ^ td) == q) x = v[j][q];
-                        v[j + 2][t] = x;
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < U; j++) {
-                    const uint64_t u0 = ab ^ a_g ^ ((j & 1) ? d0 : 0) ^ ((j & 2) ? D : 0);
-#pragma unroll
-                    for (int t = 0; t < NKS; t++) v[j][t] = old[(u0 ^ ks[t]) & lowmask];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < U; j++) {
-                const uint64_t u0 = ab ^ a_g ^ ((j & 1) ? d0 : 0) ^ ((j & 2) ? D : 0);
-                output(v[j], u0, (c_g | (uint64_t(j & 1) << jit) | cb) ^ ((j & 2) ? dc : 0));
-            }
-        }
-    } else {
-        uint64_t a_it = 0, c_it = 0;
-        for (int it = 0; it < niter; it++) {
-            if (it) {
-                const int b = __builtin_ctz(unsigned(it));
-                a_it ^= s.dep[jit + b];
-                c_it ^= uint64_t(1) << (jit + b);
-            }
-            if (!active) continue;
-            const uint64_t u0 = ab ^ a_it;
-            S v[NKS];
-#pragma unroll
-            for (int t = 0; t < NKS; t++) v[t] = old[(u0 ^ ks[t]) & lowmask];
-            output(v, u0, c_it | cb);
-        }
-    }
-    sweep_epilogue<2>(acc, part, ctl, epi, SWEEP);
-}
-
-// Entry 0 of a table set to 1 (start of a chain).
-template <class S>
-__global__ void table_one_kernel(S* t) { t[0] = Cx<S>::narrow(make_double2(1.0, 0.0)); }
-
-// ---------------------------------------------------------------------------------------------------------------
 // dispatch table
 
 // Kernel for (storage 0 = c64 / 1 = c128, log2 run, vg, ntq, route, sweep, next route); nullptr when not built.
@@ -483,26 +342,5 @@ void* run_apply_gram_kernel_ptr(int storage, int route2) {
 void* reduce_stored_gram_kernel_ptr() { return reinterpret_cast<void*>(&sweep_reduce_kernel<5>); }
 void* run_chunk_kernel_ptr() { return reinterpret_cast<void*>(&run_chunk_kernel); }
 void* run_decide_kernel_ptr() { return reinterpret_cast<void*>(&run_decide_kernel); }
-// Two-table kernels: sweep kDirect (norm pass) or kWrite; storage 0 = complex64, 1 = complex128.
-template <class S, int NKS>
-void* gather_for(int sweep) {
-    return sweep == kDirect ? reinterpret_cast<void*>(&gather_kernel<S, kDirect, NKS>)
-                            : reinterpret_cast<void*>(&gather_kernel<S, kWrite, NKS>);
-}
-template <class S>
-void* gather_by_nks(int sweep, int nks) {
-    switch (nks) {
-        case 1: return gather_for<S, 1>(sweep);
-        case 2: return gather_for<S, 2>(sweep);
-        case 4: return gather_for<S, 4>(sweep);
-    }
-    return nullptr;
-}
-void* gather_kernel_ptr(int storage, int sweep, int nks) {
-    return storage == 0 ? gather_by_nks<float2>(sweep, nks) : gather_by_nks<double2>(sweep, nks);
-}
-void* table_one_kernel_ptr(int storage) {
-    return storage == 0 ? reinterpret_cast<void*>(&table_one_kernel<float2>)
-                        : reinterpret_cast<void*>(&table_one_kernel<double2>);
-}
+
 }  // namespace gs

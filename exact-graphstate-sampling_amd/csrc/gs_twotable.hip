@@ -18,11 +18,13 @@
 
 #include "../../include/gsamp_amd.h"
 #include "gs_device.h"
+#include "gs_gf2.h"
 
 using namespace gs;
 
 namespace gs {
 void* gather_kernel_ptr(int storage, int sweep, int nks);
+void* gather_fold_kernel_ptr(int storage, int nks, int nd2, int share, int pure);
 void* table_one_kernel_ptr(int storage);
 void* decide_kernel_ptr();
 void* publish_kernel_ptr();
@@ -75,6 +77,10 @@ struct gs_tt_engine {
     void* tab[2] = {nullptr, nullptr};   // the two tables, 2^maxr entries each
     TStep* dsteps = nullptr;
     KStep* dplain = nullptr;             // M of each step (read by the decision)
+    std::vector<TFold> hfold;            // per step: its write folds in the next step's norms ...
+    std::vector<void*> fold_fn;          // ... with this kernel (nullptr: it does not)
+    std::vector<char> growth;            // per step: both branch norms follow from the stored table's norm
+    TFold* dfold = nullptr;
     std::vector<TStep> hsteps;
     double* part = nullptr;
     unsigned* counter = nullptr;
@@ -96,6 +102,7 @@ struct gs_tt_engine {
     unsigned char* h_amp = nullptr;
     int cur = 0;                         // table holding the current step's input after the last enqueue
     int grid_cap = kDefaultTTGridLog2;   // log2 of the most blocks a gather sweep launches
+    int fold_cap = kDefaultTTFoldGridLog2;   // ... one that folds in the next step's norms
 };
 
 namespace {
@@ -140,7 +147,7 @@ int parse_tt(FILE* f, bool with_m, gs_tt_plan& P) {
 void free_tt(gs_tt_engine* e) {
     if (!e) return;
     if (e->stream) (void)hipStreamSynchronize(e->stream);
-    for (void* p : {e->tab[0], e->tab[1], (void*)e->dsteps, (void*)e->dplain, (void*)e->part, (void*)e->counter,
+    for (void* p : {e->tab[0], e->tab[1], (void*)e->dsteps, (void*)e->dplain, (void*)e->dfold, (void*)e->part, (void*)e->counter,
                     (void*)e->ctl, (void*)e->d_forced, (void*)e->d_U, (void*)e->d_bits, (void*)e->d_cond,
                     (void*)e->d_out, (void*)e->d_w, (void*)e->d_amp})
         (void)hipFree(p);
@@ -177,7 +184,7 @@ int launch_gather(gs_tt_engine* e, int k, int sweep, int in, const Epi& epi, con
     void* fn = gather_kernel_ptr(e->storage, sweep, e->hsteps[size_t(k)].nks);
     if (!fn) return ttfail(15, "no gather kernel for step " + std::to_string(k));
     TT_TRY(hipLaunchKernel(fn, dim3(grid), dim3(kThreads), args, 0, e->stream));
-    if (grid > kFenceBlocks) {
+    if (!reduces_in_kernel(unsigned(grid), 1)) {
         const double* cpart = part;
         unsigned nblk = unsigned(grid);
         int sw = sweep;
@@ -187,10 +194,34 @@ int launch_gather(gs_tt_engine* e, int k, int sweep, int in, const Epi& epi, con
     return 0;
 }
 
-// Norms a step needs (gsamp.cpp chain: both branch norms directly; chain1 and forced run_steps steps: none).
-int tt_norm(int mode, int forced_bit) {
+// The write of step k with step k+1's norms folded in, reading table `in` and writing `1 - in`.
+int launch_fold(gs_tt_engine* e, int k, int in, const Epi& epi) {
+    const TStep* sp = e->dsteps + k;
+    const TFold* fp = e->dfold + k;
+    const void* old = e->tab[in];
+    void* nw = e->tab[1 - in];
+    double* part = e->part;
+    Ctl* ctl = e->ctl;
+    Epi ep = epi;
+    void* args[] = {&sp, &fp, &old, &nw, &part, &ctl, &ep};
+    const int grid = 1 << e->hfold[size_t(k)].lg_grid;
+    TT_TRY(hipLaunchKernel(e->fold_fn[size_t(k)], dim3(grid), dim3(kThreads), args, 0, e->stream));
+    if (!reduces_in_kernel(unsigned(grid), 1)) {
+        const double* cpart = part;
+        unsigned nblk = unsigned(grid);
+        int sw = kWriteDirect;
+        void* rargs[] = {&cpart, &nblk, &ctl, &ep, &sw};
+        TT_TRY(hipLaunchKernel(reduce_kernel_ptr(sw), dim3(1), dim3(kThreads), rargs, 0, e->stream));
+    }
+    return 0;
+}
+
+// Norms a step needs (gsamp.cpp chain: both branch norms directly; chain1, forced run_steps steps and growth steps:
+// none).
+int tt_norm(const gs_tt_engine* e, int mode, int k, int forced_bit) {
     if (mode == kChain1) return -1;
     if (mode == kRun && forced_bit >= 0) return -1;
+    if (e->growth[size_t(k)]) return -1;
     return kDirect;
 }
 
@@ -213,7 +244,7 @@ int tt_enqueue(gs_tt_engine* e, int mode, int k0, int k1, const int8_t* forced_h
     bool decided = false;
     for (int k = k0; k < k1; k++) {
         if (!decided && !wext) {
-            const int nm = tt_norm(mode, fb(k));
+            const int nm = tt_norm(e, mode, k, fb(k));
             Epi ep = base;
             ep.k = k;
             ep.role = kRoleNorm;
@@ -228,11 +259,15 @@ int tt_enqueue(gs_tt_engine* e, int mode, int k0, int k1, const int8_t* forced_h
         ep.role = kRoleWrite;
         if (k + 1 == k1) ep.next = kNextPublish;
         else if (wext) ep.next = kNextSweep;              // amplitude engine: weights given, no decision
-        else if (tt_norm(mode, fb(k + 1)) < 0) ep.next = kNextDecide;
-        else ep.next = kNextSweep;
-        if (int rc = launch_gather(e, k, kWrite, e->cur, ep, wext)) return rc;
+        else if (tt_norm(e, mode, k + 1, fb(k + 1)) < 0) ep.next = kNextDecide;
+        else ep.next = e->fold_fn[size_t(k)] ? int(kNextFusedDirect) : int(kNextSweep);
+        if (ep.next == kNextFusedDirect) {
+            if (int rc = launch_fold(e, k, e->cur, ep)) return rc;
+        } else {
+            if (int rc = launch_gather(e, k, kWrite, e->cur, ep, wext)) return rc;
+        }
         e->cur = 1 - e->cur;
-        decided = ep.next == kNextDecide;
+        decided = ep.next != kNextPublish && ep.next != kNextSweep;
     }
     return 0;
 }
@@ -342,6 +377,89 @@ void tt_geometry(gs_tt_engine* e) {
     }
 }
 
+// Which writes fold in the next step's norms: step k+1 must gather every (entry, x) exactly once, and the group of
+// outputs that holds one of its outputs' entries must leave at least a block of other coordinates.  A step whose every
+// output gathers one (entry, x) needs no pass at all.
+void tt_folds(gs_tt_engine* e) {
+    const int ns = e->plan.ns;
+    const size_t nsz = size_t(std::max(ns, 1));
+    e->hfold.assign(nsz, TFold{});
+    e->fold_fn.assign(nsz, nullptr);
+    e->growth.assign(nsz, 0);
+    auto once = [&](const TTStep& s) {                    // pivots and kernel span every address (c, x)
+        GfBasis b;
+        for (int i = 0; i <= s.r; i++)
+            if ((s.pivmask >> i) & 1) (void)b.add(uint64_t(1) << i);
+        for (uint64_t x : s.ker)
+            if (!b.add(x)) return false;
+        return b.n == s.r + 1;
+    };
+    for (int k = 0; k < ns; k++)
+        e->growth[size_t(k)] = e->plan.steps[size_t(k)].ker.empty() && once(e->plan.steps[size_t(k)]);
+    for (int k = 0; k + 1 < ns; k++) {
+        const TTStep &s0 = e->plan.steps[size_t(k)], &s1 = e->plan.steps[size_t(k) + 1];
+        const TStep& t0 = e->hsteps[size_t(k)];
+        if (s1.r != s0.rn || e->growth[size_t(k) + 1] || !once(s1)) continue;
+        TFold& f = e->hfold[size_t(k)];
+        const uint64_t xbit = uint64_t(1) << s1.r, low = xbit - 1;
+        std::vector<uint64_t> span{0};
+        for (uint64_t x : s1.ker) {
+            const size_t n = span.size();
+            for (size_t i = 0; i < n; i++) span.push_back(span[i] ^ x);
+        }
+        f.pure = std::find(span.begin(), span.end(), xbit) != span.end();
+        std::vector<uint64_t> dir;                        // kernel vectors with independent low parts
+        GfBasis lows;
+        for (uint64_t x : s1.ker)
+            if (lows.add(x & low)) dir.push_back(x);
+        f.nd2 = int(dir.size());
+        if (f.nd2 != int(s1.ker.size()) - (f.pure ? 1 : 0)) continue;
+        auto image = [&](uint64_t v) {
+            uint64_t a = 0;
+            for (int j = 0; j < s0.rn; j++)
+                if ((v >> j) & 1) a ^= t0.dep[j];
+            return a;
+        };
+        GfBasis W;
+        for (int i = 0; i < f.nd2; i++) {
+            f.dvec[i] = dir[size_t(i)] & low;
+            f.dimg[i] = image(f.dvec[i]);
+            (void)W.add(f.dvec[i]);
+        }
+        f.xk = 0;
+        for (int q = 0; q < (1 << f.nd2); q++) {
+            const uint64_t x = ((q & 1) ? dir[0] : 0) ^ ((q & 2) ? dir[1] : 0);
+            if (x & xbit) f.xk |= 1u << q;
+        }
+        f.rho = s1.rho;
+        // the partner direction of step k's outputs, when it is not one of the group's already
+        for (int q = 0; q < t0.nks && !f.share; q++) {
+            const uint64_t D = t0.xbit ^ t0.kspan[q];
+            uint64_t delta = 0, rest = D;
+            for (int j = 0; j < s0.rn; j++)
+                if (D & t0.dep[j]) {
+                    delta |= uint64_t(1) << j;
+                    rest &= ~t0.dep[j];
+                }
+            if (rest || !delta) continue;
+            if (W.add(delta)) {
+                f.share = 1;
+                f.pdelta = delta;
+                f.pimg = D;
+                f.ptd = q;
+            }
+            break;
+        }
+        int n = 0;
+        for (int b = 0; b < s0.rn; b++)
+            if (W.add(uint64_t(1) << b)) f.pos[n++] = uint8_t(b);
+        if (W.n != s0.rn || n < 8) continue;
+        f.lg_grid = std::min(n - 8, e->fold_cap);
+        f.lg_iter = n - 8 - f.lg_grid;
+        e->fold_fn[size_t(k)] = gather_fold_kernel_ptr(e->storage, t0.nks, f.nd2, f.share, f.pure);
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -414,6 +532,7 @@ int gs_tt_engine_create(const gs_tt_plan* plan, int storage, int device, gs_tt_e
             }
     }
     tt_geometry(e);
+    tt_folds(e);
     const size_t tbytes = (size_t(1) << e->plan.maxr) * e->esz;
     for (int i = 0; i < 2; i++)
         if (hipMalloc(&e->tab[i], tbytes) != hipSuccess) {
@@ -424,7 +543,8 @@ int gs_tt_engine_create(const gs_tt_plan* plan, int storage, int device, gs_tt_e
     const size_t C = gs_tt_engine::kChunk;
     auto dev_alloc = [&](void** p, size_t n) { return hipMalloc(p, std::max<size_t>(n, 16)) == hipSuccess; };
     auto host_alloc = [&](void** p, size_t n) { return hipHostMalloc(p, std::max<size_t>(n, 16), 0) == hipSuccess; };
-    bool ok = dev_alloc((void**)&e->dsteps, sizeof(TStep) * nsz) && dev_alloc((void**)&e->dplain, sizeof(KStep) * nsz) &&
+    bool ok = dev_alloc((void**)&e->dsteps, sizeof(TStep) * nsz) && dev_alloc((void**)&e->dfold, sizeof(TFold) * nsz) &&
+              dev_alloc((void**)&e->dplain, sizeof(KStep) * nsz) &&
               dev_alloc((void**)&e->part, sizeof(double) * kPartDoubles) &&
               dev_alloc((void**)&e->counter, sizeof(unsigned) * kCounters) && dev_alloc((void**)&e->ctl, sizeof(Ctl)) &&
               dev_alloc((void**)&e->d_forced, C * nsz) && dev_alloc((void**)&e->d_U, sizeof(double) * C * nsz) &&
@@ -438,6 +558,7 @@ int gs_tt_engine_create(const gs_tt_plan* plan, int storage, int device, gs_tt_e
     if (!ok) return bail(ttfail(11, "allocation of engine buffers failed"));
     if (hipStreamCreate(&e->stream) != hipSuccess) return bail(ttfail(17, "stream creation failed"));
     if (hipMemcpy(e->dsteps, e->hsteps.data(), sizeof(TStep) * nsz, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(e->dfold, e->hfold.data(), sizeof(TFold) * nsz, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(e->dplain, hplain.data(), sizeof(KStep) * nsz, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(e->counter, 0, sizeof(unsigned) * kCounters) != hipSuccess || hipDeviceSynchronize() != hipSuccess)
         return bail(ttfail(17, "plan upload failed"));
@@ -453,9 +574,12 @@ int gs_tt_set_grid_log2(gs_tt_engine* eng, int lg) {
     if (hipSetDevice(eng->device) != hipSuccess || hipStreamSynchronize(eng->stream) != hipSuccess)
         return ttfail(17, "device synchronisation failed");
     eng->grid_cap = lg ? lg : kDefaultTTGridLog2;
+    eng->fold_cap = lg ? lg : kDefaultTTFoldGridLog2;
     tt_geometry(eng);
+    tt_folds(eng);
     if (hipMemcpy(eng->dsteps, eng->hsteps.data(), sizeof(TStep) * eng->hsteps.size(), hipMemcpyHostToDevice) !=
-        hipSuccess)
+            hipSuccess ||
+        hipMemcpy(eng->dfold, eng->hfold.data(), sizeof(TFold) * eng->hfold.size(), hipMemcpyHostToDevice) != hipSuccess)
         return ttfail(17, "step upload failed");
     return 0;
 }
