@@ -46,7 +46,7 @@ using gs::PairSteps;
 
 constexpr int kLanes = 64;           // strings per wave (one lane group)
 constexpr int kWaves = 4;            // waves per block, each on its own part of the coset range
-constexpr int kRChunks = 64;         // chunks of the first reduction stage per lane group
+constexpr int kItemGroup = 64;       // items whose partials are reduced together before the groups are
 constexpr int kBThreads = kLanes * kWaves;
 constexpr int64_t kMinItems = 1024;  // work items (blocks) a step launch should have before tiles get coarser
 constexpr int kMaxSums = 8;          // per-lane sums of one item: the norms of one or two steps, or their G_k(x)
@@ -83,9 +83,9 @@ struct BInst {           // device view of one instance
     double* logp;        // [B]
     double* amp;         // [B][2]
     double* grad;        // [B][ns][2][2]: G_k(x) re, im (gradient mode)
-    double* part;        // [groups][items of the step per group][nq][64]: the items' nq sums
-    double* cpart;       // [groups][kRChunks][nq][64]: chunk sums of the item partials
-    int B, ns, pad0, pad1;
+    double* part;        // [lane groups][items of the step per lane group][nq][64]: the items' nq sums
+    unsigned* arrived;   // [lane groups][1 + narrived]: items (or item groups), and items of each item group, finished
+    int B, ns, narrived, pad;
 };
 
 // Per launch: what each instance's step sweep does besides the forward butterfly.
@@ -93,6 +93,7 @@ struct BLaunch {
     int k;
     int bookkeeping;     // 1: chain-mode conditionals / dead flags (scoring), 0: recomputation
     void* const* copy;   // [ninst] destination of a compact copy of this step's input table, or nullptr entries
+    unsigned long long* clock;   // [1 + ns]: device clock at the start and after each step (latest of its reductions)
 };
 
 typedef float f2v __attribute__((ext_vector_type(2)));
@@ -200,24 +201,110 @@ struct Walk {
     __device__ uint64_t coset(uint64_t t, int u) const { return cstart | ((t ^ (t >> 1)) << lu) | uint64_t(u); }
 };
 
-// Per-lane sum of NQ values over the block's waves (fixed order), stored as this item's partial (plain stores: the
-// per-(instance, lane group) reduction runs in batch_reduce_kernel after the step, at a launch boundary).
+// End of an item: its per-lane sums (over the block's waves, in order) become its partial, and the last item of its
+// (instance, lane group) to finish adds up the partials in a fixed order and ends the sweep of STEPS steps from step k
+// for those 64 lanes: chain1 bookkeeping (GRAD false: cond, prev, dead; gsamp2.cpp:67) or the gradient entries G_k.
+// With more than 2 kItemGroup items the last item of each kItemGroup consecutive ones reduces those first.  Partials are
+// published by atomic exchanges, which take effect where the counter does, before the counter is raised: no release
+// fence (each would write back the XCD's L2), and no reduction launches, which cost 8-20 us per step against the
+// 2-4 us an item's last block needs.
 template <int NQ>
-__device__ void lane_store(const BInst& I, const BItem& it, int wave, int lane, const double (&v)[NQ]) {
+__device__ __forceinline__ void add_partials(const double* from, int n, size_t stride, int wave, int lane,
+                                             double (&sh)[kWaves][NQ][kLanes]) {
+    double tot[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) tot[q] = 0;
+    for (int i = wave; i < n; i += kWaves)
+#pragma unroll
+        for (int q = 0; q < NQ; q++)
+            tot[q] += __hip_atomic_load(from + size_t(i) * stride + q * kLanes + lane, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();                                       // sh may still be read
+#pragma unroll
+    for (int q = 0; q < NQ; q++) sh[wave][q][lane] = tot[q];
+    __syncthreads();
+}
+
+template <int STEPS, bool GRAD>
+__device__ void item_end(const BInst& I, const BItem& it, int k, int wave, int lane,
+                         const double (&v)[STEPS * (GRAD ? 4 : 1)], unsigned long long* clock) {
+    constexpr int NQ = STEPS * (GRAD ? 4 : 1);
     __shared__ double sh[kWaves][NQ][kLanes];
+    __shared__ int s_last;
 #pragma unroll
     for (int q = 0; q < NQ; q++) sh[wave][q][lane] = v[q];
     __syncthreads();
-    double* part = I.part + (size_t(it.group) * size_t(it.count) + size_t(it.index)) * (NQ * kLanes);
+    const size_t stride = NQ * kLanes;
+    double* part = I.part + size_t(it.group) * size_t(it.count) * stride;
+    unsigned* total = I.arrived + size_t(it.group) * (1 + I.narrived);
+    // wave w adds up sums w, w + 4, ... of the block and publishes them at `to`; thread 0 then raises the counter: true
+    // for the block that makes it n
+    auto publish = [&](double* to, unsigned* counter, unsigned n) {
+        unsigned long long old = 0;
 #pragma unroll
-    for (int q0 = 0; q0 < NQ; q0 += kWaves) {            // wave w adds up sums w, w + 4, ...
-        const int q = q0 + wave;
-        if (q >= NQ) break;
-        double t = sh[0][q][lane];
+        for (int q0 = 0; q0 < NQ; q0 += kWaves) {
+            const int q = q0 + wave;
+            if (q >= NQ) break;
+            double t = sh[0][q][lane];
 #pragma unroll
-        for (int w = 1; w < kWaves; w++) t += sh[w][q][lane];
-        part[q * kLanes + lane] = t;
+            for (int w = 1; w < kWaves; w++) t += sh[w][q][lane];
+            old |= __hip_atomic_exchange(reinterpret_cast<unsigned long long*>(to + q * kLanes + lane),
+                                         (unsigned long long)__double_as_longlong(t), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(old) : : "memory");           // every exchange has returned
+        __syncthreads();
+        if (threadIdx.x == 0)
+            s_last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+        __syncthreads();
+        if (!s_last) return false;
+        __atomic_thread_fence(__ATOMIC_ACQUIRE);
+        if (threadIdx.x == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return true;
+    };
+    if (it.count > 1) {
+        double* mine = part + size_t(it.index) * stride;
+        if (it.count <= 2 * kItemGroup) {
+            if (!publish(mine, total, unsigned(it.count))) return;
+            add_partials<NQ>(part, it.count, stride, wave, lane, sh);
+        } else {                                           // a power of two, as kItemGroup
+            const int g = it.index / kItemGroup;
+            double* first = part + size_t(g) * kItemGroup * stride;
+            if (!publish(mine, total + 1 + g, unsigned(kItemGroup))) return;
+            add_partials<NQ>(first, kItemGroup, stride, wave, lane, sh);
+            if (!publish(first, total, unsigned(it.count / kItemGroup))) return;
+            add_partials<NQ>(part, it.count / kItemGroup, kItemGroup * stride, wave, lane, sh);
+        }
     }
+    if (wave != 0) return;
+    double tot[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        tot[q] = sh[0][q][lane];
+#pragma unroll
+        for (int w = 1; w < kWaves; w++) tot[q] += sh[w][q][lane];
+    }
+    const int b = it.group * kLanes + lane, ns = I.ns;
+    if constexpr (GRAD) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) I.grad[(size_t(b) * ns + k) * 4 + q] = tot[q];
+    } else {
+        double prev = I.prev[b];
+        bool dead = I.dead[b] != 0;
+#pragma unroll
+        for (int j = 0; j < STEPS; j++) {
+            if (dead) break;
+            I.cond[size_t(b) * ns + k + j] = tot[j] / (2 * prev);
+            prev = tot[j];
+            if (prev <= 0) {
+                for (int q = k + j; q < ns; q++) I.cond[size_t(b) * ns + q] = 0;
+                I.dead[b] = 1;
+                dead = true;
+            }
+        }
+        I.prev[b] = prev;
+    }
+    if (clock && lane == 0) atomicMax(clock + 1 + k, (unsigned long long)wall_clock64());
 }
 
 // The fields of a step that the inner loops use, copied to registers once per block (read through a reference to
@@ -319,7 +406,7 @@ __global__ __launch_bounds__(kBThreads) void batch_step_kernel(const BInst* __re
     }
     if (!L.bookkeeping) return;
     const double val[1] = {nb};
-    lane_store<1>(I, it, wave, lane, val);
+    item_end<1, false>(I, it, k, wave, lane, val, L.clock);
 }
 
 // Put a compact copy of step k's input table back into the forward arena (restart of a checkpoint segment).
@@ -435,7 +522,7 @@ __global__ __launch_bounds__(kBThreads) void batch_back_kernel(const BInst* __re
         }
     }
     const double val[4] = {g0.x, g0.y, g1.x, g1.y};
-    lane_store<4>(I, it, wave, lane, val);
+    item_end<1, true>(I, it, k, wave, lane, val, nullptr);
 }
 
 // ---- two steps per sweep (PairDesc)
@@ -593,7 +680,7 @@ __global__ __launch_bounds__(kBThreads) void pair_step_kernel(const BInst* __res
         }
     }
     if (!L.bookkeeping) return;
-    lane_store<2>(I, it, wave, lane, nb);
+    item_end<2, false>(I, it, k, wave, lane, nb, L.clock);
 }
 
 // Put a compact copy of a pair's input table back into the forward arena.
@@ -747,106 +834,15 @@ __global__ __launch_bounds__(kBThreads) void pair_back_kernel(const BInst* __res
         }
     }
     const double val[8] = {ga[0].x, ga[0].y, ga[1].x, ga[1].y, gb[0].x, gb[0].y, gb[1].x, gb[1].y};
-    lane_store<8>(I, it, wave, lane, val);
-}
-
-// After a sweep of STEPS steps from step k, batch_reduce_kernel sums the items' partials (cnt[inst] items per lane
-// group) per (instance, lane) in a fixed order over kRWaves waves and runs chain1 bookkeeping (GRAD false: cond, prev,
-// dead; gsamp2.cpp:67) or stores the gradient entries G_k.  Above kDirectItems items batch_chunk_kernel first sums
-// kRChunks chunks of consecutive items over many blocks, and the reduction takes the chunks.  One stage for few items:
-// the second launch costs 4 us and the 64 chunk sums of a lane were a serial chain of 12-16 us.
-constexpr int kRWaves = 8;
-constexpr int kDirectItems = 256;
-__host__ __device__ inline int chunk_items(int count) { return (count + kRChunks - 1) / kRChunks; }
-
-template <int NQ>
-__global__ __launch_bounds__(kBThreads) void batch_chunk_kernel(const BInst* __restrict__ insts,
-                                                               const int* __restrict__ cnt) {
-    const int inst = blockIdx.y, group = blockIdx.x / kRChunks, chunk = blockIdx.x % kRChunks;
-    const int lane = threadIdx.x & (kLanes - 1), wave = threadIdx.x / kLanes;
-    const BInst& I = insts[inst];
-    const int count = cnt[inst];
-    if (count <= kDirectItems || group >= I.B / kLanes) return;
-    const int per = chunk_items(count);
-    const int i0 = chunk * per, i1 = min(count, i0 + per);
-    if (i0 >= i1) return;
-    const double* gp = I.part + size_t(group) * size_t(count) * (NQ * kLanes);
-    double tot[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) tot[q] = 0;
-    for (int i = i0 + wave; i < i1; i += kWaves)
-#pragma unroll
-        for (int q = 0; q < NQ; q++) tot[q] += gp[(size_t(i) * NQ + q) * kLanes + lane];
-    __shared__ double sh[kWaves][NQ][kLanes];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) sh[wave][q][lane] = tot[q];
-    __syncthreads();
-    if (wave != 0) return;
-    double* out = I.cpart + (size_t(group) * kRChunks + chunk) * (NQ * kLanes);
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        double t = sh[0][q][lane];
-        for (int w = 1; w < kWaves; w++) t += sh[w][q][lane];
-        out[q * kLanes + lane] = t;
-    }
-}
-
-template <int STEPS, bool GRAD>
-__global__ __launch_bounds__(kLanes * kRWaves) void batch_reduce_kernel(const BInst* __restrict__ insts,
-                                                                        const int* __restrict__ cnt, int k) {
-    constexpr int NQ = STEPS * (GRAD ? 4 : 1);
-    const int inst = blockIdx.y, group = blockIdx.x;
-    const int lane = threadIdx.x & (kLanes - 1), wave = threadIdx.x / kLanes;
-    const BInst& I = insts[inst];
-    const int count = cnt[inst];
-    if (count == 0 || group >= I.B / kLanes) return;
-    const bool direct = count <= kDirectItems;
-    const int n = direct ? count : (count + chunk_items(count) - 1) / chunk_items(count);
-    const double* gp = direct ? I.part + size_t(group) * size_t(count) * (NQ * kLanes)
-                              : I.cpart + size_t(group) * kRChunks * (NQ * kLanes);
-    double tot[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) tot[q] = 0;
-    for (int c = wave; c < n; c += kRWaves)
-#pragma unroll
-        for (int q = 0; q < NQ; q++) tot[q] += gp[(size_t(c) * NQ + q) * kLanes + lane];
-    __shared__ double sh[kRWaves][NQ][kLanes];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) sh[wave][q][lane] = tot[q];
-    __syncthreads();
-    if (wave != 0) return;
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        tot[q] = sh[0][q][lane];
-#pragma unroll
-        for (int w = 1; w < kRWaves; w++) tot[q] += sh[w][q][lane];
-    }
-    const int b = group * kLanes + lane, ns = I.ns;
-    if constexpr (GRAD) {
-#pragma unroll
-        for (int q = 0; q < NQ; q++) I.grad[(size_t(b) * ns + k) * 4 + q] = tot[q];
-    } else {
-        double prev = I.prev[b];
-        bool dead = I.dead[b] != 0;
-#pragma unroll
-        for (int j = 0; j < STEPS; j++) {
-            if (dead) break;
-            I.cond[size_t(b) * ns + k + j] = tot[j] / (2 * prev);
-            prev = tot[j];
-            if (prev <= 0) {
-                for (int q = k + j; q < ns; q++) I.cond[size_t(b) * ns + q] = 0;
-                I.dead[b] = 1;
-                dead = true;
-            }
-        }
-        I.prev[b] = prev;
-    }
+    item_end<2, true>(I, it, k, wave, lane, val, nullptr);
 }
 
 template <class S>
-__global__ void batch_init_kernel(const BInst* __restrict__ insts, int ninst) {
+__global__ void batch_init_kernel(const BInst* __restrict__ insts, int ninst, unsigned long long* clock, int ns) {
     const int i = blockIdx.x;
     if (i >= ninst) return;
+    if (i == 0)
+        for (int k = threadIdx.x; k <= ns; k += blockDim.x) clock[k] = k ? 0 : (unsigned long long)wall_clock64();
     const BInst& I = insts[i];
     S* mem = static_cast<S*>(I.mem);
     for (int b = threadIdx.x; b < I.B; b += blockDim.x) {
@@ -909,7 +905,6 @@ struct gs_batch {
     std::vector<BItem*> ditems;           // in item_mem
     void* item_mem = nullptr;
     std::vector<int> nitems;
-    std::vector<char> chunked;            // per step: some lane group has more than kDirectItems items
     std::vector<std::vector<int>> lg;     // [inst][step]
     int lg_default = 8;                   // smallest tile (sizes the partial buffers); steps start at 2^9
     std::vector<int> nq;                  // per step: most slots per coset among the instances (kernel variant)
@@ -917,8 +912,6 @@ struct gs_batch {
     std::vector<std::vector<PairDesc>> hpairs;   // [inst][step]: steps k and k+1 as one sweep (ni 0: not possible)
     std::vector<char> unit;               // per step: steps of the sweep that starts there (1, 2; 0: inside a pair)
     bool pairs_on = true;
-    int* dcnt = nullptr;                  // device [maxns][ninst]: items per lane group of instance i at step k
-    int maxgroups = 1;
     int lu = 2;                           // log2 cosets a lane gathers at once
     bool items_dirty = false;             // tiles changed since the work lists were built
     int xcd_items = 1;                    // work lists ordered so each XCD takes consecutive items (2: coset-major)
@@ -928,7 +921,13 @@ struct gs_batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    std::vector<hipEvent_t> step_ev;      // event after each step (latency)
+    unsigned long long *dclock = nullptr, *hclock = nullptr;   // [1 + maxns]: device clock at the start, after each step
+    int clock_khz = 0;
+    // every instance's strings, and its results: log2 Pr, Z, the clock, then the conditionals of all; pinned copies
+    int8_t *dbits = nullptr, *hbits = nullptr;
+    double *dout = nullptr, *hout = nullptr;
+    size_t nbits = 0, nhead = 0, nout = 0;   // bytes of strings; doubles before the conditionals; in all
+    std::vector<size_t> at_bits, at_logp, at_amp, at_cond;
     double last_ms = 0;
     std::vector<double> step_ms;          // end of step k, ms after the start (last call)
     // gradient mode
@@ -1024,12 +1023,8 @@ int build_items(gs_batch* bt) {
     std::vector<BItem> all;                               // the lists of every step, in one allocation
     std::vector<size_t> at(size_t(bt->maxns), 0);
     const size_t ni = bt->plans.size();
-    std::vector<int> cnt(size_t(bt->maxns) * ni, 0);
-    bt->maxgroups = 1;
-    for (size_t i = 0; i < ni; i++) bt->maxgroups = std::max(bt->maxgroups, bt->B[i] / kLanes);
     bt->ditems.assign(size_t(bt->maxns), nullptr);
     bt->nitems.assign(size_t(bt->maxns), 0);
-    bt->chunked.assign(size_t(bt->maxns), 0);
     bt->nq.assign(size_t(bt->maxns), 1);
     bt->nq_exact.assign(size_t(bt->maxns), 0);
     choose_units(bt);
@@ -1055,8 +1050,6 @@ int build_items(gs_batch* bt) {
             sweep_size(bt, i, k, nk, inner);
             const int lg = item_lg(bt, i, k, shrink, finer);
             const int count = 1 << (nk - lg);
-            cnt[size_t(k) * ni + i] = count;
-            if (count > kDirectItems) bt->chunked[size_t(k)] = 1;
             const int ng = bt->B[i] / kLanes;
             for (int o = 0; o < ng * count; o++) {
                 // group-major (every coset range of lane group 0, then group 1, ...) or, with xcd_items == 2,
@@ -1100,24 +1093,22 @@ int build_items(gs_batch* bt) {
     if (hipMemcpy(bt->item_mem, all.data(), all.size() * sizeof(BItem), hipMemcpyHostToDevice) != hipSuccess)
         return bfail(17, "work-item upload failed");
     for (int k = 0; k < bt->maxns; k++) bt->ditems[size_t(k)] = static_cast<BItem*>(bt->item_mem) + at[size_t(k)];
-    if (!bt->dcnt && hipMalloc(&bt->dcnt, std::max<size_t>(cnt.size() * sizeof(int), 16)) != hipSuccess) {
-        bt->dcnt = nullptr;
-        return bfail(11, "count table allocation failed");
-    }
-    if (hipMemcpy(bt->dcnt, cnt.data(), cnt.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
-        return bfail(17, "count table upload failed");
     return 0;
 }
 
-// Doubles of one lane group's partials of instance i: four sums per lane of every item of a step at the smallest tile
-// gs_batch_set_tile accepts (2^lg_default cosets; a pair's eight at twice that tile), and the items of a launch that
-// was made finer (fewer than 2 kMinItems over all groups).
-size_t part_doubles(const gs_batch* bt, size_t i) {
+// Most items of one lane group of instance i in a launch: a step at the smallest tile gs_batch_set_tile accepts
+// (2^lg_default cosets), or a launch that was made finer (fewer than 2 kMinItems over all groups).
+size_t part_items(const gs_batch* bt, size_t i) {
     size_t m = 1;
     for (const gs::StepInfo& s : bt->plans[i].steps)
         m = std::max(m, size_t(1) << (s.nk - std::min(s.nk, bt->lg_default)));
+    return std::max(m, 2 * size_t(kMinItems) * kLanes / size_t(bt->B[i]));
+}
+
+// Doubles of one lane group's partials: four sums per lane of every item (a pair's eight at twice the smallest tile).
+size_t part_doubles(const gs_batch* bt, size_t i) {
     const size_t fine = 2 * size_t(kMinItems) * kLanes / size_t(bt->B[i]);
-    return kLanes * std::max(4 * m, size_t(kMaxSums) * std::max<size_t>(fine, 1));
+    return kLanes * std::max(4 * part_items(bt, i), size_t(kMaxSums) * std::max<size_t>(fine, 1));
 }
 
 // Instantiation of kernel K<S, NQ, LU, EX> for NQ in {1, 2, 4}, LU in 0..3, EX (every instance has NQ slots at the
@@ -1176,48 +1167,27 @@ int launch_batch(gs_batch* bt, BKernel kind, int k, BLaunch L) {
                                                                                       : bfail(17, "step launch failed");
 }
 
-// Per-(instance, lane) reduction of the item partials of the sweep at step k: chain bookkeeping or gradient entries.
-template <int STEPS, bool GRAD>
-int launch_reduce_t(gs_batch* bt, int k) {
-    const int* cnt = bt->dcnt + size_t(k) * bt->plans.size();
-    const int ninst = int(bt->plans.size());
-    if (bt->chunked[size_t(k)])
-        hipLaunchKernelGGL((batch_chunk_kernel<STEPS * (GRAD ? 4 : 1)>), dim3(bt->maxgroups * kRChunks, ninst),
-                           dim3(kBThreads), 0, bt->stream, bt->dinst, cnt);
-    hipLaunchKernelGGL((batch_reduce_kernel<STEPS, GRAD>), dim3(bt->maxgroups, ninst), dim3(kLanes * kRWaves), 0,
-                       bt->stream, bt->dinst, cnt, k);
-    return hipGetLastError() == hipSuccess ? 0 : bfail(17, "reduce launch failed");
-}
-
-int launch_reduce(gs_batch* bt, int k, bool grad) {
-    if (bt->nitems[size_t(k)] == 0) return 0;
-    if (bt->unit[size_t(k)] == 2) return grad ? launch_reduce_t<2, true>(bt, k) : launch_reduce_t<2, false>(bt, k);
-    return grad ? launch_reduce_t<1, true>(bt, k) : launch_reduce_t<1, false>(bt, k);
-}
-
 template <class S>
 int launch_step(gs_batch* bt, int k, int bookkeeping, void* const* copy) {
-    if (int rc = launch_batch<S>(bt, kBStep, k, BLaunch{k, bookkeeping, copy})) return rc;
-    return bookkeeping ? launch_reduce(bt, k, false) : 0;
+    return launch_batch<S>(bt, kBStep, k, BLaunch{k, bookkeeping, copy, bt->dclock});
 }
 
 template <class S>
-int enqueue_t(gs_batch* bt, bool record_steps) {
+int enqueue_t(gs_batch* bt) {
     const int ninst = int(bt->plans.size());
-    hipLaunchKernelGGL(batch_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
+    hipLaunchKernelGGL(batch_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst,
+                       bt->dclock, bt->maxns);
     for (int k = 0; k < bt->maxns; k++) {
         if (!bt->unit[size_t(k)]) continue;               // the second step of a pair
         if (int rc = launch_step<S>(bt, k, 1, nullptr)) return rc;
-        if (record_steps && bt->nitems[size_t(k)] && hipEventRecord(bt->step_ev[size_t(k)], bt->stream) != hipSuccess)
-            return bfail(17, "event record failed");
     }
     hipLaunchKernelGGL(batch_finish_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
     if (hipGetLastError() != hipSuccess) return bfail(17, "batch launch failed");
     return 0;
 }
 
-int enqueue(gs_batch* bt, bool record_steps) {
-    return bt->storage == GS_C64 ? enqueue_t<float2>(bt, record_steps) : enqueue_t<double2>(bt, record_steps);
+int enqueue(gs_batch* bt) {
+    return bt->storage == GS_C64 ? enqueue_t<float2>(bt) : enqueue_t<double2>(bt);
 }
 
 void drop_graph(gs_batch* bt) {
@@ -1231,7 +1201,7 @@ int build_graph(gs_batch* bt) {
     drop_graph(bt);
     if (hipStreamBeginCapture(bt->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
         return bfail(17, "stream capture failed");
-    const int rc = enqueue(bt, false);
+    const int rc = enqueue(bt);
     hipGraph_t g = nullptr;
     if (hipStreamEndCapture(bt->stream, &g) != hipSuccess || rc) return rc ? rc : bfail(17, "stream capture failed");
     bt->graph = g;
@@ -1239,20 +1209,23 @@ int build_graph(gs_batch* bt) {
     return 0;
 }
 
+// The strings of every instance, transposed to step-major, in one copy.
 int upload_bits(gs_batch* bt, const int8_t* const* bits) {
+    int8_t bad = 0;
     for (size_t i = 0; i < bt->plans.size(); i++) {
         const int B = bt->B[i], ns = bt->plans[i].ns;
-        std::vector<int8_t> t(size_t(B) * ns);
-        for (int b = 0; b < B; b++)
-            for (int k = 0; k < ns; k++) {
-                const int8_t v = bits[i][size_t(b) * ns + k];
-                if (v != 0 && v != 1) return bfail(16, "bits must be 0 or 1");
-                t[size_t(k) * B + b] = v;
-            }
-        if (hipMemcpyAsync(const_cast<int8_t*>(bt->hinst[i].bitsT), t.data(), t.size(), hipMemcpyHostToDevice, bt->stream) != hipSuccess ||
-            hipStreamSynchronize(bt->stream) != hipSuccess)
-            return bfail(17, "bits upload failed");
+        int8_t* to = bt->hbits + bt->at_bits[i];
+        for (int b0 = 0; b0 < B; b0 += kLanes)            // 64 strings at a time: whole cache lines of the result
+            for (int k = 0; k < ns; k++)
+                for (int b = b0; b < b0 + kLanes; b++) {
+                    const int8_t v = bits[i][size_t(b) * ns + k];
+                    bad |= v & ~int8_t(1);
+                    to[size_t(k) * B + b] = v;
+                }
     }
+    if (bad) return bfail(16, "bits must be 0 or 1");
+    if (bt->nbits && hipMemcpyAsync(bt->dbits, bt->hbits, bt->nbits, hipMemcpyHostToDevice, bt->stream) != hipSuccess)
+        return bfail(17, "bits upload failed");
     return 0;
 }
 
@@ -1398,7 +1371,7 @@ int grad_t(gs_batch* bt) {
     hipEvent_t e0 = bt->ev0, e1 = bt->ev1, em;
     if (hipEventCreate(&em) != hipSuccess) return bfail(17, "event creation failed");
     (void)hipEventRecord(e0, bt->stream);
-    hipLaunchKernelGGL(batch_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
+    hipLaunchKernelGGL(batch_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst, bt->dclock, ns);
     for (int k = 0; k < ns; k++)
         if (bt->unit[size_t(k)])
             if (int rc = launch_step<S>(bt, k, 1, fwd_ptr(k))) return rc;
@@ -1409,15 +1382,14 @@ int grad_t(gs_batch* bt) {
         const int k0 = s * seg, k1 = std::min(ns, k0 + seg);
         const int kf = seg_first(bt, seg, s);
         if (s != last && kf < k1) {                         // recompute the segment from its checkpoint
-            if (int rc = launch_batch<S>(bt, kBRestore, kf, BLaunch{kf, 0, ck_ptr(s)})) return rc;
+            if (int rc = launch_batch<S>(bt, kBRestore, kf, BLaunch{kf, 0, ck_ptr(s), nullptr})) return rc;
             for (int k = kf; k < k1; k++)
                 if (bt->unit[size_t(k)])
                     if (int rc = launch_step<S>(bt, k, 0, rec_ptr(k - k0))) return rc;
         }
         for (int k = k1 - 1; k >= kf; k--) {
             if (!bt->unit[size_t(k)]) continue;
-            if (int rc = launch_batch<S>(bt, kBBack, k, BLaunch{k, 0, rec_ptr(k - k0)})) return rc;
-            if (int rc = launch_reduce(bt, k, true)) return rc;
+            if (int rc = launch_batch<S>(bt, kBBack, k, BLaunch{k, 0, rec_ptr(k - k0), nullptr})) return rc;
         }
     }
     (void)hipEventRecord(e1, bt->stream);
@@ -1451,6 +1423,8 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
     auto bail = [&](int rc) {
         for (void* p : bt->allocs) (void)hipFree(p);
         (void)hipFree(bt->item_mem);
+        (void)hipHostFree(bt->hbits);
+        (void)hipHostFree(bt->hout);
         delete bt;
         return rc;
     };
@@ -1466,9 +1440,29 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
     if (hipStreamCreate(&bt->stream) != hipSuccess || hipEventCreate(&bt->ev0) != hipSuccess ||
         hipEventCreate(&bt->ev1) != hipSuccess)
         return bail(bfail(17, "stream creation failed"));
-    bt->step_ev.resize(size_t(bt->maxns));
-    for (auto& ev : bt->step_ev)
-        if (hipEventCreate(&ev) != hipSuccess) return bail(bfail(17, "event creation failed"));
+    if (hipDeviceGetAttribute(&bt->clock_khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || bt->clock_khz <= 0)
+        return bail(bfail(17, "device clock rate unknown"));
+    for (int i = 0; i < nplans; i++) {                    // strings and results of all instances, one buffer each
+        bt->at_bits.push_back(bt->nbits);
+        bt->nbits += size_t(lanes[i]) * size_t(bt->plans[size_t(i)].ns);
+        bt->at_logp.push_back(bt->nout);
+        bt->at_amp.push_back(bt->nout + size_t(lanes[i]));
+        bt->nout += 3 * size_t(lanes[i]);
+    }
+    const size_t at_clock = bt->nout;
+    bt->nhead = bt->nout += size_t(1 + bt->maxns);
+    for (int i = 0; i < nplans; i++) {
+        bt->at_cond.push_back(bt->nout);
+        bt->nout += size_t(lanes[i]) * size_t(bt->plans[size_t(i)].ns);
+    }
+    bt->dbits = dalloc<int8_t>(bt, bt->nbits);
+    bt->dout = dalloc<double>(bt, bt->nout);
+    bt->dclock = reinterpret_cast<unsigned long long*>(bt->dout + at_clock);
+    if (!bt->dbits || !bt->dout ||
+        hipHostMalloc(reinterpret_cast<void**>(&bt->hbits), std::max<size_t>(bt->nbits, 16), 0) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void**>(&bt->hout), std::max<size_t>(bt->nout * sizeof(double), 16), 0) != hipSuccess)
+        return bail(bfail(11, "batch buffer allocation failed"));
+    bt->hclock = reinterpret_cast<unsigned long long*>(bt->hout + at_clock);
     for (int i = 0; i < nplans; i++) {
         const gs::Plan& P = bt->plans[size_t(i)];
         const int B = lanes[i];
@@ -1514,10 +1508,10 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
             return at;
         };
         const size_t o_steps = take(hs.size() * sizeof(BStep)), o_pairs = take(hp.size() * sizeof(PairDesc)), head = used;
-        const size_t o_bits = take(size_t(P.ns) * B), o_prev = take(sizeof(double) * B), o_dead = take(sizeof(int) * B),
-                     o_cond = take(sizeof(double) * size_t(B) * P.ns), o_logp = take(sizeof(double) * B),
-                     o_amp = take(sizeof(double) * 2 * B),
-                     o_cpart = take(sizeof(double) * size_t(B / kLanes) * kRChunks * kLanes * kMaxSums),
+        I.narrived = int(part_items(bt, size_t(i)) / kItemGroup);
+        const size_t n_arrived = size_t(B / kLanes) * size_t(1 + I.narrived);
+        const size_t o_prev = take(sizeof(double) * B), o_dead = take(sizeof(int) * B),
+                     o_arrived = take(sizeof(unsigned) * n_arrived),
                      o_part = take(sizeof(double) * size_t(B / kLanes) * part_doubles(bt, size_t(i)));
         char* mem = dalloc<char>(bt, used);
         if (!mem) return bail(bfail(11, "batch buffer allocation failed"));
@@ -1530,13 +1524,15 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
         bt->hpairs.push_back(std::move(hp));
         I.steps = reinterpret_cast<BStep*>(mem + o_steps);
         I.pairs = reinterpret_cast<PairDesc*>(mem + o_pairs);
-        I.bitsT = reinterpret_cast<int8_t*>(mem + o_bits);
+        I.bitsT = bt->dbits + bt->at_bits[size_t(i)];
         I.prev = reinterpret_cast<double*>(mem + o_prev);
         I.dead = reinterpret_cast<int*>(mem + o_dead);
-        I.cond = reinterpret_cast<double*>(mem + o_cond);
-        I.logp = reinterpret_cast<double*>(mem + o_logp);
-        I.amp = reinterpret_cast<double*>(mem + o_amp);
-        I.cpart = reinterpret_cast<double*>(mem + o_cpart);
+        I.cond = bt->dout + bt->at_cond[size_t(i)];
+        I.logp = bt->dout + bt->at_logp[size_t(i)];
+        I.amp = bt->dout + bt->at_amp[size_t(i)];
+        I.arrived = reinterpret_cast<unsigned*>(mem + o_arrived);
+        if (hipMemset(I.arrived, 0, sizeof(unsigned) * n_arrived) != hipSuccess)
+            return bail(bfail(17, "counter initialisation failed"));
         I.part = reinterpret_cast<double*>(mem + o_part);
         bt->hinst.push_back(I);
     }
@@ -1559,8 +1555,8 @@ void gs_batch_destroy(gs_batch* bt) {
     free_grad(bt);
     for (void* p : bt->allocs) (void)hipFree(p);
     (void)hipFree(bt->item_mem);
-    (void)hipFree(bt->dcnt);
-    for (auto& ev : bt->step_ev) (void)hipEventDestroy(ev);
+    (void)hipHostFree(bt->hbits);
+    (void)hipHostFree(bt->hout);
     (void)hipEventDestroy(bt->ev0);
     (void)hipEventDestroy(bt->ev1);
     (void)hipStreamDestroy(bt->stream);
@@ -1659,28 +1655,30 @@ int gs_batch_score(gs_batch* bt, const int8_t* const* bits, double* const* log2p
             if (int rc = build_graph(bt)) return rc;
         if (hipGraphLaunch(bt->gexec, bt->stream) != hipSuccess) return bfail(17, "graph launch failed");
     } else {
-        if (int rc = enqueue(bt, true)) return rc;
+        if (int rc = enqueue(bt)) return rc;
     }
-    if (hipEventRecord(bt->ev1, bt->stream) != hipSuccess || hipEventSynchronize(bt->ev1) != hipSuccess)
+    bool any_cond = false;
+    for (size_t i = 0; i < bt->plans.size(); i++) any_cond = any_cond || (cond && cond[i]);
+    if (hipEventRecord(bt->ev1, bt->stream) != hipSuccess ||
+        hipMemcpyAsync(bt->hout, bt->dout, sizeof(double) * (any_cond ? bt->nout : bt->nhead), hipMemcpyDeviceToHost,
+                       bt->stream) != hipSuccess ||
+        hipStreamSynchronize(bt->stream) != hipSuccess)
         return bfail(17, "batch failed");
     float ms = 0;
     (void)hipEventElapsedTime(&ms, bt->ev0, bt->ev1);
     bt->last_ms = ms;
     bt->step_ms.assign(size_t(bt->maxns), -1.0);
     if (!bt->use_graph)
-        for (int k = 0; k < bt->maxns; k++) {
-            float t = 0;
-            if (bt->nitems[size_t(k)] && hipEventElapsedTime(&t, bt->ev0, bt->step_ev[size_t(k)]) == hipSuccess)
-                bt->step_ms[size_t(k)] = t;
-            else if (k > 0 && !bt->unit[size_t(k)]) bt->step_ms[size_t(k)] = bt->step_ms[size_t(k) - 1];   // pair
+        for (int k = 0; k < bt->maxns; k++) {             // the second step of a pair ends with the first
+            const int u = bt->unit[size_t(k)] ? k : k - 1;
+            if (bt->nitems[size_t(u)])
+                bt->step_ms[size_t(k)] = double(bt->hclock[size_t(1 + u)] - bt->hclock[0]) / bt->clock_khz;
         }
     for (size_t i = 0; i < bt->plans.size(); i++) {
-        const BInst& I = bt->hinst[i];
-        const int B = bt->B[i], ns = bt->plans[i].ns;
-        if (hipMemcpy(log2p[i], I.logp, sizeof(double) * size_t(B), hipMemcpyDeviceToHost) != hipSuccess ||
-            (cond && cond[i] && hipMemcpy(cond[i], I.cond, sizeof(double) * size_t(B) * ns, hipMemcpyDeviceToHost) != hipSuccess) ||
-            (amp && amp[i] && hipMemcpy(amp[i], I.amp, sizeof(double) * size_t(B) * 2, hipMemcpyDeviceToHost) != hipSuccess))
-            return bfail(17, "readback failed");
+        const size_t B = size_t(bt->B[i]), ns = size_t(bt->plans[i].ns);
+        memcpy(log2p[i], bt->hout + bt->at_logp[i], sizeof(double) * B);
+        if (cond && cond[i]) memcpy(cond[i], bt->hout + bt->at_cond[i], sizeof(double) * B * ns);
+        if (amp && amp[i]) memcpy(amp[i], bt->hout + bt->at_amp[i], sizeof(double) * B * 2);
     }
     return 0;
 }
@@ -1709,12 +1707,13 @@ int gs_batch_grad(gs_batch* bt, const int8_t* const* bits, double* const* log2p,
     if (seg_used) *seg_used = seg;
     if (int rc = upload_bits(bt, bits)) return rc;
     if (int rc = bt->storage == GS_C64 ? grad_t<float2>(bt) : grad_t<double2>(bt)) return rc;
+    if (hipMemcpy(bt->hout, bt->dout, sizeof(double) * bt->nhead, hipMemcpyDeviceToHost) != hipSuccess)
+        return bfail(17, "readback failed");
     for (size_t i = 0; i < bt->plans.size(); i++) {
-        const BInst& I = bt->hinst[i];
-        const int B = bt->B[i], ns = bt->plans[i].ns;
-        if (hipMemcpy(log2p[i], I.logp, sizeof(double) * size_t(B), hipMemcpyDeviceToHost) != hipSuccess ||
-            hipMemcpy(G[i], I.grad, sizeof(double) * size_t(B) * ns * 4, hipMemcpyDeviceToHost) != hipSuccess ||
-            (amp && amp[i] && hipMemcpy(amp[i], I.amp, sizeof(double) * size_t(B) * 2, hipMemcpyDeviceToHost) != hipSuccess))
+        const size_t B = size_t(bt->B[i]), ns = size_t(bt->plans[i].ns);
+        memcpy(log2p[i], bt->hout + bt->at_logp[i], sizeof(double) * B);
+        if (amp && amp[i]) memcpy(amp[i], bt->hout + bt->at_amp[i], sizeof(double) * B * 2);
+        if (hipMemcpy(G[i], bt->hinst[i].grad, sizeof(double) * B * ns * 4, hipMemcpyDeviceToHost) != hipSuccess)
             return bfail(17, "readback failed");
     }
     return 0;
