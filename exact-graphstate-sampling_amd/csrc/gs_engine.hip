@@ -328,7 +328,7 @@ struct gs_engine {
     double* d_U = nullptr;
     int8_t* d_bits = nullptr;
     double* d_cond = nullptr;
-    double* d_out = nullptr;        // [kChunk][4]
+    double* d_out = nullptr;        // [kChunk][4], followed by d_amp, d_bits and d_cond
     unsigned char* d_amp = nullptr; // [kChunk][16]
     int8_t* h_forced = nullptr;     // pinned mirrors
     double* h_U = nullptr;
@@ -1542,20 +1542,14 @@ void free_engine(gs_engine* e) {
     (void)hipFree(e->ctl_base);
     (void)hipFree(e->d_forced);
     (void)hipFree(e->d_U);
-    (void)hipFree(e->d_bits);
-    (void)hipFree(e->d_cond);
     (void)hipFree(e->d_out);
-    (void)hipFree(e->d_amp);
     (void)hipFree(e->drun);
     (void)hipFree(e->hpart);
     (void)hipFree(e->hchunk);
     (void)hipFree(e->rfac);
     (void)hipHostFree(e->h_forced);
     (void)hipHostFree(e->h_U);
-    (void)hipHostFree(e->h_bits);
-    (void)hipHostFree(e->h_cond);
     (void)hipHostFree(e->h_out);
-    (void)hipHostFree(e->h_amp);
     if (e->ev0) (void)hipEventDestroy(e->ev0);
     if (e->ev1) (void)hipEventDestroy(e->ev1);
     if (e->stream) (void)hipStreamDestroy(e->stream);
@@ -1571,12 +1565,26 @@ int begin_timing(gs_engine* e) {
 }
 
 int end_timing(gs_engine* e) {
-    if (!e->ev1) {
-        HIP_TRY(hipStreamSynchronize(e->stream));
-        return 0;
+    if (e->ev1) HIP_TRY(hipEventRecord(e->ev1, e->stream));
+    return 0;
+}
+
+// Results of strings 0 .. cnt-1 of the chunk (their scalars and bits; conditionals and amplitudes where asked for) to
+// the host, once the work is done: one copy behind the kernels and one wait for both.
+int finish_chunk(gs_engine* e, int cnt, bool bits, bool cond, bool amp) {
+    const size_t n = size_t(cnt), ns = size_t(ns_of(e));
+    if (e->own_buffers) {
+        unsigned char* const from = reinterpret_cast<unsigned char*>(e->d_out);
+        const unsigned char* end = cond ? reinterpret_cast<unsigned char*>(e->d_cond + n * ns)
+                                 : bits ? reinterpret_cast<unsigned char*>(e->d_bits + n * ns) : e->d_amp + 16 * n;
+        HIP_TRY(hipMemcpyAsync(e->h_out, from, size_t(end - from), hipMemcpyDeviceToHost, e->stream));
+    } else {
+        HIP_TRY(hipMemcpyAsync(e->h_out, e->d_out, n * 4 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
+        if (cond) HIP_TRY(hipMemcpyAsync(e->h_cond, e->d_cond, n * ns * sizeof(double), hipMemcpyDeviceToHost, e->stream));
+        if (amp) HIP_TRY(hipMemcpyAsync(e->h_amp, e->d_amp, n * 16, hipMemcpyDeviceToHost, e->stream));
     }
-    HIP_TRY(hipEventRecord(e->ev1, e->stream));
-    HIP_TRY(hipEventSynchronize(e->ev1));
+    HIP_TRY(hipStreamSynchronize(e->stream));
+    if (!e->ev1) return 0;
     float ms = 0;
     HIP_TRY(hipEventElapsedTime(&ms, e->ev0, e->ev1));
     e->last_ms += ms;
@@ -1655,11 +1663,7 @@ int run_forced(gs_engine* e, int mode, const int8_t* bits, int64_t nstr, double*
         if (int rc = begin_timing(e)) return rc;
         if (int rc = enqueue_strings(e, mode, cnt, true, amp != nullptr)) return rc;
         if (int rc = end_timing(e)) return rc;
-        HIP_TRY(hipMemcpyAsync(e->h_out, e->d_out, size_t(cnt) * 4 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        if (cond)
-            HIP_TRY(hipMemcpyAsync(e->h_cond, e->d_cond, size_t(cnt) * ns * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        if (amp) HIP_TRY(hipMemcpyAsync(e->h_amp, e->d_amp, size_t(cnt) * 16, hipMemcpyDeviceToHost, e->stream));
-        HIP_TRY(hipStreamSynchronize(e->stream));
+        if (int rc = finish_chunk(e, cnt, false, cond != nullptr, amp != nullptr)) return rc;
         for (int i = 0; i < cnt; i++) {
             log2p[s0 + i] = e->h_out[i * 4];
             if (cond) memcpy(cond + (s0 + i) * ns, e->h_cond + size_t(i) * ns, size_t(ns) * sizeof(double));
@@ -1744,19 +1748,24 @@ int gs_engine_create(const gs_plan* plan, int storage, int device, gs_engine** o
     auto host_alloc = [&](void** p, size_t n) { return hipHostMalloc(p, std::max<size_t>(n, 16), 0) == hipSuccess; };
     const size_t C = gs_engine::kChunk;
     const size_t nsz = size_t(std::max(ns, 1));
+    // a chunk's results in one buffer, so that one copy brings them back: scalars, amplitudes, bits, conditionals
+    const size_t out_bytes = C * (4 * sizeof(double) + 16 + nsz + sizeof(double) * nsz);
     bool ok = dev_alloc((void**)&e->dplain, sizeof(KStep) * nsz) && dev_alloc((void**)&e->dfused, sizeof(KStep) * nsz) &&
               dev_alloc((void**)&e->dlogical, sizeof(KStep) * nsz) &&
               dev_alloc((void**)&e->dsmall, sizeof(SStep) * nsz) && dev_alloc((void**)&e->dpair, sizeof(PStep) * nsz) &&
               dev_alloc((void**)&e->part_buf[0], 2 * sizeof(double) * kPartDoubles) &&
               dev_alloc((void**)&e->counter, sizeof(unsigned) * kCounters) &&
               dev_alloc((void**)&e->ctl_base, 2 * C * sizeof(Ctl)) && dev_alloc((void**)&e->d_forced, C * nsz) &&
-              dev_alloc((void**)&e->d_U, sizeof(double) * C * nsz) && dev_alloc((void**)&e->d_bits, C * nsz) &&
-              dev_alloc((void**)&e->d_cond, sizeof(double) * C * nsz) &&
-              dev_alloc((void**)&e->d_out, sizeof(double) * C * 4) && dev_alloc((void**)&e->d_amp, 16 * C) &&
-              host_alloc((void**)&e->h_forced, C * nsz) && host_alloc((void**)&e->h_U, sizeof(double) * C * nsz) &&
-              host_alloc((void**)&e->h_bits, C * nsz) && host_alloc((void**)&e->h_cond, sizeof(double) * C * nsz) &&
-              host_alloc((void**)&e->h_out, sizeof(double) * C * 4) && host_alloc((void**)&e->h_amp, 16 * C);
+              dev_alloc((void**)&e->d_U, sizeof(double) * C * nsz) && dev_alloc((void**)&e->d_out, out_bytes) &&
+              host_alloc((void**)&e->h_forced, C * nsz) && host_alloc((void**)&e->h_U, sizeof(double) * C * nsz) && host_alloc((void**)&e->h_out, out_bytes);
     if (!ok) return bail(fail(11, "allocation of engine buffers failed"));
+    auto place = [&](double* out, unsigned char*& amp, int8_t*& bits, double*& cond) {
+        amp = reinterpret_cast<unsigned char*>(out + 4 * C);
+        bits = reinterpret_cast<int8_t*>(amp + 16 * C);
+        cond = reinterpret_cast<double*>(bits + C * nsz);
+    };
+    place(e->d_out, e->d_amp, e->d_bits, e->d_cond);
+    place(e->h_out, e->h_amp, e->h_bits, e->h_cond);
     e->part_buf[1] = e->part_buf[0] + kPartDoubles;
     e->part = e->part_buf[0];
     e->ctl = e->ctl_base;
@@ -1810,9 +1819,7 @@ int gs_sample(gs_engine* eng, uint64_t seed, int64_t first, int64_t count, int s
         if (int rc = begin_timing(e)) return rc;
         if (int rc = enqueue_strings(e, kChain, cnt, false, false)) return rc;
         if (int rc = end_timing(e)) return rc;
-        HIP_TRY(hipMemcpyAsync(e->h_bits, e->d_bits, size_t(cnt) * ns, hipMemcpyDeviceToHost, e->stream));
-        HIP_TRY(hipMemcpyAsync(e->h_out, e->d_out, size_t(cnt) * 4 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        HIP_TRY(hipStreamSynchronize(e->stream));
+        if (int rc = finish_chunk(e, cnt, true, false, false)) return rc;
         memcpy(bits + s0 * ns, e->h_bits, size_t(cnt) * ns);
         for (int i = 0; i < cnt; i++) log2p[s0 + i] = e->h_out[i * 4];
     }
@@ -1842,10 +1849,7 @@ int gs_hybrid(gs_engine* eng, const int8_t* bits, int64_t nstr, uint64_t seed, i
         if (int rc = begin_timing(e)) return rc;
         if (int rc = enqueue_strings(e, kRun, cnt, true, false)) return rc;
         if (int rc = end_timing(e)) return rc;
-        HIP_TRY(hipMemcpyAsync(e->h_bits, e->d_bits, size_t(cnt) * ns, hipMemcpyDeviceToHost, e->stream));
-        HIP_TRY(hipMemcpyAsync(e->h_cond, e->d_cond, size_t(cnt) * ns * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        HIP_TRY(hipMemcpyAsync(e->h_out, e->d_out, size_t(cnt) * 4 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        HIP_TRY(hipStreamSynchronize(e->stream));
+        if (int rc = finish_chunk(e, cnt, true, true, false)) return rc;
         memcpy(out_bits + s0 * ns, e->h_bits, size_t(cnt) * ns);
         memcpy(cond + s0 * ns, e->h_cond, size_t(cnt) * ns * sizeof(double));
         for (int i = 0; i < cnt; i++) log2p[s0 + i] = e->h_out[i * 4];
@@ -1877,6 +1881,7 @@ int gs_prefix(gs_engine* eng, const int8_t* bits, int K, double* table_reim, int
     if (int rc = start_chain(e)) return rc;
     if (int rc = enqueue_run(e, kRun, 0, K, e->h_forced, e->d_forced, e->d_U, e->d_bits, e->d_cond, e->d_out)) return rc;
     if (int rc = end_timing(e)) return rc;
+    if (int rc = finish_chunk(e, 1, false, false, false)) return rc;
     void* doffs = nullptr;
     void* dtab = nullptr;
     HIP_TRY(hipMalloc(&doffs, sizeof(uint64_t) * offs.size()));
@@ -1896,7 +1901,6 @@ int gs_prefix(gs_engine* eng, const int8_t* bits, int K, double* table_reim, int
                            static_cast<const double2*>(e->arena), static_cast<const uint64_t*>(doffs), *ntq, n,
                            static_cast<double2*>(dtab));
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(e->h_out, e->d_out, 4 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipMemcpyAsync(table_reim, dtab, sizeof(double2) * size_t(n), hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
     (void)hipFree(doffs);
@@ -2004,13 +2008,7 @@ int gs_resume(gs_engine* eng, const int8_t* bits, int K, int nslices, const doub
         if ((rc = begin_timing(e))) break;
         if ((rc = enqueue_run(e, kRun, K, ns, e->h_forced, e->d_forced, e->d_U, e->d_bits, e->d_cond, e->d_out))) break;
         if ((rc = end_timing(e))) break;
-        if (hipMemcpyAsync(e->h_bits, e->d_bits, size_t(ns), hipMemcpyDeviceToHost, e->stream) != hipSuccess ||
-            hipMemcpyAsync(e->h_cond, e->d_cond, size_t(ns) * sizeof(double), hipMemcpyDeviceToHost, e->stream) != hipSuccess ||
-            hipMemcpyAsync(e->h_out, e->d_out, 4 * sizeof(double), hipMemcpyDeviceToHost, e->stream) != hipSuccess ||
-            hipStreamSynchronize(e->stream) != hipSuccess) {
-            rc = fail(17, "resume readback failed");
-            break;
-        }
+        if ((rc = finish_chunk(e, 1, true, true, false))) break;
         for (int k = 0; k < ns; k++) out_bits[k] = k < K ? bits[k] : e->h_bits[k];
         for (int k = K; k < ns; k++) cond[k] = e->h_cond[k];
         *log2p_prefix = lp_prefix;
