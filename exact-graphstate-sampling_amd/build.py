@@ -32,8 +32,8 @@ def _run(cmd, quiet_warn=True):
 def build_library():
     os.makedirs(BIN, exist_ok=True)
     cmds, objs = [], []
-    for src in ("gs_sweep_c64.hip", "gs_sweep_c128.hip", "gs_kernels.hip", "gs_gather.hip", "gs_small.hip",
-                "gs_pair.hip", "gs_engine.hip", "gs_batch.hip", "gs_twotable.hip", "gs_plan.cpp"):
+    for src in ("gs_sweep_c64.hip", "gs_sweep_c128.hip", "gs_kernels.hip", "gs_gather.hip", "gs_small.hip", "gs_pair.hip", "gs_fly.hip",
+                "gs_engine.hip", "gs_batch.hip", "gs_twotable.hip", "gs_plan.cpp"):
         obj = os.path.join(BIN, src.split(".")[0] + ".o")
         lang = [] if src.endswith(".hip") else ["-x", "hip"]
         cmds.append([HIPCC] + HIP_FLAGS + lang + ["-c", os.path.join(CSRC, src), "-o", obj])

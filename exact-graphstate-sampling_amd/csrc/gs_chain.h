@@ -137,15 +137,23 @@ __device__ void chain_step(const double (&red)[NQ], Ctl* ctl, const Epi& e, int 
         return;
     } else if (e.role == kRoleNorm) {
         decide(c, e, e.k, sweep, red);
-    } else if (NQ == 2 && e.role == kRolePair) {
-        finish_write(c, e, e.k, red[0], red[0]);
-        if (!c.dead) {
-            decide(c, e, e.k + 1, -1, nullptr);
-            finish_write(c, e, e.k + 1, red[1], red[1]);
+    } else if (NQ <= 4 && e.role == kRolePair) {
+        for (int i = 0; i < NQ && !c.dead; i++) {
+            if (i) decide(c, e, e.k + i, -1, nullptr);
+            finish_write(c, e, e.k + i, red[i], red[i]);
         }
         if (!c.dead) {
-            if (e.k + 2 == e.k1) publish(c, e);
-            else if (e.next == kNextDecide) decide(c, e, e.k + 2, -1, nullptr);
+            if (e.k + NQ == e.k1) publish(c, e);
+            else if (e.next == kNextDecide) decide(c, e, e.k + NQ, -1, nullptr);
+        }
+    } else if ((NQ == 4 || NQ == 6) && e.role == kRolePeek) {
+        double w[4];
+        for (int q = 0; q < 4; q++) w[q] = c.w[q];
+        finish_write(c, e, e.k, red[0], red[1]);
+        if (!c.dead) decide(c, e, e.k + 1, NQ == 6 ? kGram : kDirect, red + 2);
+        for (int q = 0; q < 4; q++) {
+            c.w2[q] = c.w[q];
+            c.w[q] = w[q];
         }
     } else {
         finish_write(c, e, e.k, red[0], red[1]);

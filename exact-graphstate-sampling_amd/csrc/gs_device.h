@@ -14,6 +14,12 @@ constexpr int kDefaultGridLog2 = 9;     // measured best for the width-30 sweeps
 // blocks a complex64 string takes 584 / 581 / 689 us at width 24 and 8.74 / 8.60 / 8.34 ms at width 29, a complex128 one
 // 89 / 97 / 97 us at width 20 and 4.13 / 4.56 / 4.42 ms at width 26.
 constexpr int kDefaultGridLog2Pair = 10, kDefaultGridLog2PairBig = 12, kBigPairLog2 = 26, kDefaultGridLog2PairWide = 9;
+constexpr int kDefaultGridLog2Fly = 10;   // butterfly sweeps (width 29 chain mode: 7.77 / 7.44 / 7.44 / 7.39 ms per
+                                          // string at 2^9 .. 2^12 blocks; complex128 width 23 0.635 / 0.639 / 0.635 / 0.655)
+// Sampled and forced complex128 strings take butterflies from 2^21 cosets on: below, a step's launches cost more than its
+// table (width 21: 235 us per string either way), and the allocation-free prob, whose results are those of prob bit for
+// bit, holds plans of at most 2^20.
+constexpr int kFlyMinNk = 21;
 constexpr int kDefaultGridLog2One = 12; // plain sweeps of one-slot steps: one load per thread and tile, so more waves
                                         // (width 34, 1-slot norm passes: 691 -> 343 ms per sample at 2^12 blocks)
 constexpr int kBigStepLog2 = 30;        // one-slot steps of at least 2^30 cosets take more blocks still:
@@ -163,6 +169,7 @@ struct Ctl {
     double logscale;       // run_steps: stored table = true table * 2^-logscale
     double sc;             // scale of the pending write
     double w[4];           // M[bv][0]*sc, M[bv][1]*sc as re, im pairs (read by the write sweep)
+    double w2[4];          // the same of the step after, decided before the pending write (kRolePeek)
     int bv;                // decision of the pending write
     int dead;              // a zero-probability branch was hit: later kernels do nothing
     int qidx;              // index of the next pre-drawn uniform (run_steps mode)
@@ -180,8 +187,10 @@ enum ChainMode { kChain = 0, kChain1 = 1, kRun = 2 };
 // What the last block of a sweep does after the sweep (kRoleStored: record the stored table's norm only -- the
 // product pass of a run of diagonal steps, whose decisions and bookkeeping were made before it).
 // kRoleStoredGram: the same, then the next step's decision from the Gram matrix the product pass summed.
-// kRolePair: a chain-mode sweep of steps k and k+1, whose sums are the two steps' written norms.
-enum EpiRole { kRoleNorm = 0, kRoleWrite = 1, kRoleStored = 2, kRoleStoredGram = 3, kRolePair = 4 };
+// kRolePair: a chain-mode sweep of two or three steps from step k on, whose sums are the steps' written norms.
+// kRolePeek: a read-only pass that applied step k in registers; step k+1's decision goes to w2, step k's write is still
+// to come.
+enum EpiRole { kRoleNorm = 0, kRoleWrite = 1, kRoleStored = 2, kRoleStoredGram = 3, kRolePair = 4, kRolePeek = 5 };
 // Write role: what follows step k.
 enum Next { kNextPublish = -2, kNextDecide = -1, kNextFusedGram = kGram, kNextFusedDirect = kDirect, kNextSweep = 3 };
 

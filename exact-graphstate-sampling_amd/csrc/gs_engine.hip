@@ -25,6 +25,7 @@
 
 #include "../../include/gsamp_amd.h"
 #include "gs_device.h"
+#include "gs_fly.h"
 #include "gs_gf2.h"
 #include "gs_plan.h"
 #include "gs_pstep.h"
@@ -39,11 +40,14 @@ void* reduce_kernel_ptr(int sweep);
 void* small_run_kernel_ptr(int storage);
 size_t small_run_lds(size_t tab_bytes);
 void* pair_sweep_kernel_ptr(int storage, int nq, int ni, int mo, int deg);
+void* fly_kernel_ptr(int storage, int ns);
+void* fly_norm_kernel_ptr(int norm, bool write);
+void* reduce3_kernel_ptr();
 void* reduce1_kernel_ptr();
+void* reduce_stored_gram_kernel_ptr();
 void* run_hist_kernel_ptr(int storage);
 void* run_apply_kernel_ptr(int storage);
 void* run_apply_gram_kernel_ptr(int storage, int route2);
-void* reduce_stored_gram_kernel_ptr();
 void* run_chunk_kernel_ptr();
 void* run_decide_kernel_ptr();
 }  // namespace gs
@@ -287,7 +291,8 @@ struct gs_engine {
     std::vector<KStep> hplain, hfused;
     std::vector<KStep> hlogical;    // plain steps in the plan's own coset coordinates (prefix/resume dump order)
     std::vector<char> fusable;
-    KStep* dplain = nullptr;
+    void *dmem = nullptr, *hmem = nullptr;   // the small device buffers, the pinned mirrors
+    KStep* dplain = nullptr;        // descriptors: see place_descriptors
     KStep* dfused = nullptr;
     KStep* dlogical = nullptr;
     struct Launch {
@@ -318,7 +323,7 @@ struct gs_engine {
     int fold_r = -1;                // sweeps of steps of at most 2^fold_r live slots reduce the partials the previous
                                     // sweep left (-1: none; every sweep measured slower on the width-26 plan: 4.560
                                     // against 4.484 ms per sample)
-    const double* pend_part = nullptr;
+    double* pend_part = nullptr;
     unsigned pend_nblk = 0;
     int pend_sweep = 0;
     Epi pend_epi{};
@@ -349,11 +354,16 @@ struct gs_engine {
     std::vector<SStep> hsmall;
     std::vector<int> small_at, small_dim;
     SStep* dsmall = nullptr;
-    // chain mode: steps k and k+1 as one sweep (gs_pair.hip)
-    bool allow_pairs = true;
+    // several steps per sweep: pairs of any two steps (gs_pair.hip), butterflies of two or three (gs_fly.hip)
+    bool allow_pairs = true;        // chain mode
+    bool allow_fly = true;          // the other modes
     std::vector<PStep> hpair;
-    std::vector<void*> pair_fn;     // the sweep of the pair that starts at a step, or nullptr
     PStep* dpair = nullptr;
+    std::vector<FlyDesc> hfly;      // [ns][kMaxFly - 1]: butterflies of the 2, 3, .. steps from each step on (d 0: none)
+    FlyDesc* dfly = nullptr;
+    std::vector<void*> unit_fn;     // chain mode: the sweep of several steps that starts at a step, or nullptr ...
+    std::vector<char> unit_len;     // ... its steps (a butterfly when unit_fly)
+    std::vector<char> unit_fly;
     bool fresh = false;             // the next launch starts the strings' chains
     int walk = 0;                   // tile order: 0 forward, 1 reverse on odd steps, 2 reverse on every step
     int fused_run = -1;             // log2 run of the fused layout (-1: the storage's default)
@@ -496,24 +506,39 @@ int launch_sweep(gs_engine* e, int k, int sweep, const Epi& epi) {
     return 0;
 }
 
-// The sweep of steps k and k+1 of a chain-mode string (both weights known, no scale).
-int launch_pair(gs_engine* e, int k, const Epi& epi) {
+size_t fly_at(size_t k, int d) { return (kMaxFly - 1) * k + size_t(d - 2); }
+
+// One sweep of several steps: kernel fn on descriptor desc, 2^lg_grid blocks, followed by the reduction of `sums` partial
+// sums where its blocks leave them.  k, tag: the step and sweep it is timed as.
+int launch_multi(gs_engine* e, void* fn, const void* desc, int lg_grid, const Epi& epi, int sums, int k, int tag) {
     if (int rc = launch_init(e)) return rc;
     if (int rc = flush_pending(e)) return rc;
-    const PStep* pp = e->dpair + k;
     void* mem = arena_of(e);
     double* part = e->strings > 1 ? e->slot_part[0] : e->part_buf[0];
     Ctl* ctl = e->ctl;
     Epi ep = epi;
-    const int grid = 1 << e->hpair[size_t(k)].lg_grid;
-    void* args[] = {&pp, &mem, &part, &ctl, &ep};
-    HIP_TRY(hipLaunchKernel(e->pair_fn[size_t(k)], dim3(grid, e->strings), dim3(kThreads), args, 0, e->stream));
+    const int grid = 1 << lg_grid;
+    void* args[] = {&desc, &mem, &part, &ctl, &ep};
+    hipEvent_t a = nullptr, b = nullptr;
+    if (e->profile) {
+        HIP_TRY(hipEventCreate(&a));
+        HIP_TRY(hipEventCreate(&b));
+        HIP_TRY(hipEventRecord(a, e->stream));
+    }
+    HIP_TRY(hipLaunchKernel(fn, dim3(grid, e->strings), dim3(kThreads), args, 0, e->stream));
+    if (e->profile) {
+        HIP_TRY(hipEventRecord(b, e->stream));
+        e->pev.push_back(a);
+        e->pev.push_back(b);
+        e->pev_tag.push_back(k * 8 + tag);
+    }
     if (!reduces_in_kernel(unsigned(grid), unsigned(e->strings))) {
         const double* cpart = part;
         unsigned nblk = unsigned(grid);
-        int sw = kWrite;
+        int sw = sums == 6 ? kWriteGram : sums == 4 ? kWriteDirect : kWrite;
         void* rargs[] = {&cpart, &nblk, &ctl, &ep, &sw};
-        HIP_TRY(hipLaunchKernel(reduce_kernel_ptr(sw), dim3(1, e->strings), dim3(kThreads), rargs, 0, e->stream));
+        HIP_TRY(hipLaunchKernel(sums == 3 ? reduce3_kernel_ptr() : reduce_kernel_ptr(sw), dim3(1, e->strings),
+                                dim3(kThreads), rargs, 0, e->stream));
     }
     return 0;
 }
@@ -725,13 +750,41 @@ int enqueue_run(gs_engine* e, int mode, int k0, int k1, const int8_t* forced_h, 
         Epi ep = base;
         ep.k = k;
         ep.role = kRoleWrite;
-        if (mode == kChain1 && e->allow_pairs && !e->profile && k + 1 < k1 && e->pair_fn[size_t(k)]) {
+        if (mode == kChain1 && e->allow_pairs && !e->profile && e->unit_fn[size_t(k)] && k + e->unit_len[size_t(k)] <= k1) {
+            const int n = e->unit_len[size_t(k)];
+            const bool fly = e->unit_fly[size_t(k)] != 0;
             ep.role = kRolePair;
-            ep.next = k + 2 == k1 ? kNextPublish : run_from(e, k + 2, k1) >= 0 ? kNextSweep : kNextDecide;
-            if (int rc = launch_pair(e, k, ep)) return rc;
+            ep.next = k + n == k1 ? kNextPublish : run_from(e, k + n, k1) >= 0 ? kNextSweep : kNextDecide;
+            const size_t at = fly_at(size_t(k), n);
+            const void* desc = fly ? static_cast<const void*>(e->dfly + at) : e->dpair + k;
+            if (int rc = launch_multi(e, e->unit_fn[size_t(k)], desc,
+                                      fly ? e->hfly[at].lg_grid : e->hpair[size_t(k)].lg_grid, ep, n, k, 0))
+                return rc;
             decided = ep.next != kNextSweep;
-            k++;
+            k += n - 1;
             continue;
+        }
+        // steps k, k+1 and the norms of k+2: a read-only pass decides step k+1, one write does both steps
+        if (mode != kChain1 && e->storage == GS_C128 && e->allow_fly && e->allow_fusion && e->fold_r < 0 && k + 2 < k1 &&
+            e->hfly[fly_at(size_t(k), 3)].d && e->hplain[size_t(k)].nk >= kFlyMinNk) {
+            const int n1 = norm_for(e, mode, k + 1, fb(k + 1), fstr), n2 = norm_for(e, mode, k + 2, fb(k + 2), fstr);
+            if (n1 >= 0 && n1 == n2) {
+                const int norm = n1 == kGram ? 1 : 2, sums = n1 == kGram ? 6 : 4;
+                ep.role = kRolePeek;
+                if (int rc = launch_multi(e, fly_norm_kernel_ptr(norm, false), e->dfly + fly_at(size_t(k), 2),
+                                          e->hfly[fly_at(size_t(k), 2)].lg_grid, ep, sums, k + 1, n1))
+                    return rc;
+                ep.k = k + 1;
+                ep.role = kRoleWrite;
+                ep.next = n1;
+                if (int rc = launch_multi(e, fly_norm_kernel_ptr(norm, true), e->dfly + fly_at(size_t(k), 3),
+                                          e->hfly[fly_at(size_t(k), 3)].lg_grid, ep, sums, k + 1,
+                                          n1 == kGram ? kWriteGram : kWriteDirect))
+                    return rc;
+                decided = true;
+                k++;
+                continue;
+            }
         }
         int sweep = kWrite;
         if (k + 1 == k1) {
@@ -1340,24 +1393,44 @@ void build_small(gs_engine* e) {
     }
 }
 
-// Pairs of steps of the chain mode: steps outside the runs of small and of diagonal steps whose super-cosets give a
-// thread one aligned 16-byte run per slot and leave step k+1's slot index the same over the threads' coordinates.  Each
-// saves the write and the read of the table between its steps and a launch; the pairs are the disjoint ones that save
-// the most.
-void build_pairs(gs_engine* e) {
+// Sweeps of several steps: steps outside the runs of small and of diagonal steps whose groups give a thread one aligned
+// 16-byte run per slot and leave the later steps' slot indices the same over the threads' coordinates.  In chain mode
+// each saves the write and the read of the tables between its steps and a launch; the units are the disjoint ones that
+// save the most.
+void build_units(gs_engine* e) {
     const Plan& P = e->plan;
     const size_t ns = size_t(P.ns);
     e->hpair.assign(std::max<size_t>(ns, 1), PStep{});
-    e->pair_fn.assign(std::max<size_t>(ns, 1), nullptr);
+    e->hfly.assign((kMaxFly - 1) * std::max<size_t>(ns, 1), FlyDesc{});
+    e->unit_fn.assign(std::max<size_t>(ns, 1), nullptr);
+    e->unit_len.assign(std::max<size_t>(ns, 1), 0);
+    e->unit_fly.assign(std::max<size_t>(ns, 1), 0);
     if (!e->own_buffers) return;                          // prob only
     const int lr = e->storage == GS_C64 ? 1 : 0;
     std::vector<char> taken(ns, 0);
     for (size_t k = 0; k < ns; k++) taken[k] = e->small_at[k] >= 0;
     for (const RStep& r : e->hrun)
         for (int i = 0; i < r.j; i++) taken[size_t(r.k0 + i)] = 1;
-    std::vector<double> best(ns + 2, 0.0), gain(ns, 0.0);
+    std::vector<double> best(ns + kMaxFly, 0.0), gain(ns, 0.0);
     std::vector<void*> fn(ns, nullptr);
     for (size_t k = 0; k + 1 < ns; k++) {
+        for (int d = 2; d <= kMaxFly; d++) {
+            FlyDesc& f = e->hfly[fly_at(k, d)];
+            const StepInfo* p[kMaxFly] = {};
+            bool ok = k + size_t(d) <= ns;
+            for (int i = 0; i < d && ok; i++) {
+                ok = !taken[k + size_t(i)];
+                p[i] = &P.steps[k + size_t(i)];
+            }
+            if (!ok || !make_fly(p, d, lr, 8, f)) {
+                f.d = 0;
+                break;
+            }
+            f.xcd = e->xcd_blocks;
+            const int tiles = f.nk - lr - 8;
+            f.lg_grid = std::min(tiles, e->grid_cap2 ? e->grid_cap2 : kDefaultGridLog2Fly);
+            f.lg_iter = tiles - f.lg_grid;
+        }
         if (taken[k] || taken[k + 1]) continue;
         const StepInfo &s0 = P.steps[k], &s1 = P.steps[k + 1];
         PStep& p = e->hpair[k];
@@ -1394,12 +1467,19 @@ void build_pairs(gs_engine* e) {
         fn[k] = pair_sweep_kernel_ptr(e->storage, s0.ntq, p.d.ni, p.d.mo, p.d.deg);
         if (fn[k]) gain[k] = 20e6 + 2.0 * double(e->esz) * double(uint64_t(s0.m) << s0.nk);
     }
-    for (size_t k = ns; k-- > 0;) best[k] = std::max(best[k + 1], fn[k] ? gain[k] + best[k + 2] : 0.0);
-    for (size_t k = 0; k < ns; k++)
-        if (fn[k] && gain[k] + best[k + 2] > best[k + 1]) {
-            e->pair_fn[k] = fn[k];
-            k++;
+    for (size_t k = ns; k-- > 0;) {
+        best[k] = best[k + 1];
+        for (int n = 2; n <= kMaxFly && k + size_t(n) <= ns; n++) {
+            const bool fly = e->hfly[fly_at(k, n)].d == n;
+            if (!fly && (n > 2 || !fn[k])) continue;
+            const double g = fly ? (n - 1) * (20e6 + 2.0 * double(e->esz) * double(uint64_t(2) << P.steps[k].nk)) : gain[k];
+            if (g + best[k + size_t(n)] <= best[k]) continue;
+            best[k] = g + best[k + size_t(n)];
+            e->unit_len[k] = char(n);
+            e->unit_fly[k] = fly;
+            e->unit_fn[k] = fly ? fly_kernel_ptr(e->storage, n) : fn[k];
         }
+    }
 }
 
 int build_steps(gs_engine* e) {
@@ -1492,20 +1572,43 @@ int build_steps(gs_engine* e) {
     }
     build_runs(e);
     build_small(e);
-    build_pairs(e);
+    build_units(e);
     return 0;
 }
 
 // Copy the step and run descriptors to the device, growing the run arrays (and allocating the pattern-sum buffers the
 // first time the plan has a run).
-int upload_descriptors(gs_engine* e, bool logical) {
-    const size_t ns = size_t(e->plan.ns);
-    if (ns) {
-        HIP_TRY(hipMemcpy(e->dplain, e->hplain.data(), sizeof(KStep) * ns, hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(e->dfused, e->hfused.data(), sizeof(KStep) * ns, hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(e->dpair, e->hpair.data(), sizeof(PStep) * ns, hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(e->dsmall, e->hsmall.data(), sizeof(SStep) * ns, hipMemcpyHostToDevice));
-        if (logical) HIP_TRY(hipMemcpy(e->dlogical, e->hlogical.data(), sizeof(KStep) * ns, hipMemcpyHostToDevice));
+// Bytes of the step descriptors on the device, and their places in one buffer there.
+size_t place_descriptors(gs_engine* e, unsigned char* base) {
+    const size_t ns = size_t(std::max(e->plan.ns, 1));
+    size_t used = 0;
+    auto put = [&](auto*& p, size_t n) {
+        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + used);
+        used += (n * sizeof(*p) + 255) & ~size_t(255);
+    };
+    put(e->dplain, ns);
+    put(e->dfused, ns);
+    put(e->dlogical, ns);
+    put(e->dsmall, ns);
+    put(e->dpair, ns);
+    put(e->dfly, (kMaxFly - 1) * ns);
+    return used;
+}
+
+int upload_descriptors(gs_engine* e) {
+    if (e->plan.ns) {
+        unsigned char* const base = reinterpret_cast<unsigned char*>(e->dplain);
+        std::vector<unsigned char> up(place_descriptors(e, base));
+        auto put = [&](const auto& from, const void* to) {
+            memcpy(up.data() + (static_cast<const unsigned char*>(to) - base), from.data(), from.size() * sizeof(from[0]));
+        };
+        put(e->hplain, e->dplain);
+        put(e->hfused, e->dfused);
+        put(e->hlogical, e->dlogical);
+        put(e->hsmall, e->dsmall);
+        put(e->hpair, e->dpair);
+        put(e->hfly, e->dfly);
+        HIP_TRY(hipMemcpy(base, up.data(), up.size(), hipMemcpyHostToDevice));
     }
     if (e->hrun.empty()) return 0;
     if (e->hrun.size() > e->drun_cap) {
@@ -1531,25 +1634,13 @@ void free_engine(gs_engine* e) {
     (void)hipSetDevice(e->device);
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     (void)hipFree(e->arena);
-    (void)hipFree(e->dplain);
-    (void)hipFree(e->dfused);
-    (void)hipFree(e->dlogical);
-    (void)hipFree(e->dsmall);
-    (void)hipFree(e->dpair);
-    (void)hipFree(e->part_buf[0]);
+    (void)hipFree(e->dmem);
     (void)hipFree(e->slots);
-    (void)hipFree(e->counter);
-    (void)hipFree(e->ctl_base);
-    (void)hipFree(e->d_forced);
-    (void)hipFree(e->d_U);
-    (void)hipFree(e->d_out);
     (void)hipFree(e->drun);
     (void)hipFree(e->hpart);
     (void)hipFree(e->hchunk);
     (void)hipFree(e->rfac);
-    (void)hipHostFree(e->h_forced);
-    (void)hipHostFree(e->h_U);
-    (void)hipHostFree(e->h_out);
+    (void)hipHostFree(e->hmem);
     if (e->ev0) (void)hipEventDestroy(e->ev0);
     if (e->ev1) (void)hipEventDestroy(e->ev1);
     if (e->stream) (void)hipStreamDestroy(e->stream);
@@ -1744,21 +1835,35 @@ int gs_engine_create(const gs_plan* plan, int storage, int device, gs_engine** o
         e->arena = nullptr;
         return bail(fail(11, "allocation of " + std::to_string(bytes) + " bytes failed"));
     }
-    auto dev_alloc = [&](void** p, size_t n) { return hipMalloc(p, std::max<size_t>(n, 16)) == hipSuccess; };
-    auto host_alloc = [&](void** p, size_t n) { return hipHostMalloc(p, std::max<size_t>(n, 16), 0) == hipSuccess; };
     const size_t C = gs_engine::kChunk;
     const size_t nsz = size_t(std::max(ns, 1));
     // a chunk's results in one buffer, so that one copy brings them back: scalars, amplitudes, bits, conditionals
     const size_t out_bytes = C * (4 * sizeof(double) + 16 + nsz + sizeof(double) * nsz);
-    bool ok = dev_alloc((void**)&e->dplain, sizeof(KStep) * nsz) && dev_alloc((void**)&e->dfused, sizeof(KStep) * nsz) &&
-              dev_alloc((void**)&e->dlogical, sizeof(KStep) * nsz) &&
-              dev_alloc((void**)&e->dsmall, sizeof(SStep) * nsz) && dev_alloc((void**)&e->dpair, sizeof(PStep) * nsz) &&
-              dev_alloc((void**)&e->part_buf[0], 2 * sizeof(double) * kPartDoubles) &&
-              dev_alloc((void**)&e->counter, sizeof(unsigned) * kCounters) &&
-              dev_alloc((void**)&e->ctl_base, 2 * C * sizeof(Ctl)) && dev_alloc((void**)&e->d_forced, C * nsz) &&
-              dev_alloc((void**)&e->d_U, sizeof(double) * C * nsz) && dev_alloc((void**)&e->d_out, out_bytes) &&
-              host_alloc((void**)&e->h_forced, C * nsz) && host_alloc((void**)&e->h_U, sizeof(double) * C * nsz) && host_alloc((void**)&e->h_out, out_bytes);
-    if (!ok) return bail(fail(11, "allocation of engine buffers failed"));
+    // the small buffers in one allocation, the pinned mirrors in another
+    size_t used = place_descriptors(e, nullptr), pinned = 0;
+    auto take = [](size_t& at, size_t n) {
+        const size_t a = at;
+        at += (n + 255) & ~size_t(255);
+        return a;
+    };
+    const size_t o_part = take(used, 2 * sizeof(double) * kPartDoubles), o_counter = take(used, sizeof(unsigned) * kCounters),
+                 o_ctl = take(used, 2 * C * sizeof(Ctl)), o_forced = take(used, C * nsz),
+                 o_U = take(used, sizeof(double) * C * nsz), o_out = take(used, out_bytes);
+    const size_t p_forced = take(pinned, C * nsz), p_U = take(pinned, sizeof(double) * C * nsz),
+                 p_out = take(pinned, out_bytes);
+    if (hipMalloc(&e->dmem, used) != hipSuccess || hipHostMalloc(&e->hmem, pinned, 0) != hipSuccess)
+        return bail(fail(11, "allocation of engine buffers failed"));
+    unsigned char *const db = static_cast<unsigned char*>(e->dmem), *const hb = static_cast<unsigned char*>(e->hmem);
+    (void)place_descriptors(e, db);
+    e->part_buf[0] = reinterpret_cast<double*>(db + o_part);
+    e->counter = reinterpret_cast<unsigned*>(db + o_counter);
+    e->ctl_base = reinterpret_cast<Ctl*>(db + o_ctl);
+    e->d_forced = reinterpret_cast<int8_t*>(db + o_forced);
+    e->d_U = reinterpret_cast<double*>(db + o_U);
+    e->d_out = reinterpret_cast<double*>(db + o_out);
+    e->h_forced = reinterpret_cast<int8_t*>(hb + p_forced);
+    e->h_U = reinterpret_cast<double*>(hb + p_U);
+    e->h_out = reinterpret_cast<double*>(hb + p_out);
     auto place = [&](double* out, unsigned char*& amp, int8_t*& bits, double*& cond) {
         amp = reinterpret_cast<unsigned char*>(out + 4 * C);
         bits = reinterpret_cast<int8_t*>(amp + 16 * C);
@@ -1772,7 +1877,7 @@ int gs_engine_create(const gs_plan* plan, int storage, int device, gs_engine** o
     if (hipStreamCreate(&e->stream) != hipSuccess || hipEventCreate(&e->ev0) != hipSuccess ||
         hipEventCreate(&e->ev1) != hipSuccess)
         return bail(fail(17, "stream/event creation failed"));
-    if (int rc = upload_descriptors(e, true)) return bail(rc);
+    if (int rc = upload_descriptors(e)) return bail(rc);
     if (hipMemset(e->counter, 0, sizeof(unsigned) * kCounters) != hipSuccess || hipDeviceSynchronize() != hipSuccess)
         return bail(fail(17, "counter initialisation failed"));
     e->prof_ms.assign(nsz * kNumSweeps, 0.0);
@@ -2105,7 +2210,7 @@ static int set_grid_caps(gs_engine* eng, int lg, bool one_slot_only) {
     eng->grid_cap1 = lg ? lg : kDefaultGridLog2One;
     eng->grid_cap1_big = lg ? lg : kDefaultGridLog2OneBig;
     if (int rc = build_steps(eng)) return rc;
-    return upload_descriptors(eng, true);
+    return upload_descriptors(eng);
 }
 
 int gs_set_grid_log2(gs_engine* eng, int lg) { return set_grid_caps(eng, lg, false); }
@@ -2130,7 +2235,7 @@ int gs_set_fused_run(gs_engine* eng, int lr) {
     HIP_TRY(hipStreamSynchronize(eng->stream));
     eng->fused_run = lr;
     if (int rc = build_steps(eng)) return rc;
-    return upload_descriptors(eng, false);
+    return upload_descriptors(eng);
 }
 
 // Plain sweeps of steps with at most ntq_max slots per coset (0: none, at most 2) take two runs per thread, the second
@@ -2144,7 +2249,7 @@ int gs_set_plain_pairs(gs_engine* eng, int ntq_max, int far) {
     eng->pair_ntq = ntq_max;
     eng->pair_far = far;
     if (int rc = build_steps(eng)) return rc;
-    return upload_descriptors(eng, false);
+    return upload_descriptors(eng);
 }
 
 // Give each XCD a contiguous eighth of every sweep's block coordinates (on = 1) or deal them round-robin (0); results
@@ -2155,7 +2260,7 @@ int gs_set_xcd_blocks(gs_engine* eng, int on) {
     HIP_TRY(hipStreamSynchronize(eng->stream));
     eng->xcd_blocks = on ? 1 : 0;
     if (int rc = build_steps(eng)) return rc;
-    return upload_descriptors(eng, false);
+    return upload_descriptors(eng);
 }
 
 // Tile order of the sweeps: 0 forward, 1 reverse on odd steps, 2 reverse on every step (results do not depend on it).
@@ -2166,7 +2271,7 @@ int gs_set_walk(gs_engine* eng, int mode) {
     HIP_TRY(hipStreamSynchronize(eng->stream));
     eng->walk = mode;
     if (int rc = build_steps(eng)) return rc;
-    return upload_descriptors(eng, false);
+    return upload_descriptors(eng);
 }
 
 // Steps with at most 2^nk cosets run, in runs of two or more, in one single-block launch (nk -1: never; default 10; runs
@@ -2178,8 +2283,8 @@ int gs_set_small_steps(gs_engine* eng, int nk) {
     HIP_TRY(hipStreamSynchronize(eng->stream));
     eng->small_nk = nk;
     build_small(eng);
-    build_pairs(eng);
-    return upload_descriptors(eng, false);
+    build_units(eng);
+    return upload_descriptors(eng);
 }
 
 // Runs of at most max_steps consecutive diagonal steps (2..8; 0 or 1: off; default 8) of at least 2^min_nk cosets
@@ -2194,7 +2299,7 @@ int gs_set_diag_runs(gs_engine* eng, int max_steps, int min_nk) {
     eng->run_max = max_steps;
     eng->run_min_nk = min_nk;
     if (int rc = build_steps(eng)) return rc;
-    return upload_descriptors(eng, false);
+    return upload_descriptors(eng);
 }
 
 // The run of diagonal steps that step k belongs to: out[0] its first step, out[1] its length, out[2] log2 blocks of
@@ -2267,7 +2372,7 @@ int gs_race_check(gs_engine* eng, int k, int layout, int64_t* counts) {
 // Chain mode: two steps per sweep where the plan allows it (default on) or one.
 int gs_set_pairs(gs_engine* eng, int on) {
     if (!eng) return fail(16, "null engine");
-    eng->allow_pairs = on != 0;
+    eng->allow_pairs = eng->allow_fly = on != 0;
     return 0;
 }
 
@@ -2284,7 +2389,7 @@ int gs_set_fused4(gs_engine* eng, int on) {
     if (!eng) return fail(16, "null engine");
     eng->allow_fused4 = on != 0;
     if (int rc = build_steps(eng)) return rc;
-    return upload_descriptors(eng, false);
+    return upload_descriptors(eng);
 }
 
 }  // extern "C"

@@ -29,6 +29,13 @@ struct GfBasis {
         reduce(x, coef);
         return x == 0;
     }
+    // Mask m with parity(x & m) == parity(combination of x & f) for every x of the span.
+    uint64_t form(uint64_t f) const {
+        uint64_t m = 0;
+        for (int b = 0; b < 64; b++)
+            if (row[b] && (parity(comb[b] & f) ^ parity(row[b] & m))) m |= uint64_t(1) << b;
+        return m;
+    }
     bool has(uint64_t x) const {
         uint64_t c;
         return solve(x, c);

@@ -316,6 +316,7 @@ void* reduce_kernel_ptr(int sweep) {
     return nullptr;
 }
 void* publish_kernel_ptr() { return reinterpret_cast<void*>(&publish_kernel); }
+void* reduce3_kernel_ptr() { return reinterpret_cast<void*>(&sweep_reduce_kernel<3>); }
 void* reduce1_kernel_ptr() { return reinterpret_cast<void*>(&sweep_reduce_kernel<1>); }
 void* run_hist_kernel_ptr(int storage) {
     return storage == 0 ? reinterpret_cast<void*>(&run_hist_kernel<float2>)

@@ -48,13 +48,13 @@ inline bool make_pair(const StepInfo& s0, const StepInfo& s1, bool units, PairDe
         if (!live.has(d[j]) || !next.add(d[j])) return false;
     if (next.n != live.n || !live.has(s1.off[0])) return false;
     // parities of an address of L1: bit 0 step k's sign, bit 1 step k+1's, bits 2-3 its slot, bit 4 step k's output
+    const uint64_t forms[5] = {live.form(s0.rhoc & ((uint64_t(1) << s0.nk) - 1)),
+                               next.form(s1.rhoc & ((uint64_t(1) << s1.nk) - 1)), next.form(uint64_t(1) << s1.nk),
+                               next.form(uint64_t(2) << s1.nk), live.form(uint64_t(1) << s0.nk)};
     auto nib = [&](uint64_t x) {
-        uint64_t c0 = 0, c1 = 0;
-        (void)live.solve(x, c0);
-        (void)next.solve(x, c1);
-        const uint64_t m0 = (uint64_t(1) << s0.nk) - 1, m1 = (uint64_t(1) << s1.nk) - 1;
-        return uint8_t(parity(c0 & m0 & s0.rhoc) | (parity(c1 & m1 & s1.rhoc) << 1) | (int((c1 >> s1.nk) & 3) << 2) |
-                       (int((c0 >> s0.nk) & 1) << 4));
+        int n = 0;
+        for (int i = 0; i < 5; i++) n |= parity(x & forms[i]) << i;
+        return uint8_t(n);
     };
     GfBasis slots;
     for (int j = 1; j <= lg1; j++) (void)slots.add(d[j]);

@@ -381,7 +381,8 @@ class Engine:
         _check(library().gs_set_fusion(self._h, 1 if on else 0))
 
     def set_pairs(self, on):
-        """Chain mode: two consecutive steps per sweep where the plan allows it (default on)."""
+        """Several consecutive steps per sweep where the plan allows it (default on): chain mode, and sampled and forced
+        complex128 strings."""
         _check(library().gs_set_pairs(self._h, 1 if on else 0))
 
     def set_fused4(self, on):

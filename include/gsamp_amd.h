@@ -181,8 +181,8 @@ int gs_step_geometry(const gs_engine* eng, int k, int* out);
 int gs_step_columns(const gs_engine* eng, int k, int fused, uint64_t* cols, int cap);
 /* Fold the next step's norm pass into the previous write (on, default) or run it as its own sweep (off). */
 int gs_set_fusion(gs_engine* eng, int on);
-/* Chain mode: two consecutive steps per sweep where the plan allows it (on, default) or one (off); the tables are the
-   same, the norms agree up to the order of their FP64 sums. */
+/* Several consecutive steps per sweep where the plan allows it (on, default) or one (off), in chain mode and for sampled
+   and forced complex128 strings; the tables are the same, the norms agree up to the order of their FP64 sums. */
 int gs_set_pairs(gs_engine* eng, int on);
 /* Fold the norms of a four-slot next step into the previous write (two pairing coordinates per thread) on or off
    (default on; off: such a step takes its own norm sweep). */
