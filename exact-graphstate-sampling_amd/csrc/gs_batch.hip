@@ -31,13 +31,21 @@
 #include <vector>
 
 #include "../../include/gsamp_amd.h"
+#include "gs_fly.h"
 #include "gs_pair.h"
 #include "gs_plan.h"
 
 namespace {
 
 using gs::flip_if;
+using gs::fly_each;
+using gs::fly_pair;
+using gs::fly_pair_back;
+using gs::fly_route_of;
+using gs::FlyDesc;
+using gs::make_fly;
 using gs::make_pair;
+using gs::uniform_byte;
 using gs::pair_route0;
 using gs::pair_route1;
 using gs::PairDesc;
@@ -49,7 +57,8 @@ constexpr int kWaves = 4;            // waves per block, each on its own part of
 constexpr int kItemGroup = 64;       // items whose partials are reduced together before the groups are
 constexpr int kBThreads = kLanes * kWaves;
 constexpr int64_t kMinItems = 1024;  // work items (blocks) a step launch should have before tiles get coarser
-constexpr int kMaxSums = 8;          // per-lane sums of one item: the norms of one or two steps, or their G_k(x)
+constexpr int kMaxUnit = 3;          // most steps of one sweep
+constexpr int kMaxSums = 4 * kMaxUnit;   // per-lane sums of one item: the norms of its steps, or their G_k(x)
 
 struct BStep {
     uint64_t cols[40];
@@ -76,6 +85,7 @@ struct BInst {           // device view of one instance
     void* lam;           // [2^R][B] adjoint arena (gradient mode)
     const BStep* steps;  // [ns]
     const PairDesc* pairs;  // [ns]: the sweep of steps k and k+1, where one is taken
+    const FlyDesc* flys;    // [ns][kMaxUnit - 2]: ... of 3 steps and more from k on
     const int8_t* bitsT; // [ns][B] forced bits, step-major
     double* prev;        // [B]
     int* dead;           // [B]
@@ -115,6 +125,9 @@ struct Sto<float2> {
         const f2v t = {v.x, v.y};
         __builtin_nontemporal_store(t, (GS_GLOBAL f2v*)(p));
     }
+    // entry i of a wave-uniform row
+    static __device__ __forceinline__ float2 ld(const float2* row, int i) { return ld(row + i); }
+    static __device__ __forceinline__ void st(float2* row, int i, float2 v) { st(row + i, v); }
     static __device__ __forceinline__ double2 wide(float2 v) { return make_double2(v.x, v.y); }
     static __device__ __forceinline__ float2 narrow(double2 v) { return make_float2(float(v.x), float(v.y)); }
 };
@@ -128,6 +141,8 @@ struct Sto<double2> {
         const d2v t = {v.x, v.y};
         __builtin_nontemporal_store(t, (GS_GLOBAL d2v*)(p));
     }
+    static __device__ __forceinline__ double2 ld(const double2* row, int i) { return ld(row + i); }
+    static __device__ __forceinline__ void st(double2* row, int i, double2 v) { st(row + i, v); }
     static __device__ __forceinline__ double2 wide(double2 v) { return v; }
     static __device__ __forceinline__ double2 narrow(double2 v) { return v; }
 };
@@ -556,7 +571,8 @@ struct PairWalk {
     bool on;
     __device__ __forceinline__ uint64_t col(int j) const { return uniform64(cols[j]); }
     __device__ __forceinline__ uint32_t nib(int j) const { return uint32_t(__builtin_amdgcn_readfirstlane(pn[j])); }
-    __device__ PairWalk(const BItem& it, const PairDesc& P, uint64_t* scols, int* spn, int wave) : cols(scols), pn(spn) {
+    template <class Desc>
+    __device__ PairWalk(const BItem& it, const Desc& P, uint64_t* scols, int* spn, int wave) : cols(scols), pn(spn) {
         for (int j = threadIdx.x; j < P.nk; j += blockDim.x) {
             scols[j] = P.cols[j];
             spn[j] = P.pn[j];
@@ -837,6 +853,219 @@ __global__ __launch_bounds__(kBThreads) void pair_back_kernel(const BInst* __res
     item_end<2, true>(I, it, k, wave, lane, val, nullptr);
 }
 
+// ---- three steps and more per sweep (FlyDesc): a run of butterfly steps, whose outputs take the places of their slots
+//
+// A lane holds the 2^NS entries of a group of its string; addresses, signs and slot indices are wave-uniform (the fields
+// are made so by hand: bytes and loads through the instance table land in vector registers, and with them the routes
+// became divergent branches and a step took 168 VGPRs instead of 128).  The pairs' saving goes on: 64 strings of the
+// n = 70 band 26 instance, which has 17 such steps in a row, take 18.2 ms instead of 24.6, 128 gradients of n = 60
+// band 24 11.8 ms instead of 16.0.  Sixteen entries (four steps) and their weights take 290 VGPRs.
+template <int NS>
+struct FlyGroup {
+    static constexpr int NE = 1 << NS;
+    uint64_t de[NE];                          // entries relative to the group's base, and their parities
+    uint32_t pe[NE];
+    int route[NS];
+    uint32_t par[NS];
+    __device__ explicit FlyGroup(const FlyDesc& f) {
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+            route[i] = int(uniform_byte(f.route[i]));
+            par[i] = uniform_byte(f.par[i]);
+        }
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            de[e] = 0;
+            pe[e] = uniform_byte(f.cn);
+#pragma unroll
+            for (int i = 0; i < NS; i++)
+                if ((e >> i) & 1) {
+                    de[e] ^= uniform64(f.dir[i]);
+                    pe[e] ^= uniform_byte(f.dn[i]);
+                }
+        }
+    }
+    __device__ uint32_t slot(uint32_t p, int e, int i) const { return ((p ^ pe[e]) >> (4 + i)) & 1; }
+    __device__ uint32_t sign(uint32_t p, int e, int i) const { return ((p ^ pe[e]) >> i) & 1; }
+};
+
+template <class S, int NS, int I>
+__device__ __forceinline__ void fly_step(const FlyGroup<NS>& g, uint32_t p, const double2 (&w)[2], const S (&x)[1 << NS],
+                                         S (&y)[1 << NS], double& nb) {
+    fly_route_of(g.route[I], [&](auto r) {
+#pragma unroll
+        for (int e = 0; e < (1 << NS); e++) {
+            if ((e >> I) & 1) continue;
+            double2 ylo, yhi;
+            fly_pair<decltype(r)::value>(g.par[I], g.slot(p, e, I), g.sign(p, e, I), Sto<S>::wide(x[e]),
+                                         Sto<S>::wide(x[e | (1 << I)]), w[0], w[1], ylo, yhi);
+            nb += norm2(ylo);
+            nb += norm2(yhi);
+            y[e] = Sto<S>::narrow(ylo);
+            y[e | (1 << I)] = Sto<S>::narrow(yhi);
+        }
+    });
+}
+
+// Forgets that v was widened before: its FP64 copy need not stay in registers.
+__device__ __forceinline__ void forget(float2& v) { asm("" : "+v"(v.x), "+v"(v.y)); }
+__device__ __forceinline__ void forget(double2&) {}
+
+template <int NS>
+__device__ __forceinline__ void fly_weights(const BInst& I, int k, int b, double2 (&w)[NS][2]) {
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+        const BStep& s = I.steps[k + i];
+        const int bv = I.bitsT[size_t(k + i) * I.B + b];
+#pragma unroll
+        for (int x = 0; x < 2; x++) w[i][x] = make_double2(s.mre[bv][x], s.mim[bv][x]);
+    }
+}
+
+template <class S, int NS>
+__global__ __launch_bounds__(kBThreads) void fly_step_kernel(const BInst* __restrict__ insts,
+                                                             const BItem* __restrict__ items, BLaunch L) {
+    constexpr int NE = 1 << NS;
+    const BItem it = items[blockIdx.x];
+    const BInst& I = insts[it.inst];
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int B = I.B;
+    const int b = it.group * kLanes + lane;
+    double2 w[NS][2];
+    fly_weights<NS>(I, L.k, b, w);
+    S* __restrict__ mem = static_cast<S*>(I.mem);
+    S* __restrict__ cp = L.copy ? static_cast<S*>(L.copy[it.inst]) : nullptr;
+    const FlyDesc& f = I.flys[size_t(L.k) * (kMaxUnit - 2) + NS - 3];
+    const FlyGroup<NS> g(f);
+    __shared__ uint64_t scols[40];
+    __shared__ int spn[40];
+    PairWalk<0> wk(it, f, scols, spn, wave);
+    const uint64_t ng = wk.groups();
+    double nb[NS];
+#pragma unroll
+    for (int i = 0; i < NS; i++) nb[i] = 0;
+    for (uint64_t t = 0; t < ng; t++) {
+        if (t) wk.next(t);
+        const uint64_t base = uniform64(wk.base);
+        const uint32_t p = uint32_t(__builtin_amdgcn_readfirstlane(int(wk.p)));
+        S v[NE];
+#pragma unroll
+        for (int e = 0; e < NE; e++) v[e] = Sto<S>::ld(mem + (base ^ g.de[e]) * uint64_t(B), b);
+        if (cp)
+#pragma unroll
+            for (int e = 0; e < NE; e++) Sto<S>::st(cp + (wk.index(t, 0) * NE + e) * uint64_t(B), b, v[e]);
+        fly_each([&](auto i) { fly_step<S, NS, decltype(i)::value>(g, p, w[decltype(i)::value], v, v, nb[decltype(i)::value]); },
+                 std::make_integer_sequence<int, NS>{});
+#pragma unroll
+        for (int e = 0; e < NE; e++) Sto<S>::st(mem + (base ^ g.de[e]) * uint64_t(B), b, v[e]);
+    }
+    if (!L.bookkeeping) return;
+    item_end<NS, false>(I, it, L.k, wave, lane, nb, L.clock);
+}
+
+// Put a compact copy of the run's input table back into the forward arena.
+template <class S, int NS>
+__global__ __launch_bounds__(kBThreads) void fly_restore_kernel(const BInst* __restrict__ insts,
+                                                                const BItem* __restrict__ items, BLaunch L) {
+    constexpr int NE = 1 << NS;
+    const BItem it = items[blockIdx.x];
+    const BInst& I = insts[it.inst];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int B = I.B;
+    const int b = it.group * kLanes + (threadIdx.x & (kLanes - 1));
+    S* __restrict__ mem = static_cast<S*>(I.mem);
+    const S* __restrict__ cp = static_cast<const S*>(L.copy[it.inst]);
+    if (!cp) return;
+    const FlyDesc& f = I.flys[size_t(L.k) * (kMaxUnit - 2) + NS - 3];
+    const FlyGroup<NS> g(f);
+    __shared__ uint64_t scols[40];
+    __shared__ int spn[40];
+    PairWalk<0> wk(it, f, scols, spn, wave);
+    const uint64_t ng = wk.groups();
+    for (uint64_t t = 0; t < ng; t++) {
+        if (t) wk.next(t);
+        const uint64_t base = uniform64(wk.base);
+        S v[NE];
+#pragma unroll
+        for (int e = 0; e < NE; e++) v[e] = Sto<S>::ld(cp + (wk.index(t, 0) * NE + e) * uint64_t(B), b);
+#pragma unroll
+        for (int e = 0; e < NE; e++) Sto<S>::st(mem + (base ^ g.de[e]) * uint64_t(B), b, v[e]);
+    }
+}
+
+// Backward through the run: the copy of its first input gives the tables between the steps again (in registers), lambda
+// goes from the last step's outputs to the first one's inputs, and every step's gradient is summed.
+template <class S, int NS>
+__global__ __launch_bounds__(kBThreads, 2) void fly_back_kernel(const BInst* __restrict__ insts,
+                                                             const BItem* __restrict__ items, BLaunch L) {
+    constexpr int NE = 1 << NS;
+    const BItem it = items[blockIdx.x];
+    const BInst& I = insts[it.inst];
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int B = I.B;
+    const int b = it.group * kLanes + lane;
+    double2 w[NS][2];
+    fly_weights<NS>(I, L.k, b, w);
+    S* __restrict__ lam = static_cast<S*>(I.lam);
+    const S* __restrict__ cp = static_cast<const S*>(L.copy[it.inst]);
+    const FlyDesc& f = I.flys[size_t(L.k) * (kMaxUnit - 2) + NS - 3];
+    const FlyGroup<NS> g(f);
+    __shared__ uint64_t scols[40];
+    __shared__ int spn[40];
+    PairWalk<0> wk(it, f, scols, spn, wave);
+    const uint64_t ng = wk.groups();
+    double2 G[NS][2];
+#pragma unroll
+    for (int i = 0; i < NS; i++) G[i][0] = G[i][1] = make_double2(0, 0);
+    for (uint64_t t = 0; t < ng; t++) {
+        if (t) wk.next(t);
+        const uint64_t base = uniform64(wk.base);
+        const uint32_t p = uint32_t(__builtin_amdgcn_readfirstlane(int(wk.p)));
+        S x[NS][NE], l[NE];
+#pragma unroll
+        for (int e = 0; e < NE; e++) x[0][e] = Sto<S>::ld(cp + (wk.index(t, 0) * NE + e) * uint64_t(B), b);
+#pragma unroll
+        for (int e = 0; e < NE; e++) l[e] = Sto<S>::ld(lam + (base ^ g.de[e]) * uint64_t(B), b);
+        fly_each([&](auto i) {
+            constexpr int J = decltype(i)::value;
+            double unused = 0;
+            fly_step<S, NS, J>(g, p, w[J], x[J], x[J + 1], unused);
+        }, std::make_integer_sequence<int, NS - 1>{});
+#pragma unroll
+        for (int i = 0; i < NS; i++)
+#pragma unroll
+            for (int e = 0; e < NE; e++) forget(x[i][e]);
+        fly_each([&](auto i) {
+            constexpr int J = NS - 1 - decltype(i)::value;
+            fly_route_of(g.route[J], [&](auto r) {
+#pragma unroll
+                for (int e = 0; e < NE; e++) {
+                    if ((e >> J) & 1) continue;
+                    double2 llo = Sto<S>::wide(l[e]), lhi = Sto<S>::wide(l[e | (1 << J)]);
+                    fly_pair_back<decltype(r)::value>(g.par[J], g.slot(p, e, J), g.sign(p, e, J),
+                                                      Sto<S>::wide(x[J][e]), Sto<S>::wide(x[J][e | (1 << J)]), w[J][0],
+                                                      w[J][1], llo, lhi, G[J]);
+                    l[e] = Sto<S>::narrow(llo);
+                    l[e | (1 << J)] = Sto<S>::narrow(lhi);
+                }
+            });
+        }, std::make_integer_sequence<int, NS>{});
+#pragma unroll
+        for (int e = 0; e < NE; e++) Sto<S>::st(lam + (base ^ g.de[e]) * uint64_t(B), b, l[e]);
+    }
+    double val[4 * NS];
+#pragma unroll
+    for (int i = 0; i < NS; i++)
+#pragma unroll
+        for (int x = 0; x < 2; x++) {
+            val[4 * i + 2 * x] = G[i][x].x;
+            val[4 * i + 2 * x + 1] = G[i][x].y;
+        }
+    item_end<NS, true>(I, it, L.k, wave, lane, val, nullptr);
+}
+
 template <class S>
 __global__ void batch_init_kernel(const BInst* __restrict__ insts, int ninst, unsigned long long* clock, int ns) {
     const int i = blockIdx.x;
@@ -910,7 +1139,8 @@ struct gs_batch {
     std::vector<int> nq;                  // per step: most slots per coset among the instances (kernel variant)
     std::vector<int> nq_exact;            // per step: 1 if every instance at the step has nq slots per coset
     std::vector<std::vector<PairDesc>> hpairs;   // [inst][step]: steps k and k+1 as one sweep (ni 0: not possible)
-    std::vector<char> unit;               // per step: steps of the sweep that starts there (1, 2; 0: inside a pair)
+    std::vector<std::vector<FlyDesc>> hflys;     // [inst][step][kMaxUnit - 2]: 3 steps and more (d 0: not possible)
+    std::vector<char> unit;               // per step: steps of the sweep that starts there (0: inside another's)
     bool pairs_on = true;
     int lu = 2;                           // log2 cosets a lane gathers at once
     bool items_dirty = false;             // tiles changed since the work lists were built
@@ -950,51 +1180,65 @@ T* dalloc(gs_batch* b, size_t n) {
     return static_cast<T*>(p);
 }
 
-// Which sweeps the step sequence takes: single steps, or two at once where every instance that is still running has
-// the same kind of pair.  A pair saves the write and the read of the table between its steps (and a launch), so the
-// pairs are the disjoint ones that save the most.
+// Which sweeps the step sequence takes: single steps, or several at once where every instance that is still running has
+// the same kind of pair, or a run of butterfly steps.  A sweep of n steps saves n - 1 writes and reads of the table (and
+// launches); the sweeps are the disjoint ones that save the most.
 void choose_units(gs_batch* bt) {
     const int ns = bt->maxns;
     bt->unit.assign(size_t(ns), 1);
     if (!bt->pairs_on) return;
     constexpr double kLaunch = 40e6;                      // bytes moved in the time a launch and its reduction take
-    std::vector<double> gain(size_t(ns), -1.0), best(size_t(ns) + 2, 0.0);
-    for (int k = 0; k + 1 < ns; k++) {
-        double g = kLaunch;
-        const PairDesc* first = nullptr;
-        int ntq = 0;
-        bool ok = true;
-        for (size_t i = 0; i < bt->plans.size() && ok; i++) {
-            const gs::Plan& P = bt->plans[i];
-            if (k >= P.ns) continue;
-            const PairDesc& p = bt->hpairs[i][size_t(k)];
-            if (k + 1 >= P.ns || !p.ni) {
-                ok = false;
-            } else if (!first) {
-                first = &p;
-                ntq = P.steps[size_t(k)].ntq;
-            } else {
-                ok = p.ni == first->ni && p.mo == first->mo && p.deg == first->deg && P.steps[size_t(k)].ntq == ntq;
+    std::vector<double> best(size_t(ns + kMaxUnit), 0.0);
+    std::vector<char> take(size_t(ns), 1);
+    for (int k = ns - 1; k >= 0; k--) {
+        best[size_t(k)] = best[size_t(k) + 1];
+        for (int n = 2; n <= kMaxUnit && k + n <= ns; n++) {
+            double g = kLaunch;
+            const PairDesc* first = nullptr;
+            int ntq = 0;
+            bool ok = true;
+            for (size_t i = 0; i < bt->plans.size() && ok; i++) {
+                const gs::Plan& P = bt->plans[i];
+                if (k >= P.ns) continue;
+                const PairDesc& p = bt->hpairs[i][size_t(k)];
+                if (k + n > P.ns) {
+                    ok = false;
+                } else if (n > 2) {
+                    ok = bt->hflys[i][size_t(k) * (kMaxUnit - 2) + size_t(n - 3)].d == n;
+                } else if (!first) {
+                    first = &p;
+                    ntq = P.steps[size_t(k)].ntq;
+                    ok = p.ni != 0;
+                } else {
+                    ok = p.ni == first->ni && p.mo == first->mo && p.deg == first->deg && P.steps[size_t(k)].ntq == ntq;
+                }
+                g += 2.0 * double(bt->B[i]) * double(bt->esz) *
+                     double(uint64_t(n > 2 ? 2 : p.mo) << P.steps[size_t(k)].nk);
             }
-            g += 2.0 * double(bt->B[i]) * double(bt->esz) * double(uint64_t(p.mo) << P.steps[size_t(k)].nk);
+            g *= n - 1;
+            if (ok && g + best[size_t(k + n)] > best[size_t(k)]) {
+                best[size_t(k)] = g + best[size_t(k + n)];
+                take[size_t(k)] = char(n);
+            }
         }
-        if (ok && first) gain[size_t(k)] = g;
     }
-    for (int k = ns - 1; k >= 0; k--)
-        best[size_t(k)] = std::max(best[size_t(k) + 1], gain[size_t(k)] + best[size_t(k) + 2]);
-    for (int k = 0; k < ns; k++)
-        if (gain[size_t(k)] > 0 && gain[size_t(k)] + best[size_t(k) + 2] > best[size_t(k) + 1]) {
-            bt->unit[size_t(k)] = 2;
-            bt->unit[size_t(k) + 1] = 0;
-            k++;
-        }
+    for (int k = 0; k < ns; k += take[size_t(k)]) {
+        bt->unit[size_t(k)] = take[size_t(k)];
+        for (int j = 1; j < take[size_t(k)]; j++) bt->unit[size_t(k + j)] = 0;
+    }
 }
 
-// Cosets (or super-cosets of a pair) of instance i's sweep at step k, log2, and log2 of the step-k cosets in each.
+// Cosets (or super-cosets of several steps) of instance i's sweep at step k, log2, and log2 of the step-k cosets in each.
 void sweep_size(const gs_batch* bt, size_t i, int k, int& nk, int& inner) {
     nk = bt->plans[i].steps[size_t(k)].nk;
     inner = 0;
-    if (bt->unit[size_t(k)] != 2) return;
+    const int n = bt->unit[size_t(k)];
+    if (n < 2) return;
+    if (n > 2) {
+        inner = n - 1;
+        nk -= inner;
+        return;
+    }
     const PairDesc& p = bt->hpairs[i][size_t(k)];
     inner = p.ni == 4 ? 2 : p.ni == 2 ? 1 : 0;
     nk = p.nk;
@@ -1003,15 +1247,16 @@ void sweep_size(const gs_batch* bt, size_t i, int k, int& nk, int& inner) {
 // log2 (super-)cosets per work item.  Tiles set per step index (by hand or by the autotuner, often on a larger batch)
 // are made finer, down to 2^kFinestTile cosets, while the launch has fewer than kMinItems items: one item per block,
 // and a launch of a few dozen blocks leaves the chip idle while each wave walks a long range (five width-11 plans of
-// 128 lanes: 40 blocks of 2^8 cosets took 30 us a step).  A pair's backward sums take twice the room per item, so its
-// tiles start one step coarser.
+// 128 lanes: 40 blocks of 2^8 cosets took 30 us a step).  The backward sums of several steps take more room per item, so their
+// tiles start coarser.
 constexpr int kFinestTile = 4;
 int item_lg(const gs_batch* bt, size_t i, int k, int shrink, bool& finer) {
     int nk, inner;
     sweep_size(bt, i, k, nk, inner);
     const int floor = std::min(nk, std::max(0, kFinestTile - inner));
     int lg = bt->lg[i][size_t(k)];
-    if (bt->unit[size_t(k)] == 2) lg = std::max(lg, bt->lg_default + 1);
+    const int n = bt->unit[size_t(k)];
+    if (n > 1) lg = std::max(lg, bt->lg_default + (n > 2 ? 2 : 1));
     lg = std::min(nk, std::max(lg - inner - shrink, floor));
     finer = finer || lg > floor;
     return lg;
@@ -1105,7 +1350,7 @@ size_t part_items(const gs_batch* bt, size_t i) {
     return std::max(m, 2 * size_t(kMinItems) * kLanes / size_t(bt->B[i]));
 }
 
-// Doubles of one lane group's partials: four sums per lane of every item (a pair's eight at twice the smallest tile).
+// Doubles of one lane group's partials: four sums per lane of every item (a pair's eight at twice the smallest tile, ...).
 size_t part_doubles(const gs_batch* bt, size_t i) {
     const size_t fine = 2 * size_t(kMinItems) * kLanes / size_t(bt->B[i]);
     return kLanes * std::max(4 * part_items(bt, i), size_t(kMaxSums) * std::max<size_t>(fine, 1));
@@ -1144,6 +1389,15 @@ size_t part_doubles(const gs_batch* bt, size_t i) {
 enum BKernel { kBStep, kBRestore, kBBack };
 
 template <class S>
+const void* fly_variant(BKernel kind, int n) {
+#define GS_FV(n) (kind == kBStep ? reinterpret_cast<const void*>(&fly_step_kernel<S, n>)                            \
+                  : kind == kBRestore ? reinterpret_cast<const void*>(&fly_restore_kernel<S, n>)                     \
+                                      : reinterpret_cast<const void*>(&fly_back_kernel<S, n>))
+    return n == 3 ? GS_FV(3) : nullptr;
+#undef GS_FV
+}
+
+template <class S>
 int launch_batch(gs_batch* bt, BKernel kind, int k, BLaunch L) {
     const int n = bt->nitems[size_t(k)];
     if (n == 0) return 0;
@@ -1153,7 +1407,9 @@ int launch_batch(gs_batch* bt, BKernel kind, int k, BLaunch L) {
     if (bt->unit[size_t(k)] == 2)
         for (size_t i = 0; i < bt->plans.size() && !pair; i++)
             if (k < bt->plans[i].ns) pair = &bt->hpairs[i][size_t(k)];
-    const void* fn = pair ? (kind == kBStep ? GS_PAIR_VARIANT(pair_step_kernel, S, nq, *pair)
+    const int n_steps = bt->unit[size_t(k)];
+    const void* fn = n_steps > 2 ? fly_variant<S>(kind, n_steps)
+                   : pair ? (kind == kBStep ? GS_PAIR_VARIANT(pair_step_kernel, S, nq, *pair)
                              : kind == kBRestore ? GS_PAIR_VARIANT(pair_restore_kernel, S, nq, *pair)
                                                  : GS_PAIR_VARIANT(pair_back_kernel, S, nq, *pair))
                    : kind == kBStep ? GS_BATCH_VARIANT(batch_step_kernel, S, nq, lu, ex)
@@ -1178,7 +1434,7 @@ int enqueue_t(gs_batch* bt) {
     hipLaunchKernelGGL(batch_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst,
                        bt->dclock, bt->maxns);
     for (int k = 0; k < bt->maxns; k++) {
-        if (!bt->unit[size_t(k)]) continue;               // the second step of a pair
+        if (!bt->unit[size_t(k)]) continue;               // inside another step's sweep
         if (int rc = launch_step<S>(bt, k, 1, nullptr)) return rc;
     }
     hipLaunchKernelGGL(batch_finish_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
@@ -1500,6 +1756,14 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
         std::vector<PairDesc> hp(size_t(P.ns));
         for (int k = 0; k < P.ns; k++)
             if (k + 1 >= P.ns || !make_pair(P.steps[size_t(k)], P.steps[size_t(k) + 1], false, hp[size_t(k)])) hp[size_t(k)].ni = 0;
+        std::vector<FlyDesc> hf(size_t(P.ns) * (kMaxUnit - 2));
+        for (int k = 0; k < P.ns; k++)
+            for (int n = 3; n <= kMaxUnit; n++) {
+                const gs::StepInfo* st[kMaxUnit] = {};
+                for (int j = 0; j < n && k + j < P.ns; j++) st[j] = &P.steps[size_t(k + j)];
+                FlyDesc& f = hf[size_t(k) * (kMaxUnit - 2) + size_t(n - 3)];
+                if (!st[n - 1] || !make_fly(st, n, 0, 0, f)) f.d = 0;
+            }
         // the instance's small buffers in one allocation: descriptors first, uploaded in one copy
         size_t used = 0;
         auto take = [&](size_t bytes) {
@@ -1507,7 +1771,8 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
             used += (bytes + 255) & ~size_t(255);
             return at;
         };
-        const size_t o_steps = take(hs.size() * sizeof(BStep)), o_pairs = take(hp.size() * sizeof(PairDesc)), head = used;
+        const size_t o_steps = take(hs.size() * sizeof(BStep)), o_pairs = take(hp.size() * sizeof(PairDesc)),
+                     o_flys = take(hf.size() * sizeof(FlyDesc)), head = used;
         I.narrived = int(part_items(bt, size_t(i)) / kItemGroup);
         const size_t n_arrived = size_t(B / kLanes) * size_t(1 + I.narrived);
         const size_t o_prev = take(sizeof(double) * B), o_dead = take(sizeof(int) * B),
@@ -1518,12 +1783,15 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
         std::vector<char> up(head);
         if (!hs.empty()) memcpy(up.data() + o_steps, hs.data(), hs.size() * sizeof(BStep));
         if (!hp.empty()) memcpy(up.data() + o_pairs, hp.data(), hp.size() * sizeof(PairDesc));
+        if (!hf.empty()) memcpy(up.data() + o_flys, hf.data(), hf.size() * sizeof(FlyDesc));
         if (head && hipMemcpy(mem, up.data(), head, hipMemcpyHostToDevice) != hipSuccess)
             return bail(bfail(17, "plan upload failed"));
         bt->hsteps.push_back(std::move(hs));
         bt->hpairs.push_back(std::move(hp));
+        bt->hflys.push_back(std::move(hf));
         I.steps = reinterpret_cast<BStep*>(mem + o_steps);
         I.pairs = reinterpret_cast<PairDesc*>(mem + o_pairs);
+        I.flys = reinterpret_cast<FlyDesc*>(mem + o_flys);
         I.bitsT = bt->dbits + bt->at_bits[size_t(i)];
         I.prev = reinterpret_cast<double*>(mem + o_prev);
         I.dead = reinterpret_cast<int*>(mem + o_dead);
@@ -1669,8 +1937,8 @@ int gs_batch_score(gs_batch* bt, const int8_t* const* bits, double* const* log2p
     bt->last_ms = ms;
     bt->step_ms.assign(size_t(bt->maxns), -1.0);
     if (!bt->use_graph)
-        for (int k = 0; k < bt->maxns; k++) {             // the second step of a pair ends with the first
-            const int u = bt->unit[size_t(k)] ? k : k - 1;
+        for (int k = 0, u = 0; k < bt->maxns; k++) {      // the steps of one sweep end together
+            if (bt->unit[size_t(k)]) u = k;
             if (bt->nitems[size_t(u)])
                 bt->step_ms[size_t(k)] = double(bt->hclock[size_t(1 + u)] - bt->hclock[0]) / bt->clock_khz;
         }

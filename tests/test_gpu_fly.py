@@ -38,3 +38,36 @@ def test_butterflies_equal_single_steps(shape, storage, tol, grid, tmp_path):
             assert np.array_equal(a, b)                     # chain mode: the same tables
         else:
             assert np.allclose(a, b, rtol=tol, atol=tol), np.max(np.abs(a - b))
+
+
+# plateaus of 24 and 20 steps; gadgets; two instances whose plateaus overlap in part
+BATCHES = [[((40, 8, 1, 0), 64)], [((52, 16, 4, 0), 128)], [((40, 12, 3, 6), 64)],
+           [((40, 8, 1, 0), 64), ((44, 10, 2, 0), 64)]]
+
+
+@pytest.mark.parametrize("storage", [gs.C64, gs.C128])
+@pytest.mark.parametrize("batch", BATCHES)
+def test_batched_butterflies_equal_single_steps(batch, storage, tmp_path):
+    """The tables are the same bit for bit; norms and gradients are FP64 sums over up to 2^16 cosets in another order
+    (2^16 terms x 2^-53, with room: 1e-11)."""
+    plans, bits = [], []
+    rng = np.random.default_rng(19)
+    for i, ((n, band, seed, gadgets), lanes) in enumerate(batch):
+        inst = egs.instances.Instance(n, band, seed, gadgets_count=gadgets)
+        plans.append(str(tmp_path / f"p{i}.txt"))
+        inst.write_plan(plans[-1])
+        bits.append(rng.integers(0, 2, size=(lanes, inst.N)).astype(np.int8))
+    print(batch, storage, flush=True)
+    with gs.BatchEngine(plans, [lanes for _, lanes in batch], storage=storage) as bt:
+        many = bt.score(bits)
+        gmany, _ = bt.grad(bits)
+        gseg, _ = bt.grad(bits, seg=5)
+        bt.set_pairs(False)
+        one = bt.score(bits)
+        gone, _ = bt.grad(bits)
+    for i in range(len(batch)):
+        assert np.array_equal(many[2][i], one[2][i])
+        assert np.max(np.abs(many[0][i] - one[0][i])) < 1e-11
+        assert np.allclose(many[1][i], one[1][i], rtol=1e-11, atol=0)
+        assert np.max(np.abs(gmany[i][2] - gone[i][2])) < 1e-11 * np.max(np.abs(gone[i][2]))
+        assert np.array_equal(gmany[i][2], gseg[i][2]) and np.array_equal(gmany[i][1], gseg[i][1])
