@@ -176,6 +176,10 @@ struct Ctl {
     int pad;
 };
 
+// Sweeps of at least this many blocks are reduced by several waves (see wide_reduce_kernel): one block takes 5.2 / 8.0 /
+// 12.7 / 28.7 us for the partials of 2^11 .. 2^14 blocks, they take 6.4 / 6.6 / 6.5 / 10.2.
+constexpr int kWideReduce = 1 << 12;
+
 // Whether a sweep's blocks reduce their own partials (one block per string, or few blocks in all): see sweep_epilogue.
 __device__ __host__ __forceinline__ bool reduces_in_kernel(unsigned blocks, unsigned strings) {
     return blocks == 1 || blocks * strings <= unsigned(kFenceBlocks);
@@ -188,9 +192,11 @@ enum ChainMode { kChain = 0, kChain1 = 1, kRun = 2 };
 // product pass of a run of diagonal steps, whose decisions and bookkeeping were made before it).
 // kRoleStoredGram: the same, then the next step's decision from the Gram matrix the product pass summed.
 // kRolePair: a chain-mode sweep of two or three steps from step k on, whose sums are the steps' written norms.
+// kRoleSilent: nothing (a write whose norms nobody needs).
 // kRolePeek: a read-only pass that applied step k in registers; step k+1's decision goes to w2, step k's write is still
 // to come.
-enum EpiRole { kRoleNorm = 0, kRoleWrite = 1, kRoleStored = 2, kRoleStoredGram = 3, kRolePair = 4, kRolePeek = 5 };
+enum EpiRole { kRoleNorm = 0, kRoleWrite = 1, kRoleStored = 2, kRoleStoredGram = 3, kRolePair = 4, kRolePeek = 5,
+               kRoleSilent = 6 };
 // Write role: what follows step k.
 enum Next { kNextPublish = -2, kNextDecide = -1, kNextFusedGram = kGram, kNextFusedDirect = kDirect, kNextSweep = 3 };
 

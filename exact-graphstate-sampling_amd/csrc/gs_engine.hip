@@ -36,15 +36,13 @@ int plain_lr(int storage);
 int fused_lr(int storage);
 void* decide_kernel_ptr();
 void* publish_kernel_ptr();
-void* reduce_kernel_ptr(int sweep);
+hipError_t launch_reduce(int nq, double* part, unsigned nblk, Ctl* ctl, const Epi& epi, int sweep, unsigned strings,
+                         hipStream_t stream);
 void* small_run_kernel_ptr(int storage);
 size_t small_run_lds(size_t tab_bytes);
 void* pair_sweep_kernel_ptr(int storage, int nq, int ni, int mo, int deg);
 void* fly_kernel_ptr(int storage, int ns);
 void* fly_norm_kernel_ptr(int norm, bool write);
-void* reduce3_kernel_ptr();
-void* reduce1_kernel_ptr();
-void* reduce_stored_gram_kernel_ptr();
 void* run_hist_kernel_ptr(int storage);
 void* run_apply_kernel_ptr(int storage);
 void* run_apply_gram_kernel_ptr(int storage, int route2);
@@ -437,14 +435,10 @@ int ensure_slots(gs_engine* e, int64_t want) {
 // Reduce the partials the last sweep left (one-block kernel) before a launch that does not reduce them itself.
 int flush_pending(gs_engine* e) {
     if (!e->pend_nblk) return 0;
-    const double* cpart = e->pend_part;
-    unsigned nblk = e->pend_nblk;
-    Ctl* ctl = e->ctl;
-    Epi ep = e->pend_epi;
-    int sw = e->pend_sweep;
+    const unsigned nblk = e->pend_nblk;
     e->pend_nblk = 0;
-    void* rargs[] = {&cpart, &nblk, &ctl, &ep, &sw};
-    HIP_TRY(hipLaunchKernel(reduce_kernel_ptr(sw), dim3(1, e->strings), dim3(kThreads), rargs, 0, e->stream));
+    HIP_TRY(launch_reduce(partials_of(e->pend_sweep), e->pend_part, nblk, e->ctl, e->pend_epi, e->pend_sweep,
+                          unsigned(e->strings), e->stream));
     return 0;
 }
 
@@ -533,12 +527,8 @@ int launch_multi(gs_engine* e, void* fn, const void* desc, int lg_grid, const Ep
         e->pev_tag.push_back(k * 8 + tag);
     }
     if (!reduces_in_kernel(unsigned(grid), unsigned(e->strings))) {
-        const double* cpart = part;
-        unsigned nblk = unsigned(grid);
-        int sw = sums == 6 ? kWriteGram : sums == 4 ? kWriteDirect : kWrite;
-        void* rargs[] = {&cpart, &nblk, &ctl, &ep, &sw};
-        HIP_TRY(hipLaunchKernel(sums == 3 ? reduce3_kernel_ptr() : reduce_kernel_ptr(sw), dim3(1, e->strings),
-                                dim3(kThreads), rargs, 0, e->stream));
+        const int sw = sums == 6 ? kWriteGram : sums == 4 ? kWriteDirect : kWrite;
+        HIP_TRY(launch_reduce(sums, part, unsigned(grid), ctl, ep, sw, unsigned(e->strings), e->stream));
     }
     return 0;
 }
@@ -664,13 +654,8 @@ int launch_run(gs_engine* e, int ri, const Epi& base, bool gram) {
             return 0;
         }))
         return rc;
-    if (!reduces_in_kernel(nblk, 1)) {
-        const double* cpart = part;
-        int sw = kWrite;
-        void* rargs[] = {&cpart, &nblk, &ctl, &ea, &sw};
-        HIP_TRY(hipLaunchKernel(gram ? reduce_stored_gram_kernel_ptr() : reduce1_kernel_ptr(), dim3(1), dim3(kThreads),
-                                rargs, 0, e->stream));
-    }
+    if (!reduces_in_kernel(nblk, 1))
+        HIP_TRY(launch_reduce(gram ? 5 : 1, part, nblk, ctl, ea, kWrite, 1, e->stream));
     return 0;
 }
 

@@ -136,7 +136,7 @@ __global__ __launch_bounds__(kThreads) void gather_kernel(const TStep* __restric
             output(v, u0, c_it | cb);
         }
     }
-    sweep_epilogue<2>(acc, part, ctl, epi, SWEEP);
+    if (epi.role != kRoleSilent) sweep_epilogue<2>(acc, part, ctl, epi, SWEEP);
 }
 
 // The write pass of step k that also sums step k+1's branch norms, from the values it stores (TFold).  A thread takes

@@ -25,6 +25,55 @@ __global__ __launch_bounds__(kThreads) void sweep_reduce_kernel(const double* __
     chain_step<NQ>(red, ctl, slot_epi(e), sweep);
 }
 
+// The same for many blocks, in the same order: thread t of the one-block kernel sums partials t, t + 256, ...; here a
+// wave does that for one quantity and 64 of the t, and the last of the 4 NQ waves adds up and runs the chain.  One block
+// reads the 64-byte partials of 2^14 blocks in 28.7 us, bound by the loads one CU has in flight; the waves in 10.2 us.
+template <int NQ>
+__global__ __launch_bounds__(64) void wide_reduce_kernel(double* __restrict__ part, unsigned nblk, Ctl* __restrict__ ctl,
+                                                         Epi e, int sweep) {
+    constexpr int NW = kThreads / 64, U = 16;
+    ctl += blockIdx.y;
+    part += size_t(blockIdx.y) * e.slot_part;
+    if (ctl->dead) return;
+    const int lane = threadIdx.x, q = int(blockIdx.x) % NQ, w = int(blockIdx.x) / NQ;
+    double r = 0;
+    for (unsigned i = unsigned(w * 64 + lane); i < nblk; i += U * kThreads) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            v[u] = part[size_t(min(i + unsigned(u) * kThreads, nblk - 1)) * kPartStride + q];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i + unsigned(u) * kThreads < nblk) r += v[u];
+    }
+    for (int o = 32; o > 0; o >>= 1) r += __shfl_xor(r, o, 64);
+    // the wave's sum in the last, unused double of partial w * NQ + q; published before the counter is raised
+    auto slot = [&](int i) { return reinterpret_cast<unsigned long long*>(part + size_t(i) * kPartStride + kPartStride - 1); };
+    int last = 0;
+    if (lane == 0) {
+        unsigned long long old = __hip_atomic_exchange(slot(w * NQ + q), (unsigned long long)__double_as_longlong(r),
+                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(old) : : "memory");
+        last = __hip_atomic_fetch_add(e.counter + blockIdx.y, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+               unsigned(NW * NQ - 1);
+    }
+    if (!__shfl(last, 0, 64)) return;
+    __atomic_thread_fence(__ATOMIC_ACQUIRE);
+    double v = 0;
+    if (lane < NW * NQ)
+        v = __longlong_as_double((long long)__hip_atomic_load(slot(lane), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    double red[NQ];
+#pragma unroll
+    for (int k = 0; k < NQ; k++) {
+        red[k] = __shfl(v, k, 64);
+#pragma unroll
+        for (int j = 1; j < NW; j++) red[k] += __shfl(v, j * NQ + k, 64);
+    }
+    if (lane != 0) return;
+    chain_step<NQ>(red, ctl, slot_epi(e), sweep);
+    __hip_atomic_store(e.counter + blockIdx.y, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // single-thread chain kernels
 
@@ -304,20 +353,31 @@ int plain_lr(int) { return 1; }
 int fused_lr(int storage) { return storage == 0 ? 1 : 0; }
 
 void* decide_kernel_ptr() { return reinterpret_cast<void*>(&decide_kernel); }
-// Reduce kernel of a sweep kind (number of partial sums: Gram 4, direct 2, write 2, write + Gram 6, write + direct 4).
-void* reduce_kernel_ptr(int sweep) {
-    switch (sweep) {
-        case kGram: return reinterpret_cast<void*>(&sweep_reduce_kernel<4>);
-        case kDirect: return reinterpret_cast<void*>(&sweep_reduce_kernel<2>);
-        case kWrite: return reinterpret_cast<void*>(&sweep_reduce_kernel<2>);
-        case kWriteGram: return reinterpret_cast<void*>(&sweep_reduce_kernel<6>);
-        case kWriteDirect: return reinterpret_cast<void*>(&sweep_reduce_kernel<4>);
+template <int NQ>
+hipError_t reduce_for(double* part, unsigned nblk, Ctl* ctl, const Epi& epi, int sweep, unsigned strings, hipStream_t stream) {
+    Epi e = epi;
+    void* args[] = {&part, &nblk, &ctl, &e, &sweep};
+    if (nblk >= unsigned(kWideReduce))
+        return hipLaunchKernel(reinterpret_cast<void*>(&wide_reduce_kernel<NQ>), dim3(kThreads / 64 * NQ, strings), dim3(64),
+                               args, 0, stream);
+    return hipLaunchKernel(reinterpret_cast<void*>(&sweep_reduce_kernel<NQ>), dim3(1, strings), dim3(kThreads), args, 0,
+                           stream);
+}
+// Reduction of nq partial sums per block after a sweep of nblk blocks and strings (Gram 4, direct 2, write 2, write +
+// Gram 6, write + direct 4; a product pass 1, with the next step's Gram 5; chain-mode sweeps one per step).
+hipError_t launch_reduce(int nq, double* part, unsigned nblk, Ctl* ctl, const Epi& epi, int sweep, unsigned strings,
+                         hipStream_t stream) {
+    switch (nq) {
+        case 1: return reduce_for<1>(part, nblk, ctl, epi, sweep, strings, stream);
+        case 2: return reduce_for<2>(part, nblk, ctl, epi, sweep, strings, stream);
+        case 3: return reduce_for<3>(part, nblk, ctl, epi, sweep, strings, stream);
+        case 4: return reduce_for<4>(part, nblk, ctl, epi, sweep, strings, stream);
+        case 5: return reduce_for<5>(part, nblk, ctl, epi, sweep, strings, stream);
+        case 6: return reduce_for<6>(part, nblk, ctl, epi, sweep, strings, stream);
     }
-    return nullptr;
+    return hipErrorInvalidValue;
 }
 void* publish_kernel_ptr() { return reinterpret_cast<void*>(&publish_kernel); }
-void* reduce3_kernel_ptr() { return reinterpret_cast<void*>(&sweep_reduce_kernel<3>); }
-void* reduce1_kernel_ptr() { return reinterpret_cast<void*>(&sweep_reduce_kernel<1>); }
 void* run_hist_kernel_ptr(int storage) {
     return storage == 0 ? reinterpret_cast<void*>(&run_hist_kernel<float2>)
                         : reinterpret_cast<void*>(&run_hist_kernel<double2>);
@@ -340,7 +400,6 @@ void* run_apply_gram_for(int route2) {
 void* run_apply_gram_kernel_ptr(int storage, int route2) {
     return storage == 0 ? run_apply_gram_for<float2>(route2) : run_apply_gram_for<double2>(route2);
 }
-void* reduce_stored_gram_kernel_ptr() { return reinterpret_cast<void*>(&sweep_reduce_kernel<5>); }
 void* run_chunk_kernel_ptr() { return reinterpret_cast<void*>(&run_chunk_kernel); }
 void* run_decide_kernel_ptr() { return reinterpret_cast<void*>(&run_decide_kernel); }
 

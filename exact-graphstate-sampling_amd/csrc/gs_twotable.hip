@@ -28,7 +28,8 @@ void* gather_fold_kernel_ptr(int storage, int nks, int nd2, int share, int pure)
 void* table_one_kernel_ptr(int storage);
 void* decide_kernel_ptr();
 void* publish_kernel_ptr();
-void* reduce_kernel_ptr(int sweep);
+hipError_t launch_reduce(int nq, double* part, unsigned nblk, Ctl* ctl, const Epi& epi, int sweep, unsigned strings,
+                         hipStream_t stream);
 }  // namespace gs
 
 namespace {
@@ -184,13 +185,8 @@ int launch_gather(gs_tt_engine* e, int k, int sweep, int in, const Epi& epi, con
     void* fn = gather_kernel_ptr(e->storage, sweep, e->hsteps[size_t(k)].nks);
     if (!fn) return ttfail(15, "no gather kernel for step " + std::to_string(k));
     TT_TRY(hipLaunchKernel(fn, dim3(grid), dim3(kThreads), args, 0, e->stream));
-    if (!reduces_in_kernel(unsigned(grid), 1)) {
-        const double* cpart = part;
-        unsigned nblk = unsigned(grid);
-        int sw = sweep;
-        void* rargs[] = {&cpart, &nblk, &ctl, &ep, &sw};
-        TT_TRY(hipLaunchKernel(reduce_kernel_ptr(sweep), dim3(1), dim3(kThreads), rargs, 0, e->stream));
-    }
+    if (ep.role != kRoleSilent && !reduces_in_kernel(unsigned(grid), 1))
+        TT_TRY(launch_reduce(2, part, unsigned(grid), ctl, ep, sweep, 1, e->stream));
     return 0;
 }
 
@@ -206,13 +202,8 @@ int launch_fold(gs_tt_engine* e, int k, int in, const Epi& epi) {
     void* args[] = {&sp, &fp, &old, &nw, &part, &ctl, &ep};
     const int grid = 1 << e->hfold[size_t(k)].lg_grid;
     TT_TRY(hipLaunchKernel(e->fold_fn[size_t(k)], dim3(grid), dim3(kThreads), args, 0, e->stream));
-    if (!reduces_in_kernel(unsigned(grid), 1)) {
-        const double* cpart = part;
-        unsigned nblk = unsigned(grid);
-        int sw = kWriteDirect;
-        void* rargs[] = {&cpart, &nblk, &ctl, &ep, &sw};
-        TT_TRY(hipLaunchKernel(reduce_kernel_ptr(sw), dim3(1), dim3(kThreads), rargs, 0, e->stream));
-    }
+    if (!reduces_in_kernel(unsigned(grid), 1))
+        TT_TRY(launch_reduce(4, part, unsigned(grid), ctl, ep, kWriteDirect, 1, e->stream));
     return 0;
 }
 
@@ -261,6 +252,8 @@ int tt_enqueue(gs_tt_engine* e, int mode, int k0, int k1, const int8_t* forced_h
         else if (wext) ep.next = kNextSweep;              // amplitude engine: weights given, no decision
         else if (tt_norm(e, mode, k + 1, fb(k + 1)) < 0) ep.next = kNextDecide;
         else ep.next = e->fold_fn[size_t(k)] ? int(kNextFusedDirect) : int(kNextSweep);
+        // a renormalised string's write before a norm pass has no use for its own norms
+        if (mode == kChain && ep.next == kNextSweep) ep.role = kRoleSilent;
         if (ep.next == kNextFusedDirect) {
             if (int rc = launch_fold(e, k, e->cur, ep)) return rc;
         } else {
