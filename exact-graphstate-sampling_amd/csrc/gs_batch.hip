@@ -34,6 +34,7 @@
 #include "gs_fly.h"
 #include "gs_pair.h"
 #include "gs_plan.h"
+#include "gs_wave.h"
 
 namespace {
 
@@ -58,6 +59,8 @@ constexpr int kItemGroup = 64;       // items whose partials are reduced togethe
 constexpr int kBThreads = kLanes * kWaves;
 constexpr int64_t kMinItems = 1024;  // work items (blocks) a step launch should have before tiles get coarser
 constexpr int kMaxUnit = 3;          // most steps of one sweep
+// Plans whose table fits the LDS (score_lds_kernel): most steps, log2 most slots
+constexpr int kLdsSteps = 128, kLdsMaxR = 14;
 constexpr int kMaxSums = 4 * kMaxUnit;   // per-lane sums of one item: the norms of its steps, or their G_k(x)
 
 struct BStep {
@@ -69,6 +72,18 @@ struct BStep {
     int tau0[4], tau1[4], par[4];
     uint32_t t0m, t1m, parm;     // tau0, tau1, par as bit masks over the offsets
 };
+
+// A step with its table in LDS at the arena's own slot numbers.  Coordinates: those first whose columns fall on different
+// LDS banks.
+struct LStep {
+    uint32_t cols[kLdsMaxR];
+    uint32_t off[4], g;
+    uint32_t rho;                // sign mask over the coordinates
+    uint32_t t0m, t1m, parm;     // as in BStep
+    int nk, ntq, m;
+    int pad[2];                  // whole 16-byte words
+};
+static_assert(sizeof(LStep) % 16 == 0, "the weights behind the descriptors are read as 16-byte words");
 
 struct BItem {
     uint64_t c0;         // first coset of the range (aligned to 2^lg)
@@ -86,6 +101,7 @@ struct BInst {           // device view of one instance
     const BStep* steps;  // [ns]
     const PairDesc* pairs;  // [ns]: the sweep of steps k and k+1, where one is taken
     const FlyDesc* flys;    // [ns][kMaxUnit - 2]: ... of 3 steps and more from k on
+    const LStep* lsteps;    // [ns]: where the plan's table fits the LDS
     const int8_t* bitsT; // [ns][B] forced bits, step-major
     double* prev;        // [B]
     int* dead;           // [B]
@@ -1095,6 +1111,163 @@ __global__ void batch_finish_kernel(const BInst* __restrict__ insts, int ninst) 
     }
 }
 
+// ---- whole strings in LDS
+//
+// Small plans are bound by launches: five width-11 plans of 128 lanes took 40 launches of 10 us for tables of 17 KB a
+// string, and plans of unlike steps share no sweep of several steps.  Where every plan's table fits the LDS, one block
+// takes a string from its first step to its last: one barrier per step (none while 64 cosets or fewer keep one wave busy),
+// the steps' norms left as a sum per wave and put together at the end.  Those five plans take 146 us a call instead of
+// 514; what is left is the chain of 45 steps (0.9 us each) and 60 us of launch, copies and transposition of the bits.
+// Device time of 64 / 1024 / 4096 strings, sweeps against this: 140 / 173 / 306 us and 43 / 70 / 200 at 2^11 complex64
+// slots, 178 / 239 / 533 and 58 / 116 / 381 at 2^12, 178 / 288 / 777 and 56 / 142 / 506 at 2^12 complex128 ones, and at
+// 2^4 and 4096 strings, the one place where they are level, 56 and 64.
+template <class S, int NTQ>
+__device__ __forceinline__ double lds_step(const LStep& s, S* tab, double2 w0, double2 w1, int t, int lt) {
+    auto uni = [](uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); };
+    const int nk = int(uni(uint32_t(s.nk))), m = int(uni(uint32_t(s.m)));
+    const uint32_t rho = uni(s.rho), t0m = uni(s.t0m), t1m = uni(s.t1m), parm = uni(s.parm), g = uni(s.g);
+    uint32_t off[NTQ], a = 0;
+#pragma unroll
+    for (int q = 0; q < NTQ; q++) off[q] = uni(s.off[q]);
+#pragma unroll
+    for (int j = 0; j < 9; j++)
+        if (j < lt) a ^= ((t >> j) & 1) ? s.cols[j] : 0;      // columns beyond nk are 0
+    double nb = 0;
+    if (nk < lt && (t >> nk)) return nb;
+    uint32_t sg = uint32_t(__popc(uint32_t(t) & rho)) & 1;
+    const int groups = nk > lt ? 1 << (nk - lt) : 1;
+    for (int it = 0; it < groups; it++) {
+        if (it) {
+            const int j = lt + __builtin_ctz(unsigned(it));
+            a ^= uni(s.cols[j]);
+            sg ^= (rho >> j) & 1;
+        }
+        S v[NTQ];
+#pragma unroll
+        for (int q = 0; q < NTQ; q++) v[q] = tab[a ^ off[q]];
+        double2 A[2][2];
+        A[0][0] = A[0][1] = A[1][0] = A[1][1] = make_double2(-0.0, -0.0);
+#pragma unroll
+        for (int q = 0; q < NTQ; q++)
+            gs::route_one(A, Sto<S>::wide(v[q]), (t0m >> q) & 1, (t1m >> q) & 1, sg ^ ((parm >> q) & 1));
+        const double2 o0 = cfma(w0, A[0][0], cmul(w1, A[0][1]));
+        tab[a] = Sto<S>::narrow(o0);
+        nb += norm2(o0);
+        if (m == 2) {
+            const double2 o1 = cfma(w0, A[1][0], cmul(w1, A[1][1]));
+            tab[a ^ g] = Sto<S>::narrow(o1);
+            nb += norm2(o1);
+        }
+    }
+    return nb;
+}
+
+// Blocks blk0[j] .. blk0[j + 1] - 1 take the strings of instance order[j].
+template <class S, int NT>
+__global__ __launch_bounds__(NT) void score_lds_kernel(const BInst* __restrict__ insts, int ninst,
+                                                                const int* __restrict__ order,
+                                                                const int* __restrict__ blk0, int tab_bytes,
+                                                                unsigned long long* __restrict__ clock) {
+    constexpr int NW = NT / 64, LT = NT == 64 ? 6 : NT == 256 ? 8 : 9;
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ double nbs[kLdsSteps];
+    __shared__ int s_dead;
+    int j = 0;
+    while (j + 1 < ninst && int(blockIdx.x) >= blk0[j + 1]) j++;
+    const BInst& I = insts[order[j]];
+    const int b = int(blockIdx.x) - blk0[j], B = I.B, ns = I.ns;
+    S* tab = reinterpret_cast<S*>(lds);
+    LStep* st = reinterpret_cast<LStep*>(lds + tab_bytes);
+    double2* wt = reinterpret_cast<double2*>(st + ns);          // [ns][2]
+    double* part = reinterpret_cast<double*>(wt + 2 * ns);      // [ns][NW]
+    unsigned long long* at = reinterpret_cast<unsigned long long*>(nbs);
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const bool times = b == B - 1;                              // the instance's last string tells the steps' times
+    for (int i = t; i < ns * int(sizeof(LStep) / 4); i += NT)
+        reinterpret_cast<uint32_t*>(st)[i] = reinterpret_cast<const uint32_t*>(I.lsteps)[i];
+    for (int i = t; i < ns * NW; i += NT) part[i] = 0;
+    for (int k = t; k < ns; k += NT) {
+        const BStep& s = I.steps[k];
+        const int bv = I.bitsT[size_t(k) * B + b];
+        wt[2 * k] = make_double2(s.mre[bv][0], s.mim[bv][0]);
+        wt[2 * k + 1] = make_double2(s.mre[bv][1], s.mim[bv][1]);
+    }
+    if (t == 0) {
+        tab[0] = Sto<S>::narrow(make_double2(1.0, 0.0));
+        s_dead = ns;
+    }
+    __syncthreads();
+    for (int k = 0; k < ns; k++) {
+        const LStep& s = st[k];
+        const bool wide = NW > 1 && __builtin_amdgcn_readfirstlane(s.nk) > 6;
+        if (wide || wave == 0) {
+            const int ntq = __builtin_amdgcn_readfirstlane(s.ntq), lt = wide ? LT : 6;
+            const double2 w0 = wt[2 * k], w1 = wt[2 * k + 1];
+            double nb = ntq == 1   ? lds_step<S, 1>(s, tab, w0, w1, t, lt)
+                        : ntq == 2 ? lds_step<S, 2>(s, tab, w0, w1, t, lt)
+                                   : lds_step<S, 4>(s, tab, w0, w1, t, lt);
+            nb = gs::wave_sum(nb);
+            if (lane == 0) part[k * NW + wave] = nb;
+            if (times && t == 0) at[k] = wall_clock64();
+            gs::wave_fence();
+        }
+        const bool next = NW > 1 && k + 1 < ns && __builtin_amdgcn_readfirstlane(st[k + 1].nk) > 6;
+        if (wide || next) __syncthreads();
+    }
+    if (times) {
+        __syncthreads();
+        for (int k = t; k < ns && clock; k += NT) atomicMax(clock + 1 + k, at[k]);
+    }
+    __syncthreads();
+    for (int k = t; k < ns; k += NT) {
+        double nb = part[k * NW];
+#pragma unroll
+        for (int w = 1; w < NW; w++) nb += part[k * NW + w];
+        nbs[k] = nb;
+        if (nb <= 0) atomicMin(&s_dead, k);
+    }
+    __syncthreads();
+    const int dead = s_dead;
+    for (int k = t; k < ns; k += NT)
+        I.cond[size_t(b) * ns + k] = k >= dead ? 0 : nbs[k] / (2 * (k ? nbs[k - 1] : 1.0));
+    if (t != 0) return;
+    I.logp[b] = dead < ns ? -INFINITY : log2(ns ? nbs[ns - 1] : 1.0) - ns;
+    const double2 z = Sto<S>::wide(tab[0]);
+    I.amp[2 * b] = z.x;
+    I.amp[2 * b + 1] = z.y;
+    if (clock && ns) atomicMax(clock + ns, (unsigned long long)wall_clock64());
+}
+
+// A step for score_lds_kernel; esz: bytes of an entry.
+LStep make_lstep(const gs::StepInfo& s, int R, size_t esz) {
+    LStep d{};
+    gs::GfBasis span, taken, banks;
+    for (uint64_t c : s.cols) (void)span.add(c);
+    const uint64_t form = span.form(s.rhoc & ((uint64_t(1) << s.nk) - 1)), bank = 256 / esz - 1;
+    std::vector<uint64_t> cand;
+    for (int i = 0; i < R; i++)
+        if (span.has(uint64_t(1) << i)) cand.push_back(uint64_t(1) << i);
+    cand.insert(cand.end(), s.cols.begin(), s.cols.end());
+    for (int pass = 0; pass < 2; pass++)
+        for (uint64_t c : cand) {
+            if (pass == 0 && banks.has(c & bank)) continue;
+            if (!taken.add(c)) continue;
+            (void)banks.add(c & bank);
+            d.rho |= uint32_t(gs::parity(c & form)) << d.nk;
+            d.cols[d.nk++] = uint32_t(c);
+        }
+    for (int q = 0; q < s.ntq; q++) {
+        d.off[q] = uint32_t(s.off[q]);
+        d.t0m |= uint32_t(s.tau0[q] & 1) << q;
+        d.t1m |= uint32_t(s.tau1[q] & 1) << q;
+        d.parm |= uint32_t(s.par[q] & 1) << q;
+    }
+    d.g = uint32_t(s.g);
+    d.ntq = s.ntq;
+    d.m = s.m;
+    return d;
+}
+
 // lambda at the end of the chain: dZ/d(final single entry) = 1
 template <class S>
 __global__ void batch_lambda_init_kernel(const BInst* __restrict__ insts, int ninst) {
@@ -1140,6 +1313,9 @@ struct gs_batch {
     std::vector<int> nq_exact;            // per step: 1 if every instance at the step has nq slots per coset
     std::vector<std::vector<PairDesc>> hpairs;   // [inst][step]: steps k and k+1 as one sweep (ni 0: not possible)
     std::vector<std::vector<FlyDesc>> hflys;     // [inst][step][kMaxUnit - 2]: 3 steps and more (d 0: not possible)
+    // scoring with whole strings in LDS (score_lds_kernel): bytes of its table and of all its LDS (0: not all plans fit)
+    int lds_table = 0, lds_bytes = 0, lds_blocks = 0, lds_threads = 512;
+    int *dorder = nullptr, *dblk0 = nullptr;
     std::vector<char> unit;               // per step: steps of the sweep that starts there (0: inside another's)
     bool pairs_on = true;
     int lu = 2;                           // log2 cosets a lane gathers at once
@@ -1433,6 +1609,13 @@ int enqueue_t(gs_batch* bt) {
     const int ninst = int(bt->plans.size());
     hipLaunchKernelGGL(batch_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst,
                        bt->dclock, bt->maxns);
+    if (bt->lds_bytes && bt->pairs_on) {
+        const int nt = bt->lds_threads;
+        hipLaunchKernelGGL((nt == 64 ? score_lds_kernel<S, 64> : nt == 256 ? score_lds_kernel<S, 256> : score_lds_kernel<S, 512>),
+                           dim3(bt->lds_blocks), dim3(nt), bt->lds_bytes, bt->stream, bt->dinst, ninst, bt->dorder, bt->dblk0,
+                           bt->lds_table, bt->dclock);
+        return hipGetLastError() == hipSuccess ? 0 : bfail(17, "batch launch failed");
+    }
     for (int k = 0; k < bt->maxns; k++) {
         if (!bt->unit[size_t(k)]) continue;               // inside another step's sweep
         if (int rc = launch_step<S>(bt, k, 1, nullptr)) return rc;
@@ -1679,7 +1862,6 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
     auto bail = [&](int rc) {
         for (void* p : bt->allocs) (void)hipFree(p);
         (void)hipFree(bt->item_mem);
-        (void)hipHostFree(bt->hbits);
         (void)hipHostFree(bt->hout);
         delete bt;
         return rc;
@@ -1715,10 +1897,28 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
     bt->dout = dalloc<double>(bt, bt->nout);
     bt->dclock = reinterpret_cast<unsigned long long*>(bt->dout + at_clock);
     if (!bt->dbits || !bt->dout ||
-        hipHostMalloc(reinterpret_cast<void**>(&bt->hbits), std::max<size_t>(bt->nbits, 16), 0) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&bt->hout), std::max<size_t>(bt->nout * sizeof(double), 16), 0) != hipSuccess)
+        hipHostMalloc(reinterpret_cast<void**>(&bt->hout), bt->nout * sizeof(double) + std::max<size_t>(bt->nbits, 16), 0) !=
+            hipSuccess)
         return bail(bfail(11, "batch buffer allocation failed"));
+    bt->hbits = reinterpret_cast<int8_t*>(bt->hout + bt->nout);
     bt->hclock = reinterpret_cast<unsigned long long*>(bt->hout + at_clock);
+    // whether every plan's strings fit the LDS: the table, then per step its descriptor, weights and sums.  One wave per
+    // string up to 2^9 slots, else eight while the chip has a CU per string, four where several tables share a CU: with
+    // 1 / 4 / 8 waves 4096 strings take 83 / 112 / 173 us at 2^9 complex64 slots, 261 / 200 / 280 at 2^11, 659 / 381 /
+    // 438 at 2^12, 1096 / 526 / 506 at 2^12 complex128 ones; 64 strings 34 / 32 / 33, 72 / 45 / 43 and 136 / 65 / 58.
+    int maxR = 0, lds_most = 0;
+    for (const gs::Plan& P : bt->plans) maxR = std::max(maxR, P.R);
+    bool lds_fits = maxR <= kLdsMaxR && bt->maxns <= kLdsSteps;
+    if (lds_fits) {
+        bt->lds_table = int(std::max<size_t>(bt->esz << maxR, 16));
+        for (int b : bt->B) bt->lds_blocks += b;
+        bt->lds_threads = maxR <= 9 ? 64 : bt->lds_blocks > 256 && bt->lds_table <= (32 << 10) ? 256 : 512;
+        bt->lds_bytes = bt->lds_table + bt->maxns * int(sizeof(LStep) + 2 * sizeof(double2) + sizeof(double) * size_t(bt->lds_threads / 64));
+        if (hipDeviceGetAttribute(&lds_most, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
+            return bail(bfail(17, "device LDS size unknown"));
+        lds_fits = bt->lds_bytes + int(sizeof(double)) * kLdsSteps + 64 <= lds_most;
+        if (!lds_fits) bt->lds_bytes = 0;
+    }
     for (int i = 0; i < nplans; i++) {
         const gs::Plan& P = bt->plans[size_t(i)];
         const int B = lanes[i];
@@ -1764,6 +1964,9 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
                 FlyDesc& f = hf[size_t(k) * (kMaxUnit - 2) + size_t(n - 3)];
                 if (!st[n - 1] || !make_fly(st, n, 0, 0, f)) f.d = 0;
             }
+        std::vector<LStep> hl;
+        if (lds_fits)
+            for (const gs::StepInfo& si : P.steps) hl.push_back(make_lstep(si, P.R, bt->esz));
         // the instance's small buffers in one allocation: descriptors first, uploaded in one copy
         size_t used = 0;
         auto take = [&](size_t bytes) {
@@ -1771,12 +1974,12 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
             used += (bytes + 255) & ~size_t(255);
             return at;
         };
-        const size_t o_steps = take(hs.size() * sizeof(BStep)), o_pairs = take(hp.size() * sizeof(PairDesc)),
-                     o_flys = take(hf.size() * sizeof(FlyDesc)), head = used;
         I.narrived = int(part_items(bt, size_t(i)) / kItemGroup);
         const size_t n_arrived = size_t(B / kLanes) * size_t(1 + I.narrived);
+        const size_t o_steps = take(hs.size() * sizeof(BStep)), o_pairs = take(hp.size() * sizeof(PairDesc)),
+                     o_flys = take(hf.size() * sizeof(FlyDesc)), o_lsteps = take(hl.size() * sizeof(LStep)),
+                     o_arrived = take(sizeof(unsigned) * n_arrived), head = used;   // counters start at 0
         const size_t o_prev = take(sizeof(double) * B), o_dead = take(sizeof(int) * B),
-                     o_arrived = take(sizeof(unsigned) * n_arrived),
                      o_part = take(sizeof(double) * size_t(B / kLanes) * part_doubles(bt, size_t(i)));
         char* mem = dalloc<char>(bt, used);
         if (!mem) return bail(bfail(11, "batch buffer allocation failed"));
@@ -1784,6 +1987,7 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
         if (!hs.empty()) memcpy(up.data() + o_steps, hs.data(), hs.size() * sizeof(BStep));
         if (!hp.empty()) memcpy(up.data() + o_pairs, hp.data(), hp.size() * sizeof(PairDesc));
         if (!hf.empty()) memcpy(up.data() + o_flys, hf.data(), hf.size() * sizeof(FlyDesc));
+        if (!hl.empty()) memcpy(up.data() + o_lsteps, hl.data(), hl.size() * sizeof(LStep));
         if (head && hipMemcpy(mem, up.data(), head, hipMemcpyHostToDevice) != hipSuccess)
             return bail(bfail(17, "plan upload failed"));
         bt->hsteps.push_back(std::move(hs));
@@ -1792,6 +1996,7 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
         I.steps = reinterpret_cast<BStep*>(mem + o_steps);
         I.pairs = reinterpret_cast<PairDesc*>(mem + o_pairs);
         I.flys = reinterpret_cast<FlyDesc*>(mem + o_flys);
+        I.lsteps = reinterpret_cast<LStep*>(mem + o_lsteps);
         I.bitsT = bt->dbits + bt->at_bits[size_t(i)];
         I.prev = reinterpret_cast<double*>(mem + o_prev);
         I.dead = reinterpret_cast<int*>(mem + o_dead);
@@ -1799,14 +2004,24 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
         I.logp = bt->dout + bt->at_logp[size_t(i)];
         I.amp = bt->dout + bt->at_amp[size_t(i)];
         I.arrived = reinterpret_cast<unsigned*>(mem + o_arrived);
-        if (hipMemset(I.arrived, 0, sizeof(unsigned) * n_arrived) != hipSuccess)
-            return bail(bfail(17, "counter initialisation failed"));
         I.part = reinterpret_cast<double*>(mem + o_part);
         bt->hinst.push_back(I);
     }
     bt->dinst = dalloc<BInst>(bt, bt->hinst.size());
     if (!bt->dinst || hipMemcpy(bt->dinst, bt->hinst.data(), bt->hinst.size() * sizeof(BInst), hipMemcpyHostToDevice) != hipSuccess)
         return bail(bfail(17, "instance upload failed"));
+    if (bt->lds_bytes) {                                  // the largest plans' strings first
+        std::vector<int> list(size_t(2 * nplans + 1), 0);
+        for (int i = 0; i < nplans; i++) list[size_t(i)] = i;
+        std::stable_sort(list.begin(), list.begin() + nplans,
+                         [&](int a, int b) { return bt->plans[size_t(a)].R > bt->plans[size_t(b)].R; });
+        for (int i = 0; i < nplans; i++)
+            list[size_t(nplans + i + 1)] = list[size_t(nplans + i)] + lanes[list[size_t(i)]];
+        bt->dorder = dalloc<int>(bt, list.size());
+        bt->dblk0 = bt->dorder + nplans;
+        if (!bt->dorder || hipMemcpy(bt->dorder, list.data(), list.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
+            return bail(bfail(17, "work list upload failed"));
+    }
     bt->dptrs = dalloc<void*>(bt, size_t(4 * bt->maxns + 4) * size_t(nplans));
     if (!bt->dptrs) return bail(bfail(11, "allocation failed"));
     if (int rc = build_items(bt)) return bail(rc);
@@ -1823,7 +2038,6 @@ void gs_batch_destroy(gs_batch* bt) {
     free_grad(bt);
     for (void* p : bt->allocs) (void)hipFree(p);
     (void)hipFree(bt->item_mem);
-    (void)hipHostFree(bt->hbits);
     (void)hipHostFree(bt->hout);
     (void)hipEventDestroy(bt->ev0);
     (void)hipEventDestroy(bt->ev1);
@@ -1938,7 +2152,7 @@ int gs_batch_score(gs_batch* bt, const int8_t* const* bits, double* const* log2p
     bt->step_ms.assign(size_t(bt->maxns), -1.0);
     if (!bt->use_graph)
         for (int k = 0, u = 0; k < bt->maxns; k++) {      // the steps of one sweep end together
-            if (bt->unit[size_t(k)]) u = k;
+            if (bt->unit[size_t(k)] || (bt->lds_bytes && bt->pairs_on)) u = k;
             if (bt->nitems[size_t(u)])
                 bt->step_ms[size_t(k)] = double(bt->hclock[size_t(1 + u)] - bt->hclock[0]) / bt->clock_khz;
         }

@@ -36,10 +36,16 @@ struct GfBasis {
             if (row[b] && (parity(comb[b] & f) ^ parity(row[b] & m))) m |= uint64_t(1) << b;
         return m;
     }
-    bool has(uint64_t x) const {
-        uint64_t c;
-        return solve(x, c);
+    // What is left of x modulo the span: equal for x and y when their difference is in it.
+    uint64_t residue(uint64_t x) const {
+        for (uint64_t left = x; left;) {
+            const int b = 63 - __builtin_clzll(left);
+            x ^= row[b];
+            left = x & ((uint64_t(1) << b) - 1);
+        }
+        return x;
     }
+    bool has(uint64_t x) const { return residue(x) == 0; }
 
 private:
     void reduce(uint64_t& v, uint64_t& c) const {

@@ -117,13 +117,18 @@ inline bool make_pair(const StepInfo& s0, const StepInfo& s1, bool units, PairDe
             wr.push_back(at);
             if (s1.m == 2) wr.push_back(at ^ s1.g);
         }
-    auto clash = [&](const std::vector<uint64_t>& x, const std::vector<uint64_t>& y) {
-        for (uint64_t u : x)
-            for (uint64_t v : y)
-                if (u != v && C.has(u ^ v)) return true;
+    const std::vector<uint64_t> rd0 = rd, wr0 = wr;
+    for (auto* v : {&rd, &wr})
+        for (uint64_t& u : *v) u = C.residue(u);
+    // one and the same slot of a super-coset meets itself only
+    auto clash = [&](const std::vector<uint64_t>& x, const std::vector<uint64_t>& y, const std::vector<uint64_t>& x0,
+                     const std::vector<uint64_t>& y0) {
+        for (size_t i = 0; i < x.size(); i++)
+            for (size_t j = 0; j < y.size(); j++)
+                if (x[i] == y[j] && x0[i] != y0[j]) return true;
         return false;
     };
-    if (clash(wr, rd) || clash(wr, wr) || clash(rd, rd)) return false;
+    if (clash(wr, rd, wr0, rd0) || clash(wr, wr, wr0, wr0) || clash(rd, rd, rd0, rd0)) return false;
     p.ni = ni;
     return true;
 }

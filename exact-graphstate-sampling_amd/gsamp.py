@@ -475,7 +475,8 @@ class BatchEngine:
         self._check(library().gs_batch_set_unroll(self._h, int(lu)))
 
     def set_pairs(self, on):
-        """Two or three consecutive steps per sweep where the plans allow it (True, default) or one."""
+        """Several consecutive steps per sweep where the plans allow it, and whole strings in LDS where all of them fit (True,
+        default), or one step per sweep."""
         self._check(library().gs_batch_set_pairs(self._h, 1 if on else 0))
 
     def score(self, bits, want_cond=True, want_amp=True):

@@ -101,10 +101,11 @@ int gs_batch_set_tile(gs_batch* batch, int i, int k, int lg);
 int gs_batch_set_xcd_items(gs_batch* batch, int on);
 /* log2 cosets each lane gathers at once (0..3; default 2 for complex64, 1 for complex128). */
 int gs_batch_set_unroll(gs_batch* batch, int lu);
-/* Two or three consecutive steps per sweep where the plans allow it (on, default) or one (off): scores and gradients differ at
-   most by the order of FP64 sums. */
+/* Several consecutive steps per sweep where the plans allow it, and whole strings in LDS where all of them fit (on,
+   default), or one step per sweep (off): scores and gradients differ at most by the order of FP64 sums. */
 int gs_batch_set_pairs(gs_batch* batch, int on);
-/* Device time of the last gs_batch_score (ms); step_end_ms (may be NULL) [max ns]: end of each step after the start. */
+/* Device time of the last gs_batch_score (ms); step_end_ms (may be NULL) [max ns]: end of each step after the start (strings
+   in LDS: an instance's last step for all of its strings, the steps before for its last string). */
 double gs_batch_last_ms(const gs_batch* batch, double* step_end_ms);
 /* Replace instance i's measurement matrices M[ns][2][2] (complex as re, im pairs; M[k][b][x]). */
 int gs_batch_set_matrices(gs_batch* batch, int i, const double* M);
