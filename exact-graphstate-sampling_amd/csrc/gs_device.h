@@ -96,8 +96,8 @@ struct SStep {
     uint32_t cols[kSmallMaxNk];     // LDS index of each coset coordinate's column (0 beyond nk), as the plain descriptor's
     uint32_t off[4], g;             // of the coset offsets (beyond ntq: the first again) and of g
     uint32_t rho;                   // sign mask over the coordinates
-    uint32_t route;                 // a bit per offset: output of its x = 0 term | of its x = 1 term << 4 | its par << 8
-    int nk, ntq, m, growth, pad;
+    uint32_t par;                   // a bit per offset
+    int nk, ntq, m, growth, kind;   // kind: ntq * 4 + Route
     double mre[2][2], mim[2][2];
 };
 

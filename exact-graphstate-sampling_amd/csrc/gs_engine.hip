@@ -1363,12 +1363,8 @@ void build_small(gs_engine* e) {
             d.ntq = s.ntq;
             d.m = s.m;
             d.growth = s.growth;
-            for (int j = 0; j < s.ntq; j++) {             // the canonical routes (see Route)
-                const int t0 = s.route == kRouteMixA || s.route == kRouteMixB ? j & 1 : 0;
-                const int t1 = s.route == kRoute1 ? 0 : s.route == kRouteSplit ? 1 : s.route == kRouteMixA ? 1 - (j & 1)
-                                                                                                        : (j & 1);
-                d.route |= uint32_t(t0) << j | uint32_t(t1) << (4 + j) | ((s.parmask >> j) & 1) << (8 + j);
-            }
+            d.kind = s.ntq * 4 + s.route;
+            d.par = s.parmask;
             memcpy(d.mre, s.mre, sizeof d.mre);
             memcpy(d.mim, s.mim, sizeof d.mim);
             e->small_at[size_t(q)] = int(e->small_dim.size());

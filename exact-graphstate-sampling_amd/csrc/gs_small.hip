@@ -8,11 +8,11 @@
 //
 // What bounds it is latency: a step has little to compute and two sums over the cosets that the next pass needs.  So
 // the chain state lives in registers of every thread (each makes the decision itself, no broadcast), sums go through
-// DPP inside a wave and one barrier across waves, steps of at most 64 cosets run on the first wave with no barrier at
-// all, every descriptor, bit and uniform is in LDS before the first step, and the logarithms, which no decision needs,
-// are taken for all steps at once at the end.  A version with the table in the arena, state changes by one thread and
-// two barriers per pass took 4.6 us per step; this one takes 2.0 us
-// (the n = 24 plan, 24 steps, complex64: 115 -> 49.5 us).
+// lane swaps and DPP inside a wave and one barrier across waves, steps of at most 64 cosets run on the first wave with no
+// barrier at all (narrow_steps), every descriptor, bit and uniform is in LDS before the first step, and the logarithms,
+// which no decision needs, are taken for all steps at once at the end.  A version with the table in the arena, state
+// changes by one thread and two barriers per pass took 4.6 us per step; with one code for all steps it was 2.0 us, and
+// this one takes 1.3 us (the n = 24 plan, 24 steps, complex64: 115 -> 49.5 -> 33.6 us).
 #include "gs_math.h"
 #include "gs_wave.h"
 
@@ -22,8 +22,17 @@ namespace {
 
 constexpr int kWavesS = kSmallThreads / 64;
 
+// A step of at most 64 cosets, as the first wave reads it: offsets two to a word, g, and kind | m << 5 | par << 8 |
+// growth << 12 | next step's growth << 13 | nk << 16.
+struct NStep {
+    uint32_t o01, o23, g, bits;
+};
+
 struct Shared {                       // after the table in LDS
     SStep s[kSmallSteps];
+    NStep n[kSmallSteps];
+    double coef[kSmallSteps][2][4];   // per branch |m0|^2, |m1|^2, Re and Im of m0 conj(m1)
+    uint32_t word[kSmallSteps][64];   // per lane: index of its coset's base, its sign in bit 31
     double U[kSmallSteps];
     double pfac[kSmallSteps], plog[kSmallSteps];      // factors of Pr, and their log2 at the end of the run
     double sfac[kSmallSteps], slog[kSmallSteps];      // table norms of the rescalings (kRun), and their log2
@@ -45,33 +54,71 @@ struct State {
     bool neglog;                      // a zero-probability branch: log2 Pr = -inf
 };
 
-// Sums of a pass over the threads that run it, in every one of them.
+// Sums of a pass over the threads that run it, in every one of them.  nw: waves with cosets (the others' sums are zeros);
+// across waves lane q adds up value q, in wave order.
 template <bool WIDE, int NQ>
-__device__ __forceinline__ void pass_sum(Shared& sh, int& buf, const double (&v)[4], double (&out)[4]) {
-    double r[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) r[q] = wave_sum(v[q]);
+__device__ __forceinline__ void pass_sum(Shared& sh, int& buf, const double (&v)[4], double (&out)[4], int nw) {
+    const int lane = threadIdx.x & 63;
+    const double r = NQ == 4 ? sum4(v) : NQ == 2 ? sum2(v) : wave_sum(v[0]);
     if constexpr (WIDE) {
-        const int wave = threadIdx.x >> 6;
-        if ((threadIdx.x & 63) == 0)
-#pragma unroll
-            for (int q = 0; q < NQ; q++) sh.sum[buf][wave][q] = r[q];
+        const int wave = threadIdx.x >> 6, row = lane >> 4;
+        if ((lane & 15) == 0) sh.sum[buf][wave][NQ == 4 ? (row >> 1) | (row & 1) << 1 : row >> 1] = r;   // see sum2, sum4
         __syncthreads();
+        double x = sh.sum[buf][0][lane & 3];
 #pragma unroll
-        for (int q = 0; q < NQ; q++) {
-            double x = sh.sum[buf][0][q];
-#pragma unroll
-            for (int w = 1; w < kWavesS; w++) x += sh.sum[buf][w][q];
-            r[q] = x;
+        for (int w = 1; w < kWavesS; w++) {
+            if (w >= nw) break;
+            x += sh.sum[buf][w][lane & 3];
         }
         buf ^= 1;
-    }
 #pragma unroll
-    for (int q = 0; q < NQ; q++) out[q] = r[q];
+        for (int q = 0; q < NQ; q++) out[q] = lane_value(x, q);
+    } else {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) out[q] = lane_value(r, NQ == 4 ? 32 * (q & 1) + 16 * (q >> 1) : 32 * q);
+    }
+}
+
+// Routed slot sums A[tau][x] of the coset at a (sign pc), slots in ascending order; kind: slots * 4 + Route, uniform.
+template <class S, int NTQ, int ROUTE>
+__device__ __forceinline__ void slot_sums(const S* tab, uint32_t a, const uint32_t (&off)[4], uint32_t pc, uint32_t par,
+                                          double2 (&A)[2][2]) {
+    S v[NTQ];
+#pragma unroll
+    for (int j = 0; j < NTQ; j++) v[j] = tab[a ^ off[j]];
+    A[0][0] = A[0][1] = A[1][0] = A[1][1] = make_double2(-0.0, -0.0);
+#pragma unroll
+    for (int j = 0; j < NTQ; j++) {
+        const double2 w = Cx<S>::widen(v[j]);
+        const int neg = int((pc ^ (par >> j)) << 31);
+        const double2 ws = make_double2(__hiloint2double(__double2hiint(w.x) ^ neg, __double2loint(w.x)),
+                                        __hiloint2double(__double2hiint(w.y) ^ neg, __double2loint(w.y)));
+        constexpr bool MIX = ROUTE == kRouteMixA || ROUTE == kRouteMixB;
+        const int t0 = MIX ? j & 1 : 0;
+        const int t1 = ROUTE == kRoute1 ? 0 : ROUTE == kRouteSplit ? 1 : ROUTE == kRouteMixA ? 1 - (j & 1) : (j & 1);
+        A[t0][0] = cadd(A[t0][0], w);
+        A[t1][1] = cadd(A[t1][1], ws);
+    }
+}
+template <class S>
+__device__ __forceinline__ void slot_sums_of(int kind, const S* tab, uint32_t a, const uint32_t (&off)[4], uint32_t pc,
+                                             uint32_t par, double2 (&A)[2][2]) {
+    switch (kind) {
+        case 1 * 4 + kRoute1: slot_sums<S, 1, kRoute1>(tab, a, off, pc, par, A); break;
+        case 1 * 4 + kRouteSplit: slot_sums<S, 1, kRouteSplit>(tab, a, off, pc, par, A); break;
+        case 2 * 4 + kRoute1: slot_sums<S, 2, kRoute1>(tab, a, off, pc, par, A); break;
+        case 2 * 4 + kRouteSplit: slot_sums<S, 2, kRouteSplit>(tab, a, off, pc, par, A); break;
+        case 2 * 4 + kRouteMixA: slot_sums<S, 2, kRouteMixA>(tab, a, off, pc, par, A); break;
+        case 2 * 4 + kRouteMixB: slot_sums<S, 2, kRouteMixB>(tab, a, off, pc, par, A); break;
+        case 4 * 4 + kRoute1: slot_sums<S, 4, kRoute1>(tab, a, off, pc, par, A); break;
+        case 4 * 4 + kRouteSplit: slot_sums<S, 4, kRouteSplit>(tab, a, off, pc, par, A); break;
+        case 4 * 4 + kRouteMixA: slot_sums<S, 4, kRouteMixA>(tab, a, off, pc, par, A); break;
+        default: slot_sums<S, 4, kRouteMixB>(tab, a, off, pc, par, A); break;
+    }
 }
 
 // One step on one wave (at most 64 cosets) or on the whole block.  last: the run's last step, whose outputs go to the
-// arena.
+// arena.  A thread with one coset keeps its slot sums from the norm pass for the write.
 template <class S, bool WIDE>
 __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KStep* plain, const Epi& e, State& st, int k,
                                            int k0, bool decided, bool last) {
@@ -79,13 +126,12 @@ __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KSt
     const int t = threadIdx.x;
     constexpr int T = WIDE ? kSmallThreads : 64;
     constexpr int LT = WIDE ? 9 : 6;
-    const int nk = __builtin_amdgcn_readfirstlane(s.nk), ntq = __builtin_amdgcn_readfirstlane(s.ntq);
-    const int m = __builtin_amdgcn_readfirstlane(s.m);
-    const uint32_t route = __builtin_amdgcn_readfirstlane(int(s.route));   // t0 | t1 << 4 | par << 8, a bit per offset
-    const uint32_t rho = s.rho, g = s.g;
+    auto uni = [](uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); };
+    const int nk = int(uni(uint32_t(s.nk))), m = int(uni(uint32_t(s.m))), kind = int(uni(uint32_t(s.kind)));
+    const uint32_t par = uni(s.par), rho = uni(s.rho), g = uni(s.g);
     uint32_t off[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) off[j] = s.off[j];
+    for (int j = 0; j < 4; j++) off[j] = uni(s.off[j]);
     uint32_t bt = 0;
 #pragma unroll
     for (int j = 0; j < LT; j++)                               // columns beyond nk are 0
@@ -96,6 +142,8 @@ __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KSt
 #pragma unroll
         for (int x = 0; x < 2; x++) M[b][x] = make_double2(s.mre[b][x], s.mim[b][x]);
     const uint32_t n = 1u << nk;
+    const bool one = !WIDE || n <= uint32_t(T);
+    const int nw = n >= uint32_t(T) ? kWavesS : int(n >> 6);    // only the wide path asks
     // index of coset c (c = t mod T) and its routed slot sums
     auto index_of = [&](uint32_t c) {
         uint32_t a = bt;
@@ -104,29 +152,15 @@ __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KSt
             for (int j = LT; j < kSmallMaxNk; j++) a ^= ((c >> j) & 1) ? s.cols[j] : 0;
         return a;
     };
-    auto sums = [&](uint32_t a, uint32_t c, double2 (&A)[2][2]) {
-        S v[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = tab[a ^ off[j]];    // offsets beyond ntq repeat the first
-        const uint32_t pc = __popc(c & rho) & 1;
-        A[0][0] = A[0][1] = A[1][0] = A[1][1] = make_double2(-0.0, -0.0);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (j >= ntq) break;
-            const double2 w = Cx<S>::widen(v[j]);
-            const int neg = int((pc ^ (route >> (8 + j))) << 31);
-            const double2 ws = make_double2(__hiloint2double(__double2hiint(w.x) ^ neg, __double2loint(w.x)),
-                                            __hiloint2double(__double2hiint(w.y) ^ neg, __double2loint(w.y)));
-            if ((route >> j) & 1) A[1][0] = cadd(A[1][0], w); else A[0][0] = cadd(A[0][0], w);       // uniform branches
-            if ((route >> (4 + j)) & 1) A[1][1] = cadd(A[1][1], ws); else A[0][1] = cadd(A[0][1], ws);
-        }
-    };
+    double2 A[2][2];
+    auto sums = [&](uint32_t a, uint32_t c) { slot_sums_of<S>(kind, tab, a, off, uint32_t(__popc(c & rho)) & 1, par, A); };
+    bool have = false;                                         // A holds the sums of this thread's only coset
     // Norms the decision needs: none when it is forced or made without them (chain1, forced hybrid steps) or follows
     // from the stored norm (growth steps), direct branch norms for a forced string, else the Gram matrix.
     if (!decided) {
         int bv = e.forced ? int(sh.forced[k - k0]) : -1;
         const bool need_p = e.mode == kChain || (e.mode == kRun && bv < 0);
-        const int growth = __builtin_amdgcn_readfirstlane(s.growth);
+        const int growth = int(uni(uint32_t(s.growth)));
         double n2[2] = {0, 0};
         if (need_p && growth) {
 #pragma unroll
@@ -135,8 +169,7 @@ __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KSt
             double acc[4] = {0, 0, 0, 0}, red[4];
             const bool direct = e.mode == kChain && e.forced;
             for (uint32_t c = t; c < n; c += T) {
-                double2 A[2][2];
-                sums(index_of(c), c, A);
+                sums(index_of(c), c);
 #pragma unroll
                 for (int q = 0; q < 2; q++) {
                     const double2 a = A[q][0], b = A[q][1];
@@ -151,7 +184,9 @@ __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KSt
                     }
                 }
             }
-            pass_sum<WIDE, 4>(sh, st.buf, acc, red);
+            have = one;
+            if (direct) pass_sum<WIDE, 2>(sh, st.buf, acc, red, nw);
+            else pass_sum<WIDE, 4>(sh, st.buf, acc, red, nw);
 #pragma unroll
             for (int b = 0; b < 2; b++) {
                 const double2 m0 = M[b][0], m1 = M[b][1];
@@ -161,7 +196,10 @@ __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KSt
         }
         double sc = 1.0;
         if (e.mode == kChain) {
-            const double p1 = n2[1] / (n2[0] + n2[1]);
+            double both = 1.0 / sqrt((t & 1) ? n2[1] : n2[0]);  // lane 0: branch 0, lane 1: branch 1
+            double p1 = n2[1] / (n2[0] + n2[1]);
+            here(both);                                         // the two beside each other
+            here(p1);
             if (bv < 0) bv = sh.U[k - k0] < p1;
             const double pb = bv ? p1 : 1 - p1;
             if (pb <= 0) {
@@ -171,7 +209,7 @@ __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KSt
             }
             if (t == 0) sh.pfac[st.np] = pb;
             st.np++;
-            sc = 1.0 / sqrt(bv ? n2[1] : n2[0]);
+            sc = lane_value(both, __builtin_amdgcn_readfirstlane(bv));
         } else if (e.mode == kRun) {
             sc = 1.0 / sqrt(st.prev);
             if (bv < 0) bv = sh.U[st.qidx++] < n2[1] / (n2[0] + n2[1]);
@@ -186,9 +224,8 @@ __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KSt
     }
     double acc[4] = {0, 0, 0, 0}, red[4];
     for (uint32_t c = t; c < n; c += T) {
-        double2 A[2][2];
         const uint32_t a = index_of(c);
-        sums(a, c, A);
+        if (!have) sums(a, c);
         uint64_t pa = 0;
         if (last)
             for (int j = 0; j < nk; j++)
@@ -205,8 +242,15 @@ __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KSt
         }
     }
     if constexpr (!WIDE) wave_fence();
-    pass_sum<WIDE, 2>(sh, st.buf, acc, red);
-    st.nstored = red[1];
+    // the written norm is used outside the renormalised chain, the stored one by a growth step or after the run
+    const bool stored = e.mode != kChain1 && (last || uni(uint32_t(sh.s[k + 1 - k0].growth)) != 0);
+    if (e.mode == kChain && !stored) {
+        if constexpr (WIDE) __syncthreads();
+        return;
+    }
+    if (stored) pass_sum<WIDE, 2>(sh, st.buf, acc, red, nw);
+    else pass_sum<WIDE, 1>(sh, st.buf, acc, red, nw);
+    if (stored) st.nstored = red[1];
     const double nb = red[0];
     if (e.mode == kChain1) {                                   // gsamp2.cpp:67
         if (t == 0) sh.cond[k - k0] = nb / (2 * st.prev);
@@ -225,6 +269,151 @@ __device__ __forceinline__ void small_step(Shared& sh, S* tab, S* mem, const KSt
         else st.np++;
     }
     if (e.mode != kChain && nb <= 0) st.neglog = true;
+}
+
+// Steps from k on while they have at most 64 cosets (before step `to`), on the first wave alone; returns the step it
+// stopped at.  The chain from one step to the next is all latency -- slots from LDS, sums over the wave, a square root and
+// a division, the outputs -- so everything else is out of it: bases and signs of every lane were computed for all steps
+// at once, the next step's are fetched during this one, four sums share one butterfly, and both branches' scales are
+// taken on two lanes while p1 is divided.
+template <class S, int MODE>
+__device__ __forceinline__ int narrow_steps(Shared& sh, S* tab, bool forced, State& st, int k, int k0, int to) {
+    const int t = threadIdx.x;
+    auto uni = [](uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); };
+    NStep nx = sh.n[k - k0];
+    uint32_t word = sh.word[k - k0][t];
+    while (k < to) {
+        const uint32_t o01 = uni(nx.o01), o23 = uni(nx.o23), g = uni(nx.g), bits = uni(nx.bits);
+        const uint32_t a = word & 0xffffu, pc = word >> 31;
+        const uint32_t off[4] = {o01 & 0xffffu, o01 >> 16, o23 & 0xffffu, o23 >> 16};
+        const int i = k - k0, m = int(bits >> 5) & 3;
+        const bool on = uint32_t(t) < (1u << (bits >> 16));
+        double2 A[2][2];
+        if (on) slot_sums_of<S>(int(bits & 31), tab, a, off, pc, (bits >> 8) & 15, A);
+        else A[0][0] = A[0][1] = A[1][0] = A[1][1] = make_double2(0, 0);
+        if (k + 1 < to) {
+            nx = sh.n[i + 1];
+            word = sh.word[i + 1][t];
+        }
+        const SStep& s = sh.s[i];
+        const double2 M[2][2] = {{make_double2(s.mre[0][0], s.mim[0][0]), make_double2(s.mre[0][1], s.mim[0][1])},
+                                 {make_double2(s.mre[1][0], s.mim[1][0]), make_double2(s.mre[1][1], s.mim[1][1])}};
+        int bv = forced ? int(sh.forced[i]) : -1;
+        double u = MODE == kChain ? sh.U[i] : MODE == kRun ? sh.U[st.qidx] : 0;
+        double cf[2][4];
+        if constexpr (MODE != kChain1) {
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) cf[b][j] = sh.coef[i][b][j];
+        }
+        bv = __builtin_amdgcn_readfirstlane(bv);
+        const bool growth = (bits >> 12) & 1;
+        double sc = 1.0;
+        if constexpr (MODE == kRun) sc = 1.0 / sqrt(st.prev);
+        if (MODE == kChain || (MODE == kRun && bv < 0)) {
+            double n2[2];
+            if (growth) {
+#pragma unroll
+                for (int b = 0; b < 2; b++) n2[b] = (cf[b][0] + cf[b][1]) * st.nstored;
+            } else if (MODE == kChain && forced) {
+                double acc[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    if (q >= m) break;
+                    add_norm(acc[0], cfma(M[0][0], A[q][0], cmul(M[0][1], A[q][1])));
+                    add_norm(acc[1], cfma(M[1][0], A[q][0], cmul(M[1][1], A[q][1])));
+                }
+                const double r = sum2(acc);
+                n2[0] = lane_value(r, 0);
+                n2[1] = lane_value(r, 32);
+            } else {
+                double acc[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    if (q >= m) break;
+                    const double2 x = A[q][0], y = A[q][1];
+                    add_norm(acc[0], x);
+                    add_norm(acc[1], y);
+                    acc[2] = fma(x.x, y.x, fma(x.y, y.y, acc[2]));
+                    acc[3] = fma(x.y, y.x, fma(-x.x, y.y, acc[3]));
+                }
+                const double r = sum4(acc);
+                const double r0 = lane_value(r, 0), r1 = lane_value(r, 32), r2 = lane_value(r, 16), r3 = lane_value(r, 48);
+#pragma unroll
+                for (int b = 0; b < 2; b++) n2[b] = cf[b][0] * r0 + cf[b][1] * r1 + 2 * (cf[b][2] * r2 - cf[b][3] * r3);
+            }
+            double p1 = n2[1] / (n2[0] + n2[1]);
+            if constexpr (MODE == kChain) {
+                double both = 1.0 / sqrt((t & 1) ? n2[1] : n2[0]);   // lane 0: branch 0, lane 1: branch 1
+                here(both);
+                here(p1);
+                if (bv < 0) bv = __builtin_amdgcn_readfirstlane(int(u < p1));
+                const double pb = bv ? p1 : 1 - p1;
+                if (__builtin_amdgcn_readfirstlane(int(pb <= 0))) {
+                    st.neglog = true;
+                    st.dead = 1;
+                    return k;
+                }
+                if (t == 0) sh.pfac[st.np] = pb;
+                st.np++;
+                sc = lane_value(both, bv);
+            } else {
+                bv = __builtin_amdgcn_readfirstlane(int(u < p1));
+                st.qidx++;
+            }
+        }
+        if (t == 0) sh.bits[i] = int8_t(bv);
+        st.bv = bv;
+        st.sc = sc;
+        const double2 m0 = bv ? M[1][0] : M[0][0], m1 = bv ? M[1][1] : M[0][1];
+        st.w0 = make_double2(m0.x * sc, m0.y * sc);
+        st.w1 = make_double2(m1.x * sc, m1.y * sc);
+        double acc[4] = {0, 0, 0, 0};
+        if (on) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                if (q >= m) break;
+                const double2 v = cfma(st.w0, A[q][0], cmul(st.w1, A[q][1]));
+                const S sv = Cx<S>::narrow(v);
+                tab[q ? a ^ g : a] = sv;
+                add_norm(acc[0], v);
+                add_norm(acc[1], Cx<S>::widen(sv));
+            }
+        }
+        wave_fence();
+        k++;
+        const bool stored = MODE != kChain1 && ((bits >> 13) & 1);
+        if (MODE == kChain && !stored) continue;
+        double nb;
+        if (stored) {
+            const double r = sum2(acc);
+            nb = lane_value(r, 0);
+            st.nstored = lane_value(r, 32);
+        } else {
+            nb = wave_sum(acc[0]);
+        }
+        if constexpr (MODE == kChain1) {                       // gsamp2.cpp:67
+            if (t == 0) sh.cond[i] = nb / (2 * st.prev);
+            st.prev = nb;
+        } else if constexpr (MODE == kRun) {                   // gsamp2.cpp:93-95
+            const double cd = nb / 2;
+            if (t == 0) {
+                sh.sfac[st.nsf] = st.prev;
+                sh.cond[i] = cd;
+                sh.pfac[st.np] = cd;
+            }
+            st.nsf++;
+            st.prev = nb;
+            if (!__builtin_amdgcn_readfirstlane(int(nb <= 0))) st.np++;
+        }
+        if (MODE != kChain && __builtin_amdgcn_readfirstlane(int(nb <= 0))) {
+            st.dead = 1;
+            st.neglog = true;
+            return k - 1;
+        }
+    }
+    return k;
 }
 
 // Steps k0 .. k1-1 of one chain, one block per string.  start: the chain begins here (table 1, fresh state); decided0:
@@ -269,11 +458,32 @@ __global__ __launch_bounds__(kSmallThreads) void small_run_kernel(const SStep* _
         }
     }
     st.qidx = 0;
-    if (start) {
-        if (t == 0) tab[0] = Cx<S>::narrow(make_double2(1.0, 0.0));
-        __syncthreads();
-    } else {
-        __syncthreads();
+    if (start && t == 0) tab[0] = Cx<S>::narrow(make_double2(1.0, 0.0));
+    __syncthreads();
+    for (int i = t >> 6; i < steps_n; i += kWavesS) {
+        const SStep& s = sh.s[i];
+        if (s.nk > 6) continue;
+        const int lane = t & 63;
+        uint32_t a = 0;
+#pragma unroll
+        for (int j = 0; j < 6; j++) a ^= ((lane >> j) & 1) ? s.cols[j] : 0;
+        sh.word[i][lane] = a | (uint32_t(__popc(uint32_t(lane) & s.rho)) << 31);
+        if (lane < 2) {
+            const double2 m0 = make_double2(s.mre[lane][0], s.mim[lane][0]), m1 = make_double2(s.mre[lane][1], s.mim[lane][1]);
+            sh.coef[i][lane][0] = norm2(m0);
+            sh.coef[i][lane][1] = norm2(m1);
+            sh.coef[i][lane][2] = m0.x * m1.x + m0.y * m1.y;   // m0 conj(m1)
+            sh.coef[i][lane][3] = m0.y * m1.x - m0.x * m1.y;
+        }
+        if (lane == 0) {
+            const uint32_t next = i + 1 < steps_n ? uint32_t(sh.s[i + 1].growth != 0) : 1u;
+            sh.n[i] = NStep{s.off[0] | s.off[1] << 16, s.off[2] | s.off[3] << 16, s.g,
+                            uint32_t(s.kind) | uint32_t(s.m) << 5 | s.par << 8 | uint32_t(s.growth != 0) << 12 | next << 13 |
+                                uint32_t(s.nk) << 16};
+        }
+    }
+    __syncthreads();
+    if (!start) {
         const SStep& s = sh.s[0];
         const KStep& p = plain[k0];
         for (int i = t; i < (s.ntq << s.nk); i += kSmallThreads) {     // the live slots of step k0
@@ -301,10 +511,19 @@ __global__ __launch_bounds__(kSmallThreads) void small_run_kernel(const SStep* _
         int to = k;                                            // steps of one wave
         while (to < k1 && sh.s[to - k0].nk <= 6) to++;
         if (t < 64) {
-            for (; k < to && !st.dead;) {
-                small_step<S, false>(sh, tab, mem, plain, e, st, k, k0, decided, k + 1 == k1);
-                decided = false;
-                if (!st.dead) k++;
+            while (k < to && !st.dead) {
+                const int stop = to == k1 ? k1 - 1 : to;       // the run's last step writes to the arena
+                if (decided || k >= stop) {
+                    small_step<S, false>(sh, tab, mem, plain, e, st, k, k0, decided, k + 1 == k1);
+                    decided = false;
+                    if (!st.dead) k++;
+                } else if (e.mode == kChain) {
+                    k = narrow_steps<S, kChain>(sh, tab, e.forced != nullptr, st, k, k0, stop);
+                } else if (e.mode == kChain1) {
+                    k = narrow_steps<S, kChain1>(sh, tab, true, st, k, k0, stop);
+                } else {
+                    k = narrow_steps<S, kRun>(sh, tab, e.forced != nullptr, st, k, k0, stop);
+                }
             }
             if (t == 0) {
                 Ctl c{};
