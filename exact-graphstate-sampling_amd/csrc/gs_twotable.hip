@@ -82,7 +82,7 @@ struct gs_tt_engine {
     std::vector<void*> fold_fn;          // ... with this kernel (nullptr: it does not)
     std::vector<char> growth;            // per step: both branch norms follow from the stored table's norm
     TFold* dfold = nullptr;
-    std::vector<TStep> hsteps;
+    std::vector<TStep> hsteps;           // [2 ns]: see tt_geometry
     double* part = nullptr;
     unsigned* counter = nullptr;
     Ctl* ctl = nullptr;
@@ -173,7 +173,8 @@ int launch_one(gs_tt_engine* e, void* fn, Epi epi, int k) {
 
 // One gather sweep of step k reading table `in` (norm pass) or reading `in` and writing `1 - in` (write pass).
 int launch_gather(gs_tt_engine* e, int k, int sweep, int in, const Epi& epi, const double* wext) {
-    const TStep* sp = e->dsteps + k;
+    const size_t at = size_t(k) + (sweep == kWrite && epi.mode != kRun ? e->hsteps.size() / 2 : 0);
+    const TStep* sp = e->dsteps + at;
     const void* old = e->tab[in];
     void* nw = e->tab[1 - in];
     double* part = e->part;
@@ -181,7 +182,7 @@ int launch_gather(gs_tt_engine* e, int k, int sweep, int in, const Epi& epi, con
     Epi ep = epi;
     const double* w = wext;
     void* args[] = {&sp, &old, &nw, &part, &ctl, &ep, &w};
-    const int grid = 1 << e->hsteps[size_t(k)].lg_grid;
+    const int grid = 1 << e->hsteps[at].lg_grid;
     void* fn = gather_kernel_ptr(e->storage, sweep, e->hsteps[size_t(k)].nks);
     if (!fn) return ttfail(15, "no gather kernel for step " + std::to_string(k));
     TT_TRY(hipLaunchKernel(fn, dim3(grid), dim3(kThreads), args, 0, e->stream));
@@ -334,21 +335,29 @@ int run_forced(gs_tt_engine* e, int mode, const int8_t* bits, int64_t nstr, doub
     return 0;
 }
 
+// Writes whose sums are free: log2 blocks, up to 2^kWriteFewLog2 outputs and above (renormalised samples at 2^10 / 2^12 /
+// 2^14 blocks: width 26 8.63 / 8.83 / 8.86 ms, width 27 15.0 / 15.7 / 15.4, width 29 64.0 / 65.4 / 61.9), and the fewest
+// that a partner direction is worth.
+constexpr int kWriteGridFew = 10, kWriteGridMany = 14, kWriteFewLog2 = 27, kMinPartnerGrid = 9;
+
 // Blocks and tiles per block of every step's gather sweep (2^rn outputs, one per thread and tile), and its partner
 // direction: an output-space vector pdelta whose image pD = pdep(pdelta) is xbit ^ kspan[q] for some q.  Output
 // u0 ^ pD then gathers the entries (u0 ^ kspan[t ^ q]) & lowmask, the same as output u0: the x bit is not an address
 // bit of the old table.  Used when the top bit of pdelta is a tile bit above the first (the kernel's groups of 4
 // tiles pair j with j + 2 along pdelta).
+// The second half of the descriptors is for writes whose norms have no bearing on later values (renormalised strings,
+// whose scales come from norm passes, and strings with given weights): they take fewer blocks where that makes a partner
+// direction's top bit a tile bit, so that each entry is read once (a width-26 plateau step's write 270 - 330 -> 200 us).
 void tt_geometry(gs_tt_engine* e) {
-    for (auto& t : e->hsteps) {
+    const size_t n = e->hsteps.size() / 2;
+    std::copy_n(e->hsteps.begin(), n, e->hsteps.begin() + std::ptrdiff_t(n));
+    for (size_t i = 0; i < 2 * n; i++) {
+        TStep& t = e->hsteps[i];
         const int tiles = std::max(0, t.rn - 8);
         t.lg_grid = std::min(tiles, e->grid_cap);
-        t.lg_iter = tiles - t.lg_grid;
         t.ph = -1;
         t.pdelta = t.pD = 0;
         t.ptd = 0;
-        if (t.lg_iter < 2) continue;
-        const int jit = 8 + t.lg_grid;
         for (int q = 0; q < t.nks; q++) {
             const uint64_t D = t.xbit ^ t.kspan[q];
             uint64_t delta = 0, rest = D;
@@ -359,7 +368,9 @@ void tt_geometry(gs_tt_engine* e) {
                 }
             if (rest || !delta) continue;             // D outside the outputs' image
             const int h = 63 - __builtin_clzll(delta);
-            if (h >= jit + 1) {
+            if (i >= n && h - 9 >= kMinPartnerGrid)
+                t.lg_grid = std::min({t.lg_grid, h - 9, std::max(tiles - 2, 0), t.rn <= kWriteFewLog2 ? kWriteGridFew : kWriteGridMany});
+            if (tiles - t.lg_grid >= 2 && h >= 9 + t.lg_grid) {
                 t.ph = h;
                 t.pdelta = delta;
                 t.pD = D;
@@ -367,6 +378,7 @@ void tt_geometry(gs_tt_engine* e) {
             }
             break;
         }
+        t.lg_iter = tiles - t.lg_grid;
     }
 }
 
@@ -508,7 +520,7 @@ int gs_tt_engine_create(const gs_tt_plan* plan, int storage, int device, gs_tt_e
     if (hipSetDevice(device) != hipSuccess) return bail(ttfail(17, "hipSetDevice failed"));
     const int ns = e->plan.ns;
     const size_t nsz = size_t(std::max(ns, 1));
-    e->hsteps.assign(nsz, TStep{});
+    e->hsteps.assign(2 * nsz, TStep{});
     std::vector<KStep> hplain(nsz, KStep{});
     for (int k = 0; k < ns; k++) {
         const TTStep& s = e->plan.steps[size_t(k)];
@@ -544,7 +556,7 @@ int gs_tt_engine_create(const gs_tt_plan* plan, int storage, int device, gs_tt_e
     const size_t C = gs_tt_engine::kChunk;
     auto dev_alloc = [&](void** p, size_t n) { return hipMalloc(p, std::max<size_t>(n, 16)) == hipSuccess; };
     auto host_alloc = [&](void** p, size_t n) { return hipHostMalloc(p, std::max<size_t>(n, 16), 0) == hipSuccess; };
-    bool ok = dev_alloc((void**)&e->dsteps, sizeof(TStep) * nsz) && dev_alloc((void**)&e->dfold, sizeof(TFold) * nsz) &&
+    bool ok = dev_alloc((void**)&e->dsteps, 2 * sizeof(TStep) * nsz) && dev_alloc((void**)&e->dfold, sizeof(TFold) * nsz) &&
               dev_alloc((void**)&e->dplain, sizeof(KStep) * nsz) &&
               dev_alloc((void**)&e->part, sizeof(double) * kPartDoubles) &&
               dev_alloc((void**)&e->counter, sizeof(unsigned) * kCounters) && dev_alloc((void**)&e->ctl, sizeof(Ctl)) &&
@@ -558,7 +570,7 @@ int gs_tt_engine_create(const gs_tt_plan* plan, int storage, int device, gs_tt_e
               host_alloc((void**)&e->h_amp, 16 * C);
     if (!ok) return bail(ttfail(11, "allocation of engine buffers failed"));
     if (hipStreamCreate(&e->stream) != hipSuccess) return bail(ttfail(17, "stream creation failed"));
-    if (hipMemcpy(e->dsteps, e->hsteps.data(), sizeof(TStep) * nsz, hipMemcpyHostToDevice) != hipSuccess ||
+    if (hipMemcpy(e->dsteps, e->hsteps.data(), 2 * sizeof(TStep) * nsz, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(e->dfold, e->hfold.data(), sizeof(TFold) * nsz, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(e->dplain, hplain.data(), sizeof(KStep) * nsz, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(e->counter, 0, sizeof(unsigned) * kCounters) != hipSuccess || hipDeviceSynchronize() != hipSuccess)
