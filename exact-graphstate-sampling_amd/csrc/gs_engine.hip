@@ -1641,11 +1641,20 @@ int end_timing(gs_engine* e) {
     return 0;
 }
 
+// Whether a chunk's launches read its strings and uniforms from the pinned mirrors and write its results there: a plan that
+// is one run of small steps reads each once, at its start, and writes each once, at its end, so copies before and behind
+// it (3.4 us each, and a gap) would only add to it.  Amplitudes are copied from the arenas.
+bool reads_host(const gs_engine* e, bool amp) {
+    const size_t ns = size_t(ns_of(e));
+    return e->own_buffers && !amp && ns >= 2 && e->small_at[0] >= 0 && e->small_at[ns - 1] == e->small_at[0] && e->hrun.empty();
+}
+
 // Results of strings 0 .. cnt-1 of the chunk (their scalars and bits; conditionals and amplitudes where asked for) to
 // the host, once the work is done: one copy behind the kernels and one wait for both.
-int finish_chunk(gs_engine* e, int cnt, bool bits, bool cond, bool amp) {
+int finish_chunk(gs_engine* e, int cnt, bool bits, bool cond, bool amp, bool direct) {
     const size_t n = size_t(cnt), ns = size_t(ns_of(e));
-    if (e->own_buffers) {
+    if (direct) {                                         // there already
+    } else if (e->own_buffers) {
         unsigned char* const from = reinterpret_cast<unsigned char*>(e->d_out);
         const unsigned char* end = cond ? reinterpret_cast<unsigned char*>(e->d_cond + n * ns)
                                  : bits ? reinterpret_cast<unsigned char*>(e->d_bits + n * ns) : e->d_amp + 16 * n;
@@ -1694,6 +1703,7 @@ int enqueue_amp(gs_engine* e, int slot) {
 // decide which sweeps a step needs.
 int enqueue_strings(gs_engine* e, int mode, int cnt, bool forced, bool amp) {
     const int ns = ns_of(e);
+    const bool direct = reads_host(e, amp);
     const int most = ensure_slots(e, cnt);
     auto alike = [&](int a, int b) {
         for (int k = 0; k < ns; k++)
@@ -1706,8 +1716,10 @@ int enqueue_strings(gs_engine* e, int mode, int cnt, bool forced, bool amp) {
         while (e->strings < most && i + e->strings < cnt && (mode != kRun || alike(i, i + e->strings))) e->strings++;
         if ((rc = start_chain(e))) break;
         const size_t at = size_t(i) * ns;
-        if ((rc = enqueue_run(e, mode, 0, ns, forced ? e->h_forced + at : nullptr, forced ? e->d_forced + at : nullptr,
-                              e->d_U + at, e->d_bits + at, e->d_cond + at, e->d_out + size_t(i) * 4)))
+        if ((rc = enqueue_run(e, mode, 0, ns, forced ? e->h_forced + at : nullptr,
+                              forced ? (direct ? e->h_forced : e->d_forced) + at : nullptr, (direct ? e->h_U : e->d_U) + at,
+                              (direct ? e->h_bits : e->d_bits) + at, (direct ? e->h_cond : e->d_cond) + at,
+                              (direct ? e->h_out : e->d_out) + size_t(i) * 4)))
             break;
         if (amp) rc = enqueue_amp(e, i);
     }
@@ -1731,11 +1743,12 @@ int run_forced(gs_engine* e, int mode, const int8_t* bits, int64_t nstr, double*
     for (int64_t s0 = 0; s0 < nstr; s0 += gs_engine::kChunk) {
         const int cnt = int(std::min<int64_t>(gs_engine::kChunk, nstr - s0));
         memcpy(e->h_forced, bits + s0 * ns, size_t(cnt) * ns);
-        HIP_TRY(hipMemcpyAsync(e->d_forced, e->h_forced, size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
+        if (!reads_host(e, amp != nullptr))
+            HIP_TRY(hipMemcpyAsync(e->d_forced, e->h_forced, size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
         if (int rc = begin_timing(e)) return rc;
         if (int rc = enqueue_strings(e, mode, cnt, true, amp != nullptr)) return rc;
         if (int rc = end_timing(e)) return rc;
-        if (int rc = finish_chunk(e, cnt, false, cond != nullptr, amp != nullptr)) return rc;
+        if (int rc = finish_chunk(e, cnt, false, cond != nullptr, amp != nullptr, reads_host(e, amp != nullptr))) return rc;
         for (int i = 0; i < cnt; i++) {
             log2p[s0 + i] = e->h_out[i * 4];
             if (cond) memcpy(cond + (s0 + i) * ns, e->h_cond + size_t(i) * ns, size_t(ns) * sizeof(double));
@@ -1901,11 +1914,12 @@ int gs_sample(gs_engine* eng, uint64_t seed, int64_t first, int64_t count, int s
             std::uniform_real_distribution<double> U(0, 1);
             for (int k = 0; k < ns; k++) e->h_U[size_t(i) * ns + k] = U(rng);
         }
-        HIP_TRY(hipMemcpyAsync(e->d_U, e->h_U, sizeof(double) * size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
+        if (!reads_host(e, false))
+            HIP_TRY(hipMemcpyAsync(e->d_U, e->h_U, sizeof(double) * size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
         if (int rc = begin_timing(e)) return rc;
         if (int rc = enqueue_strings(e, kChain, cnt, false, false)) return rc;
         if (int rc = end_timing(e)) return rc;
-        if (int rc = finish_chunk(e, cnt, true, false, false)) return rc;
+        if (int rc = finish_chunk(e, cnt, true, false, false, reads_host(e, false))) return rc;
         memcpy(bits + s0 * ns, e->h_bits, size_t(cnt) * ns);
         for (int i = 0; i < cnt; i++) log2p[s0 + i] = e->h_out[i * 4];
     }
@@ -1930,12 +1944,14 @@ int gs_hybrid(gs_engine* eng, const int8_t* bits, int64_t nstr, uint64_t seed, i
             for (int k = 0; k < ns; k++)
                 if (e->h_forced[size_t(i) * ns + k] < 0) e->h_U[size_t(i) * ns + q++] = U(rng);
         }
-        HIP_TRY(hipMemcpyAsync(e->d_forced, e->h_forced, size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
-        HIP_TRY(hipMemcpyAsync(e->d_U, e->h_U, sizeof(double) * size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
+        if (!reads_host(e, false)) {
+            HIP_TRY(hipMemcpyAsync(e->d_forced, e->h_forced, size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
+            HIP_TRY(hipMemcpyAsync(e->d_U, e->h_U, sizeof(double) * size_t(cnt) * ns, hipMemcpyHostToDevice, e->stream));
+        }
         if (int rc = begin_timing(e)) return rc;
         if (int rc = enqueue_strings(e, kRun, cnt, true, false)) return rc;
         if (int rc = end_timing(e)) return rc;
-        if (int rc = finish_chunk(e, cnt, true, true, false)) return rc;
+        if (int rc = finish_chunk(e, cnt, true, true, false, reads_host(e, false))) return rc;
         memcpy(out_bits + s0 * ns, e->h_bits, size_t(cnt) * ns);
         memcpy(cond + s0 * ns, e->h_cond, size_t(cnt) * ns * sizeof(double));
         for (int i = 0; i < cnt; i++) log2p[s0 + i] = e->h_out[i * 4];
@@ -1967,7 +1983,7 @@ int gs_prefix(gs_engine* eng, const int8_t* bits, int K, double* table_reim, int
     if (int rc = start_chain(e)) return rc;
     if (int rc = enqueue_run(e, kRun, 0, K, e->h_forced, e->d_forced, e->d_U, e->d_bits, e->d_cond, e->d_out)) return rc;
     if (int rc = end_timing(e)) return rc;
-    if (int rc = finish_chunk(e, 1, false, false, false)) return rc;
+    if (int rc = finish_chunk(e, 1, false, false, false, false)) return rc;
     void* doffs = nullptr;
     void* dtab = nullptr;
     HIP_TRY(hipMalloc(&doffs, sizeof(uint64_t) * offs.size()));
@@ -2094,7 +2110,7 @@ int gs_resume(gs_engine* eng, const int8_t* bits, int K, int nslices, const doub
         if ((rc = begin_timing(e))) break;
         if ((rc = enqueue_run(e, kRun, K, ns, e->h_forced, e->d_forced, e->d_U, e->d_bits, e->d_cond, e->d_out))) break;
         if ((rc = end_timing(e))) break;
-        if ((rc = finish_chunk(e, 1, true, true, false))) break;
+        if ((rc = finish_chunk(e, 1, true, true, false, false))) break;
         for (int k = 0; k < ns; k++) out_bits[k] = k < K ? bits[k] : e->h_bits[k];
         for (int k = K; k < ns; k++) cond[k] = e->h_cond[k];
         *log2p_prefix = lp_prefix;
