@@ -90,7 +90,8 @@ struct KStep {
 
 // Runs of small steps (gs_small.hip): one block of kSmallThreads per string, the slots a run touches in LDS.
 constexpr int kSmallThreads = 512;
-constexpr int kSmallMaxNk = 12;     // cosets of a step, log2
+constexpr int kSmallMaxNk = 13;     // cosets of a step, log2
+constexpr size_t kLdsBytes = size_t(160) << 10;
 constexpr int kSmallSteps = 64;     // steps of a run
 struct SStep {
     uint32_t cols[kSmallMaxNk];     // LDS index of each coset coordinate's column (0 beyond nk), as the plain descriptor's

@@ -348,7 +348,8 @@ struct gs_engine {
     int grid_cap1 = kDefaultGridLog2One;  // ... a plain sweep of a one-slot step
     int grid_cap1_big = kDefaultGridLog2OneBig;  // ... of a one-slot step with at least 2^kBigStepLog2 cosets
     // runs of small steps (gs_small.hip): descriptors, the run each step belongs to (-1: none), log2 slots of each run
-    int small_nk = 10;              // steps with at most 2^small_nk cosets (-1: no runs)
+    int small_nk = 10;              // steps with at most 2^small_nk cosets (-1: no runs) ...
+    bool small_whole = true;        // ... and a plan whose steps all fit one run, as long as nobody sets small_nk
     std::vector<SStep> hsmall;
     std::vector<int> small_at, small_dim;
     SStep* dsmall = nullptr;
@@ -1302,8 +1303,17 @@ void build_small(gs_engine* e) {
     e->hsmall.assign(size_t(std::max(P.ns, 1)), SStep{});
     e->small_at.assign(size_t(std::max(P.ns, 1)), -1);
     e->small_dim.clear();
-    const size_t room = size_t(64) << 10;                 // bytes of table
-    const int lim = std::min(e->small_nk, kSmallMaxNk);
+    size_t room = size_t(64) << 10;                       // bytes of table
+    int lim = std::min(e->small_nk, kSmallMaxNk);
+    // A plan that fits a run as a whole is one launch a call, without copies: 64 samples of 2^12 / 2^13 / 2^14 complex64
+    // slots take 250 / 369 / 431 us with runs of up to 2^10 cosets and 186 / 222 / 326 in one, one sample 169 / 263 / 307
+    // and 122 / 158 / 260, one string in chain mode, which has the fewest launches to save, 126 / 175 / 186 and 106 / 131 /
+    // 194.  A table of 2^14 slots is also the largest that fits.
+    if (e->small_whole && small_run_lds(e->esz << P.R) <= kLdsBytes && P.ns <= kSmallSteps &&
+        std::all_of(P.steps.begin(), P.steps.end(), [](const StepInfo& s) { return s.nk <= kSmallMaxNk; })) {
+        lim = kSmallMaxNk;
+        room = std::max(room, e->esz << P.R);
+    }
     auto slots_of = [](const KStep& s) {
         std::vector<uint64_t> v(s.cols, s.cols + s.nk);
         v.insert(v.end(), s.off, s.off + s.ntq);
@@ -2279,6 +2289,7 @@ int gs_set_small_steps(gs_engine* eng, int nk) {
     HIP_TRY(hipSetDevice(eng->device));
     HIP_TRY(hipStreamSynchronize(eng->stream));
     eng->small_nk = nk;
+    eng->small_whole = false;
     build_small(eng);
     build_units(eng);
     return upload_descriptors(eng);

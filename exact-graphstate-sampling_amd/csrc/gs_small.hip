@@ -21,6 +21,7 @@ namespace gs {
 namespace {
 
 constexpr int kWavesS = kSmallThreads / 64;
+static_assert(kSmallMaxNk < 15, "narrow_steps keeps an index and a sign in 16 bits");
 
 // A step of at most 64 cosets, as the first wave reads it: offsets two to a word, g, and kind | m << 5 | par << 8 |
 // growth << 12 | next step's growth << 13 | nk << 16.
@@ -32,7 +33,7 @@ struct Shared {                       // after the table in LDS
     SStep s[kSmallSteps];
     NStep n[kSmallSteps];
     double coef[kSmallSteps][2][4];   // per branch |m0|^2, |m1|^2, Re and Im of m0 conj(m1)
-    uint32_t word[kSmallSteps][64];   // per lane: index of its coset's base, its sign in bit 31
+    uint16_t word[kSmallSteps][64];   // per lane: index of its coset's base, its sign in bit 15
     double U[kSmallSteps];
     double pfac[kSmallSteps], plog[kSmallSteps];      // factors of Pr, and their log2 at the end of the run
     double sfac[kSmallSteps], slog[kSmallSteps];      // table norms of the rescalings (kRun), and their log2
@@ -284,7 +285,7 @@ __device__ __forceinline__ int narrow_steps(Shared& sh, S* tab, bool forced, Sta
     uint32_t word = sh.word[k - k0][t];
     while (k < to) {
         const uint32_t o01 = uni(nx.o01), o23 = uni(nx.o23), g = uni(nx.g), bits = uni(nx.bits);
-        const uint32_t a = word & 0xffffu, pc = word >> 31;
+        const uint32_t a = word & 0x7fffu, pc = word >> 15;
         const uint32_t off[4] = {o01 & 0xffffu, o01 >> 16, o23 & 0xffffu, o23 >> 16};
         const int i = k - k0, m = int(bits >> 5) & 3;
         const bool on = uint32_t(t) < (1u << (bits >> 16));
@@ -467,7 +468,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_run_kernel(const SStep* _
         uint32_t a = 0;
 #pragma unroll
         for (int j = 0; j < 6; j++) a ^= ((lane >> j) & 1) ? s.cols[j] : 0;
-        sh.word[i][lane] = a | (uint32_t(__popc(uint32_t(lane) & s.rho)) << 31);
+        sh.word[i][lane] = uint16_t(a | (uint32_t(__popc(uint32_t(lane) & s.rho)) & 1) << 15);
         if (lane < 2) {
             const double2 m0 = make_double2(s.mre[lane][0], s.mim[lane][0]), m1 = make_double2(s.mre[lane][1], s.mim[lane][1]);
             sh.coef[i][lane][0] = norm2(m0);
