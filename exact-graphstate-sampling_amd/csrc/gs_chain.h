@@ -124,8 +124,9 @@ __device__ __forceinline__ void block_tree_sum(double (&sh)[NT / 64][NQ], const 
     __syncthreads();
 }
 
-// Chain logic after a sweep, from its reduced sums (one thread).
-template <int NQ>
+// Chain logic after a sweep, from its reduced sums (one thread).  MULTI: the sweep may be one of several steps (the others
+// are spared the code, which costs them registers and scratch: 6 hybrid strings of 60 steps, 712 us with it, 650 without).
+template <int NQ, bool MULTI = false>
 __device__ void chain_step(const double (&red)[NQ], Ctl* ctl, const Epi& e, int sweep) {
     Ctl& c = *ctl;
     if constexpr (NQ == 1) {            // one sum: the product pass of a run (role kRoleStored), the stored norm
@@ -137,8 +138,10 @@ __device__ void chain_step(const double (&red)[NQ], Ctl* ctl, const Epi& e, int 
         return;
     } else if (e.role == kRoleNorm) {
         decide(c, e, e.k, sweep, red);
-    } else if (NQ <= 4 && e.role == kRolePair) {
-        for (int i = 0; i < NQ && !c.dead; i++) {
+    } else if (MULTI && NQ <= 4 && e.role == kRolePair) {
+#pragma unroll
+        for (int i = 0; i < NQ; i++) {
+            if (c.dead) break;
             if (i) decide(c, e, e.k + i, -1, nullptr);
             finish_write(c, e, e.k + i, red[i], red[i]);
         }
@@ -146,11 +149,13 @@ __device__ void chain_step(const double (&red)[NQ], Ctl* ctl, const Epi& e, int 
             if (e.k + NQ == e.k1) publish(c, e);
             else if (e.next == kNextDecide) decide(c, e, e.k + NQ, -1, nullptr);
         }
-    } else if ((NQ == 4 || NQ == 6) && e.role == kRolePeek) {
+    } else if (MULTI && (NQ == 4 || NQ == 6) && e.role == kRolePeek) {
         double w[4];
+#pragma unroll
         for (int q = 0; q < 4; q++) w[q] = c.w[q];
         finish_write(c, e, e.k, red[0], red[1]);
         if (!c.dead) decide(c, e, e.k + 1, NQ == 6 ? kGram : kDirect, red + 2);
+#pragma unroll
         for (int q = 0; q < 4; q++) {
             c.w2[q] = c.w[q];
             c.w[q] = w[q];
@@ -186,7 +191,7 @@ __device__ __forceinline__ void reduce_partials(double (&sh)[kThreads / 64][NQ],
 // the kernel: the last block of a string to arrive (agent-scope counter) reduces and runs the chain; a string's only
 // block does so at once.  Larger launches end here and sweep_reduce_kernel follows on the stream: an agent-scope
 // release per block writes back the XCD's L2 each time (tens of ns per block), which a launch boundary does once.
-template <int NQ>
+template <int NQ, bool MULTI = false>
 __device__ void sweep_epilogue(double (&acc)[NQ], double* part, Ctl* ctl, const Epi& e, int sweep) {
     // block sum (wave butterfly, then the 4 waves in order)
 #pragma unroll
@@ -212,7 +217,7 @@ __device__ void sweep_epilogue(double (&acc)[NQ], double* part, Ctl* ctl, const 
             red[q] = v;
         }
         if (nblk == 1) {
-            chain_step<NQ>(red, ctl, slot_epi(e), sweep);
+            chain_step<NQ, MULTI>(red, ctl, slot_epi(e), sweep);
         } else {
 #pragma unroll
             for (int q = 0; q < NQ; q++) {
@@ -235,7 +240,7 @@ __device__ void sweep_epilogue(double (&acc)[NQ], double* part, Ctl* ctl, const 
     double red[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; q++) red[q] = sh[0][q];
-    chain_step<NQ>(red, ctl, slot_epi(e), sweep);
+    chain_step<NQ, MULTI>(red, ctl, slot_epi(e), sweep);
     __hip_atomic_store(e.counter + blockIdx.y, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

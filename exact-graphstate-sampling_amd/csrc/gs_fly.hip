@@ -200,7 +200,7 @@ __global__ __launch_bounds__(kThreads) void fly_kernel(const FlyDesc* __restrict
     }
     if constexpr (NORM == kNormGram)
         if (route[NS] != kRouteSplit) acc[3] = acc[2];
-    sweep_epilogue<NA>(acc, part, ctl, epi, NORM == kNormGram ? kWriteGram : NORM == kNormDirect ? kWriteDirect : kWrite);
+    sweep_epilogue<NA, true>(acc, part, ctl, epi, NORM == kNormGram ? kWriteGram : NORM == kNormDirect ? kWriteDirect : kWrite);
 }
 
 namespace {

@@ -22,7 +22,7 @@ __global__ __launch_bounds__(kThreads) void sweep_reduce_kernel(const double* __
     double red[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; q++) red[q] = sh[0][q];
-    chain_step<NQ>(red, ctl, slot_epi(e), sweep);
+    chain_step<NQ, true>(red, ctl, slot_epi(e), sweep);
 }
 
 // The same for many blocks, in the same order: thread t of the one-block kernel sums partials t, t + 256, ...; here a
@@ -70,7 +70,7 @@ __global__ __launch_bounds__(64) void wide_reduce_kernel(double* __restrict__ pa
         for (int j = 1; j < NW; j++) red[k] += __shfl(v, j * NQ + k, 64);
     }
     if (lane != 0) return;
-    chain_step<NQ>(red, ctl, slot_epi(e), sweep);
+    chain_step<NQ, true>(red, ctl, slot_epi(e), sweep);
     __hip_atomic_store(e.counter + blockIdx.y, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

@@ -107,7 +107,7 @@ __global__ __launch_bounds__(kThreads) void pair_sweep_kernel(const PStep* __res
                 Run<S, VR>::store(mem, at & ~uint64_t(VR - 1), f[c][t]);
             }
     }
-    sweep_epilogue<2>(acc, part, ctl, epi, kWrite);
+    sweep_epilogue<2, true>(acc, part, ctl, epi, kWrite);
 }
 
 namespace {
