@@ -24,8 +24,8 @@ constexpr int kDefaultGridLog2One = 12; // plain sweeps of one-slot steps: one l
                                         // (width 34, 1-slot norm passes: 691 -> 343 ms per sample at 2^12 blocks)
 constexpr int kBigStepLog2 = 30;        // one-slot steps of at least 2^30 cosets take more blocks still:
 constexpr int kDefaultGridLog2OneBig = 14;  // width 34: 1.231 -> 1.196 s per sample; width 30 prefers 2^12
-// The write that folds in the next step's norms holds 4-8 outputs per thread and wants fewer blocks: width 26 5.65 ms per
-// sample at 2^11 blocks, 5.72 / 5.78 / 7.30 at 2^10 / 2^12 / 2^14; width 29 18.1 ms at 2^10 - 2^12, 18.3 at 2^14.
+// The write that folds in the next step's norms holds 4-8 outputs per thread; its grid hardly matters (complex128 width 26
+// 9.47 / 9.45 / 9.53 ms per sample at 2^10 / 2^11 / 2^12 blocks, width 20 706 / 711 / 709 us).
 constexpr int kDefaultTTFoldGridLog2 = 11;
 constexpr int kDefaultTTGridLog2 = 14;  // gather sweeps of the two-table engine (latency-bound gathers: the
                                          // width-31 IBM sample 0.276 s at 2^9 blocks, 0.121 s at 2^14)
