@@ -1291,6 +1291,16 @@ struct gs_plan {
     gs::Plan p;
 };
 
+// A launch of the batch: steps k .. k + n - 1 of the instances of its work items.
+struct Sweep {
+    int k, n;
+    const PairDesc* pair;                 // n == 2: the kind of pair
+    int nq;                               // most slots per coset among the instances at step k (kernel variant)
+    bool exact;                           // ... every one has nq
+    BItem* items;
+    int nitems;
+};
+
 struct gs_batch {
     int device = 0;
     int storage = GS_C64;
@@ -1303,20 +1313,17 @@ struct gs_batch {
     BInst* dinst = nullptr;
     std::vector<void*> allocs;
     int maxns = 0;
-    // per step: work items (device) and their count; tuning: log2 cosets per item per step
-    std::vector<BItem*> ditems;           // in item_mem
-    void* item_mem = nullptr;
-    std::vector<int> nitems;
-    std::vector<std::vector<int>> lg;     // [inst][step]
+    void* item_mem = nullptr;             // the launches' work items (device)
+    std::vector<std::vector<int>> lg;     // [inst][step]: log2 cosets per item
     int lg_default = 8;                   // smallest tile (sizes the partial buffers); steps start at 2^9
-    std::vector<int> nq;                  // per step: most slots per coset among the instances (kernel variant)
-    std::vector<int> nq_exact;            // per step: 1 if every instance at the step has nq slots per coset
     std::vector<std::vector<PairDesc>> hpairs;   // [inst][step]: steps k and k+1 as one sweep (ni 0: not possible)
     std::vector<std::vector<FlyDesc>> hflys;     // [inst][step][kMaxUnit - 2]: 3 steps and more (d 0: not possible)
     // scoring with whole strings in LDS (score_lds_kernel): bytes of its table and of all its LDS (0: not all plans fit)
     int lds_table = 0, lds_bytes = 0, lds_blocks = 0, lds_threads = 512;
     int *dorder = nullptr, *dblk0 = nullptr;
     std::vector<char> unit;               // per step: steps of the sweep that starts there (0: inside another's)
+    std::vector<Sweep> common;            // the launches of these sweeps, every instance in each (gradients)
+    std::vector<Sweep> sweeps;            // scoring: the launches, by first step; instances may take sweeps of their own
     bool pairs_on = true;
     int lu = 2;                           // log2 cosets a lane gathers at once
     bool items_dirty = false;             // tiles changed since the work lists were built
@@ -1356,14 +1363,23 @@ T* dalloc(gs_batch* b, size_t n) {
     return static_cast<T*>(p);
 }
 
-// Which sweeps the step sequence takes: single steps, or several at once where every instance that is still running has
-// the same kind of pair, or a run of butterfly steps.  A sweep of n steps saves n - 1 writes and reads of the table (and
-// launches); the sweeps are the disjoint ones that save the most.
-void choose_units(gs_batch* bt) {
-    const int ns = bt->maxns;
-    bt->unit.assign(size_t(ns), 1);
-    if (!bt->pairs_on) return;
-    constexpr double kLaunch = 40e6;                      // bytes moved in the time a launch and its reduction take
+constexpr double kLaunch = 40e6;                          // bytes moved in the time a launch and its reduction take
+
+// Bytes that one sweep of instance i over the n steps from k saves against a sweep more of the table.
+double unit_bytes(const gs_batch* bt, size_t i, int k, int n) {
+    return 2.0 * double(bt->B[i]) * double(bt->esz) *
+           double(uint64_t(n > 2 ? 2 : bt->hpairs[i][size_t(k)].mo) << bt->plans[i].steps[size_t(k)].nk);
+}
+
+// Which sweeps the members' step sequence takes (per step: the steps of the sweep that starts there): single steps, or
+// several at once where every member that is still running has the same kind of pair, or a run of butterfly steps.  A
+// sweep of n steps saves n - 1 writes and reads of the table (and launches); the sweeps are the disjoint ones that save
+// the most.
+std::vector<char> choose_units(const gs_batch* bt, const std::vector<size_t>& members) {
+    int ns = 0;
+    for (size_t i : members) ns = std::max(ns, bt->plans[i].ns);
+    std::vector<char> unit(size_t(bt->maxns), 1);
+    if (!bt->pairs_on) return unit;
     std::vector<double> best(size_t(ns + kMaxUnit), 0.0);
     std::vector<char> take(size_t(ns), 1);
     for (int k = ns - 1; k >= 0; k--) {
@@ -1373,7 +1389,7 @@ void choose_units(gs_batch* bt) {
             const PairDesc* first = nullptr;
             int ntq = 0;
             bool ok = true;
-            for (size_t i = 0; i < bt->plans.size() && ok; i++) {
+            for (size_t i : members) {
                 const gs::Plan& P = bt->plans[i];
                 if (k >= P.ns) continue;
                 const PairDesc& p = bt->hpairs[i][size_t(k)];
@@ -1388,8 +1404,8 @@ void choose_units(gs_batch* bt) {
                 } else {
                     ok = p.ni == first->ni && p.mo == first->mo && p.deg == first->deg && P.steps[size_t(k)].ntq == ntq;
                 }
-                g += 2.0 * double(bt->B[i]) * double(bt->esz) *
-                     double(uint64_t(n > 2 ? 2 : p.mo) << P.steps[size_t(k)].nk);
+                if (!ok) break;
+                g += unit_bytes(bt, i, k, n);
             }
             g *= n - 1;
             if (ok && g + best[size_t(k + n)] > best[size_t(k)]) {
@@ -1399,16 +1415,89 @@ void choose_units(gs_batch* bt) {
         }
     }
     for (int k = 0; k < ns; k += take[size_t(k)]) {
-        bt->unit[size_t(k)] = take[size_t(k)];
-        for (int j = 1; j < take[size_t(k)]; j++) bt->unit[size_t(k + j)] = 0;
+        unit[size_t(k)] = take[size_t(k)];
+        for (int j = 1; j < take[size_t(k)]; j++) unit[size_t(k + j)] = 0;
     }
+    return unit;
 }
 
-// Cosets (or super-cosets of several steps) of instance i's sweep at step k, log2, and log2 of the step-k cosets in each.
-void sweep_size(const gs_batch* bt, size_t i, int k, int& nk, int& inner) {
+// The instances whose sweeps at step k can share a launch, as groups (first member first).
+std::vector<std::vector<size_t>> sweep_groups(const gs_batch* bt, const std::vector<const std::vector<char>*>& unit, int k) {
+    std::vector<std::vector<size_t>> groups;
+    for (size_t i = 0; i < bt->plans.size(); i++) {
+        if (k >= bt->plans[i].ns || !(*unit[i])[size_t(k)]) continue;
+        const int n = (*unit[i])[size_t(k)];
+        bool found = false;
+        for (auto& g : groups) {
+            const size_t f = g[0];
+            if ((*unit[f])[size_t(k)] != n) continue;
+            if (n == 2) {
+                const PairDesc &a = bt->hpairs[i][size_t(k)], &b = bt->hpairs[f][size_t(k)];
+                if (a.ni != b.ni || a.mo != b.mo || a.deg != b.deg ||
+                    bt->plans[i].steps[size_t(k)].ntq != bt->plans[f].steps[size_t(k)].ntq)
+                    continue;
+            }
+            g.push_back(i);
+            found = true;
+            break;
+        }
+        if (!found) groups.push_back({i});
+    }
+    return groups;
+}
+
+// What a choice of sweeps costs, in bytes, up to a constant: its launches, less the bytes its sweeps save.
+double units_cost(const gs_batch* bt, const std::vector<const std::vector<char>*>& unit) {
+    double c = 0;
+    for (int k = 0; k < bt->maxns; k++)
+        for (const auto& g : sweep_groups(bt, unit, k)) {
+            c += kLaunch;
+            for (size_t i : g) {
+                const int n = (*unit[i])[size_t(k)];
+                if (n > 1) c -= (n - 1) * unit_bytes(bt, i, k, n);
+            }
+        }
+    return c;
+}
+
+// Scoring: instances do not wait for each other, so an instance may take the sweeps that suit its own plan, in launches
+// of its own where no other takes the same kind at that step.  The widest instances leave the common sequence first,
+// while what the sweeps save is more than the launches cost.  64 lanes each of four plans of bands 19 to 21: 4.00 -> 2.83
+// ms complex64, 6.77 -> 3.84 complex128; 96 plans of widths 13 to 24: 11,800 strings/s one batch each, 13,200 in two.
+std::vector<std::vector<char>> score_units(const gs_batch* bt) {
+    const size_t ni = bt->plans.size();
+    std::vector<size_t> order(ni);
+    for (size_t i = 0; i < ni; i++) order[i] = i;
+    auto bytes = [&](size_t i) {
+        int nk = 0;
+        for (const gs::StepInfo& st : bt->plans[i].steps) nk = std::max(nk, st.nk);
+        return double(bt->B[i]) * double(uint64_t(1) << nk);
+    };
+    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return bytes(a) > bytes(b); });
+    std::vector<std::vector<char>> best(ni, bt->unit), own(ni);
+    if (ni == 1 || !bt->pairs_on || bt->lds_bytes) return best;
+    for (size_t i = 0; i < ni; i++) own[i] = choose_units(bt, {i});
+    auto view = [&](const std::vector<char>& common, size_t leave) {
+        std::vector<const std::vector<char>*> v(ni, &common);
+        for (size_t j = 0; j < leave; j++) v[order[j]] = &own[order[j]];
+        return v;
+    };
+    double cost = units_cost(bt, view(bt->unit, 0));
+    for (size_t leave = 1; leave <= ni; leave++) {
+        const std::vector<char> common = choose_units(bt, std::vector<size_t>(order.begin() + ptrdiff_t(leave), order.end()));
+        const auto v = view(common, leave);
+        const double c = units_cost(bt, v);
+        if (c >= cost) continue;
+        cost = c;
+        for (size_t i = 0; i < ni; i++) best[i] = *v[i];
+    }
+    return best;
+}
+
+// Cosets (or super-cosets of several steps) of instance i's sweep of the n steps from k, log2, and log2 of the step-k cosets in each.
+void sweep_size(const gs_batch* bt, size_t i, int k, int n, int& nk, int& inner) {
     nk = bt->plans[i].steps[size_t(k)].nk;
     inner = 0;
-    const int n = bt->unit[size_t(k)];
     if (n < 2) return;
     if (n > 2) {
         inner = n - 1;
@@ -1426,94 +1515,110 @@ void sweep_size(const gs_batch* bt, size_t i, int k, int& nk, int& inner) {
 // 128 lanes: 40 blocks of 2^8 cosets took 30 us a step).  The backward sums of several steps take more room per item, so their
 // tiles start coarser.
 constexpr int kFinestTile = 4;
-int item_lg(const gs_batch* bt, size_t i, int k, int shrink, bool& finer) {
+int item_lg(const gs_batch* bt, size_t i, int k, int n, int shrink, bool& finer) {
     int nk, inner;
-    sweep_size(bt, i, k, nk, inner);
+    sweep_size(bt, i, k, n, nk, inner);
     const int floor = std::min(nk, std::max(0, kFinestTile - inner));
     int lg = bt->lg[i][size_t(k)];
-    const int n = bt->unit[size_t(k)];
     if (n > 1) lg = std::max(lg, bt->lg_default + (n > 2 ? 2 : 1));
     lg = std::min(nk, std::max(lg - inner - shrink, floor));
     finer = finer || lg > floor;
     return lg;
 }
 
+// The work items of one launch: the n steps from k of the instances in `group`.
+std::vector<BItem> sweep_items(const gs_batch* bt, const std::vector<size_t>& group, int k, int n) {
+    int shrink = 0;
+    for (;; shrink++) {
+        int64_t tot = 0;
+        bool finer = false;
+        for (size_t i : group) {
+            int nk, inner;
+            sweep_size(bt, i, k, n, nk, inner);
+            tot += int64_t(bt->B[i] / kLanes) << (nk - item_lg(bt, i, k, n, shrink, finer));
+        }
+        if (tot >= kMinItems || !finer) break;
+    }
+    std::vector<BItem> items;
+    for (size_t i : group) {
+        int nk, inner;
+        bool finer = false;
+        sweep_size(bt, i, k, n, nk, inner);
+        const int lg = item_lg(bt, i, k, n, shrink, finer);
+        const int count = 1 << (nk - lg);
+        const int ng = bt->B[i] / kLanes;
+        for (int o = 0; o < ng * count; o++) {
+            // group-major (every coset range of lane group 0, then group 1, ...) or, with xcd_items == 2,
+            // coset-major (all lane groups of a coset range next to each other: whole slot rows)
+            const int g = bt->xcd_items == 2 ? o % ng : o / count;
+            const int q = bt->xcd_items == 2 ? o / ng : o % count;
+            BItem it{};
+            it.c0 = uint64_t(q) << lg;
+            it.inst = int(i);
+            it.group = g;
+            it.lg = lg;
+            it.index = q;
+            it.count = count;
+            items.push_back(it);
+        }
+    }
+    if (bt->xcd_items && items.size() >= 8 && items.size() % 8 == 0) {
+        // blocks are dealt round-robin to the 8 XCDs (block i on XCD i mod 8): list position b = (j mod n/8) * 8
+        // + j / (n/8) gives XCD x the consecutive items x n/8 .. (x+1) n/8 - 1 (adjacent coset ranges)
+        const size_t m = items.size(), chunk = m / 8;
+        std::vector<BItem> order(m);
+        for (size_t j = 0; j < m; j++) order[(j % chunk) * 8 + j / chunk] = items[j];
+        items.swap(order);
+    }
+    return items;
+}
+
 int build_items(gs_batch* bt) {
     (void)hipFree(bt->item_mem);
     bt->item_mem = nullptr;
-    std::vector<BItem> all;                               // the lists of every step, in one allocation
-    std::vector<size_t> at(size_t(bt->maxns), 0);
+    std::vector<BItem> all;                               // the lists of every launch, in one allocation
+    std::vector<size_t> at;                               // ... where each begins
     const size_t ni = bt->plans.size();
-    bt->ditems.assign(size_t(bt->maxns), nullptr);
-    bt->nitems.assign(size_t(bt->maxns), 0);
-    bt->nq.assign(size_t(bt->maxns), 1);
-    bt->nq_exact.assign(size_t(bt->maxns), 0);
-    choose_units(bt);
-    for (int k = 0; k < bt->maxns; k++) {
-        if (!bt->unit[size_t(k)]) continue;
-        int shrink = 0;
-        for (;; shrink++) {
-            int64_t tot = 0;
-            bool finer = false;
-            for (size_t i = 0; i < ni; i++) {
-                if (k >= bt->plans[i].ns) continue;
-                int nk, inner;
-                sweep_size(bt, i, k, nk, inner);
-                tot += int64_t(bt->B[i] / kLanes) << (nk - item_lg(bt, i, k, shrink, finer));
-            }
-            if (tot >= kMinItems || !finer) break;
-        }
-        std::vector<BItem> items;
-        for (size_t i = 0; i < ni; i++) {
-            if (k >= bt->plans[i].ns) continue;
-            int nk, inner;
-            bool finer = false;
-            sweep_size(bt, i, k, nk, inner);
-            const int lg = item_lg(bt, i, k, shrink, finer);
-            const int count = 1 << (nk - lg);
-            const int ng = bt->B[i] / kLanes;
-            for (int o = 0; o < ng * count; o++) {
-                // group-major (every coset range of lane group 0, then group 1, ...) or, with xcd_items == 2,
-                // coset-major (all lane groups of a coset range next to each other: whole slot rows)
-                const int g = bt->xcd_items == 2 ? o % ng : o / count;
-                const int q = bt->xcd_items == 2 ? o / ng : o % count;
-                BItem it{};
-                it.c0 = uint64_t(q) << lg;
-                it.inst = int(i);
-                it.group = g;
-                it.lg = lg;
-                it.index = q;
-                it.count = count;
-                items.push_back(it);
-            }
-        }
-        if (bt->xcd_items && items.size() >= 8 && items.size() % 8 == 0) {
-            // blocks are dealt round-robin to the 8 XCDs (block i on XCD i mod 8): list position b = (j mod n/8) * 8
-            // + j / (n/8) gives XCD x the consecutive items x n/8 .. (x+1) n/8 - 1 (adjacent coset ranges)
-            const size_t n = items.size(), chunk = n / 8;
-            std::vector<BItem> order(n);
-            for (size_t j = 0; j < n; j++) order[(j % chunk) * 8 + j / chunk] = items[j];
-            items.swap(order);
-        }
-        int nqk = 1;
-        for (size_t i = 0; i < bt->plans.size(); i++)
-            if (k < bt->plans[i].ns) nqk = std::max(nqk, bt->plans[i].steps[size_t(k)].ntq);
-        bt->nq[size_t(k)] = nqk;
-        int exact = 1;
-        for (size_t i = 0; i < bt->plans.size(); i++)
-            if (k < bt->plans[i].ns && bt->plans[i].steps[size_t(k)].ntq != nqk) exact = 0;
-        bt->nq_exact[size_t(k)] = exact;
-        bt->nitems[size_t(k)] = int(items.size());
-        at[size_t(k)] = all.size();
+    std::vector<size_t> everyone(ni);
+    for (size_t i = 0; i < ni; i++) everyone[i] = i;
+    bt->unit = choose_units(bt, everyone);
+    auto add = [&](std::vector<Sweep>& to, const std::vector<size_t>& group, int k, int n) {
+        Sweep w{k, n, n == 2 ? &bt->hpairs[group[0]][size_t(k)] : nullptr, 1, true, nullptr, 0};
+        for (size_t i : group) w.nq = std::max(w.nq, bt->plans[i].steps[size_t(k)].ntq);
+        for (size_t i : group) w.exact = w.exact && bt->plans[i].steps[size_t(k)].ntq == w.nq;
+        const std::vector<BItem> items = sweep_items(bt, group, k, n);
+        w.nitems = int(items.size());
+        at.push_back(all.size());
         all.insert(all.end(), items.begin(), items.end());
+        to.push_back(w);
+    };
+    bt->common.clear();
+    bt->sweeps.clear();
+    for (int k = 0; k < bt->maxns; k++) {
+        std::vector<size_t> group;
+        for (size_t i = 0; i < ni; i++)
+            if (k < bt->plans[i].ns) group.push_back(i);
+        if (bt->unit[size_t(k)]) add(bt->common, group, k, bt->unit[size_t(k)]);
     }
+    const std::vector<std::vector<char>> own = score_units(bt);
+    std::vector<const std::vector<char>*> view(ni);
+    bool same = true;
+    for (size_t i = 0; i < ni; i++) {
+        view[i] = &own[i];
+        same = same && own[i] == bt->unit;
+    }
+    for (int k = 0; k < bt->maxns && !same; k++)
+        for (const auto& g : sweep_groups(bt, view, k)) add(bt->sweeps, g, k, own[g[0]][size_t(k)]);
     if (hipMalloc(&bt->item_mem, std::max<size_t>(all.size() * sizeof(BItem), 16)) != hipSuccess) {
         bt->item_mem = nullptr;
         return bfail(11, "work-item allocation failed");
     }
     if (hipMemcpy(bt->item_mem, all.data(), all.size() * sizeof(BItem), hipMemcpyHostToDevice) != hipSuccess)
         return bfail(17, "work-item upload failed");
-    for (int k = 0; k < bt->maxns; k++) bt->ditems[size_t(k)] = static_cast<BItem*>(bt->item_mem) + at[size_t(k)];
+    size_t a = 0;
+    for (Sweep& w : bt->common) w.items = static_cast<BItem*>(bt->item_mem) + at[a++];
+    for (Sweep& w : bt->sweeps) w.items = static_cast<BItem*>(bt->item_mem) + at[a++];
+    if (same) bt->sweeps = bt->common;
     return 0;
 }
 
@@ -1574,34 +1679,28 @@ const void* fly_variant(BKernel kind, int n) {
 }
 
 template <class S>
-int launch_batch(gs_batch* bt, BKernel kind, int k, BLaunch L) {
-    const int n = bt->nitems[size_t(k)];
-    if (n == 0) return 0;
-    const int nq = bt->nq[size_t(k)], lu = bt->lu;
-    const bool ex = bt->nq_exact[size_t(k)] != 0;
-    const PairDesc* pair = nullptr;
-    if (bt->unit[size_t(k)] == 2)
-        for (size_t i = 0; i < bt->plans.size() && !pair; i++)
-            if (k < bt->plans[i].ns) pair = &bt->hpairs[i][size_t(k)];
-    const int n_steps = bt->unit[size_t(k)];
-    const void* fn = n_steps > 2 ? fly_variant<S>(kind, n_steps)
-                   : pair ? (kind == kBStep ? GS_PAIR_VARIANT(pair_step_kernel, S, nq, *pair)
-                             : kind == kBRestore ? GS_PAIR_VARIANT(pair_restore_kernel, S, nq, *pair)
-                                                 : GS_PAIR_VARIANT(pair_back_kernel, S, nq, *pair))
+int launch_batch(gs_batch* bt, BKernel kind, const Sweep& w, BLaunch L) {
+    if (w.nitems == 0) return 0;
+    const int nq = w.nq, lu = bt->lu;
+    const bool ex = w.exact;
+    const void* fn = w.n > 2 ? fly_variant<S>(kind, w.n)
+                   : w.pair ? (kind == kBStep ? GS_PAIR_VARIANT(pair_step_kernel, S, nq, *w.pair)
+                               : kind == kBRestore ? GS_PAIR_VARIANT(pair_restore_kernel, S, nq, *w.pair)
+                                                   : GS_PAIR_VARIANT(pair_back_kernel, S, nq, *w.pair))
                    : kind == kBStep ? GS_BATCH_VARIANT(batch_step_kernel, S, nq, lu, ex)
                    : kind == kBRestore ? GS_BATCH_VARIANT(batch_restore_kernel, S, nq, lu, ex)
                                        : GS_BATCH_VARIANT(batch_back_kernel, S, nq, lu, ex);
     if (!fn) return bfail(16, "no kernel variant");
     const BInst* insts = bt->dinst;
-    const BItem* items = bt->ditems[size_t(k)];
+    const BItem* items = w.items;
     void* args[] = {&insts, &items, &L};
-    return hipLaunchKernel(fn, dim3(n), dim3(kBThreads), args, 0, bt->stream) == hipSuccess ? 0
-                                                                                      : bfail(17, "step launch failed");
+    return hipLaunchKernel(fn, dim3(w.nitems), dim3(kBThreads), args, 0, bt->stream) == hipSuccess
+               ? 0 : bfail(17, "step launch failed");
 }
 
 template <class S>
-int launch_step(gs_batch* bt, int k, int bookkeeping, void* const* copy) {
-    return launch_batch<S>(bt, kBStep, k, BLaunch{k, bookkeeping, copy, bt->dclock});
+int launch_step(gs_batch* bt, const Sweep& w, int bookkeeping, void* const* copy) {
+    return launch_batch<S>(bt, kBStep, w, BLaunch{w.k, bookkeeping, copy, bt->dclock});
 }
 
 template <class S>
@@ -1616,10 +1715,8 @@ int enqueue_t(gs_batch* bt) {
                            bt->lds_table, bt->dclock);
         return hipGetLastError() == hipSuccess ? 0 : bfail(17, "batch launch failed");
     }
-    for (int k = 0; k < bt->maxns; k++) {
-        if (!bt->unit[size_t(k)]) continue;               // inside another step's sweep
-        if (int rc = launch_step<S>(bt, k, 1, nullptr)) return rc;
-    }
+    for (const Sweep& w : bt->sweeps)
+        if (int rc = launch_step<S>(bt, w, 1, nullptr)) return rc;
     hipLaunchKernelGGL(batch_finish_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
     if (hipGetLastError() != hipSuccess) return bfail(17, "batch launch failed");
     return 0;
@@ -1811,24 +1908,25 @@ int grad_t(gs_batch* bt) {
     if (hipEventCreate(&em) != hipSuccess) return bfail(17, "event creation failed");
     (void)hipEventRecord(e0, bt->stream);
     hipLaunchKernelGGL(batch_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst, bt->dclock, ns);
-    for (int k = 0; k < ns; k++)
-        if (bt->unit[size_t(k)])
-            if (int rc = launch_step<S>(bt, k, 1, fwd_ptr(k))) return rc;
+    for (const Sweep& w : bt->common)
+        if (int rc = launch_step<S>(bt, w, 1, fwd_ptr(w.k))) return rc;
     hipLaunchKernelGGL(batch_finish_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
     (void)hipEventRecord(em, bt->stream);
     hipLaunchKernelGGL(batch_lambda_init_kernel<S>, dim3(ninst), dim3(256), 0, bt->stream, bt->dinst, ninst);
     for (int s = last; s >= 0; s--) {
         const int k0 = s * seg, k1 = std::min(ns, k0 + seg);
-        const int kf = seg_first(bt, seg, s);
-        if (s != last && kf < k1) {                         // recompute the segment from its checkpoint
-            if (int rc = launch_batch<S>(bt, kBRestore, kf, BLaunch{kf, 0, ck_ptr(s), nullptr})) return rc;
-            for (int k = kf; k < k1; k++)
-                if (bt->unit[size_t(k)])
-                    if (int rc = launch_step<S>(bt, k, 0, rec_ptr(k - k0))) return rc;
+        size_t a = 0, b = 0;                                // the segment's sweeps: a .. b - 1
+        while (a < bt->common.size() && bt->common[a].k < k0) a++;
+        for (b = a; b < bt->common.size() && bt->common[b].k < k1;) b++;
+        if (s != last && a < b) {                           // recompute the segment from its checkpoint
+            const Sweep& f = bt->common[a];
+            if (int rc = launch_batch<S>(bt, kBRestore, f, BLaunch{f.k, 0, ck_ptr(s), nullptr})) return rc;
+            for (size_t j = a; j < b; j++)
+                if (int rc = launch_step<S>(bt, bt->common[j], 0, rec_ptr(bt->common[j].k - k0))) return rc;
         }
-        for (int k = k1 - 1; k >= kf; k--) {
-            if (!bt->unit[size_t(k)]) continue;
-            if (int rc = launch_batch<S>(bt, kBBack, k, BLaunch{k, 0, rec_ptr(k - k0), nullptr})) return rc;
+        for (size_t j = b; j-- > a;) {
+            const Sweep& w = bt->common[j];
+            if (int rc = launch_batch<S>(bt, kBBack, w, BLaunch{w.k, 0, rec_ptr(w.k - k0), nullptr})) return rc;
         }
     }
     (void)hipEventRecord(e1, bt->stream);
@@ -2150,12 +2248,15 @@ int gs_batch_score(gs_batch* bt, const int8_t* const* bits, double* const* log2p
     (void)hipEventElapsedTime(&ms, bt->ev0, bt->ev1);
     bt->last_ms = ms;
     bt->step_ms.assign(size_t(bt->maxns), -1.0);
-    if (!bt->use_graph)
+    if (!bt->use_graph) {
+        const bool lds = bt->lds_bytes && bt->pairs_on;
+        size_t a = 0;
         for (int k = 0, u = 0; k < bt->maxns; k++) {      // the steps of one sweep end together
-            if (bt->unit[size_t(k)] || (bt->lds_bytes && bt->pairs_on)) u = k;
-            if (bt->nitems[size_t(u)])
-                bt->step_ms[size_t(k)] = double(bt->hclock[size_t(1 + u)] - bt->hclock[0]) / bt->clock_khz;
+            while (a < bt->sweeps.size() && bt->sweeps[a].k <= k) u = bt->sweeps[a++].k;
+            if (lds) u = k;
+            bt->step_ms[size_t(k)] = double(bt->hclock[size_t(1 + u)] - bt->hclock[0]) / bt->clock_khz;
         }
+    }
     for (size_t i = 0; i < bt->plans.size(); i++) {
         const size_t B = size_t(bt->B[i]), ns = size_t(bt->plans[i].ns);
         memcpy(log2p[i], bt->hout + bt->at_logp[i], sizeof(double) * B);
