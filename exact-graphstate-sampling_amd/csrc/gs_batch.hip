@@ -1462,10 +1462,13 @@ double units_cost(const gs_batch* bt, const std::vector<const std::vector<char>*
 
 // Scoring: instances do not wait for each other, so an instance may take the sweeps that suit its own plan, in launches
 // of its own where no other takes the same kind at that step.  The widest instances leave the common sequence first,
-// while what the sweeps save is more than the launches cost.  64 lanes each of four plans of bands 19 to 21: 4.00 -> 2.83
-// ms complex64, 6.77 -> 3.84 complex128; 96 plans of widths 13 to 24: 11,800 strings/s one batch each, 13,200 in two.
+// while what the sweeps save is more than the launches cost; at most kLeave of them, so that the choice takes a time
+// proportional to the number of plans (400 plans: the batch is made in 50 ms instead of 60, its scores take 7.2 ms either
+// way).  64 lanes each of four plans of bands 19 to 21: 4.00 -> 2.83 ms complex64, 6.77 -> 3.84 complex128; 96 plans of
+// widths 13 to 24: 11,800 strings/s one batch each, 13,200 in two.
+constexpr size_t kLeave = 64;
 std::vector<std::vector<char>> score_units(const gs_batch* bt) {
-    const size_t ni = bt->plans.size();
+    const size_t ni = bt->plans.size(), most = std::min(ni, kLeave);
     std::vector<size_t> order(ni);
     for (size_t i = 0; i < ni; i++) order[i] = i;
     auto bytes = [&](size_t i) {
@@ -1476,14 +1479,14 @@ std::vector<std::vector<char>> score_units(const gs_batch* bt) {
     std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return bytes(a) > bytes(b); });
     std::vector<std::vector<char>> best(ni, bt->unit), own(ni);
     if (ni == 1 || !bt->pairs_on || bt->lds_bytes) return best;
-    for (size_t i = 0; i < ni; i++) own[i] = choose_units(bt, {i});
+    for (size_t j = 0; j < most; j++) own[order[j]] = choose_units(bt, {order[j]});
     auto view = [&](const std::vector<char>& common, size_t leave) {
         std::vector<const std::vector<char>*> v(ni, &common);
         for (size_t j = 0; j < leave; j++) v[order[j]] = &own[order[j]];
         return v;
     };
     double cost = units_cost(bt, view(bt->unit, 0));
-    for (size_t leave = 1; leave <= ni; leave++) {
+    for (size_t leave = 1; leave <= most; leave++) {
         const std::vector<char> common = choose_units(bt, std::vector<size_t>(order.begin() + ptrdiff_t(leave), order.end()));
         const auto v = view(common, leave);
         const double c = units_cost(bt, v);
