@@ -1994,6 +1994,12 @@ int gs_prefix(gs_engine* eng, const int8_t* bits, int K, double* table_reim, int
     if (int rc = enqueue_run(e, kRun, 0, K, e->h_forced, e->d_forced, e->d_U, e->d_bits, e->d_cond, e->d_out)) return rc;
     if (int rc = end_timing(e)) return rc;
     if (int rc = finish_chunk(e, 1, false, false, false, false)) return rc;
+    if (logscale) *logscale = e->h_out[1];
+    if (log2p_prefix) *log2p_prefix = e->h_out[0];
+    if (e->h_out[3] != 0) {            // probability 0: the chain stopped there, and the arena holds what it held before
+        std::fill_n(table_reim, 2 * n, 0.0);
+        return 0;
+    }
     void* doffs = nullptr;
     void* dtab = nullptr;
     HIP_TRY(hipMalloc(&doffs, sizeof(uint64_t) * offs.size()));
@@ -2017,8 +2023,6 @@ int gs_prefix(gs_engine* eng, const int8_t* bits, int K, double* table_reim, int
     HIP_TRY(hipStreamSynchronize(e->stream));
     (void)hipFree(doffs);
     (void)hipFree(dtab);
-    if (logscale) *logscale = e->h_out[1];
-    if (log2p_prefix) *log2p_prefix = e->h_out[0];
     return 0;
 }
 

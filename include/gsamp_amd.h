@@ -69,7 +69,8 @@ int gs_hybrid(gs_engine* eng, const int8_t* bits, int64_t nstr, uint64_t seed, i
  * return the live table of step K in logical order (c-major, sorted coset offsets of step K; {0} past the end)
  * as complex doubles table_reim [2 * 2^nk * ntq] (capacity table_cap complex entries; the reference's dump
  * stores the arena's type, the caller narrows), plus nk, ntq, logscale (true = stored * 2^logscale) and
- * log2 Pr(prefix).  Pass table_reim = NULL to query nk and ntq only (no steps are run). */
+ * log2 Pr(prefix).  A prefix of probability 0 has a table of zeros, the logscale of the steps before the impossible
+ * one and log2 Pr = -inf.  Pass table_reim = NULL to query nk and ntq only (no steps are run). */
 int gs_prefix(gs_engine* eng, const int8_t* bits, int K, double* table_reim, int64_t table_cap, int* nk, int* ntq,
               double* logscale, double* log2p_prefix);
 
