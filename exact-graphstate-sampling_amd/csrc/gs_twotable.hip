@@ -701,6 +701,12 @@ int gs_tt_prefix(gs_tt_engine* e, const int8_t* bits, int K, double* table_reim,
     TT_TRY(hipMemcpyAsync(raw.data(), e->tab[e->cur], raw.size(), hipMemcpyDeviceToHost, e->stream));
     TT_TRY(hipMemcpyAsync(e->h_out, e->d_out, 4 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
     TT_TRY(hipStreamSynchronize(e->stream));
+    *log2p_prefix = e->h_out[0];
+    *logscale = e->h_out[1];
+    if (e->h_out[3] != 0) {            // probability 0: the chain stopped there, and the tables hold what they held before
+        std::fill_n(table_reim, 2 * n, 0.0);
+        return 0;
+    }
     for (int64_t i = 0; i < n; i++) {
         if (e->storage == GS_C64) {
             float v[2];
@@ -711,8 +717,6 @@ int gs_tt_prefix(gs_tt_engine* e, const int8_t* bits, int K, double* table_reim,
             memcpy(table_reim + 2 * i, raw.data() + size_t(i) * 16, 16);
         }
     }
-    *log2p_prefix = e->h_out[0];
-    *logscale = e->h_out[1];
     return 0;
 }
 
