@@ -325,8 +325,8 @@ int run_forced(gs_tt_engine* e, int mode, const int8_t* bits, int64_t nstr, doub
         for (int i = 0; i < cnt; i++) {
             log2p[s0 + i] = e->h_out[i * 4];
             if (cond) memcpy(cond + (s0 + i) * ns, e->h_cond + size_t(i) * ns, size_t(ns) * sizeof(double));
-            if (amp) {
-                const std::complex<double> z = read_amp(e, i);
+            if (amp) {                  // a string of probability 0 stopped early: its amplitude is 0
+                const std::complex<double> z = e->h_out[i * 4 + 3] != 0 ? std::complex<double>() : read_amp(e, i);
                 amp[2 * (s0 + i)] = z.real();
                 amp[2 * (s0 + i) + 1] = z.imag();
             }

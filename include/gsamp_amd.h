@@ -131,8 +131,9 @@ int gs_tt_plan_info(const gs_tt_plan* plan, int* n, int* ns, int* maxr);
 void gs_tt_plan_destroy(gs_tt_plan* plan);
 int gs_tt_engine_create(const gs_tt_plan* plan, int storage, int device, gs_tt_engine** out);
 void gs_tt_engine_destroy(gs_tt_engine* eng);
-/* prob (gsamp.cpp:39-55 forced, both branch norms per step), chain (chain1, gsamp.cpp:59-70; amp_reim may be NULL),
- * sample (mt19937_64(seed + first + i), gsamp.cpp:111-117), hybrid ('?' = -1 sampled, gsamp.cpp:118-123). */
+/* prob (gsamp.cpp:39-55 forced, both branch norms per step), chain (chain1, gsamp.cpp:59-70; amp_reim may be NULL,
+ * and is 0 for a string that meets a zero-probability branch), sample (mt19937_64(seed + first + i),
+ * gsamp.cpp:111-117), hybrid ('?' = -1 sampled, gsamp.cpp:118-123). */
 int gs_tt_prob(gs_tt_engine* eng, const int8_t* bits, int64_t nstr, double* log2p);
 int gs_tt_chain(gs_tt_engine* eng, const int8_t* bits, int64_t nstr, double* log2p, double* cond, double* amp_reim);
 int gs_tt_sample(gs_tt_engine* eng, uint64_t seed, int64_t first, int64_t count, int8_t* bits, double* log2p);

@@ -1,5 +1,5 @@
-"""Two-table engine, strings that meet a branch of probability zero: the table of such a prefix is zero,
-whatever the two tables held before (the steps behind the branch do not run)."""
+"""Two-table engine, strings that meet a branch of probability zero: the table of such a prefix is zero and so is the
+amplitude, whatever the two tables held before (the steps behind the branch do not run)."""
 import numpy as np
 import pytest
 
@@ -33,3 +33,17 @@ def test_dead_prefix_is_a_zero_table(shape, step, storage, tmp_path):
             assert np.any(e.prefix(other, K)[0])
             tab, _, ls, lp = e.prefix(bits, K)
             assert not np.any(tab) and lp == -np.inf and np.isfinite(ls)
+
+
+@pytest.mark.parametrize("storage", [gs.C64, gs.C128])
+@pytest.mark.parametrize("shape", PLANS)
+@pytest.mark.parametrize("step", STEPS)
+def test_dead_string_has_no_amplitude(shape, step, storage, tmp_path):
+    inst, d, _, dead = zeroed(shape, tmp_path, two_table=True, step=step)
+    bits, other = strings(inst, d)
+    print(shape, step, storage, flush=True)
+    with gs.TwoTableEngine(dead, storage=storage) as e:
+        lp, cond, amp = e.chain(np.array([other, bits, other]))
+    assert np.isfinite(lp[0]) and lp[1] == -np.inf and lp[2] == lp[0]
+    assert np.all(cond[1, d:] == 0)
+    assert amp[1] == 0 and amp[0] != 0 and amp[0] == amp[2]
