@@ -90,7 +90,8 @@ struct KStep {
 
 // Runs of small steps (gs_small.hip): one block of kSmallThreads per string, the slots a run touches in LDS.
 constexpr int kSmallThreads = 512;
-constexpr int kSmallMaxNk = 13;     // cosets of a step, log2
+constexpr int kSmallMaxNk = 13;     // cosets of a step, log2: the most a run can take ...
+constexpr int kSmallDefaultNk = 10; // ... and does take unless the plan fits a run as a whole (gs_set_small_steps)
 constexpr size_t kLdsBytes = size_t(160) << 10;
 constexpr int kSmallSteps = 64;     // steps of a run
 struct SStep {

@@ -348,8 +348,8 @@ struct gs_engine {
     int grid_cap1 = kDefaultGridLog2One;  // ... a plain sweep of a one-slot step
     int grid_cap1_big = kDefaultGridLog2OneBig;  // ... of a one-slot step with at least 2^kBigStepLog2 cosets
     // runs of small steps (gs_small.hip): descriptors, the run each step belongs to (-1: none), log2 slots of each run
-    int small_nk = 10;              // steps with at most 2^small_nk cosets (-1: no runs) ...
-    bool small_whole = true;        // ... and a plan whose steps all fit one run, as long as nobody sets small_nk
+    int small_nk = kSmallDefaultNk; // steps with at most 2^small_nk cosets (-1: no runs) ...
+    bool small_whole = true;        // ... and, with the default, a plan whose steps all fit one run
     std::vector<SStep> hsmall;
     std::vector<int> small_at, small_dim;
     SStep* dsmall = nullptr;
@@ -2285,15 +2285,16 @@ int gs_set_walk(gs_engine* eng, int mode) {
     return upload_descriptors(eng);
 }
 
-// Steps with at most 2^nk cosets run, in runs of two or more, in one single-block launch (nk -1: never; default 10; runs
-// are cut where their slots would not fit the LDS, and steps beyond 2^12 cosets always take sweeps).
+// Steps with at most 2^nk cosets run, in runs of two or more, in one single-block launch (nk -1: never).  Runs are cut
+// where their slots would not fit 64 KB of the LDS or after kSmallSteps steps, and steps beyond 2^kSmallMaxNk cosets always
+// take sweeps.  With the default, kSmallDefaultNk, a plan that fits a run as a whole (build_small) is one run.
 int gs_set_small_steps(gs_engine* eng, int nk) {
     if (!eng) return fail(16, "null engine");
     if (nk < -1 || nk > 20) return fail(16, "small-step limit must be -1..20");
     HIP_TRY(hipSetDevice(eng->device));
     HIP_TRY(hipStreamSynchronize(eng->stream));
     eng->small_nk = nk;
-    eng->small_whole = false;
+    eng->small_whole = nk == kSmallDefaultNk;
     build_small(eng);
     build_units(eng);
     return upload_descriptors(eng);

@@ -408,7 +408,8 @@ class Engine:
         _check(library().gs_set_xcd_blocks(self._h, 1 if on else 0))
 
     def set_small_steps(self, nk):
-        """Run consecutive steps of at most 2^nk cosets in one single-block launch (-1: never)."""
+        """Run consecutive steps of at most 2^nk cosets in one single-block launch (-1: never; 10, the default: also a whole
+        plan whose steps fit one)."""
         _check(library().gs_set_small_steps(self._h, int(nk)))
 
     def set_grid_log2_one_slot(self, lg):

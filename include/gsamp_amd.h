@@ -217,7 +217,9 @@ int gs_step_run(const gs_engine* eng, int k, int* out);
    then needs no separate reduction launch (on = 1; on >= 2: only when the next sweep's step has at most 2^on live
    slots), or by a one-block kernel between the two (0, default); the results are bitwise the same. */
 int gs_set_fold_reduce(gs_engine* eng, int on);
-/* Runs of two or more steps with at most 2^nk cosets go to one single-block launch (nk -1: never; default 10). */
+/* Runs of two or more steps with at most 2^nk cosets go to one single-block launch (nk -1: never; at most 20, though steps
+   beyond 2^13 cosets never do).  The default, 10, also makes one run of a plan of at most 64 steps whose steps have up
+   to 2^13 cosets and whose arena fits the LDS (2^14 complex64 or 2^13 complex128 entries); other limits hold as given. */
 int gs_set_small_steps(gs_engine* eng, int nk);
 /* Device race check of step k (debug mode; overwrites the arena, used as an owner map of the slots): layout 0 the
    plain sweeps' coset coordinates, 1 the fused sweep's, 2 the plan's own, 3 the run of diagonal steps starting at k.
