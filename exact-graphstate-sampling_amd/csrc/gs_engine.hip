@@ -404,9 +404,10 @@ uint32_t slot_part_doubles(const gs_engine* e) {
     return uint32_t(kPartStride) << std::min(kMaxGridLog2, std::max(0, e->plan.R - 8));
 }
 
-// Make room for up to `want` strings per launch; returns how many the engine can run at once (1: one by one, also when
-// the memory is not there).  Runs of diagonal steps keep pattern sums for one string only, so plans with such runs
-// (2^20 cosets and more) run one string at a time, as do engines whose sweeps are timed one by one.
+// Make room for up to `want` strings per launch; returns how many the engine can run at once (1: one by one).  Where the
+// memory is not there the engine keeps what it has, or takes as many as fit.  Runs of diagonal steps keep pattern sums for
+// one string only, so plans with such runs (2^20 cosets and more) run one string at a time, as do engines whose sweeps are
+// timed one by one.
 int ensure_slots(gs_engine* e, int64_t want) {
     if (want < 2 || !e->own_buffers || e->profile || !e->hrun.empty()) return 1;
     const size_t arena = slot_entries(e) * e->esz;
@@ -416,21 +417,23 @@ int ensure_slots(gs_engine* e, int64_t want) {
     if (most < kMinSlots) return 1;
     int n = 2;
     while (n < want && n < most) n = std::min(2 * n, most);
+    if (size_t fr = 0, tot = 0; n > e->nslots && hipMemGetInfo(&fr, &tot) == hipSuccess)
+        while (n > e->nslots && each * size_t(n) > fr + each * size_t(e->nslots)) n = std::max(n / 2, e->nslots);
     if (n > e->nslots) {
         if (hipStreamSynchronize(e->stream) != hipSuccess) return 1;
         (void)hipFree(e->slots);
         e->slots = nullptr;
         e->nslots = 0;
-        if (hipMalloc(&e->slots, each * size_t(n)) != hipSuccess) {
+        for (; n > 1 && hipMalloc(&e->slots, each * size_t(n)) != hipSuccess; n /= 2) {
             (void)hipGetLastError();
             e->slots = nullptr;
-            return 1;
         }
+        if (n < 2) return 1;
         e->nslots = n;
         e->slot_part[0] = reinterpret_cast<double*>(static_cast<unsigned char*>(e->slots) + arena * size_t(n));
         e->slot_part[1] = e->slot_part[0] + size_t(slot_part_doubles(e)) * size_t(n);
     }
-    return int(std::min<int64_t>(n, want));
+    return int(std::max<int64_t>(1, std::min<int64_t>(n, want)));
 }
 
 // Reduce the partials the last sweep left (one-block kernel) before a launch that does not reduce them itself.
