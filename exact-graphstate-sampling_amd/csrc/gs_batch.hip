@@ -1316,6 +1316,7 @@ struct gs_batch {
     void* item_mem = nullptr;             // the launches' work items (device)
     std::vector<std::vector<int>> lg;     // [inst][step]: log2 cosets per item
     int lg_default = 8;                   // smallest tile (sizes the partial buffers); steps start at 2^9
+    // sweeps of several steps (build_several; empty until a batch that scores in LDS takes a gradient)
     std::vector<std::vector<PairDesc>> hpairs;   // [inst][step]: steps k and k+1 as one sweep (ni 0: not possible)
     std::vector<std::vector<FlyDesc>> hflys;     // [inst][step][kMaxUnit - 2]: 3 steps and more (d 0: not possible)
     // scoring with whole strings in LDS (score_lds_kernel): bytes of its table and of all its LDS (0: not all plans fit)
@@ -1363,6 +1364,58 @@ T* dalloc(gs_batch* b, size_t n) {
     return static_cast<T*>(p);
 }
 
+// Descriptors of every instance's sweeps of several steps, host and device, and the instances' device table with their
+// addresses.  Batches whose strings are scored in LDS have that table without them, until a gradient first asks: five plans
+// of width 11 are made in 1.6 ms with them, 1.2 without.
+int build_several(gs_batch* bt) {
+    const size_t ni = bt->plans.size();
+    std::vector<std::vector<PairDesc>> pairs(ni);
+    std::vector<std::vector<FlyDesc>> flys(ni);
+    size_t np = 0, nf = 0;
+    for (size_t i = 0; i < ni; i++) {
+        const gs::Plan& P = bt->plans[i];
+        std::vector<PairDesc>& hp = pairs[i];
+        hp.resize(size_t(P.ns));
+        for (int k = 0; k < P.ns; k++)
+            if (k + 1 >= P.ns || !make_pair(P.steps[size_t(k)], P.steps[size_t(k) + 1], false, hp[size_t(k)])) hp[size_t(k)].ni = 0;
+        std::vector<FlyDesc>& hf = flys[i];
+        hf.resize(size_t(P.ns) * (kMaxUnit - 2));
+        for (int k = 0; k < P.ns; k++)
+            for (int n = 3; n <= kMaxUnit; n++) {
+                const gs::StepInfo* st[kMaxUnit] = {};
+                for (int j = 0; j < n && k + j < P.ns; j++) st[j] = &P.steps[size_t(k + j)];
+                FlyDesc& f = hf[size_t(k) * (kMaxUnit - 2) + size_t(n - 3)];
+                if (!st[n - 1] || !make_fly(st, n, 0, 0, f)) f.d = 0;
+            }
+        np += hp.size();
+        nf += hf.size();
+    }
+    auto up256 = [](size_t n) { return (n + 255) & ~size_t(255); };
+    const size_t table = ni * sizeof(BInst), at_pair = bt->dinst ? 0 : up256(table),
+                 at_fly = at_pair + up256(np * sizeof(PairDesc));
+    std::vector<char> up(at_fly + nf * sizeof(FlyDesc));
+    char* mem = dalloc<char>(bt, up.size());
+    if (!mem) return bfail(11, "allocation of the sweep descriptors failed");
+    size_t p = at_pair, f = at_fly;
+    for (size_t i = 0; i < ni; i++) {
+        if (!pairs[i].empty()) memcpy(up.data() + p, pairs[i].data(), pairs[i].size() * sizeof(PairDesc));
+        if (!flys[i].empty()) memcpy(up.data() + f, flys[i].data(), flys[i].size() * sizeof(FlyDesc));
+        bt->hinst[i].pairs = reinterpret_cast<PairDesc*>(mem + p);
+        bt->hinst[i].flys = reinterpret_cast<FlyDesc*>(mem + f);
+        p += pairs[i].size() * sizeof(PairDesc);
+        f += flys[i].size() * sizeof(FlyDesc);
+    }
+    if (at_pair) memcpy(up.data(), bt->hinst.data(), table);
+    if (!up.empty() && hipMemcpy(mem, up.data(), up.size(), hipMemcpyHostToDevice) != hipSuccess)
+        return bfail(17, "plan upload failed");
+    if (at_pair) bt->dinst = reinterpret_cast<BInst*>(mem);
+    else if (hipMemcpy(bt->dinst, bt->hinst.data(), table, hipMemcpyHostToDevice) != hipSuccess)
+        return bfail(17, "instance upload failed");
+    bt->hpairs = std::move(pairs);
+    bt->hflys = std::move(flys);
+    return 0;
+}
+
 constexpr double kLaunch = 40e6;                          // bytes moved in the time a launch and its reduction take
 
 // Bytes that one sweep of instance i over the n steps from k saves against a sweep more of the table.
@@ -1379,7 +1432,7 @@ std::vector<char> choose_units(const gs_batch* bt, const std::vector<size_t>& me
     int ns = 0;
     for (size_t i : members) ns = std::max(ns, bt->plans[i].ns);
     std::vector<char> unit(size_t(bt->maxns), 1);
-    if (!bt->pairs_on) return unit;
+    if (!bt->pairs_on || bt->hpairs.empty()) return unit;
     std::vector<double> best(size_t(ns + kMaxUnit), 0.0);
     std::vector<char> take(size_t(ns), 1);
     for (int k = ns - 1; k >= 0; k--) {
@@ -2054,17 +2107,6 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
             s.ntq = si.ntq;
             s.m = si.m;
         }
-        std::vector<PairDesc> hp(size_t(P.ns));
-        for (int k = 0; k < P.ns; k++)
-            if (k + 1 >= P.ns || !make_pair(P.steps[size_t(k)], P.steps[size_t(k) + 1], false, hp[size_t(k)])) hp[size_t(k)].ni = 0;
-        std::vector<FlyDesc> hf(size_t(P.ns) * (kMaxUnit - 2));
-        for (int k = 0; k < P.ns; k++)
-            for (int n = 3; n <= kMaxUnit; n++) {
-                const gs::StepInfo* st[kMaxUnit] = {};
-                for (int j = 0; j < n && k + j < P.ns; j++) st[j] = &P.steps[size_t(k + j)];
-                FlyDesc& f = hf[size_t(k) * (kMaxUnit - 2) + size_t(n - 3)];
-                if (!st[n - 1] || !make_fly(st, n, 0, 0, f)) f.d = 0;
-            }
         std::vector<LStep> hl;
         if (lds_fits)
             for (const gs::StepInfo& si : P.steps) hl.push_back(make_lstep(si, P.R, bt->esz));
@@ -2077,8 +2119,7 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
         };
         I.narrived = int(part_items(bt, size_t(i)) / kItemGroup);
         const size_t n_arrived = size_t(B / kLanes) * size_t(1 + I.narrived);
-        const size_t o_steps = take(hs.size() * sizeof(BStep)), o_pairs = take(hp.size() * sizeof(PairDesc)),
-                     o_flys = take(hf.size() * sizeof(FlyDesc)), o_lsteps = take(hl.size() * sizeof(LStep)),
+        const size_t o_steps = take(hs.size() * sizeof(BStep)), o_lsteps = take(hl.size() * sizeof(LStep)),
                      o_arrived = take(sizeof(unsigned) * n_arrived), head = used;   // counters start at 0
         const size_t o_prev = take(sizeof(double) * B), o_dead = take(sizeof(int) * B),
                      o_part = take(sizeof(double) * size_t(B / kLanes) * part_doubles(bt, size_t(i)));
@@ -2086,17 +2127,11 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
         if (!mem) return bail(bfail(11, "batch buffer allocation failed"));
         std::vector<char> up(head);
         if (!hs.empty()) memcpy(up.data() + o_steps, hs.data(), hs.size() * sizeof(BStep));
-        if (!hp.empty()) memcpy(up.data() + o_pairs, hp.data(), hp.size() * sizeof(PairDesc));
-        if (!hf.empty()) memcpy(up.data() + o_flys, hf.data(), hf.size() * sizeof(FlyDesc));
         if (!hl.empty()) memcpy(up.data() + o_lsteps, hl.data(), hl.size() * sizeof(LStep));
         if (head && hipMemcpy(mem, up.data(), head, hipMemcpyHostToDevice) != hipSuccess)
             return bail(bfail(17, "plan upload failed"));
         bt->hsteps.push_back(std::move(hs));
-        bt->hpairs.push_back(std::move(hp));
-        bt->hflys.push_back(std::move(hf));
         I.steps = reinterpret_cast<BStep*>(mem + o_steps);
-        I.pairs = reinterpret_cast<PairDesc*>(mem + o_pairs);
-        I.flys = reinterpret_cast<FlyDesc*>(mem + o_flys);
         I.lsteps = reinterpret_cast<LStep*>(mem + o_lsteps);
         I.bitsT = bt->dbits + bt->at_bits[size_t(i)];
         I.prev = reinterpret_cast<double*>(mem + o_prev);
@@ -2108,10 +2143,12 @@ int gs_batch_create(const gs_plan* const* plans, const int* lanes, int nplans, i
         I.part = reinterpret_cast<double*>(mem + o_part);
         bt->hinst.push_back(I);
     }
-    bt->dinst = dalloc<BInst>(bt, bt->hinst.size());
-    if (!bt->dinst || hipMemcpy(bt->dinst, bt->hinst.data(), bt->hinst.size() * sizeof(BInst), hipMemcpyHostToDevice) != hipSuccess)
-        return bail(bfail(17, "instance upload failed"));
-    if (bt->lds_bytes) {                                  // the largest plans' strings first
+    if (!bt->lds_bytes) {
+        if (int rc = build_several(bt)) return bail(rc);
+    } else {                                              // the largest plans' strings first
+        bt->dinst = dalloc<BInst>(bt, bt->hinst.size());
+        if (!bt->dinst || hipMemcpy(bt->dinst, bt->hinst.data(), bt->hinst.size() * sizeof(BInst), hipMemcpyHostToDevice) != hipSuccess)
+            return bail(bfail(17, "instance upload failed"));
         std::vector<int> list(size_t(2 * nplans + 1), 0);
         for (int i = 0; i < nplans; i++) list[size_t(i)] = i;
         std::stable_sort(list.begin(), list.begin() + nplans,
@@ -2276,6 +2313,10 @@ int gs_batch_grad(gs_batch* bt, const int8_t* const* bits, double* const* log2p,
                   int seg, double mem_budget, int* seg_used) {
     if (!bt || !bits || !log2p || !G) return bfail(16, "bad argument");
     if (hipSetDevice(bt->device) != hipSuccess) return bfail(17, "hipSetDevice failed");
+    if (bt->pairs_on && bt->hpairs.empty()) {
+        if (int rc = build_several(bt)) return rc;
+        bt->items_dirty = true;
+    }
     if (bt->items_dirty) {
         if (int rc = build_items(bt)) return rc;
         bt->items_dirty = false;
