@@ -3,8 +3,8 @@
 Tiles.  ``gs_batch`` launches one kernel per step index covering every instance; a work item is (instance, lane group
 of 64 strings, a Gray-ordered range of 2^lg cosets) and one block takes one item.  Small lg gives many items (the
 chip fills even for one lane group) and more partial sums; large lg gives few, long items.  ``tune_tiles`` times the
-whole step sequence once per candidate lg (per-step device times from the events the engine records after every
-step), keeps for every step index the fastest candidate, applies the choice with ``set_tile`` and stores it in a JSON
+whole step sequence once per candidate lg (per-step times from the device clock, which the engine reads at the end of
+every sweep), keeps for every step index the fastest candidate (steps inside a sweep of several: that sweep's), applies the choice with ``set_tile`` and stores it in a JSON
 cache keyed by the plans' content digests, the lane counts and the storage, so a later process with the same batch
 skips the measurement.  The final choice is made on graph replays of the whole batch: the per-step choice against
 every uniform tile, each at every unroll depth.
@@ -47,7 +47,8 @@ def _store(path, table):
 
 
 def step_times(bt, bits):
-    """Device ms of every step index of one scoring run (kernel-by-kernel launches, events after each step)."""
+    """Device ms of every step index of one scoring run (kernel-by-kernel launches).  The steps of one sweep end together:
+    the first has the sweep's time, the others 0."""
     bt.use_graph(False)
     bt.score(bits, want_cond=False, want_amp=False)
     _, ends = bt.last_ms()
@@ -78,9 +79,14 @@ def tune_tiles(bt, bits, candidates=CANDIDATES, unrolls=UNROLLS, cache=None, rep
         for _ in range(repeats):
             t = np.minimum(t, step_times(bt, bits))
         times[lg] = t
-    per_step = [int(min(candidates, key=lambda c: times[c][k])) for k in range(bt.maxns)]
-    # The per-step choice comes from runs with an event after every step; the batch is then replayed as one graph,
-    # where a choice that won a step by noise can lose.  The final choice (tiles and unroll) is the fastest graph
+    per_step = []
+    for k in range(bt.maxns):
+        if per_step and all(times[c][k] <= 0 for c in candidates):
+            per_step.append(per_step[-1])
+        else:
+            per_step.append(int(min(candidates, key=lambda c: times[c][k])))
+    # The per-step choice comes from runs kernel by kernel; the batch is then replayed as one graph, where a choice
+    # that won a step by noise can lose.  The final choice (tiles and unroll) is the fastest graph
     # replay of the whole step sequence among the per-step choice and every uniform tile.
     plans = {"per_step": per_step}
     for lg in candidates:
@@ -176,7 +182,7 @@ def run_schedule(gs, plans, lanes, bits, groups, storage, tiles, graph=True, log
             t1 = time.perf_counter()
             lp, _, _ = bt.score(sub, want_cond=False, want_amp=False)
             dt = time.perf_counter() - t1
-            bt.use_graph(False)                                       # per-step events for the latencies
+            bt.use_graph(False)                                       # per-step times for the latencies
             bt.score(sub, want_cond=False, want_amp=False)
             total_ms, ends = bt.last_ms()
             for j, i in enumerate(grp):
