@@ -14,8 +14,9 @@
                                                         reads for the copy probe of MIB MiB (bench.py --calibrate-copy)
   python rocprof_summary.py gather TRACE_DIR FETCH_DIR WRITE_DIR PLAN MIB SAMPLES
                                                      -> the two-table engine's exact samples of PLAN (a gsamp plan:
-                                                        one norm pass and one write pass per step): samples 1 ..
-                                                        SAMPLES-1 of the trace (sample 0 is the warm-up), per step and
+                                                        per step one write pass, and one norm pass before it unless
+                                                        the write before that folded it in or none is needed): samples
+                                                        1 .. SAMPLES-1 of the trace (sample 0 is the warm-up), per step and
                                                         pass the kernel time, the algorithmic bytes (each old-table
                                                         entry a pass gathers read once, the writes) and the HBM bytes
                                                         of the counter runs, calibrated as in traffic
@@ -100,39 +101,51 @@ def traffic(fetch_dir, write_dir, mib):
     return "\n".join(out)
 
 
-def _gather_rows(path, key):
-    rows = [r for r in csv.DictReader(open(path)) if "gather_kernel" in r["Kernel_Name"]]
+def _gather_rows(path, ns, samples):
+    """Gather passes of the first ``samples`` samples of a plan of ns steps, in launch order: per sample
+    {(step, "norm" | "write"): row}."""
+    rows = [r for r in csv.DictReader(open(path)) if re.search("gather_(fold_)?kernel", r["Kernel_Name"])]
     rows.sort(key=lambda r: int(r["Dispatch_Id"]))
-    return rows
+    out, at = [], 0
+    for _ in range(samples):
+        one = {}
+        for k in range(ns):
+            # gather_kernel<S, kDirect = 1 / kWrite = 2, NKS>; a fold is a write
+            if "fold" not in rows[at]["Kernel_Name"] and rows[at]["Kernel_Name"].split(",")[2].strip() == "1":
+                one[k, "norm"] = rows[at]
+                at += 1
+            name = rows[at]["Kernel_Name"]
+            assert "fold" in name or name.split(",")[2].strip() == "2", (k, name)
+            one[k, "write"] = rows[at]
+            at += 1
+        out.append(one)
+    return out
 
 
 def gather(trace_dir, fetch_dir, write_dir, plan, mib, samples):
     toks = open(plan).read().split()
     ns, i, pos = int(toks[1]), 3, []
+    tr = _gather_rows(os.path.join(trace_dir, "run_kernel_trace.csv"), ns, samples)
+    fr = _gather_rows(os.path.join(fetch_dir, "run_counter_collection.csv"), ns, samples)
+    wr = _gather_rows(os.path.join(write_dir, "run_counter_collection.csv"), ns, samples)
     for k in range(ns):
         r, rn, nk = int(toks[i + 1]), int(toks[i + 2]), int(toks[i + 5])
         i += 6 + nk + 8
         rd = min(1 << r, 1 << (rn + nk)) * 8                  # c64 entries gathered, each read once
-        pos += [(k, "norm", r, rn, nk, rd), (k, "write", r, rn, nk, rd + (1 << rn) * 8)]
-    P = len(pos)
-    tr = _gather_rows(os.path.join(trace_dir, "run_kernel_trace.csv"), "Dispatch_Id")
-    fr = _gather_rows(os.path.join(fetch_dir, "run_counter_collection.csv"), "Dispatch_Id")
-    wr = _gather_rows(os.path.join(write_dir, "run_counter_collection.csv"), "Dispatch_Id")
+        pos += [(k, "norm", r, rn, nk, rd)] if (k, "norm") in tr[0] else []
+        pos += [(k, "write", r, rn, nk, rd + (1 << rn) * 8)]
     f = _counter(os.path.join(fetch_dir, "run_counter_collection.csv"), "FETCH_SIZE")
     w = _counter(os.path.join(write_dir, "run_counter_collection.csv"), "WRITE_SIZE")
     probe = next(k for k in f if "copy_probe" in k)
     ff, wf = mib * 1024.0 / f[probe][0], mib * 1024.0 / w[probe][0]
-    n = samples - 1
+    P, n = len(pos), samples - 1
     dur, hr, hw = [0.0] * P, [0.0] * P, [0.0] * P
     for s in range(1, samples):
         for p in range(P):
-            j = s * P + p
-            want = "1" if pos[p][1] == "norm" else "2"           # gather_kernel<S, kDirect = 1 / kWrite = 2, NKS>
-            for rows in (tr, fr, wr):
-                assert rows[j]["Kernel_Name"].split(",")[2].strip() == want, (j, rows[j]["Kernel_Name"])
-            dur[p] += (int(tr[j]["End_Timestamp"]) - int(tr[j]["Start_Timestamp"])) / 1e3 / n
-            hr[p] += float(fr[j]["Counter_Value"]) * ff * 1024 / n
-            hw[p] += float(wr[j]["Counter_Value"]) * wf * 1024 / n
+            at = pos[p][:2]
+            dur[p] += (int(tr[s][at]["End_Timestamp"]) - int(tr[s][at]["Start_Timestamp"])) / 1e3 / n
+            hr[p] += float(fr[s][at]["Counter_Value"]) * ff * 1024 / n
+            hw[p] += float(wr[s][at]["Counter_Value"]) * wf * 1024 / n
     T, A, H = sum(dur), sum(x[5] for x in pos), sum(hr) + sum(hw)
     out = [f"per sample ({n} samples): gather kernels {T / 1e3:.1f} ms; algorithmic {A / 1e9:.1f} GB "
            f"({A / T / 1e6:.2f} TB/s); HBM {sum(hr) / 1e9:.1f} GB read + {sum(hw) / 1e9:.1f} GB written "
