@@ -2221,8 +2221,9 @@ int gs_batch_set_unroll(gs_batch* bt, int lu) {
     return 0;
 }
 
-// Two consecutive steps per sweep where the plans allow it (on, default) or one (off); the results differ at most by
-// the order of FP64 sums.  A gradient's copies are laid out anew by its next call.
+// Two or three consecutive steps per sweep where the plans allow it, and whole strings in LDS where all plans fit (on,
+// default), or one step per sweep (off); the results differ at most by the order of FP64 sums.  A gradient's copies are
+// laid out anew by its next call.
 int gs_batch_set_pairs(gs_batch* bt, int on) {
     if (!bt) return bfail(16, "null batch");
     bt->pairs_on = on != 0;

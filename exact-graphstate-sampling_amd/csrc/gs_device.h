@@ -193,7 +193,7 @@ enum ChainMode { kChain = 0, kChain1 = 1, kRun = 2 };
 // What the last block of a sweep does after the sweep (kRoleStored: record the stored table's norm only -- the
 // product pass of a run of diagonal steps, whose decisions and bookkeeping were made before it).
 // kRoleStoredGram: the same, then the next step's decision from the Gram matrix the product pass summed.
-// kRolePair: a chain-mode sweep of two or three steps from step k on, whose sums are the steps' written norms.
+// kRolePair: a chain-mode sweep of two to four steps from step k on, whose sums are the steps' written norms.
 // kRoleSilent: nothing (a write whose norms nobody needs).
 // kRolePeek: a read-only pass that applied step k in registers; step k+1's decision goes to w2, step k's write is still
 // to come.

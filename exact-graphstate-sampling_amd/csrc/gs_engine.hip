@@ -353,7 +353,7 @@ struct gs_engine {
     std::vector<SStep> hsmall;
     std::vector<int> small_at, small_dim;
     SStep* dsmall = nullptr;
-    // several steps per sweep: pairs of any two steps (gs_pair.hip), butterflies of two or three (gs_fly.hip)
+    // several steps per sweep: pairs of any two steps (gs_pair.hip), butterflies of two to four (gs_fly.hip)
     bool allow_pairs = true;        // chain mode
     bool allow_fly = true;          // the other modes
     std::vector<PStep> hpair;
@@ -1570,8 +1570,6 @@ int build_steps(gs_engine* e) {
     return 0;
 }
 
-// Copy the step and run descriptors to the device, growing the run arrays (and allocating the pattern-sum buffers the
-// first time the plan has a run).
 // Bytes of the step descriptors on the device, and their places in one buffer there.
 size_t place_descriptors(gs_engine* e, unsigned char* base) {
     const size_t ns = size_t(std::max(e->plan.ns, 1));
@@ -1589,6 +1587,8 @@ size_t place_descriptors(gs_engine* e, unsigned char* base) {
     return used;
 }
 
+// Copy the step and run descriptors to the device, growing the run arrays (and allocating the pattern-sum buffers the
+// first time the plan has a run).
 int upload_descriptors(gs_engine* e) {
     if (e->plan.ns) {
         unsigned char* const base = reinterpret_cast<unsigned char*>(e->dplain);
@@ -2189,8 +2189,9 @@ int gs_profile_read(const gs_engine* eng, double* ms, int64_t* launches) {
     return 0;
 }
 
-// Launch geometry of step k, out[10]: plain log2 run, plain blocks, ntq, route, fusable, fused blocks, next route,
-// plain log2 tiles per block, fused log2 run and fused log2 tiles per block (-1 when the step does not fuse).
+// Launch geometry of step k, out[12]: plain log2 run, plain blocks, ntq, route, fusable, fused blocks, next route, plain
+// log2 tiles per block, fused log2 run and fused log2 tiles per block (-1 when the step does not fuse), runs per thread of
+// the plain sweeps and of the fused one (-1: no fusion).
 int gs_step_geometry(const gs_engine* eng, int k, int* out) {
     if (!eng || k < 0 || k >= eng->plan.ns || !out) return fail(16, "bad step");
     const KStep& s = eng->hplain[size_t(k)];
@@ -2385,7 +2386,8 @@ int gs_race_check(gs_engine* eng, int k, int layout, int64_t* counts) {
     return rc;
 }
 
-// Chain mode: two steps per sweep where the plan allows it (default on) or one.
+// Several steps per sweep where the plan allows it (default on) or one: two of any kind and two to four butterflies in
+// chain mode, two butterflies per write for sampled and forced complex128 strings.
 int gs_set_pairs(gs_engine* eng, int on) {
     if (!eng) return fail(16, "null engine");
     eng->allow_pairs = eng->allow_fly = on != 0;

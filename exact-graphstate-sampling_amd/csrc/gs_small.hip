@@ -2,7 +2,8 @@
 //
 // The head and tail of a plan are steps of a few thousand cosets and less, where a sweep costs far less than a launch;
 // one block runs such a run step after step -- norm pass, decision, write pass, bookkeeping -- with the run's table in
-// LDS: the arena slots a run touches span a subspace of at most 2^kSmallTab entries, and the host gives every step's
+// LDS: the arena slots a run touches span a subspace of at most 64 KB, or the whole arena where that fits (build_small in
+// gs_engine.hip), and the host gives every step's
 // columns, offsets and g as indices into that subspace.  The arithmetic per coset is the sweep kernels' (FP64 routed slot
 // sums, one rounding per store), the chain logic theirs too (gsamp2.cpp:46-49, :67, :80-95).
 //

@@ -354,8 +354,8 @@ class Engine:
         return dict(zip(("read_twice", "written_twice", "clobbered", "checked"), (int(x) for x in out)))
 
     def race_check_all(self):
-        """Race check of every layout the kernels walk (plain, fused where a step folds the next norms, runs of
-        diagonal steps); returns the summed counts, and raises AssertionError on any conflict."""
+        """Race check of every layout the single-step kernels walk (plain, fused where a step folds the next norms) and of
+        the runs of diagonal steps; returns the summed counts, and raises AssertionError on any conflict."""
         tot = dict(read_twice=0, written_twice=0, clobbered=0, checked=0)
         for k in range(self.ns):
             lays = ["plain"] + (["fused"] if self.geometry(k)["fusable"] else [])

@@ -16,7 +16,8 @@
  *     failure on the calling thread.
  *   - A zero-probability branch gives log2 Pr = -inf and zero conditionals from that step on, as the reference.
  *   - One engine owns one device arena of 2^R entries and one HIP stream; engines are not re-entrant, separate
- *     host threads may drive separate engines.
+ *     host threads may drive separate engines.  A call of several strings also gives each string in flight an arena:
+ *     up to 64 of them and 4 GiB in all, fewer where the device has less free, kept until the engine is destroyed.
  */
 #ifndef GSAMP_AMD_H
 #define GSAMP_AMD_H
